@@ -1,0 +1,625 @@
+// qiw_arcs.h -- open-arc graphs of the diagrams of an integration group, and their device
+// programs for models with sector blocks (host only; no HIP).
+//
+// Summing the diagrams of a group one by one (src/topology_eval.jl:454-556 walks the pair
+// assignments of every topology) repeats work: two partial diagrams that have reached the
+// same position in the same sector with the same open arcs continue identically, whatever
+// arcs they have closed on the way.  The compiler therefore walks the positions once and
+// keeps one state per (sector, open arcs); the partial products of all partial diagrams in
+// a state are added before they are continued.  What a closed arc leaves behind:
+//   * its sign: a perfect matching's parity is (-1)^crossings, and an arc that closes
+//     crosses exactly the arcs opened after it that are still open;
+//   * connectedness (src/diagrammatics.jl:214-254): every arc has to be linked by crossings
+//     to one that straddles the cut.  Before the cut the open arcs carry the partition into
+//     linked components (closing an arc links it to all later open ones; a component with
+//     no open arc left can no longer be linked: dead).  At the cut every open arc is
+//     linked.  After it the linked arcs are a prefix of the open ones.
+// At order 4 of the two-orbital model this takes 26 000 states where the assignment trie of
+// the same group has more than a million nodes.
+#pragma once
+#include <algorithm>
+#include <array>
+#include <cstdint>
+#include <cstring>
+#include <string>
+#include <unordered_map>
+#include <vector>
+
+namespace qiwi {
+
+enum { ARC_BOLD = 0, ARC_BARE = 1, ARC_CORR = 2, ARC_SIGMA = 3 };  // = QIW_G_*
+constexpr int kArcMax = 6;                                         // largest order
+
+// Sector maps of a model (-1: the operator annihilates the sector).
+struct ArcModel {
+    int ns = 0, np = 0;
+    std::vector<int> dims;
+    std::vector<std::vector<int>> head_sf, tail_sf;  // [np][ns]: operators at an arc's earlier / later end
+    std::vector<int> table;                          // [np] hybridization table
+    std::vector<int> a_sf, b_sf;                     // correlator operators A (at tau_w) and B (at tau_i)
+};
+
+struct ArcState {
+    uint8_t sector = 0, n = 0, good = 0;     // open arcs; the first `good` of them are linked across the cut
+    std::array<uint8_t, kArcMax> comp{};     // components of the arcs after them
+    std::array<uint8_t, kArcMax> pos{};      // point at which each arc opened
+    std::array<uint16_t, kArcMax> pair{};
+    bool operator==(const ArcState &o) const {
+        return sector == o.sector && n == o.n && good == o.good && comp == o.comp && pos == o.pos && pair == o.pair;
+    }
+    bool operator<(const ArcState &o) const {
+        if (sector != o.sector) return sector < o.sector;
+        if (n != o.n) return n < o.n;
+        if (pos != o.pos) return pos < o.pos;
+        if (comp != o.comp) return comp < o.comp;
+        if (good != o.good) return good < o.good;
+        return pair < o.pair;
+    }
+};
+struct ArcStateHash {
+    size_t operator()(const ArcState &s) const {
+        uint64_t h = 0x9E3779B97F4A7C15ull;
+        auto mix = [&](uint64_t v) {
+            h ^= v + 0x9E3779B97F4A7C15ull + (h << 6) + (h >> 2);
+            h *= 0xBF58476D1CE4E5B9ull;
+        };
+        mix(s.sector | (s.n << 8) | (s.good << 16));
+        for (int i = 0; i < s.n; ++i) mix(s.pos[i] | (s.pair[i] << 8) | ((uint64_t)s.comp[i] << 32));
+        return (size_t)h;
+    }
+};
+
+// What a position applies: nothing, the head or tail operator of a pair, or the operator A.
+enum { ARC_ID = 0, ARC_HEAD = 1, ARC_TAIL = 2, ARC_A = 3 };
+struct ArcJoin {
+    int src, dst;
+    uint16_t pair;
+    uint8_t op;    // ARC_*
+    int8_t sign;
+    int8_t head;   // configuration position of the closed arc's head (ARC_TAIL)
+};
+struct ArcStage {
+    int position;  // configuration position (1-based)
+    std::vector<ArcJoin> joins;
+};
+// One initial sector of a group: levels[0] is the root (position 1), levels[i + 1] the
+// states after stage i; the last level is the closed state (s0, no arcs).
+struct ArcGraph {
+    int s0 = 0;
+    std::vector<std::vector<ArcState>> levels;
+    std::vector<ArcStage> stages;
+    double leaves = 0;  // complete diagrams (topology, pair assignment) summed by the graph
+};
+
+// fixed: pair of the first fixed.size() arcs opened (the sum over diagrams is cut into one
+// graph per choice).  skip_w: leave out the stage of an identity node at tau_w between two
+// points (its two propagators are multiplied beforehand).  Returns false when a diagram ends
+// outside its initial sector; an empty graph (no stages, no levels) when there is none.
+inline bool arc_graph(const ArcModel &m, int kind, int order, int n_after, int s0, const std::vector<int> &fixed,
+                      bool skip_w, ArcGraph &out) {
+    out = ArcGraph{};
+    out.s0 = s0;
+    const int np2 = 2 * order;
+    const int cut = kind == ARC_BARE ? 0 : kind == ARC_SIGMA ? np2 - 1 : np2 - n_after;  // points before the cut
+    const int at_w = kind == ARC_BARE ? -1 : kind == ARC_SIGMA ? np2 : np2 - n_after;    // points before tau_w
+    ArcState root;
+    root.sector = (uint8_t)s0;
+    if (kind == ARC_CORR) {
+        if (m.b_sf[s0] < 0) return true;
+        root.sector = (uint8_t)m.b_sf[s0];
+    }
+    std::vector<std::vector<ArcState>> levels{{root}};
+    std::vector<std::vector<double>> ways{{1.0}};
+    std::vector<ArcStage> stages;
+    std::unordered_map<ArcState, int, ArcStateHash> index;
+    auto begin = [&](int position) {
+        index.clear();
+        stages.push_back(ArcStage{position, {}});
+        levels.emplace_back();
+        ways.emplace_back();
+    };
+    auto join = [&](int src, const ArcState &d, int op, int pair, int sign, int head) {
+        auto it = index.emplace(d, (int)levels.back().size());
+        if (it.second) {
+            levels.back().push_back(d);
+            ways.back().push_back(0.0);
+        }
+        const int dst = it.first->second;
+        ways.back()[dst] += ways[ways.size() - 2][src];
+        stages.back().joins.push_back(ArcJoin{src, dst, (uint16_t)pair, (uint8_t)op, (int8_t)sign, (int8_t)head});
+    };
+    auto linked = [&](ArcState &s) {  // every open arc is linked
+        s.good = s.n;
+        s.comp.fill(0);
+    };
+    auto w_node = [&](int position) {
+        begin(position);
+        const std::vector<ArcState> &src = levels[levels.size() - 2];
+        for (int i = 0; i < (int)src.size(); ++i) {
+            ArcState d = src[i];
+            if (kind == ARC_CORR) {
+                if (m.a_sf[d.sector] < 0) continue;
+                d.sector = (uint8_t)m.a_sf[d.sector];
+            }
+            join(i, d, kind == ARC_CORR ? ARC_A : ARC_ID, 0, 1, 0);
+        }
+    };
+    auto position_of = [&](int j) { return 2 + j + (at_w >= 0 && j >= at_w ? 1 : 0); };
+    for (int j = 0; j < np2; ++j) {
+        if (j == at_w && !skip_w) w_node(2 + at_w);
+        begin(position_of(j));
+        const std::vector<ArcState> src = levels[levels.size() - 2];
+        const int rem = np2 - j;
+        const bool all_linked = kind == ARC_BARE || j + 1 == cut;  // the new states stand at the cut
+        for (int i = 0; i < (int)src.size(); ++i) {
+            const ArcState &s = src[i];
+            if (s.n + 1 <= rem - 1) {  // open an arc
+                const int nth = (j + s.n) / 2;  // arcs opened so far
+                for (int p = 0; p < m.np; ++p) {
+                    const int t = m.head_sf[p][s.sector];
+                    if (t < 0 || (nth < (int)fixed.size() && fixed[nth] != p)) continue;
+                    ArcState d = s;
+                    d.sector = (uint8_t)t;
+                    d.pos[d.n] = (uint8_t)j;
+                    d.pair[d.n] = (uint16_t)p;
+                    d.comp[d.n] = d.n > d.good ? (uint8_t)(d.comp[d.n - 1] + 1) : (uint8_t)0;
+                    ++d.n;
+                    if (all_linked) linked(d);
+                    join(i, d, ARC_HEAD, p, 1, 0);
+                }
+            }
+            for (int a = 0; a < s.n; ++a) {  // close an arc
+                const int p = s.pair[a], t = m.tail_sf[p][s.sector];
+                if (t < 0) continue;
+                ArcState d = s;
+                d.sector = (uint8_t)t;
+                const int own = s.comp[a];
+                bool alive = true;
+                if (a < s.good) {
+                    linked(d);
+                } else {  // the later arcs join its component, which must not end here
+                    for (int q = a + 1; q < s.n; ++q) d.comp[q] = (uint8_t)own;
+                    alive = a + 1 < s.n || (a > s.good && s.comp[a - 1] == own);
+                }
+                if (!alive) continue;
+                for (int q = a; q + 1 < s.n; ++q) {
+                    d.comp[q] = d.comp[q + 1];
+                    d.pos[q] = d.pos[q + 1];
+                    d.pair[q] = d.pair[q + 1];
+                }
+                --d.n;
+                d.comp[d.n] = 0;
+                d.pos[d.n] = 0;
+                d.pair[d.n] = 0;
+                if (a < s.good) {
+                    d.good = d.n;
+                } else {  // components numbered from 0 without gaps
+                    int next = -1, last = -1;
+                    for (int q = d.good; q < d.n; ++q) {
+                        if (d.comp[q] != last) {
+                            last = d.comp[q];
+                            ++next;
+                        }
+                        d.comp[q] = (uint8_t)next;
+                    }
+                }
+                if (all_linked) linked(d);
+                join(i, d, ARC_TAIL, p, ((s.n - 1 - a) & 1) ? -1 : 1, position_of(s.pos[a]));
+            }
+        }
+    }
+    if (at_w == np2 && !skip_w) w_node(2 + at_w);
+    // keep what reaches the closed state
+    std::vector<char> alive(levels.back().size(), 0);
+    for (size_t i = 0; i < alive.size(); ++i) {
+        const ArcState &s = levels.back()[i];
+        if (s.n != 0) continue;
+        if (s.sector != s0) return false;
+        alive[i] = 1;
+        out.leaves += ways.back()[i];
+    }
+    if (out.leaves == 0) return true;
+    for (int l = (int)stages.size(); l >= 0; --l) {
+        std::vector<int> to(alive.size(), -1);
+        std::vector<ArcState> kept;
+        for (size_t i = 0; i < alive.size(); ++i)
+            if (alive[i]) {
+                to[i] = (int)kept.size();
+                kept.push_back(levels[l][i]);
+            }
+        levels[l].swap(kept);
+        if (l < (int)stages.size())
+            for (ArcJoin &x : stages[l].joins) x.src = to[x.src];
+        if (l == 0) break;
+        std::vector<char> below(levels[l - 1].size(), 0);
+        std::vector<ArcJoin> js;
+        for (ArcJoin &x : stages[l - 1].joins)
+            if (to[x.dst] >= 0) {
+                below[x.src] = 1;
+                x.dst = to[x.dst];
+                js.push_back(x);
+            }
+        stages[l - 1].joins.swap(js);
+        alive.swap(below);
+    }
+    out.levels.swap(levels);
+    out.stages.swap(stages);
+    return true;
+}
+
+// ---------------------------------------------------------------------------------------
+// Device programs of the arc walk for sector blocks (k_eval_arcs_t)
+// ---------------------------------------------------------------------------------------
+// A workgroup evaluates one sample at a time: a lane holds one column of one state, the
+// states of a level lie in LDS and the levels alternate between the two ends of one region.
+// A tile is the work of one wavefront in a stage: up to 64 >> lg states of one sector, times
+// 1 << lg columns of the initial sector's block.
+//
+// The program of a group is a blob of 32-bit words, offsets relative to its start:
+//   group    0 segments, 1 arc values, 2 position of the left-out node at tau_w (0: none),
+//            3 offset of the arc list, 4-7 byte offsets in LDS of the closed state's columns,
+//            the arc values, the propagators and the states, 8.. offsets of the segments
+//   arc      head position | tail position << 8 | table << 16
+//   segment  0 s0 | m0 << 8 | lg << 16, 1 stages, 2 root sector dimension | stride << 8,
+//            3 root operator block (offset, ARC_NONE: identity), 4 root propagator offset,
+//            5 root state offset, 6 parts of the closed state, 7 offset of their list,
+//            8.. per stage: tiles, offset of the tile records
+//   tile     0 operators | rows << 8 | states << 16 | stride << 24, 1 state offset,
+//            2 propagator offset (ARC_NONE: none), 3 offset of the operator records
+//   operator 0 block (offset, ARC_NONE: identity), 1 rows of the source | stride << 8 |
+//            joins per state << 16, 2 offset of the join words
+//   join     source state offset | index of the arc value << 20
+// Offsets of states and propagators are in elements of the value type.  The arc values are
+// 0: 0, 1: 1, then +v, -v of each arc in turn.  Joins are stored [join][state of the tile];
+// a state with fewer joins than its tile is filled up with value 0.
+constexpr uint32_t ARC_NONE = 0xFFFFFFFFu;
+constexpr int kArcGroupHead = 8, kArcSegHead = 8;
+
+struct ArcLayout {
+    int elem = 4;             // bytes of the value type
+    int mmax = 1;             // largest sector block
+    int bt = 0;               // elements of one segment's propagator blocks
+    std::vector<int> bt_off;  // [ns]
+    int waves = 1;            // wavefronts of the workgroup
+    size_t cap = 0;           // LDS bytes of the workgroup
+};
+
+// Elements a state of m rows takes per column, in a model whose largest block is mmax: fours
+// (one 16-byte access) where a block is wider than 8, else pairs up to 6 (6 rows of 4 bytes
+// keep the banks of neighbouring lanes apart).
+inline int arc_stride(int m, int mmax) {
+    return mmax > 8 || m > 6 ? (m + 3) & ~3 : m == 1 ? 1 : (m + 1) & ~1;
+}
+
+// LDS of a group in bytes: the times of the positions, the closed state's columns, the arc
+// values, the propagators of n - 2 segments and one product, then the states.
+struct ArcLds {
+    size_t fin, arcs, prop, states;
+};
+inline ArcLds arc_lds(const ArcLayout &l, int n, int n_arcs, int m0) {
+    auto up = [](size_t b) { return (b + 15) & ~(size_t)15; };
+    ArcLds r;
+    r.fin = 16 * 8;
+    r.arcs = r.fin + up((size_t)m0 * m0 * 8);
+    r.prop = r.arcs + up((size_t)(2 + 2 * n_arcs) * l.elem);
+    r.states = r.prop + up((size_t)(n - 1) * l.bt * l.elem);
+    return r;
+}
+
+struct ArcGroupProgram {
+    std::vector<uint32_t> blob;
+    int n_segments = 0;
+    std::vector<double> seg_cost;  // real FLOPs per sample of each segment
+    double flops = 0, leaves = 0, joins = 0;
+    size_t lds = 0;  // bytes a workgroup needs
+    int n_arcs = 0;
+};
+
+// Operator blocks as the packer names them: offset of the block of (op, pair, source sector).
+struct ArcBlocks {
+    std::vector<std::vector<uint32_t>> head, tail;  // [np][ns]
+    std::vector<uint32_t> a, b;                     // [ns]
+};
+
+struct ArcPacker {
+    const ArcModel &m;
+    const ArcLayout &l;
+    const ArcBlocks &ob;
+    int kind, order, n_after, n, w_skipped;
+    std::vector<uint32_t> arcs;  // arc list
+    std::unordered_map<uint32_t, int> arc_id;
+
+    uint32_t arc_value(int head, int tail, int table, int sign) {
+        const uint32_t key = (uint32_t)head | ((uint32_t)tail << 8) | ((uint32_t)table << 16);
+        auto it = arc_id.emplace(key, (int)arcs.size());
+        if (it.second) arcs.push_back(key);
+        return 2u + 2u * (uint32_t)it.first->second + (sign < 0 ? 1u : 0u);
+    }
+    // slot of the propagators that follow configuration position p: segment p + 1 (slots
+    // 0 .. n - 3), or the product over the left-out node at tau_w (slot n - 2)
+    int slot_after(int p) const { return w_skipped && p + 1 == w_skipped ? n - 2 : p - 1; }
+
+    struct Tile {
+        int sector;
+        std::vector<int> states;  // indices in the level
+        std::vector<int> ops;     // keys (op << 16 | pair) this tile sums
+    };
+
+    // states of a level in tiles, with the offsets of every state's parts
+    struct Placed {
+        std::vector<Tile> tiles;
+        std::vector<size_t> tile_off;
+        std::vector<std::vector<size_t>> parts;  // [state] offsets
+        size_t size = 0;
+    };
+
+    Placed place(const std::vector<ArcState> &lev, const ArcStage &st, int lg) const {
+        const int per = 64 >> lg, cg = 1 << lg;
+        std::vector<std::vector<int>> ops_of(lev.size());
+        for (const ArcJoin &x : st.joins) {
+            const int key = (x.op << 16) | x.pair;
+            auto &v = ops_of[x.dst];
+            if (std::find(v.begin(), v.end(), key) == v.end()) v.push_back(key);
+        }
+        for (auto &v : ops_of) std::sort(v.begin(), v.end());
+        // states opened at this position have one operator: tiles of one operator; the others
+        // are tiled by sector
+        std::vector<int> ord(lev.size());
+        for (size_t i = 0; i < ord.size(); ++i) ord[i] = (int)i;
+        auto head_key = [&](int i) {
+            return ops_of[i].size() == 1 && (ops_of[i][0] >> 16) == ARC_HEAD ? ops_of[i][0] : -1;
+        };
+        std::sort(ord.begin(), ord.end(), [&](int x, int y) {
+            if (lev[x].sector != lev[y].sector) return lev[x].sector < lev[y].sector;
+            const int hx = head_key(x), hy = head_key(y);
+            if (hx != hy) return hx < hy;
+            return lev[x] < lev[y];
+        });
+        Placed p;
+        for (size_t i = 0; i < ord.size();) {
+            Tile t;
+            t.sector = lev[ord[i]].sector;
+            const int hk = head_key(ord[i]);
+            while (i < ord.size() && (int)t.states.size() < per && lev[ord[i]].sector == t.sector &&
+                   head_key(ord[i]) == hk)
+                t.states.push_back(ord[i++]);
+            for (int s : t.states)
+                for (int key : ops_of[s])
+                    if (std::find(t.ops.begin(), t.ops.end(), key) == t.ops.end()) t.ops.push_back(key);
+            std::sort(t.ops.begin(), t.ops.end());
+            p.tiles.push_back(t);
+        }
+        // a stage with fewer tiles than wavefronts: cut the tiles' operator sums into parts,
+        // each a tile of its own with its own copy of the states
+        const int nt = (int)p.tiles.size();
+        if (nt > 0 && nt < l.waves) {
+            const int share = l.waves / nt;
+            std::vector<Tile> cutted;
+            for (const Tile &t : p.tiles) {
+                const int k = std::max(1, std::min<int>(share, (int)t.ops.size()));
+                for (int q = 0; q < k; ++q) {
+                    Tile c = t;
+                    c.ops.assign(t.ops.begin() + t.ops.size() * q / k, t.ops.begin() + t.ops.size() * (q + 1) / k);
+                    cutted.push_back(c);
+                }
+            }
+            p.tiles.swap(cutted);
+        }
+        p.parts.assign(lev.size(), {});
+        for (const Tile &t : p.tiles) {
+            const size_t step = (size_t)arc_stride(m.dims[t.sector], l.mmax) * cg;
+            p.size = (p.size + 3) & ~(size_t)3;
+            p.tile_off.push_back(p.size);
+            for (size_t i = 0; i < t.states.size(); ++i)  // a part without any of the state's joins is zero
+                for (int key : t.ops)
+                    if (std::binary_search(ops_of[t.states[i]].begin(), ops_of[t.states[i]].end(), key)) {
+                        p.parts[t.states[i]].push_back(p.size + i * step);
+                        break;
+                    }
+            p.size += t.states.size() * step;
+        }
+        p.size = (p.size + 3) & ~(size_t)3;
+        return p;
+    }
+
+    // Elements of the state region and wavefront passes of a graph at 1 << lg columns.
+    void measure(const ArcGraph &g, int lg, size_t *region, double *cost) const {
+        const int cg = 1 << lg, m0 = m.dims[g.s0];
+        size_t prev = (size_t)arc_stride(m.dims[g.levels[0][0].sector], l.mmax) * cg, reg = (prev + 3) & ~(size_t)3;
+        double c = 0;
+        for (size_t s = 0; s < g.stages.size(); ++s) {
+            const Placed p = place(g.levels[s + 1], g.stages[s], lg);
+            reg = std::max(reg, ((prev + 3) & ~(size_t)3) + p.size);
+            prev = p.size;
+            c += 1.0 + (double)((p.tiles.size() + l.waves - 1) / l.waves);
+        }
+        *region = reg;
+        *cost = c * ((m0 + cg - 1) / cg);
+    }
+
+    double graph_flops(const ArcGraph &g) const {
+        const double m0 = m.dims[g.s0];
+        const double mr = m.dims[g.levels[0][0].sector];
+        double f = 2.0 * mr * mr * m0 + 2.0 * m0 * m0 * m0;
+        for (size_t s = 0; s < g.stages.size(); ++s) {
+            std::vector<uint64_t> seen;
+            for (const ArcJoin &x : g.stages[s].joins) {
+                if (x.op == ARC_TAIL) f += 2.0 * m.dims[g.levels[s][x.src].sector] * m0;
+                const uint64_t key = ((uint64_t)x.dst << 20) | ((uint64_t)x.op << 16) | x.pair;
+                if (x.op != ARC_ID) seen.push_back(key);
+            }
+            std::sort(seen.begin(), seen.end());
+            seen.erase(std::unique(seen.begin(), seen.end()), seen.end());
+            for (uint64_t key : seen) {
+                const int op = (int)((key >> 16) & 15), pair = (int)(key & 0xFFFF);
+                const int sd = g.levels[s + 1][key >> 20].sector;
+                int ss = sd;  // the source sector the operator takes to sd
+                for (int q = 0; q < m.ns; ++q) {
+                    const int to = op == ARC_HEAD ? m.head_sf[pair][q] : op == ARC_TAIL ? m.tail_sf[pair][q] : m.a_sf[q];
+                    if (to == sd) ss = q;
+                }
+                f += 2.0 * m.dims[ss] * m.dims[sd] * m0;
+            }
+            if (s + 1 < g.stages.size())
+                for (const ArcState &d : g.levels[s + 1]) f += 2.0 * m.dims[d.sector] * m.dims[d.sector] * m0;
+        }
+        return f;
+    }
+
+    void emit(const ArcGraph &g, int lg, size_t region, ArcGroupProgram &out) {
+        std::vector<uint32_t> &b = out.blob;
+        while (b.size() % 4) b.push_back(0);
+        out.blob[kArcGroupHead + out.n_segments] = (uint32_t)b.size();
+        const size_t seg = b.size();
+        const int m0 = m.dims[g.s0], s1 = g.levels[0][0].sector;
+        b.resize(seg + kArcSegHead + 2 * g.stages.size(), 0u);
+        b[seg] = (uint32_t)g.s0 | ((uint32_t)m0 << 8) | ((uint32_t)lg << 16);
+        b[seg + 1] = (uint32_t)g.stages.size();
+        b[seg + 2] = (uint32_t)m.dims[s1] | ((uint32_t)arc_stride(m.dims[s1], l.mmax) << 8);
+        b[seg + 3] = kind == ARC_CORR ? ob.b[g.s0] : ARC_NONE;
+        // with no stage after it the root is the closed state, and its propagator the last one
+        b[seg + 4] = g.stages.empty() ? ARC_NONE : (uint32_t)(slot_after(1) * l.bt + l.bt_off[s1]);
+        b[seg + 5] = 0;
+        std::vector<std::vector<size_t>> src{{0}};
+        for (size_t s = 0; s < g.stages.size(); ++s) {
+            const ArcStage &st = g.stages[s];
+            const bool last = s + 1 == g.stages.size();
+            const Placed p = place(g.levels[s + 1], st, lg);
+            const size_t base = s % 2 == 0 ? region - p.size : 0;  // the levels alternate between the ends
+            std::vector<std::vector<size_t>> dst = p.parts;
+            for (auto &v : dst)
+                for (size_t &o : v) o += base;
+            // joins by destination and operator
+            std::vector<std::vector<int>> by(g.levels[s + 1].size());
+            for (size_t i = 0; i < st.joins.size(); ++i) by[st.joins[i].dst].push_back((int)i);
+            while (b.size() % 4) b.push_back(0);
+            const size_t tiles = b.size();
+            b[seg + kArcSegHead + 2 * s] = (uint32_t)p.tiles.size();
+            b[seg + kArcSegHead + 2 * s + 1] = (uint32_t)tiles;
+            b.resize(tiles + 4 * p.tiles.size(), 0u);
+            for (size_t ti = 0; ti < p.tiles.size(); ++ti) {
+                const Tile &t = p.tiles[ti];
+                const int md = m.dims[t.sector], ns = (int)t.states.size();
+                while (b.size() % 4) b.push_back(0);
+                const size_t ops = b.size();
+                b.resize(ops + 4 * t.ops.size(), 0u);
+                b[tiles + 4 * ti] = (uint32_t)t.ops.size() | ((uint32_t)md << 8) | ((uint32_t)ns << 16) |
+                                    ((uint32_t)arc_stride(md, l.mmax) << 24);
+                b[tiles + 4 * ti + 1] = (uint32_t)(base + p.tile_off[ti]);
+                b[tiles + 4 * ti + 2] = last ? ARC_NONE : (uint32_t)(slot_after(st.position) * l.bt + l.bt_off[t.sector]);
+                b[tiles + 4 * ti + 3] = (uint32_t)ops;
+                for (size_t oi = 0; oi < t.ops.size(); ++oi) {
+                    const int op = t.ops[oi] >> 16, pair = t.ops[oi] & 0xFFFF;
+                    std::vector<std::vector<uint32_t>> words(ns);
+                    int ssec = t.sector;
+                    size_t most = 0;
+                    for (int i = 0; i < ns; ++i) {
+                        for (int ji : by[t.states[i]]) {
+                            const ArcJoin &x = st.joins[ji];
+                            if (x.op != op || x.pair != pair) continue;
+                            ssec = g.levels[s][x.src].sector;
+                            const uint32_t v = op == ARC_TAIL
+                                                   ? arc_value(x.head, st.position, m.table[pair], x.sign)
+                                                   : 1u;
+                            for (size_t off : src[x.src]) words[i].push_back((uint32_t)off | (v << 20));
+                        }
+                        most = std::max(most, words[i].size());
+                    }
+                    uint32_t blk = ARC_NONE;
+                    if (op == ARC_HEAD) blk = ob.head[pair][ssec];
+                    if (op == ARC_TAIL) blk = ob.tail[pair][ssec];
+                    if (op == ARC_A) blk = ob.a[ssec];
+                    const int ms = m.dims[ssec];
+                    b[ops + 4 * oi] = blk;
+                    b[ops + 4 * oi + 1] = (uint32_t)ms | ((uint32_t)arc_stride(ms, l.mmax) << 8) | ((uint32_t)most << 16);
+                    b[ops + 4 * oi + 2] = (uint32_t)b.size();
+                    uint32_t any = 0;  // a source of the tile, for the fill words
+                    for (int i = 0; i < ns; ++i)
+                        if (!words[i].empty()) any = words[i][0] & 0xFFFFFu;
+                    for (size_t e = 0; e < most; ++e)
+                        for (int i = 0; i < ns; ++i) b.push_back(e < words[i].size() ? words[i][e] : any);
+                    out.joins += (double)most * ns;
+                }
+            }
+            src.swap(dst);
+        }
+        // the parts of the closed state
+        b[seg + 6] = (uint32_t)src[0].size();
+        b[seg + 7] = (uint32_t)b.size();
+        for (size_t off : src[0]) b.push_back((uint32_t)off);
+        out.n_segments++;
+        const double f = graph_flops(g);
+        out.seg_cost.push_back(f);
+        out.flops += f;
+        out.leaves += g.leaves;
+    }
+};
+
+// Compiles a group: all initial sectors, cut by the pairs of the first n_fixed arcs.
+// Returns 0, 1 when a diagram ends outside its initial sector, or 2 when the states do not
+// fit the layout's LDS (or the word formats).
+inline int arc_compile(const ArcModel &m, const ArcLayout &l, const ArcBlocks &ob, int kind, int order, int n_after,
+                       int n_fixed, ArcGroupProgram &out) {
+    out = ArcGroupProgram{};
+    const int n = kind == ARC_BARE ? 2 * order + 2 : 2 * order + 3;
+    const bool skip_w = kind == ARC_BOLD && order > 0;
+    const int pos_w = kind == ARC_BARE ? 0 : 2 * order - n_after + 2;
+    ArcPacker pk{m, l, ob, kind, order, n_after, n, skip_w ? pos_w : 0, {}, {}};
+    std::vector<ArcGraph> graphs;
+    std::vector<int> fix(std::min(n_fixed, order), 0);
+    double total = 1;
+    for (size_t i = 0; i < fix.size(); ++i) total *= m.np;
+    for (int s0 = 0; s0 < m.ns; ++s0)
+        for (double c = 0; c < total; ++c) {
+            double r = c;
+            for (size_t i = 0; i < fix.size(); ++i) {
+                fix[i] = (int)((long long)r % m.np);
+                r = (double)((long long)r / m.np);
+            }
+            ArcGraph g;
+            if (!arc_graph(m, kind, order, n_after, s0, fix, skip_w, g)) return 1;
+            if (!g.levels.empty()) graphs.push_back(std::move(g));
+        }
+    int m0 = 1;
+    for (const ArcGraph &g : graphs) m0 = std::max(m0, m.dims[g.s0]);
+    const int most_arcs = order * (2 * order - 1) * (1 + *std::max_element(m.table.begin(), m.table.end()));
+    const ArcLds at = arc_lds(l, n, order > 0 ? most_arcs : 0, m0);
+    if (at.states >= l.cap || 2 + 2 * most_arcs >= 4096) return 2;
+    const size_t room = (l.cap - at.states) / l.elem;
+    out.blob.assign(kArcGroupHead + graphs.size(), 0u);
+    out.lds = at.states;
+    for (const ArcGraph &g : graphs) {
+        int best = -1;
+        size_t best_region = 0;
+        double best_cost = 0;
+        for (int lg = 0; lg <= 5; ++lg) {
+            if (lg > 0 && (1 << (lg - 1)) >= m.dims[g.s0]) break;
+            size_t region;
+            double cost;
+            pk.measure(g, lg, &region, &cost);
+            if (region > room || region >= (1u << 20)) break;
+            if (best < 0 || cost < best_cost) {
+                best = lg;
+                best_region = region;
+                best_cost = cost;
+            }
+        }
+        if (best < 0) return 2;
+        pk.emit(g, best, best_region, out);
+        out.lds = std::max(out.lds, at.states + best_region * l.elem);
+    }
+    while (out.blob.size() % 4) out.blob.push_back(0);
+    out.blob[0] = (uint32_t)out.n_segments;
+    out.blob[1] = (uint32_t)pk.arcs.size();
+    out.blob[2] = (uint32_t)pk.w_skipped;
+    out.blob[3] = (uint32_t)out.blob.size();
+    out.blob[4] = (uint32_t)at.fin;
+    out.blob[5] = (uint32_t)at.arcs;
+    out.blob[6] = (uint32_t)at.prop;
+    out.blob[7] = (uint32_t)at.states;
+    out.n_arcs = (int)pk.arcs.size();
+    out.blob.insert(out.blob.end(), pk.arcs.begin(), pk.arcs.end());
+    return 0;
+}
+
+}  // namespace qiwi

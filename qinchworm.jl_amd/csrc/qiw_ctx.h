@@ -103,6 +103,7 @@ struct qiw_ctx {
     std::string model_fp;      // bytes of the model content the compiled programs depend on
     bool vec_staged = false;   // operator blocks of the vector walk are on the device
     bool mfma_staged = false;  // operator blocks of the matrix-core walk are on the device
+    int arc_staged = 0;        // tables of the arc walk are on the device: 1 float64, 2 float32
     // Sobol state
     int sob_dim = 0;
     std::vector<uint32_t> sob_m, sob_x;

@@ -273,6 +273,17 @@ struct MfmaArgs {
     int ops_zero;              // position of four 0.0 in ops (16-byte aligned, past the blocks)
     int wave_lds;              // floats of LDS per wavefront (absent-row writes and walk stack)
 };
+// Arguments of the arc walk (k_eval_arcs_t; programs as in qiw_arcs.h)
+struct ArcArgs {
+    EvalArgs e;
+    const void *ops;           // operator blocks: slice registers (float32), column-major (float64)
+    const void *ops_cm;        // the same column-major in the value type
+    const double *ediag;       // [bt] E + lambda on the diagonal positions (bare groups)
+    const uint8_t *emask;      // [bt] 1 on the diagonal positions
+    const int32_t *sector_of;  // [bt]
+    const int32_t *dims, *bt_off, *stride;  // [ns]
+    int bt;
+};
 // Wavefronts per workgroup of k_eval_mfma_t (tasks come in units of this many)
 #define QIW_MFMA_WAVES 4
 
@@ -314,6 +325,9 @@ hipError_t qiw_launch_simplex_points(hipStream_t st, const uint32_t *m, const ui
 hipError_t qiw_launch_eval_flat(hipStream_t st, const EvalArgs &a, int n_tasks, int km, int sm, int tm);
 hipError_t qiw_launch_eval_block(hipStream_t st, const BlockArgs &b, int n_tasks, size_t lds_bytes);
 hipError_t qiw_launch_eval_mfma(hipStream_t st, const MfmaArgs &m, int n_tasks, int km, int tm, size_t lds_bytes);
+hipError_t qiw_launch_eval_arcs(hipStream_t st, const ArcArgs &a, int n_tasks, int mb, int fp32, int waves, size_t lds);
+int qiw_arc_rows(int mb);
+int qiw_arc_waves(int mb, int fp32);
 hipError_t qiw_launch_eval_vec(hipStream_t st, const VecArgs &v, int n_tasks, int mb, int km, int tm, int fp32);
 hipError_t qiw_launch_ptab_cells(hipStream_t st, const double *T, int n_tau, int bt, double2 *out, double *outm,
                                  QiwCell32 *out32);

@@ -19,6 +19,7 @@
 #include <vector>
 
 #include "../../include/qiw.h"
+#include "qiw_arcs.h"
 #include "qiw_chunks.h"
 #include "qiw_ctx.h"
 #include "qiw_device.h"
@@ -212,15 +213,24 @@ int load_scalar_op(qiw_ctx *c, const qiw_sbm &in, const std::vector<int> &dims, 
 // ---------------------------------------------------------------------------------------
 enum NodeKind { N_PAIR_HEAD, N_PAIR_TAIL, N_IDENTITY, N_OPERATOR };
 
-// Program formats: the scalar structured walk, the LDS block walk, the vector walk.
-enum ProgFormat { FMT_SCALAR = 0, FMT_BLOCK = 1, FMT_VEC = 2 };
+// Program formats: the scalar structured walk, the LDS block walk, the vector walk, the arc
+// walk (sector blocks).
+enum ProgFormat { FMT_SCALAR = 0, FMT_BLOCK = 1, FMT_VEC = 2, FMT_ARC = 3 };
 
-// Vector programs also drive the matrix-core walk of wide blocks (float32 chain products).
+// Format of the assignment tries.  Vector programs also drive the matrix-core walk of wide
+// blocks (float32 chain products).
 int program_format(const HostModel &m, int max_order, int precision) {
     if (m.scalar_kernel) return FMT_SCALAR;
     if (m.vec_ok && max_order <= 4) return FMT_VEC;
     if (m.mfma_ok && max_order <= 4 && precision == QIW_PREC_FP32) return FMT_VEC;
     return FMT_BLOCK;
+}
+
+// Models with sector blocks run the arc walk wherever its states fit a CU's LDS
+// (compile_group), and the assignment tries otherwise.
+int eval_format(const HostModel &m, int max_order, int precision) {
+    const int fmt = program_format(m, max_order, precision);
+    return fmt == FMT_SCALAR || m.ns > 255 ? fmt : FMT_ARC;
 }
 
 // Stride of the W slots: the table count of the register walk instantiation that runs the
@@ -245,6 +255,9 @@ struct Compiled {
     // operator block per edge, the leaf accumulation)
     double flops_per_sample = 0;
     int n_top = 0;
+    // arc programs: initial-sector segments, wavefronts and LDS bytes of a workgroup
+    int n_segments = 0, waves = 1;
+    size_t lds_bytes = 0;
     int replica_of = -1;  // randomized qMC: another sequence of group `replica_of` (no program of its own)
 };
 
@@ -255,6 +268,10 @@ struct TrieNode {
     std::vector<int> children;
     int s_in = 0, s_out = 0, blk = 0xFFFF;  // block programs: sectors and operator block
 };
+
+constexpr char kOffDiagonal[] =
+    "A block off-diagonal contribution to a pseudo-particle propagator detected, try passing more "
+    "'symmetry_breakers' when constructing the local exact diagonalization object";
 
 struct Compiler {
     const HostModel &m;
@@ -306,8 +323,7 @@ struct Compiler {
     int dfs(int node, int pos, int s, double c) {
         if (pos > n) {
             if (s != s0) {
-                err = "A block off-diagonal contribution to a pseudo-particle propagator detected, try passing "
-                      "more 'symmetry_breakers' when constructing the local exact diagonalization object";
+                err = kOffDiagonal;
                 return -1;
             }
             trie[node].leaf = true;
@@ -596,11 +612,126 @@ struct Compiler {
     }
 };
 
+// ---- arc programs (qiw_arcs.h) ----
+ArcModel arc_model(const HostModel &m, int corr) {
+    ArcModel a;
+    a.ns = m.ns;
+    a.np = m.np;
+    a.dims = m.dims;
+    a.table = m.pair_table;
+    for (int p = 0; p < m.np; ++p) {
+        a.head_sf.push_back(m.op_i[p].sf);
+        a.tail_sf.push_back(m.op_f[p].sf);
+    }
+    if (corr >= 0) {
+        a.a_sf = m.corr_A[corr].sf;
+        a.b_sf = m.corr_B[corr].sf;
+    }
+    return a;
+}
+
+// Slice registers of the float32 operator blocks (64 floats each) in the instantiation for
+// the model's blocks.
+int arc_slice_regs(const HostModel &m) {
+    const int mb = qiw_arc_rows(m.mmax);
+    return (mb / 4 * mb + 15) / 16;
+}
+
+ArcBlocks arc_blocks(const HostModel &m, int corr, int precision) {
+    ArcBlocks o;
+    const uint32_t per = 64u * (uint32_t)arc_slice_regs(m);
+    auto offsets = [&](const ScalarOp &op, bool column_major) {
+        std::vector<uint32_t> v(m.ns, ARC_NONE);
+        for (int s = 0; s < m.ns; ++s)
+            if (op.blk[s] >= 0)
+                v[s] = column_major || precision == QIW_PREC_FP64 ? (uint32_t)m.op_desc[3 * op.blk[s]]
+                                                                  : per * (uint32_t)op.blk[s];
+        return v;
+    };
+    for (int p = 0; p < m.np; ++p) {
+        o.head.push_back(offsets(m.op_i[p], false));
+        o.tail.push_back(offsets(m.op_f[p], false));
+    }
+    if (corr >= 0) {
+        o.a = offsets(m.corr_A[corr], false);
+        o.b = offsets(m.corr_B[corr], true);  // the root reads columns of B
+    }
+    return o;
+}
+
+// Workgroup shapes of the arc walk, narrowest first: wavefronts and the LDS they may take
+// (eight, three, two and one workgroup per CU), and the widest level, in 64-state tiles,
+// that the shape is for.
+struct ArcShape {
+    int waves;
+    size_t cap;
+    int tiles;
+};
+constexpr ArcShape kArcShapes[] = {{1, 20 << 10, 2}, {4, 53 << 10, 12}, {8, 80 << 10, 32}, {16, 160 << 10, 1 << 30}};
+
 // Algorithmic real FLOPs of one sample of a compiled group: the scalar walk's multiply per
 // trie edge and leaf, or the block programs' chain products.
 double sample_flops(const Compiled &cg) {
     if (cg.flops_per_sample > 0) return cg.flops_per_sample;
     return 2.0 * cg.edges_per_sample + 2.0 * cg.leaves_per_sample;
+}
+
+// Compiles a group as an arc program.  Returns 0, 1 when a diagram ends outside its initial
+// sector, 2 when the states do not fit.
+int compile_arcs(const HostModel &m, int kind, int order, int n_after, int corr, int precision, Compiled &out) {
+    const ArcModel am = arc_model(m, corr);
+    if (m.np > 127) return 2;
+    const ArcBlocks ob = arc_blocks(m, corr, precision);
+    const bool fp32 = precision == QIW_PREC_FP32;
+    const int max_waves = qiw_arc_waves(m.mmax, fp32 ? 1 : 0);
+    ArcLayout l;
+    l.elem = fp32 ? 4 : 8;
+    l.mmax = m.mmax;
+    l.bt = m.bt;
+    l.bt_off.assign(m.bt_off.begin(), m.bt_off.end());
+    // the widest level decides the shape to start from
+    size_t widest = 0;
+    for (int s0 = 0; s0 < m.ns; ++s0) {
+        ArcGraph g;
+        if (!arc_graph(am, kind, order, n_after, s0, {}, kind == QIW_G_BOLD && order > 0, g)) return 1;
+        for (const auto &lev : g.levels) widest = std::max(widest, lev.size());
+    }
+    ArcGroupProgram pg;
+    int rc = 2;
+    for (int n_fixed = 0; n_fixed <= order && rc == 2; ++n_fixed)
+        for (const ArcShape &sh : kArcShapes) {
+            if (n_fixed == 0 && (widest + 63) / 64 > (size_t)sh.tiles) continue;
+            l.waves = std::min(sh.waves, max_waves);
+            l.cap = sh.cap;
+            rc = arc_compile(am, l, ob, kind, order, n_after, n_fixed, pg);
+            if (rc != 2) break;
+        }
+    if (rc) return rc;
+    const int d_after = (kind == QIW_G_BARE) ? 2 * order : (kind == QIW_G_SIGMA) ? 0 : n_after;
+    out.n_top = (int)((kind == QIW_G_BARE)    ? topologies_at_order(order, -1, false)
+                      : (kind == QIW_G_SIGMA) ? topologies_at_order(order, 1, false)
+                                              : topologies_at_order(order, n_after, false))
+                    .size();
+    if (pg.blob.size() % 2) pg.blob.push_back(0);
+    out.prog.resize(pg.blob.size() / 2);
+    std::memcpy(out.prog.data(), pg.blob.data(), pg.blob.size() * 4);
+    out.n_segments = pg.n_segments;
+    out.waves = l.waves;
+    out.lds_bytes = pg.lds;
+    out.leaves_per_sample = (int64_t)pg.leaves;
+    out.edges_per_sample = (int64_t)pg.joins;
+    out.flops_per_sample = pg.flops;
+    QiwGroup &g = out.g;
+    g.kind = kind;
+    g.order = order;
+    g.n_after = d_after;
+    g.n_nodes = kind == QIW_G_BARE ? 2 * order + 2 : 2 * order + 3;
+    g.d_before = 2 * order - d_after;
+    g.d_after = d_after;
+    g.pos_w = kind == QIW_G_BARE ? 0 : g.d_before + 2;
+    g.n_pslots = (g.n_nodes - 1) * m.ns;
+    g.n_wslots = order * qiw_vec_tm(m.ntab);
+    return 0;
 }
 
 // LDS doubles of one evaluator wavefront.  Scalar programs keep their state in registers;
@@ -632,6 +763,11 @@ struct Batch {
     double flops_per_launch = 0;  // algorithmic FLOPs of one launch
     int64_t leaves_per_launch = 0, diagram_evals_per_launch = 0;
     bool overflow = false;  // the launch would exceed kMaxTasks workgroups
+    struct Launch {         // arc walk: one launch per workgroup shape
+        int first, count, waves;
+        size_t lds;
+    };
+    std::vector<Launch> launches;
     int wg_waves = 1;       // wavefronts per workgroup: consecutive tasks of a workgroup share
                             // its sample block (matrix-core walk: kMfmaWaves)
 };
@@ -679,7 +815,9 @@ int upload(qiw_ctx *c, const std::string &tag, Batch &b, int64_t N, DevBatch &d,
     std::vector<QiwGroup> gs;
     // END words between and after the programs (never executed: prefetch and alignment)
     const uint64_t end_fl = (uint64_t)QIW_FL_OP_END << 28;
-    const uint64_t pad = (b.fmt == FMT_SCALAR) ? (end_fl | (end_fl << 32)) : (uint64_t)QIW_OP_END << 48;
+    const uint64_t pad = b.fmt == FMT_ARC      ? 0ull
+                         : b.fmt == FMT_SCALAR ? (end_fl | (end_fl << 32))
+                                               : (uint64_t)QIW_OP_END << 48;
     int64_t ut_total = 0, ps_total = 0;
     for (auto &cg : b.groups) {
         QiwGroup g = cg.g;
@@ -879,6 +1017,9 @@ void push_sequences(Batch &b, Compiled &&cg, int n_eval, AddTasks add_tasks) {
         rep.edges_per_sample = cg.edges_per_sample;
         rep.flops_per_sample = cg.flops_per_sample;
         rep.n_top = cg.n_top;
+        rep.n_segments = cg.n_segments;
+        rep.waves = cg.waves;
+        rep.lds_bytes = cg.lds_bytes;
         rep.replica_of = first;
     }
     b.groups.push_back(std::move(cg));
@@ -1034,6 +1175,26 @@ void order_tasks(Batch &b) {
     const size_t ng = b.groups.size();
     std::vector<int> go(ng);
     for (size_t i = 0; i < ng; ++i) go[i] = (int)i;
+    if (b.fmt == FMT_ARC) {  // one launch per workgroup shape, heaviest groups first in each
+        std::stable_sort(go.begin(), go.end(), [&](int x, int y) {
+            const Compiled &p = b.groups[x], &q = b.groups[y];
+            return p.waves != q.waves ? p.waves > q.waves : p.flops_per_sample > q.flops_per_sample;
+        });
+        std::vector<std::vector<QiwTask>> of(ng);
+        for (const QiwTask &t : b.tasks) of[t.group].push_back(t);
+        b.tasks.clear();
+        for (int gi : go) {
+            const Compiled &cg = b.groups[gi];
+            if (of[gi].empty()) continue;
+            if (b.launches.empty() || b.launches.back().waves != cg.waves)
+                b.launches.push_back({(int)b.tasks.size(), 0, cg.waves, 0});
+            Batch::Launch &ln = b.launches.back();
+            ln.count += (int)of[gi].size();
+            ln.lds = std::max(ln.lds, cg.lds_bytes);
+            b.tasks.insert(b.tasks.end(), of[gi].begin(), of[gi].end());
+        }
+        return;
+    }
     auto weight = [&](int gi) { return b.groups[gi].edges_per_sample + b.groups[gi].leaves_per_sample; };
     std::stable_sort(go.begin(), go.end(), [&](int x, int y) { return weight(x) > weight(y); });
     std::vector<size_t> count(ng, 0), start(ng, 0);
@@ -1119,6 +1280,7 @@ static int ystack_rows(const HostModel &m, int levels) {
 // Samples per task.  The scalar and vector walks map one sample to a lane (64 per task);
 // the block and matrix-core walks evaluate one sample at a time per wavefront, so their
 // tasks are cut smaller until a launch holds at least 4 tasks per SIMD of the device.
+// The arc walk takes a workgroup per sample: its tasks are cut until a launch holds 4096.
 int samples_per_task(const qiw_ctx *c, const HostModel &m, int fmt, int64_t total_samples) {
     if (fmt == FMT_SCALAR || (fmt == FMT_VEC && m.mmax <= 6)) return QIW_WAVE;
     if (c->tune.samples_per_task > 0) return c->tune.samples_per_task;
@@ -1156,8 +1318,45 @@ int64_t vec_chunk_cost(const qiw_ctx *c, int64_t N, int64_t rows) {
     return std::max<int64_t>((int64_t)1 << 14, kChunkCost * blocks / 256);
 }
 
-int build_step_batch(qiw_ctx *c, const qiw_run *run, bool bare, const std::vector<int> &oall, Batch &b,
-                     bool split = true) {
+// A group that does not fit the arc walk: the batch is built again from assignment tries.
+constexpr int kArcNoFit = 1;
+
+// Compiles one group in the batch's format.  chunk_words, chunk_cost: as in Compiler.
+int compile_group(qiw_ctx *c, const Batch &b, int kind, int order, int n_after, int corr, int chunk_words,
+                  int64_t chunk_cost, Compiled &cg) {
+    if (b.fmt == FMT_ARC) {
+        const int rc = compile_arcs(c->m, kind, order, n_after, corr, b.precision, cg);
+        return rc == 1 ? fail(c, QIW_E_OFFDIAG, kOffDiagonal) : rc == 2 ? kArcNoFit : 0;
+    }
+    Compiler comp(c->m, kind, order, n_after, corr, b.fmt, b.max_order);
+    comp.chunk_words = chunk_words;
+    comp.chunk_cost = chunk_cost;
+    return comp.compile(cg) ? 0 : fail(c, QIW_E_OFFDIAG, comp.err);
+}
+
+// Format and workgroup width of a batch (max_order and precision set).
+void set_format(const HostModel &m, Batch &b, bool arcs) {
+    b.fmt = arcs ? eval_format(m, b.max_order, b.precision) : program_format(m, b.max_order, b.precision);
+    b.wg_waves = (b.fmt == FMT_VEC && m.mmax > 6) ? kMfmaWaves : 1;
+}
+
+// The program parts of a group that get tasks of their own per sample block (QiwTask::chunk
+// and pad_): topology chunks, or for the arc walk all segments (-1), or each segment when
+// the sample blocks alone are fewer than 2048 workgroups.
+std::vector<std::pair<int32_t, int32_t>> task_parts(const Batch &b, const Compiled &cg, bool split_segments) {
+    std::vector<std::pair<int32_t, int32_t>> v;
+    if (b.fmt != FMT_ARC) {
+        for (int32_t ch : cg.chunks) v.push_back({ch, 0});
+    } else if (split_segments && cg.n_segments > 1) {
+        for (int i = 0; i < cg.n_segments; ++i) v.push_back({i, 1});
+    } else {
+        v.push_back({-1, 0});
+    }
+    return v;
+}
+
+int build_step_batch_as(qiw_ctx *c, const qiw_run *run, bool bare, const std::vector<int> &oall, Batch &b, bool split,
+                        bool arcs) {
     const HostModel &m = c->m;
     int n_o = bare ? run->n_orders_bare : run->n_orders;
     const int32_t *ord = bare ? run->orders_bare : run->orders;
@@ -1171,11 +1370,11 @@ int build_step_batch(qiw_ctx *c, const qiw_run *run, bool bare, const std::vecto
     b.n_eval = rq.n_eval();
     b.scrambled = rq.scrambled;
     b.given = rq.given;
-    b.fmt = program_format(m, max_order, run->precision);
     b.max_order = max_order;
-    b.spt = samples_per_task(c, m, b.fmt, n_groups * b.n_eval * std::max<int64_t>(run->N_samples, 1));
     b.precision = run->precision;
-    b.wg_waves = (b.fmt == FMT_VEC && m.mmax > 6) ? kMfmaWaves : 1;
+    set_format(m, b, arcs);
+    const int64_t total = n_groups * b.n_eval * std::max<int64_t>(run->N_samples, 1);
+    b.spt = samples_per_task(c, m, b.fmt, total);
     for (int oi = 0; oi < n_o; ++oi) {
         int order = ord[oi];
         if (order > 0 && run->N_samples <= 0) continue;
@@ -1188,29 +1387,28 @@ int build_step_batch(qiw_ctx *c, const qiw_run *run, bool bare, const std::vecto
             for (int na = 1; na <= 2 * order - 1; ++na)
                 if (run->n_pts_after_max <= 0 || na <= run->n_pts_after_max) nas.push_back(na);
         for (int na : nas) {
-            Compiler comp(m, bare ? QIW_G_BARE : QIW_G_BOLD, order, na, -1, b.fmt, b.max_order);
-            if (split) {
-                comp.chunk_words = c->tune.chunk_words > 0 ? c->tune.chunk_words : kChunkWords;
-                comp.chunk_cost = vec_chunk_cost(c, run->N_samples, 1);
-            }
             Compiled cg;
-            if (!comp.compile(cg)) return fail(c, QIW_E_OFFDIAG, comp.err);
+            const int words = c->tune.chunk_words > 0 ? c->tune.chunk_words : kChunkWords;
+            const int rc = compile_group(c, b, bare ? QIW_G_BARE : QIW_G_BOLD, order, na, -1, split ? words : 0,
+                                         split ? vec_chunk_cost(c, run->N_samples, 1) : 0, cg);
+            if (rc) return rc;
             if (cg.n_top == 0) continue;
             if (cg.g.n_wslots > 255 || m.ns > 255)
                 return fail(c, QIW_E_LIMIT, "too many slots");
             b.lds = std::max(b.lds, lds_slots(cg.g, m, b.fmt));
             int slot = (int)(std::find(oall.begin(), oall.end(), order) - oall.begin());
             int64_t N = order > 0 ? run->N_samples : 1;
-            const std::vector<int32_t> chunks = cg.chunks;
+            const auto parts = task_parts(b, cg, split && total / b.spt < 2048);
             const double flops = (double)N * sample_flops(cg);
             const int64_t leaves = N * cg.leaves_per_sample, evals = N * cg.n_top;
             push_sequences(b, std::move(cg), b.n_eval, [&](int gi) {
                 b.g_first.push_back((int32_t)b.tasks.size());
                 const int64_t nt64 = (N + b.spt - 1) / b.spt;
-                const int nt = tasks_fit(b, nt64 * (int64_t)chunks.size()) ? (int)nt64 : 0;
+                const int nt = tasks_fit(b, nt64 * (int64_t)parts.size()) ? (int)nt64 : 0;
                 for (int t = 0; t < nt; ++t)
-                    for (int32_t ch : chunks) b.tasks.push_back({gi, t * b.spt, 0, (int32_t)b.tasks.size(), ch, 0});
-                b.g_count.push_back(nt * (int)chunks.size());
+                    for (auto &p : parts)
+                        b.tasks.push_back({gi, t * b.spt, 0, (int32_t)b.tasks.size(), p.first, p.second});
+                b.g_count.push_back(nt * (int)parts.size());
                 b.g_slot.push_back(slot);
                 b.flops_per_launch += flops;
                 b.leaves_per_launch += leaves;
@@ -1222,6 +1420,15 @@ int build_step_batch(qiw_ctx *c, const qiw_run *run, bool bare, const std::vecto
     if (b.overflow) return fail(c, QIW_E_LIMIT, "more than 2^28 workgroups in one launch (lower N_samples)");
     order_tasks(b);
     return 0;
+}
+
+int build_step_batch(qiw_ctx *c, const qiw_run *run, bool bare, const std::vector<int> &oall, Batch &b,
+                     bool split = true) {
+    b = Batch{};
+    const int rc = build_step_batch_as(c, run, bare, oall, b, split, true);
+    if (rc != kArcNoFit) return rc;
+    b = Batch{};
+    return build_step_batch_as(c, run, bare, oall, b, split, false);
 }
 
 }  // namespace
@@ -1340,7 +1547,7 @@ int step_plan(qiw_ctx *c, const qiw_run *run, const std::vector<int> &oall, bool
     int rc = build_step_batch(c, run, bare, oall, p.b);
     if (rc) return rc;
     const bool weighted = warp && !p.b.groups.empty();
-    if (weighted && p.b.fmt == FMT_BLOCK)
+    if (weighted && program_format(c->m, p.b.max_order, p.b.precision) == FMT_BLOCK)
         return fail(c, QIW_E_LIMIT, "the learned warp needs sector blocks <= 6 and orders <= 4");
     if (!p.b.groups.empty() && (rc = upload(c, tag, p.b, run->N_samples, p.d, weighted))) return rc;
     if (!weighted) p.key = key;
@@ -1367,12 +1574,91 @@ int ensure_model_buffers(qiw_ctx *c, double **dcoef, int32_t **dkind, double **e
     return 0;
 }
 
+// Device tables of the arc walk: the operator blocks (float32: column-major and as slice
+// registers; float64: column-major, padded past the end), E + lambda and the layout of the
+// blocks.  Staged once per model and precision (synchronous copies).
+int stage_arcs(qiw_ctx *c, int precision, ArcArgs *aa) {
+    const HostModel &m = c->m;
+    const bool fp32 = precision == QIW_PREC_FP32;
+    const size_t pad = 64, nb = m.op_desc.size() / 3, regs = (size_t)arc_slice_regs(m);
+    int rc = 0;
+    float *sl = fp32 ? (float *)dev(c, "arc.slices", std::max<size_t>(nb, 1) * regs * 64 * 4, &rc) : nullptr;
+    float *cm32 = fp32 ? (float *)dev(c, "arc.ops32", (m.op_data.size() + pad) * 4, &rc) : nullptr;
+    double *cm64 = fp32 ? nullptr : (double *)dev(c, "arc.ops", (m.op_data.size() + pad) * 8, &rc);
+    double *ediag = (double *)dev(c, "arc.ediag", (size_t)m.bt * 8, &rc);
+    uint8_t *emask = (uint8_t *)dev(c, "arc.emask", (size_t)m.bt, &rc);
+    int32_t *lay = (int32_t *)dev(c, "arc.layout", ((size_t)m.bt + 3 * m.ns) * 4, &rc);
+    if (rc) return rc;
+    if (!(c->arc_staged & (fp32 ? 2 : 1))) {
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        std::vector<double> o(m.op_data);
+        o.resize(m.op_data.size() + pad, 0.0);
+        if (fp32) {
+            const int mb = qiw_arc_rows(m.mmax);
+            std::vector<float> o32(o.begin(), o.end()), s((size_t)std::max<size_t>(nb, 1) * regs * 64, 0.f);
+            for (size_t b = 0; b < nb; ++b) {
+                const int off = m.op_desc[3 * b], mf = m.op_desc[3 * b + 1], mi = m.op_desc[3 * b + 2];
+                for (int i = 0; i < mf; ++i)
+                    for (int k = 0; k < mi; ++k) {
+                        const int slice = (i / 4) * mb + k;
+                        s[(b * regs + slice / 16) * 64 + 4 * (slice % 16) + i % 4] = (float)m.op_data[off + i + k * mf];
+                    }
+            }
+            HIPCHK(c, hipMemcpy(sl, s.data(), s.size() * 4, hipMemcpyHostToDevice));
+            HIPCHK(c, hipMemcpy(cm32, o32.data(), o32.size() * 4, hipMemcpyHostToDevice));
+        } else {
+            HIPCHK(c, hipMemcpy(cm64, o.data(), o.size() * 8, hipMemcpyHostToDevice));
+        }
+        std::vector<double> ed((size_t)m.bt, 0.0);
+        std::vector<uint8_t> mk((size_t)m.bt, 0);
+        std::vector<int32_t> l((size_t)m.bt + 3 * m.ns);
+        for (int s = 0; s < m.ns; ++s) {
+            const int d = m.dims[s];
+            for (int e = 0; e < d * d; ++e) l[m.bt_off[s] + e] = s;
+            for (int i = 0; i < d; ++i) {
+                ed[m.bt_off[s] + i + i * d] = m.E[s][i] + m.lambda0;
+                mk[m.bt_off[s] + i + i * d] = 1;
+            }
+            l[m.bt + s] = d;
+            l[m.bt + m.ns + s] = m.bt_off[s];
+            l[m.bt + 2 * m.ns + s] = arc_stride(d, m.mmax);
+        }
+        HIPCHK(c, hipMemcpy(ediag, ed.data(), ed.size() * 8, hipMemcpyHostToDevice));
+        HIPCHK(c, hipMemcpy(emask, mk.data(), mk.size(), hipMemcpyHostToDevice));
+        HIPCHK(c, hipMemcpy(lay, l.data(), l.size() * 4, hipMemcpyHostToDevice));
+        c->arc_staged |= fp32 ? 2 : 1;
+    }
+    aa->ops = fp32 ? (const void *)sl : (const void *)cm64;
+    aa->ops_cm = fp32 ? (const void *)cm32 : (const void *)cm64;
+    aa->ediag = ediag;
+    aa->emask = emask;
+    aa->sector_of = lay;
+    aa->dims = lay + m.bt;
+    aa->bt_off = lay + m.bt + m.ns;
+    aa->stride = lay + m.bt + 2 * m.ns;
+    aa->bt = m.bt;
+    return 0;
+}
+
 // Launches the evaluator matching the model's sector structure.  The vector and matrix-core
 // walks stage their operator tables once per model on their first launch (synchronous
 // copies), so a launch can be captured into a hipGraph only after that
 // (c->vec_staged / c->mfma_staged).
-int launch_eval(qiw_ctx *c, const EvalArgs &a, int n_tasks, int fmt, int precision) {
+int launch_eval(qiw_ctx *c, const EvalArgs &a, const Batch &batch) {
     const HostModel &m = c->m;
+    const int n_tasks = (int)batch.tasks.size(), fmt = batch.fmt, precision = batch.precision;
+    if (fmt == FMT_ARC) {
+        ArcArgs aa{};
+        int rc = stage_arcs(c, precision, &aa);
+        if (rc) return rc;
+        aa.e = a;
+        for (const Batch::Launch &ln : batch.launches) {
+            aa.e.tasks = a.tasks + ln.first;
+            HIPCHK(c, qiw_launch_eval_arcs(c->stream, aa, ln.count, m.mmax, precision == QIW_PREC_FP32 ? 1 : 0, ln.waves,
+                                           ln.lds));
+        }
+        return 0;
+    }
     const size_t lds_bytes = (size_t)a.lds_slots * sizeof(double);
     if (lds_bytes > 160 * 1024) return fail(c, QIW_E_LIMIT, "evaluator state exceeds the 160 KiB of LDS of a CU");
     if (fmt == FMT_SCALAR) {
@@ -1778,6 +2064,7 @@ static int qiw_set_model_impl(qiw_ctx *c, const qiw_model *mi) {
     c->model_fp = fp;
     c->vec_staged = false;
     c->mfma_staged = false;
+    c->arc_staged = 0;
     atomic_ip(c->m, c->ip);
     c->n_known = (m.ppgf_kind == QIW_GF_INC_SPLINE) ? 1 : m.ntau;
     c->der0.assign(m.bt, cd(0.0));  // initial_ppgf_derivative: -i diag(-E - lambda), src/ppgf.jl:710-720
@@ -2029,7 +2316,7 @@ int run_inchworm(qiw_ctx *c, const qiw_run *run, bool do_bare, int first_w, int 
         EvalArgs a = make_eval_args(c, bare_b, bare_d, ptab, eshift, dcoef, dkind, partial);
         HIPCHK(c, coords(bare_b, bare_d, QIW_RQ_BARE, 0, gidx_bare));
         HIPCHK(c, mark());
-        if ((rc = launch_eval(c, a, (int)bare_b.tasks.size(), bare_b.fmt, bare_b.precision))) return rc;
+        if ((rc = launch_eval(c, a, bare_b))) return rc;
         HIPCHK(c, mark());
         fa.groups = bare_d.groups;
         fa.group_task_first = bare_d.g_first;
@@ -2071,10 +2358,14 @@ int run_inchworm(qiw_ctx *c, const qiw_run *run, bool do_bare, int first_w, int 
             fa.normalize = normalize ? 1 : 0;
         };
         // without the warp the whole loop is one hipGraph, replayed while the launch arguments
-        // are unchanged: the flat scalar walk, and the vector and matrix-core walks once their
+        // are unchanged: the flat scalar walk, the arc walk, and the vector and matrix-core walks once their
         // tables are staged (from the second call on); the LDS block walk copies host data per
         // launch and stays eager
-        const bool staged = bold_b.fmt == FMT_SCALAR ||
+        if (bold_b.fmt == FMT_ARC) {  // stages its tables here, before a capture
+            ArcArgs aa{};
+            if ((rc = stage_arcs(c, bold_b.precision, &aa))) return rc;
+        }
+        const bool staged = bold_b.fmt == FMT_SCALAR || bold_b.fmt == FMT_ARC ||
                             (bold_b.fmt == FMT_VEC && (m.mmax > 6 ? c->mfma_staged : c->vec_staged));
         bool graph = c->graphs && staged && !warped && !c->no_alloc && !rq.given;
         const int n_known_start = n_known;
@@ -2118,7 +2409,7 @@ int run_inchworm(qiw_ctx *c, const qiw_run *run, bool do_bare, int first_w, int 
                 for (int jw = first_w; jw <= last_w && err == hipSuccess; ++jw) {
                     step_args(jw);
                     if ((err = coords(bold_b, bold_d, QIW_RQ_BOLD, jw, nullptr)) != hipSuccess) break;  // never given
-                    if (launch_eval(c, a, n_tasks, bold_b.fmt, bold_b.precision) != 0) {
+                    if (launch_eval(c, a, bold_b) != 0) {
                         err = hipErrorUnknown;
                         break;
                     }
@@ -2164,7 +2455,7 @@ int run_inchworm(qiw_ctx *c, const qiw_run *run, bool do_bare, int first_w, int 
             HIPCHK(c, coords(bold_b, bold_d, QIW_RQ_BOLD, jw,
                              gidx_bold ? gidx_bold + (size_t)(jw - first_w) * bold_b.groups.size() : nullptr));
             HIPCHK(c, mark());
-            if ((rc = launch_eval(c, a, (int)bold_b.tasks.size(), bold_b.fmt, bold_b.precision))) return rc;
+            if ((rc = launch_eval(c, a, bold_b))) return rc;
             HIPCHK(c, mark());
             fa.jf = fa.jt = jw + 1;
             fa.tau_w = jw * m.h;
@@ -2273,7 +2564,7 @@ namespace {
 
 // Self-energy groups of run->orders (order 0 has none; order 1 is exact), slot = index in
 // run->orders.
-int build_diff_batch(qiw_ctx *c, const qiw_run *run, Batch &b) {
+int build_diff_batch_as(qiw_ctx *c, const qiw_run *run, Batch &b, bool arcs) {
     const HostModel &m = c->m;
     int max_order = 0;
     int64_t n_groups = 0;
@@ -2285,33 +2576,33 @@ int build_diff_batch(qiw_ctx *c, const qiw_run *run, Batch &b) {
     b.n_eval = rq.n_eval();
     b.scrambled = rq.scrambled;
     b.given = rq.given;
-    b.fmt = program_format(m, max_order, run->precision);
     b.max_order = max_order;
-    b.spt = samples_per_task(c, m, b.fmt, n_groups * b.n_eval * std::max<int64_t>(run->N_samples, 1));
     b.precision = run->precision;
-    b.wg_waves = (b.fmt == FMT_VEC && m.mmax > 6) ? kMfmaWaves : 1;
+    set_format(m, b, arcs);
+    const int64_t total = n_groups * b.n_eval * std::max<int64_t>(run->N_samples, 1);
+    b.spt = samples_per_task(c, m, b.fmt, total);
     for (int oi = 0; oi < run->n_orders; ++oi) {
         const int order = run->orders[oi];
         if (order == 0 || (order > 1 && run->N_samples <= 0)) continue;  // :557, :567
-        Compiler comp(m, QIW_G_SIGMA, order, 1, -1, b.fmt, b.max_order);
-        comp.chunk_words = c->tune.chunk_words > 0 ? c->tune.chunk_words : kChunkWordsDiff;
-        comp.chunk_cost = vec_chunk_cost(c, run->N_samples, 1);
         Compiled cg;
-        if (!comp.compile(cg)) return fail(c, QIW_E_OFFDIAG, comp.err);
+        const int rc = compile_group(c, b, QIW_G_SIGMA, order, 1, -1,
+                                     c->tune.chunk_words > 0 ? c->tune.chunk_words : kChunkWordsDiff,
+                                     vec_chunk_cost(c, run->N_samples, 1), cg);
+        if (rc) return rc;
         if (cg.n_top == 0) continue;
         if (cg.g.n_wslots > 255 || m.ns > 255) return fail(c, QIW_E_LIMIT, "too many slots");
         b.lds = std::max(b.lds, lds_slots(cg.g, m, b.fmt));
         const int64_t N = order == 1 ? 1 : run->N_samples;
-        const std::vector<int32_t> chunks = cg.chunks;
+        const auto parts = task_parts(b, cg, total / b.spt < 2048);
         const double flops = (double)N * sample_flops(cg);
         const int64_t leaves = N * cg.leaves_per_sample, evals = N * cg.n_top;
         push_sequences(b, std::move(cg), b.n_eval, [&](int gi) {
             b.g_first.push_back((int32_t)b.tasks.size());
             const int64_t nt64 = (N + b.spt - 1) / b.spt;
-            const int nt = tasks_fit(b, nt64 * (int64_t)chunks.size()) ? (int)nt64 : 0;
+            const int nt = tasks_fit(b, nt64 * (int64_t)parts.size()) ? (int)nt64 : 0;
             for (int t = 0; t < nt; ++t)
-                for (int32_t ch : chunks) b.tasks.push_back({gi, t * b.spt, 0, (int32_t)b.tasks.size(), ch, 0});
-            b.g_count.push_back(nt * (int)chunks.size());
+                for (auto &p : parts) b.tasks.push_back({gi, t * b.spt, 0, (int32_t)b.tasks.size(), p.first, p.second});
+            b.g_count.push_back(nt * (int)parts.size());
             b.g_slot.push_back(oi);
             b.flops_per_launch += flops;
             b.leaves_per_launch += leaves;
@@ -2322,6 +2613,14 @@ int build_diff_batch(qiw_ctx *c, const qiw_run *run, Batch &b) {
     if (b.overflow) return fail(c, QIW_E_LIMIT, "more than 2^28 workgroups in one launch (lower N_samples)");
     order_tasks(b);
     return 0;
+}
+
+int build_diff_batch(qiw_ctx *c, const qiw_run *run, Batch &b) {
+    b = Batch{};
+    const int rc = build_diff_batch_as(c, run, b, true);
+    if (rc != kArcNoFit) return rc;
+    b = Batch{};
+    return build_diff_batch_as(c, run, b, false);
 }
 
 // diff_inchworm!: n_tau - 1 steps from the atomic propagator, each one evaluator launch
@@ -2464,7 +2763,7 @@ int run_diff(qiw_ctx *c, const qiw_run *run, double *S_out, double *S_std_out) {
                                              run->N_samples > 0 ? run->N_samples : 1, sobm, rq.seed, QIW_RQ_DIFF, st,
                                              d.ut));
         HIPCHK(c, mark());
-        if ((rc = launch_eval(c, a, (int)b.tasks.size(), b.fmt, b.precision))) return rc;
+        if ((rc = launch_eval(c, a, b))) return rc;
         HIPCHK(c, mark());
         HIPCHK(c, qiw_launch_finalize_diff(c->stream, fa, rqmc ? 1 : 0));
         ++launches;
@@ -2583,15 +2882,14 @@ static int qiw_inchworm_step_bare_impl(qiw_ctx *c, const qiw_run *run, double *v
 namespace {
 // The groups of operator pair ci (src/inchworm.jl:957-981): every n_pts_after of every
 // order with topologies, compiled.
-int build_corr_groups(qiw_ctx *c, const qiw_run *run, int ci, Batch &b, bool *first_is_order0) {
+int build_corr_groups_as(qiw_ctx *c, const qiw_run *run, int ci, Batch &b, bool *first_is_order0, bool arcs) {
     const HostModel &m = c->m;
     const RandPlan rq = rand_plan(run);
     int max_order = 0;
     for (int oi = 0; oi < run->n_orders; ++oi) max_order = std::max(max_order, (int)run->orders[oi]);
-    b.fmt = program_format(m, max_order, run->precision);
     b.max_order = max_order;
     b.precision = run->precision;
-    b.wg_waves = (b.fmt == FMT_VEC && m.mmax > 6) ? kMfmaWaves : 1;
+    set_format(m, b, arcs);
     b.n_eval = rq.n_eval();
     b.scrambled = rq.scrambled;
     b.given = rq.given;
@@ -2601,11 +2899,11 @@ int build_corr_groups(qiw_ctx *c, const qiw_run *run, int ci, Batch &b, bool *fi
         if (order > 0 && run->N_samples <= 0) continue;
         int lo = order == 0 ? 0 : 1, hi = order == 0 ? 0 : 2 * order - 1;
         for (int na = lo; na <= hi; ++na) {
-            Compiler comp(m, QIW_G_CORR, order, na, ci, b.fmt, b.max_order);
-            comp.chunk_words = c->tune.chunk_words > 0 ? c->tune.chunk_words : kChunkWords;
-            comp.chunk_cost = vec_chunk_cost(c, run->N_samples, m.ntau);
             Compiled cg;
-            if (!comp.compile(cg)) return fail(c, QIW_E_OFFDIAG, comp.err);
+            const int rc = compile_group(c, b, QIW_G_CORR, order, na, ci,
+                                         c->tune.chunk_words > 0 ? c->tune.chunk_words : kChunkWords,
+                                         vec_chunk_cost(c, run->N_samples, m.ntau), cg);
+            if (rc) return rc;
             if (cg.n_top == 0) continue;
             if (b.groups.empty() && order == 0) *first_is_order0 = true;
             b.lds = std::max(b.lds, lds_slots(cg.g, m, b.fmt));
@@ -2614,6 +2912,14 @@ int build_corr_groups(qiw_ctx *c, const qiw_run *run, int ci, Batch &b, bool *fi
     }
     if (b.r_first.size() > 64) return fail(c, QIW_E_LIMIT, "more than 64 (order, n_pts_after) groups");
     return 0;
+}
+
+int build_corr_groups(qiw_ctx *c, const qiw_run *run, int ci, Batch &b, bool *first_is_order0) {
+    b = Batch{};
+    const int rc = build_corr_groups_as(c, run, ci, b, first_is_order0, true);
+    if (rc != kArcNoFit) return rc;
+    b = Batch{};
+    return build_corr_groups_as(c, run, ci, b, first_is_order0, false);
 }
 
 // correlator_2p(expansion, grid, orders, N_samples, RequestStdDev(); rand_params)
@@ -2671,22 +2977,24 @@ int run_correlator(qiw_ctx *c, const qiw_run *run, double *corr_out, double *cor
             if ((rc = build_corr_groups(c, run, ci, b, &p.first_is_order0))) return rc;
             if (!b.groups.empty()) {
                 int ng = (int)b.groups.size();
-                b.spt = samples_per_task(c, m, b.fmt, (int64_t)m.ntau * ng * std::max<int64_t>(run->N_samples, 1));
+                const int64_t total = (int64_t)m.ntau * ng * std::max<int64_t>(run->N_samples, 1);
+                b.spt = samples_per_task(c, m, b.fmt, total);
                 std::vector<int32_t> rf((size_t)m.ntau * ng, 0), rcnt((size_t)m.ntau * ng, 0);
                 for (int j = 0; j < m.ntau; ++j)
                     for (int gi = 0; gi < ng; ++gi) {
                         // tau_A = tau_B: only the leading order-0 group (src/inchworm.jl:1014-1024)
                         if (j == 0 && !(gi == 0 && p.first_is_order0)) continue;
                         int64_t N = b.groups[gi].g.order > 0 ? run->N_samples : 1;
-                        const std::vector<int32_t> &chs = b.groups[gi].chunks;
+                        const auto parts = task_parts(b, b.groups[gi], total / b.spt < 2048);
                         const int64_t nt64 = (N + b.spt - 1) / b.spt;
-                        if (!tasks_fit(b, nt64 * (int64_t)chs.size()))
+                        if (!tasks_fit(b, nt64 * (int64_t)parts.size()))
                             return fail(c, QIW_E_LIMIT, "more than 2^28 workgroups in one launch (lower N_samples)");
                         const int nt = (int)nt64;
                         rf[(size_t)j * ng + gi] = (int32_t)b.tasks.size();
-                        rcnt[(size_t)j * ng + gi] = nt * (int)chs.size();
+                        rcnt[(size_t)j * ng + gi] = nt * (int)parts.size();
                         for (int t = 0; t < nt; ++t)
-                            for (int32_t ch : chs) b.tasks.push_back({gi, t * b.spt, j, (int32_t)b.tasks.size(), ch, 0});
+                            for (auto &q : parts)
+                                b.tasks.push_back({gi, t * b.spt, j, (int32_t)b.tasks.size(), q.first, q.second});
                         b.flops_per_launch += (double)N * sample_flops(b.groups[gi]);
                         b.leaves_per_launch += N * b.groups[gi].leaves_per_sample;
                         b.diagram_evals_per_launch += N * b.groups[gi].n_top;
@@ -2764,7 +3072,7 @@ int run_correlator(qiw_ctx *c, const qiw_run *run, double *corr_out, double *cor
             a.ut = ut_rows;
             a.ut_row_stride = b.ut_total;
         }
-        if ((rc = launch_eval(c, a, (int)b.tasks.size(), b.fmt, b.precision))) return rc;
+        if ((rc = launch_eval(c, a, b))) return rc;
         HIPCHK(c, hipEventRecord(e1, c->stream));
         CorrFinalizeArgs fa{};
         fa.groups = d.groups;
@@ -2925,7 +3233,8 @@ int warp_collect(qiw_ctx *c, const qiw_run *run, const std::vector<int> &steps, 
     Batch b;
     DevBatch d;
     if ((rc = build_step_batch(c, &r, false, oall, b, false))) return rc;  // per-sample sums: one chunk
-    if (b.fmt == FMT_BLOCK) return fail(c, QIW_E_LIMIT, "the learned warp needs sector blocks <= 6 and orders <= 4");
+    if (program_format(m, b.max_order, b.precision) == FMT_BLOCK)
+        return fail(c, QIW_E_LIMIT, "the learned warp needs sector blocks <= 6 and orders <= 4");
     if (b.groups.empty()) return fail(c, QIW_E_ARG, "no sampled bold groups to train on");
     if ((rc = upload(c, "wtrain", b, n, d))) return rc;
     double *dcoef, *eshift;
@@ -2948,7 +3257,7 @@ int warp_collect(qiw_ctx *c, const qiw_run *run, const std::vector<int> &steps, 
     a.per_sample = ps;
     for (size_t si = 0; si < steps.size(); ++si) {
         a.step_w = steps[si];
-        if ((rc = launch_eval(c, a, (int)b.tasks.size(), b.fmt, b.precision))) return rc;
+        if ((rc = launch_eval(c, a, b))) return rc;
         HIPCHK(c, hipMemcpyAsync(host.data(), ps, (size_t)ps_total * 8, hipMemcpyDeviceToHost, c->stream));
         HIPCHK(c, hipStreamSynchronize(c->stream));
         for (size_t gi = 0; gi < gs.size(); ++gi)
@@ -3002,7 +3311,7 @@ int time_bold_step(qiw_ctx *c, const qiw_run *run, double *ms_out) {
     double best = 1e300;
     for (int rep = 0; rep < 3; ++rep) {
         HIPCHK(c, hipEventRecord(e0, c->stream));
-        if ((rc = launch_eval(c, a, (int)b.tasks.size(), b.fmt, b.precision))) return rc;
+        if ((rc = launch_eval(c, a, b))) return rc;
         HIPCHK(c, hipEventRecord(e1, c->stream));
         HIPCHK(c, hipEventSynchronize(e1));
         float ms = 0;
@@ -3058,7 +3367,7 @@ static int qiw_autotune_impl(qiw_ctx *c, const qiw_run *run, qiw_tuning *out) {
     const HostModel &m = c->m;
     int max_order = 0;
     for (int i = 0; i < run->n_orders; ++i) max_order = std::max(max_order, (int)run->orders[i]);
-    const int fmt = program_format(m, max_order, run->precision);
+    const int fmt = eval_format(m, max_order, run->precision);
     std::vector<qiw_tuning> cand;
     if (fmt == FMT_SCALAR) {
         for (int w : {256, 384, 512, 640, 896, 1024, 2048}) cand.push_back(qiw_tuning{w, 0, 0, 0, 0, 0.0});

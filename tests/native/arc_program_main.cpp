@@ -1,0 +1,359 @@
+// Runs the block-sector programs of qiw_arcs.h on the CPU, word for word as the arc walk
+// reads them, with every access checked, against the plain sum over topologies and pair
+// assignments.  Arguments: kind order n_after n_fixed waves cap_bytes elem modes seed [largest block, 5].
+// The model: `modes` fermionic modes, one sector per particle number with random dimensions,
+// random operator blocks, propagators and arc values.  Prints the largest deviation relative
+// to the largest element, and the count of diagrams of the program and of the plain sum.
+#include <cmath>
+#include <cstdio>
+#include <cstdlib>
+#include <functional>
+#include <map>
+#include <random>
+
+#include "qiw_arcs.h"
+
+using namespace qiwi;
+
+static std::mt19937_64 rng;
+static double rnd() { return std::uniform_real_distribution<double>(-1.0, 1.0)(rng); }
+static void die(const char *what) {
+    std::printf("FAIL %s\n", what);
+    std::exit(1);
+}
+
+typedef std::vector<std::pair<int, int>> Pairs;
+struct Topo {
+    Pairs p;
+    int parity;
+};
+static void gen(Pairs &part, int parity, std::vector<int> open, std::vector<Topo> &out) {
+    if (open.empty()) {
+        out.push_back({part, parity});
+        return;
+    }
+    for (size_t i = 1; i < open.size(); ++i) {
+        std::vector<int> rest;
+        for (size_t q = 1; q < open.size(); ++q)
+            if (q != i) rest.push_back(open[q]);
+        part.push_back({open[0], open[i]});
+        gen(part, i % 2 ? parity : -parity, rest, out);
+        part.pop_back();
+    }
+}
+static bool connected(const Pairs &t, int k) {
+    Pairs stack, rest;
+    for (auto &p : t) ((p.first <= k && p.second > k) ? stack : rest).push_back(p);
+    while (!stack.empty()) {
+        auto c = stack.back();
+        stack.pop_back();
+        for (size_t i = rest.size(); i-- > 0;) {
+            auto a = c, b = rest[i];
+            if (a.first > b.first) std::swap(a, b);
+            if (a.second > b.first && a.second < b.second) {
+                stack.push_back(rest[i]);
+                rest.erase(rest.begin() + i);
+            }
+        }
+    }
+    return rest.empty();
+}
+
+int main(int argc, char **argv) {
+    if (argc < 10) return 2;
+    const int kind = std::atoi(argv[1]), order = std::atoi(argv[2]), n_after = std::atoi(argv[3]);
+    const int n_fixed = std::atoi(argv[4]), waves = std::atoi(argv[5]), cap = std::atoi(argv[6]);
+    const int elem = std::atoi(argv[7]), modes = std::atoi(argv[8]);
+    rng.seed(std::atoi(argv[9]));
+    const int most = argc > 10 ? std::atoi(argv[10]) : 5;
+    ArcModel m;
+    m.ns = modes + 1;
+    m.np = 2 * modes;
+    for (int s = 0; s < m.ns; ++s) m.dims.push_back(1 + (int)(rng() % most));
+    if (modes > 1) m.dims[1] = 1;
+    std::vector<int> off(m.ns + 1, 0);
+    for (int s = 0; s < m.ns; ++s) off[s + 1] = off[s] + m.dims[s] * m.dims[s];
+    ArcLayout l;
+    l.elem = elem;
+    l.mmax = *std::max_element(m.dims.begin(), m.dims.end());
+    l.bt = off[m.ns];
+    l.bt_off.assign(off.begin(), off.end() - 1);
+    l.waves = waves;
+    l.cap = cap;
+    std::vector<std::vector<double>> blocks;  // operator blocks, named by index
+    std::vector<std::pair<int, int>> shape;
+    ArcBlocks ob;
+    auto block = [&](int from, int to) -> uint32_t {
+        if (to < 0) return ARC_NONE;
+        std::vector<double> v(m.dims[to] * m.dims[from]);
+        for (double &x : v) x = rnd();
+        blocks.push_back(v);
+        shape.push_back({m.dims[to], m.dims[from]});
+        return (uint32_t)blocks.size() - 1;
+    };
+    for (int p = 0; p < m.np; ++p) {
+        std::vector<int> h, t;
+        std::vector<uint32_t> hb, tb;
+        for (int s = 0; s < m.ns; ++s) {
+            const int up = s + 1 < m.ns ? s + 1 : -1, dn = s - 1;
+            h.push_back(p % 2 ? up : dn);
+            t.push_back(p % 2 ? dn : up);
+            hb.push_back(block(s, h.back()));
+            tb.push_back(block(s, t.back()));
+        }
+        m.head_sf.push_back(h);
+        m.tail_sf.push_back(t);
+        ob.head.push_back(hb);
+        ob.tail.push_back(tb);
+        m.table.push_back(p % 2);
+    }
+    for (int s = 0; s < m.ns; ++s) {
+        m.a_sf.push_back(s - 1);
+        m.b_sf.push_back(s + 1 < m.ns ? s + 1 : -1);
+        ob.a.push_back(block(s, m.a_sf[s]));
+        ob.b.push_back(block(s, m.b_sf[s]));
+    }
+    const int n = kind == ARC_BARE ? 2 * order + 2 : 2 * order + 3;
+    std::vector<std::vector<double>> prop(n + 1, std::vector<double>(l.bt));  // segment L
+    for (auto &v : prop)
+        for (double &x : v) x = rnd();
+    std::map<uint32_t, double> arcs;
+    auto arc = [&](int head, int tail, int tab) {
+        const uint32_t k = (uint32_t)head | ((uint32_t)tail << 8) | ((uint32_t)tab << 16);
+        auto it = arcs.find(k);
+        if (it == arcs.end()) it = arcs.emplace(k, rnd()).first;
+        return it->second;
+    };
+
+    // ---- the program ----
+    ArcGroupProgram pg;
+    const int rc = arc_compile(m, l, ob, kind, order, n_after, n_fixed, pg);
+    if (rc) {
+        std::printf("rc %d\n", rc);
+        return 0;
+    }
+    const std::vector<uint32_t> &b = pg.blob;
+    auto at = [&](size_t i) -> uint32_t {
+        if (i >= b.size()) die("word out of the program");
+        return b[i];
+    };
+    const size_t region = (pg.lds - at(7)) / elem;
+    if (pg.lds > l.cap) die("more LDS than the cap");
+    if (at(4) != 128 || at(5) % 16 || at(6) % 16 || at(7) % 16) die("alignment");
+    const size_t dv_size = (at(6) - at(5)) / elem, prop_size = (at(7) - at(6)) / elem;
+    std::vector<double> dv(2 + 2 * at(1));
+    if (dv.size() > dv_size) die("arc values");
+    dv[1] = 1.0;
+    for (uint32_t i = 0; i < at(1); ++i) {
+        const uint32_t a = at(at(3) + i);
+        dv[2 + 2 * i] = arc(a & 255, (a >> 8) & 255, a >> 16);
+        dv[3 + 2 * i] = -dv[2 + 2 * i];
+    }
+    std::vector<double> pl((size_t)(n - 1) * l.bt, NAN);
+    if (pl.size() > prop_size) die("propagators");
+    for (int L = 2; L < n; ++L) std::copy(prop[L].begin(), prop[L].end(), pl.begin() + (size_t)(L - 2) * l.bt);
+    if (at(2))
+        for (int s = 0; s < m.ns; ++s)
+            for (int i = 0; i < m.dims[s]; ++i)
+                for (int j = 0; j < m.dims[s]; ++j) {
+                    double v = 0;
+                    for (int q = 0; q < m.dims[s]; ++q)
+                        v += prop[at(2) + 1][off[s] + i + q * m.dims[s]] * prop[at(2)][off[s] + q + j * m.dims[s]];
+                    pl[(size_t)(n - 2) * l.bt + off[s] + i + j * m.dims[s]] = v;
+                }
+    std::vector<double> res(l.bt, 0.0), ref(l.bt, 0.0);
+    for (uint32_t sg = 0; sg < at(0); ++sg) {
+        const size_t h = at(kArcGroupHead + sg);
+        const int s0 = at(h) & 255, m0 = (at(h) >> 8) & 255, lg = at(h) >> 16, cg = 1 << lg;
+        if (m0 != m.dims[s0]) die("m0");
+        for (int c0 = 0; c0 < m0; c0 += cg) {
+            std::vector<double> st(region, NAN);
+            auto get = [&](size_t i) -> double {
+                if (i >= st.size()) die("state read out of the region");
+                return st[i];
+            };
+            auto put = [&](size_t i, double v) {
+                if (i >= st.size()) die("state write out of the region");
+                st[i] = v;
+            };
+            auto times = [&](size_t po, int mm, const std::vector<double> &x) {
+                std::vector<double> y(mm, 0.0);
+                for (int i = 0; i < mm; ++i)
+                    for (int q = 0; q < mm; ++q) {
+                        if (po + i + q * mm >= pl.size()) die("propagator read");
+                        y[i] += pl[po + i + q * mm] * x[q];
+                    }
+                return y;
+            };
+            const int m1 = at(h + 2) & 255, str1 = at(h + 2) >> 8;
+            for (int col = 0; col < cg; ++col) {
+                std::vector<double> x(m1, 0.0);
+                for (int k = 0; k < m1; ++k)
+                    if (c0 + col < m0)
+                        x[k] = at(h + 3) == ARC_NONE ? (k == c0 + col) : blocks.at(at(h + 3)).at((c0 + col) * m1 + k);
+                if (at(h + 4) != ARC_NONE) x = times(at(h + 4), m1, x);
+                for (int k = 0; k < m1; ++k) put(at(h + 5) + col * str1 + k, x[k]);
+            }
+            int stf = str1;
+            for (uint32_t s = 0; s < at(h + 1); ++s) {
+                const uint32_t n_tiles = at(h + kArcSegHead + 2 * s);
+                const size_t tiles = at(h + kArcSegHead + 2 * s + 1);
+                std::vector<std::pair<size_t, double>> writes;
+                for (uint32_t ti = 0; ti < n_tiles; ++ti) {
+                    const uint32_t t0 = at(tiles + 4 * ti);
+                    const int n_ops = t0 & 255, rows = (t0 >> 8) & 255, ns = (t0 >> 16) & 255, str = t0 >> 24;
+                    if (ns < 1 || ns > (64 >> lg) || str != arc_stride(rows, l.mmax)) die("tile");
+                    for (int lane = 0; lane < ns * cg; ++lane) {
+                        const int col = lane & (cg - 1), sl = lane >> lg;
+                        std::vector<double> acc(rows, 0.0);
+                        for (int oi = 0; oi < n_ops; ++oi) {
+                            const size_t o = at(tiles + 4 * ti + 3) + 4 * oi;
+                            const int ms = at(o + 1) & 255, ss = (at(o + 1) >> 8) & 255, ne = at(o + 1) >> 16;
+                            std::vector<double> y(ms, 0.0);
+                            for (int e = 0; e < ne; ++e) {
+                                const uint32_t q = at(at(o + 2) + e * ns + sl);
+                                for (int k = 0; k < ms; ++k) {
+                                    const double v = get((q & 0xFFFFF) + col * ss + k);
+                                    if (std::isnan(v)) die("state read before it is written");
+                                    y[k] += dv.at(q >> 20) * v;
+                                }
+                            }
+                            const uint32_t blk = at(o);
+                            if (blk == ARC_NONE) {
+                                for (int k = 0; k < ms; ++k) acc[k] += y[k];
+                            } else {
+                                if (shape.at(blk) != std::make_pair(rows, ms)) die("operator shape");
+                                for (int k = 0; k < ms; ++k)
+                                    for (int i = 0; i < rows; ++i) acc[i] += blocks[blk][i + k * rows] * y[k];
+                            }
+                        }
+                        if (at(tiles + 4 * ti + 2) != ARC_NONE) acc = times(at(tiles + 4 * ti + 2), rows, acc);
+                        for (int k = 0; k < str; ++k)
+                            writes.push_back({at(tiles + 4 * ti + 1) + lane * str + k, k < rows ? acc[k] : 0.0});
+                        stf = str;
+                    }
+                }
+                // a stage may not write what it reads: the new states are stored after all reads
+                std::vector<char> hit(region, 0);
+                for (auto &w : writes) {
+                    if (w.first >= region || hit[w.first]) die("two states in one place");
+                    hit[w.first] = 1;
+                }
+                for (uint32_t ti = 0; ti < n_tiles; ++ti) {
+                    const uint32_t t0 = at(tiles + 4 * ti);
+                    for (uint32_t oi = 0; oi < (t0 & 255); ++oi) {
+                        const size_t o = at(tiles + 4 * ti + 3) + 4 * oi;
+                        const int ms = at(o + 1) & 255, ss = (at(o + 1) >> 8) & 255, ne = at(o + 1) >> 16;
+                        for (uint32_t i = 0; i < ne * ((t0 >> 16) & 255); ++i)
+                            for (int col = 0; col < cg; ++col)
+                                for (int k = 0; k < ms; ++k)
+                                    if (hit[(at(at(o + 2) + i) & 0xFFFFF) + col * ss + k]) die("a stage overwrites its source");
+                    }
+                }
+                for (auto &w : writes) put(w.first, w.second);
+            }
+            for (int col = 0; col < cg && c0 + col < m0; ++col) {
+                std::vector<double> x(m0, 0.0);
+                for (uint32_t p = 0; p < at(h + 6); ++p)
+                    for (int k = 0; k < m0; ++k) x[k] += get(at(at(h + 7) + p) + col * stf + k);
+                for (int i = 0; i < m0; ++i)
+                    for (int q = 0; q < m0; ++q)
+                        res[off[s0] + i + (c0 + col) * m0] += prop[n][off[s0] + i + q * m0] * x[q];
+            }
+        }
+    }
+
+    // ---- the plain sum ----
+    const int pos_w = kind == ARC_BARE ? -1 : kind == ARC_SIGMA ? 2 * order + 2 : 2 * order - n_after + 2;
+    std::vector<Topo> all;
+    Pairs part;
+    std::vector<int> pts;
+    for (int i = 1; i <= 2 * order; ++i) pts.push_back(i);
+    gen(part, 1, pts, all);
+    double leaves = 0;
+    auto point_pos = [&](int pt) {  // point 1 is the latest
+        int pos = n - pt;
+        if (kind == ARC_SIGMA) return pos - 1;
+        if (pos_w > 0 && pos <= pos_w) --pos;
+        return pos;
+    };
+    const int cut = kind == ARC_SIGMA ? 1 : n_after;
+    for (const Topo &t : all) {
+        if (kind != ARC_BARE && !connected(t.p, cut)) continue;
+        std::vector<int> arc_at(n + 1, -1), is_head(n + 1, 0);
+        for (size_t a = 0; a < t.p.size(); ++a) {
+            const int head = point_pos(t.p[a].second), tail = point_pos(t.p[a].first);
+            arc_at[head] = arc_at[tail] = (int)a;
+            is_head[head] = 1;
+        }
+        for (int s0 = 0; s0 < m.ns; ++s0) {
+            std::vector<int> sel(order + 1, 0);
+            // X: dims[s] x dims[s0]
+            struct Rec {
+                static void go(int pos, int s, std::vector<double> X, double wgt, int n, int pos_w, int kind, int s0,
+                               const ArcModel &m, const std::vector<int> &off, const std::vector<std::vector<double>> &prop,
+                               const std::vector<int> &arc_at, const std::vector<int> &is_head, const Topo &t,
+                               std::vector<int> &sel, const ArcBlocks &ob, const std::vector<std::vector<double>> &blocks,
+                               const std::function<double(int, int, int)> &arc, const std::function<int(int)> &pp,
+                               std::vector<double> &ref, double &leaves) {
+                    const int ms = m.dims[s], m0 = m.dims[s0];
+                    std::vector<double> Y(ms * m0, 0.0);
+                    for (int c = 0; c < m0; ++c)
+                        for (int i = 0; i < ms; ++i)
+                            for (int q = 0; q < ms; ++q) Y[i + c * ms] += prop[pos][off[s] + i + q * ms] * X[q + c * ms];
+                    if (pos == n) {
+                        if (s != s0) die("the test's model leaves its sector");
+                        leaves += 1;
+                        for (int i = 0; i < ms * m0; ++i) ref[off[s0] + i] += wgt * Y[i];
+                        return;
+                    }
+                    auto next = [&](int to, uint32_t blk, double w2) {
+                        std::vector<double> Z(m.dims[to] * m0, 0.0);
+                        for (int c = 0; c < m0; ++c)
+                            for (int i = 0; i < m.dims[to]; ++i)
+                                for (int q = 0; q < ms; ++q) Z[i + c * m.dims[to]] += blocks[blk][i + q * m.dims[to]] * Y[q + c * ms];
+                        go(pos + 1, to, Z, w2, n, pos_w, kind, s0, m, off, prop, arc_at, is_head, t, sel, ob, blocks, arc, pp, ref, leaves);
+                    };
+                    if (pos == pos_w) {
+                        if (kind == ARC_CORR) {
+                            if (m.a_sf[s] >= 0) next(m.a_sf[s], ob.a[s], wgt);
+                        } else {
+                            go(pos + 1, s, Y, wgt, n, pos_w, kind, s0, m, off, prop, arc_at, is_head, t, sel, ob, blocks, arc, pp, ref, leaves);
+                        }
+                        return;
+                    }
+                    const int a = arc_at[pos];
+                    if (is_head[pos]) {
+                        for (int p = 0; p < m.np; ++p)
+                            if (m.head_sf[p][s] >= 0) {
+                                sel[a] = p;
+                                next(m.head_sf[p][s], ob.head[p][s], wgt);
+                            }
+                    } else {
+                        const int p = sel[a];
+                        if (m.tail_sf[p][s] >= 0) next(m.tail_sf[p][s], ob.tail[p][s], wgt * arc(pp(t.p[a].second), pos, m.table[p]));
+                    }
+                }
+            };
+            int s1 = s0;
+            std::vector<double> X;
+            if (kind == ARC_CORR) {
+                if (m.b_sf[s0] < 0) continue;
+                s1 = m.b_sf[s0];
+                X = blocks[ob.b[s0]];
+            } else {
+                X.assign(m.dims[s0] * m.dims[s0], 0.0);
+                for (int i = 0; i < m.dims[s0]; ++i) X[i + i * m.dims[s0]] = 1.0;
+            }
+            Rec::go(2, s1, X, t.parity, n, pos_w, kind, s0, m, off, prop, arc_at, is_head, t, sel, ob, blocks,
+                    [&](int x, int y, int z) { return arc(x, y, z); }, [&](int x) { return point_pos(x); }, ref, leaves);
+        }
+    }
+    double dev = 0, mx = 0;
+    for (int i = 0; i < l.bt; ++i) {
+        dev = std::max(dev, std::fabs(res[i] - ref[i]));
+        mx = std::max(mx, std::fabs(ref[i]));
+    }
+    std::printf("dev %.3e leaves %.0f %.0f lds %zu segments %d\n", mx > 0 ? dev / mx : dev, pg.leaves, leaves, pg.lds, pg.n_segments);
+    return 0;
+}

@@ -1,0 +1,65 @@
+"""The arc walk (k_eval_arcs_t) on sector blocks at the edges of its instantiations (largest
+block 3, 8 | 16, 20 | 32), from one sample to several tasks per group, against the float64
+oracle.  Tolerances as in the other block tests: 1e-10 relative in float64 (sums of the same
+products in another order) and 2e-6 with float32 chain products."""
+import numpy as np
+import pytest
+
+import oracle_lib as O
+import qiw
+from qiw import abi, model
+
+pytestmark = pytest.mark.gpu
+
+
+def rel(a, b):
+    return np.linalg.norm((np.asarray(a) - np.asarray(b)).ravel()) / np.linalg.norm(np.asarray(b).ravel())
+
+
+def fermions(n_modes, key, n_tau=6):
+    """n_modes spinless levels with densities coupled and hopping between neighbours, every
+    second one on a bath; sectors by key(basis state)."""
+    fock = model.FockSpace(list(range(n_modes)))
+    H = sum((0.1 * i - 0.3) * fock.n(i) for i in range(n_modes))
+    for i in range(n_modes - 1):
+        H = H + 0.4 * fock.n(i) @ fock.n(i + 1)
+        t = fock.c_dag(i) @ fock.c(i + 1)
+        H = H + 0.2 * (t + t.T)
+    ed = model.EDCore(H, fock, key)
+    grid = model.ImaginaryTimeGrid(5.0, n_tau)
+    delta = 0.3 * model.bethe_gf(1.0, 5.0, grid)
+    pairs = []
+    for i in range(0, n_modes, 2):
+        pairs.append(model.InteractionPair(fock.c_dag(i), fock.c(i), delta))
+        pairs.append(model.InteractionPair(fock.c(i), fock.c_dag(i), model.ph_conj(delta)))
+    return model.Expansion(ed, grid, pairs, [(-fock.c(0), fock.c_dag(0))])
+
+
+def particles(b):
+    return bin(b).count("1")
+
+
+def parity(b):
+    return bin(b).count("1") & 1
+
+
+@pytest.mark.parametrize("precision", [abi.QIW_PREC_FP64, abi.QIW_PREC_FP32])
+@pytest.mark.parametrize("n_modes,key,order,log2n", [(3, particles, 3, 0), (4, parity, 2, 4), (5, parity, 2, 1),
+                                                     (6, particles, 1, 7), (6, parity, 1, 2), (3, particles, 4, 3),
+                                                     (3, particles, 5, 1)])
+def test_arc_walk(n_modes, key, order, log2n, precision):
+    eg, ec = fermions(n_modes, key), fermions(n_modes, key)
+    orders, N = range(0, order + 1), 2 ** log2n
+    tol = 1e-10 if precision == abi.QIW_PREC_FP64 else 2e-6
+    b_c, bo_c = O.inchworm_step_bare(ec, orders, N)
+    if precision == abi.QIW_PREC_FP64:
+        b_g, bo_g = qiw.inchworm_step_bare(eg, orders, N)
+        assert rel(b_g, b_c) < tol and np.abs(bo_g - bo_c).max() < tol * np.abs(b_c).max()
+    v_g, p_g = qiw.inchworm_step(eg, 2, orders, N, precision=precision)
+    v_c, p_c = O.inchworm_step(ec, orders, N, 2)
+    assert rel(v_g, v_c) < tol
+    assert np.abs(p_g - p_c).max() < tol * np.abs(v_c).max()
+    if order <= 3:
+        g_g = qiw.correlator_2p(eg, eg.grid, orders, N, precision=precision)[0]
+        g_c = O.correlator_2p(ec, orders, N)[0]
+        assert rel(g_g, g_c) < tol
