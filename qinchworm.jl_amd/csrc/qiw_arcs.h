@@ -622,4 +622,345 @@ inline int arc_compile(const ArcModel &m, const ArcLayout &l, const ArcBlocks &o
     return 0;
 }
 
+// ---------------------------------------------------------------------------------------
+// Device programs of the scalar arc walk (all sectors 1x1; k_eval_sarcs_t)
+// ---------------------------------------------------------------------------------------
+// A lane holds one sample; a workgroup of kScalarWaves wavefronts shares 64 samples.  Per
+// sample every factor of the diagrams is one row of a table in LDS: constants, arc values,
+// and propagators per segment and sector.  Each wavefront runs its own program: a state is
+// the sum over its joins (TERM words: accumulate source slot times a row), then its product
+// with the propagator that follows (STORE: destination slot = accumulator times a row).  The
+// states live in 64 registers slots, given out in the order a greedy schedule computes them
+// (the state that frees most sources first), so order 4 of the single-orbital model needs
+// 47 slots where its two widest neighbouring levels hold 120 states.
+//   word     bits 0-7 twice the slot, 9-17 row, 31 set for all but a positive TERM, 30 set
+//            for a negative TERM (clear: STORE)
+// Slots 0-7 are the results of initial sectors 0-7, slot 8 holds 1, slot 9 takes the padding.
+// The program of a group is a blob of 32-bit words, offsets relative to its start:
+//   0 constants, 1 their offset (float64 pairs; rows 0 ..), 2 arcs, 3 their offset,
+//   4 propagators, 5 their offset, 6 scaled rows, 7 their offset, 8-11 program offsets of the
+//   wavefronts, 12-15 their lengths in blocks of 16 words
+//   arc      head | tail << 8, then the rows of tables 0, 1 and 2, 3 (16 bits each, 0xFFFF none)
+//   prop     first row (one per sector), segment, second segment of a product (0: none)
+//   scaled   row, source row, constant row
+constexpr int kScalarWaves = 4, kScalarSlots = 64, kScalarFree = 10, kScalarRows = 300;
+constexpr uint32_t SARC_SPECIAL = 1u << 31, SARC_MINUS = 1u << 30;
+
+// Operator matrix elements of a scalar model.
+struct ArcValues {
+    std::vector<std::vector<double>> head, tail;  // [np][ns]
+    std::vector<double> a, b;                     // [ns]
+};
+
+struct ScalarProgram {
+    std::vector<uint32_t> blob;
+    double leaves = 0, words = 0;
+    int rows = 0;
+};
+
+struct ScalarPacker {
+    const ArcModel &m;
+    const ArcValues &val;
+    int kind, n, w_skipped;
+    std::vector<double> consts{1.0};
+    struct Arc {
+        uint32_t ends;
+        int row[4];
+    };
+    std::vector<Arc> arcs;
+    struct Scaled {
+        int row, src, c;
+    };
+    std::vector<Scaled> scaled;
+    // rows are numbered by kind first and placed when all are known
+    enum { R_CONST = 0, R_ARC = 1, R_PROP = 2, R_SCALED = 3 };
+    struct Row {
+        int kind, a, b;  // constant index | arc, table | slot, sector | scaled index
+    };
+    std::vector<Row> rows;
+    std::unordered_map<uint64_t, int> row_id;
+    int row(int k, int a, int b) {
+        const uint64_t key = ((uint64_t)k << 48) | ((uint64_t)(uint32_t)a << 16) | (uint32_t)b;
+        auto it = row_id.emplace(key, (int)rows.size());
+        if (it.second) rows.push_back(Row{k, a, b});
+        return it.first->second;
+    }
+    int const_row(double v) {
+        size_t i = std::find(consts.begin(), consts.end(), v) - consts.begin();
+        if (i == consts.size()) consts.push_back(v);
+        return row(R_CONST, (int)i, 0);
+    }
+    int arc_row(int head, int tail, int table) {
+        const uint32_t ends = (uint32_t)head | ((uint32_t)tail << 8);
+        size_t i = 0;
+        while (i < arcs.size() && arcs[i].ends != ends) ++i;
+        if (i == arcs.size()) arcs.push_back(Arc{ends, {-1, -1, -1, -1}});
+        return row(R_ARC, (int)i, table);
+    }
+    // segment index after position p as in ArcPacker (n - 2: the product), n - 1: the last
+    int slot_after(int p) const { return w_skipped && p + 1 == w_skipped ? n - 2 : p + 1 == n ? n - 1 : p - 1; }
+
+    struct Node {
+        std::vector<int> src;
+        std::vector<double> c;   // operator element and crossing sign
+        std::vector<int> base;   // row the coefficient multiplies (-1: none)
+        int prop, level;
+    };
+    struct Segment {
+        std::vector<uint32_t> words;  // rows by id in bits 9..
+        int s0;
+    };
+
+    // One initial sector: states in the greedy order, slots from the free list.  Returns
+    // false when the states need more slots than there are.
+    bool segment(const ArcGraph &g, Segment &out) {
+        std::vector<Node> node;
+        std::vector<std::vector<int>> id(g.levels.size());
+        for (size_t l = 0; l < g.levels.size(); ++l)
+            for (size_t i = 0; i < g.levels[l].size(); ++i) {
+                id[l].push_back((int)node.size());
+                const int p = l == 0 ? 1 : g.stages[l - 1].position;
+                const bool last = l + 1 == g.levels.size();
+                Node x;
+                x.level = (int)l;
+                x.prop = row(R_PROP, last ? n - 1 : slot_after(p), g.levels[l][i].sector);
+                node.push_back(x);
+            }
+        for (size_t s = 0; s < g.stages.size(); ++s)
+            for (const ArcJoin &j : g.stages[s].joins) {
+                const int ss = g.levels[s][j.src].sector;
+                double c = j.sign;
+                if (j.op == ARC_HEAD) c *= val.head[j.pair][ss];
+                if (j.op == ARC_TAIL) c *= val.tail[j.pair][ss];
+                if (j.op == ARC_A) c *= val.a[ss];
+                Node &d = node[id[s + 1][j.dst]];
+                d.src.push_back(id[s][j.src]);
+                d.c.push_back(c);
+                d.base.push_back(j.op == ARC_TAIL ? arc_row(j.head, g.stages[s].position, m.table[j.pair]) : -1);
+            }
+        const int N = (int)node.size();
+        // sign of each state as it is kept: the majority of its joins become positive
+        std::vector<double> sg(N, 1.0);
+        for (int i = 1; i + 1 < N; ++i) {
+            int plus = 0;
+            for (size_t q = 0; q < node[i].src.size(); ++q) plus += node[i].c[q] * sg[node[i].src[q]] > 0 ? 1 : -1;
+            if (plus < 0) sg[i] = -1.0;
+        }
+        std::vector<std::vector<int>> succ(N);
+        std::vector<int> pending(N, 0), uses(N, 0), slot(N, -1);
+        for (int i = 0; i < N; ++i) {
+            std::vector<int> u(node[i].src);
+            std::sort(u.begin(), u.end());
+            u.erase(std::unique(u.begin(), u.end()), u.end());
+            for (int p : u) {
+                succ[p].push_back(i);
+                ++uses[p];
+            }
+            pending[i] = (int)u.size();
+        }
+        std::vector<int> pool;
+        for (int i = kScalarSlots - 1; i >= kScalarFree; --i) pool.push_back(i);
+        auto put = [&](uint32_t flags, int sl, int r) {
+            out.words.push_back(flags | ((uint32_t)r << 9) | (uint32_t)(2 * sl));
+        };
+        auto coef = [&](double c, int base) {  // row of |c| times a row (a constant row without one)
+            c = c < 0 ? -c : c;
+            if (base < 0) return const_row(c);
+            if (c == 1.0) return base;
+            const int cr = const_row(c);
+            for (size_t i = 0; i < scaled.size(); ++i)
+                if (scaled[i].src == base && scaled[i].c == cr) return scaled[i].row;
+            const int r = row(R_SCALED, (int)scaled.size(), 0);
+            scaled.push_back(Scaled{r, base, cr});
+            return r;
+        };
+        auto store = [&](int i) {
+            if (i + 1 == N) {  // the closed state: the result of s0
+                slot[i] = g.s0;
+            } else {
+                if (pool.empty()) return false;
+                slot[i] = pool.back();
+                pool.pop_back();
+            }
+            put(SARC_SPECIAL, slot[i], node[i].prop);
+            return true;
+        };
+        const double b0 = kind == ARC_CORR ? val.b[g.s0] : 1.0;
+        put(b0 < 0 ? SARC_SPECIAL | SARC_MINUS : 0u, 8, coef(b0, -1));
+        if (!store(0)) return false;
+        std::vector<int> ready;
+        auto done = [&](int i) {
+            for (int q : succ[i])
+                if (--pending[q] == 0) ready.push_back(q);
+        };
+        done(0);
+        while (!ready.empty()) {
+            size_t best = 0;
+            int bf = -1, bl = -1;
+            for (size_t r = 0; r < ready.size(); ++r) {
+                const Node &x = node[ready[r]];
+                int f = 0;
+                for (size_t q = 0; q < x.src.size(); ++q)
+                    if (uses[x.src[q]] == 1 && std::find(x.src.begin(), x.src.begin() + q, x.src[q]) == x.src.begin() + q) ++f;
+                if (f > bf || (f == bf && x.level > bl)) {
+                    best = r;
+                    bf = f;
+                    bl = x.level;
+                }
+            }
+            const int i = ready[best];
+            ready.erase(ready.begin() + best);
+            const Node &x = node[i];
+            for (int neg = 0; neg < 2; ++neg)
+                for (size_t q = 0; q < x.src.size(); ++q) {
+                    const double c = x.c[q] * sg[x.src[q]] * sg[i];
+                    if ((c < 0) != (neg == 1)) continue;
+                    put(neg ? SARC_SPECIAL | SARC_MINUS : 0u, slot[x.src[q]], coef(c, x.base[q]));
+                }
+            for (size_t q = 0; q < x.src.size(); ++q)
+                if (std::find(x.src.begin(), x.src.begin() + q, x.src[q]) == x.src.begin() + q && --uses[x.src[q]] == 0)
+                    pool.push_back(slot[x.src[q]]);
+            if (!store(i)) return false;
+            done(i);
+        }
+        out.s0 = g.s0;
+        return true;
+    }
+};
+
+// Compiles a scalar group.  max_words: cut the graphs by the pairs of their first arcs until
+// a segment holds at most this many words (0: as few segments as fit).  Returns 0, 1 when a diagram ends outside its initial sector, or
+// 2 when the program does not fit the slots, the rows or the tables of the walk.
+inline int arc_compile_scalar(const ArcModel &m, const ArcValues &val, int kind, int order, int n_after, int max_words,
+                              ScalarProgram &out) {
+    out = ScalarProgram{};
+    const int n = kind == ARC_BARE ? 2 * order + 2 : 2 * order + 3;
+    const bool skip_w = kind == ARC_BOLD && order > 0;
+    const int pos_w = kind == ARC_BARE ? 0 : 2 * order - n_after + 2;
+    if (m.ns > 8) return 2;
+    for (int t : m.table)
+        if (t > 3) return 2;
+    for (int n_fixed = 0; n_fixed <= order; ++n_fixed) {
+        ScalarPacker pk{m, val, kind, n, skip_w ? pos_w : 0};
+        pk.const_row(1.0);
+        std::vector<ScalarPacker::Segment> segs;
+        double leaves = 0, total = 1;
+        std::vector<int> fix(n_fixed, 0);
+        for (int i = 0; i < n_fixed; ++i) total *= m.np;
+        bool fits = total <= 4096;
+        for (int s0 = 0; s0 < m.ns && fits; ++s0)
+            for (double c = 0; c < total && fits; ++c) {
+                long long r = (long long)c;
+                for (int i = 0; i < n_fixed; ++i) {
+                    fix[i] = (int)(r % m.np);
+                    r /= m.np;
+                }
+                ArcGraph g;
+                if (!arc_graph(m, kind, order, n_after, s0, fix, skip_w, g)) return 1;
+                if (g.levels.empty()) continue;
+                leaves += g.leaves;
+                size_t states = 0;
+                for (const auto &l : g.levels) states += l.size();
+                ScalarPacker::Segment sg;
+                if (states > 20000 || !pk.segment(g, sg))
+                    fits = false;
+                else
+                    segs.push_back(std::move(sg));
+            }
+        if (!fits) continue;
+        if (max_words > 0 && n_fixed < std::min(order, 2)) {
+            size_t longest = 0;
+            for (const auto &sg : segs) longest = std::max(longest, sg.words.size());
+            if (longest > (size_t)max_words) continue;
+        }
+        if (pk.rows.size() + m.ns > (size_t)kScalarRows) return 2;
+        // rows: constants, arcs, scaled rows, then one run of sectors per propagator segment
+        std::vector<int> at(pk.rows.size(), -1), prop_row(n + 1, -1);
+        int next = (int)pk.consts.size();
+        for (size_t i = 0; i < pk.rows.size(); ++i) {
+            const auto &r = pk.rows[i];
+            if (r.kind == ScalarPacker::R_CONST) at[i] = r.a;
+            if (r.kind == ScalarPacker::R_ARC) pk.arcs[r.a].row[r.b] = at[i] = next++;
+            if (r.kind == ScalarPacker::R_SCALED) at[i] = next++;
+        }
+        for (size_t i = 0; i < pk.rows.size(); ++i) {
+            const auto &r = pk.rows[i];
+            if (r.kind != ScalarPacker::R_PROP) continue;
+            if (prop_row[r.a] < 0) {
+                prop_row[r.a] = next;
+                next += m.ns;
+            }
+            at[i] = prop_row[r.a] + r.b;
+        }
+        if (next > kScalarRows) return 2;
+        std::vector<uint32_t> &b = out.blob;
+        b.assign(16, 0u);
+        b[0] = (uint32_t)pk.consts.size();
+        b[1] = (uint32_t)b.size();
+        for (double v : pk.consts) {
+            uint32_t w[2];
+            std::memcpy(w, &v, 8);
+            b.push_back(w[0]);
+            b.push_back(w[1]);
+        }
+        b[2] = (uint32_t)pk.arcs.size();
+        b[3] = (uint32_t)b.size();
+        auto half = [](int r) { return r < 0 ? 0xFFFFu : (uint32_t)r; };
+        for (const auto &a : pk.arcs) {
+            b.push_back(a.ends);
+            b.push_back(half(a.row[0]) | (half(a.row[1]) << 16));
+            b.push_back(half(a.row[2]) | (half(a.row[3]) << 16));
+        }
+        b[5] = (uint32_t)b.size();
+        for (int q = 0; q < n; ++q)
+            if (prop_row[q] >= 0) {
+                b[4]++;
+                b.push_back((uint32_t)prop_row[q]);
+                b.push_back((uint32_t)(q == n - 2 ? pos_w : q == n - 1 ? n : q + 2));
+                b.push_back((uint32_t)(q == n - 2 ? pos_w + 1 : 0));
+            }
+        b[6] = (uint32_t)pk.scaled.size();
+        b[7] = (uint32_t)b.size();
+        for (const auto &sc : pk.scaled) {
+            b.push_back((uint32_t)at[sc.row]);
+            b.push_back((uint32_t)at[sc.src]);
+            b.push_back((uint32_t)at[sc.c]);
+        }
+        // segments to wavefronts, longest first to the least loaded
+        std::vector<size_t> ord(segs.size());
+        for (size_t i = 0; i < ord.size(); ++i) ord[i] = i;
+        std::stable_sort(ord.begin(), ord.end(), [&](size_t x, size_t y) { return segs[x].words.size() > segs[y].words.size(); });
+        std::vector<std::vector<uint32_t>> prog(kScalarWaves);
+        std::vector<std::vector<char>> seen(kScalarWaves, std::vector<char>(8, 0));
+        for (size_t i : ord) {
+            int w = 0;
+            for (int q = 1; q < kScalarWaves; ++q)
+                if (prog[q].size() < prog[w].size()) w = q;
+            std::vector<uint32_t> ws = segs[i].words;
+            for (uint32_t &x : ws) x = (x & ~(0x1FFu << 9)) | ((uint32_t)at[(x >> 9) & 0x1FFu] << 9);
+            const int s0 = segs[i].s0;
+            if (seen[w][s0]) {  // add to the sector's result of this wavefront
+                ws.back() = (ws.back() & ~0xFFu) | (2u * 9u);
+                ws.push_back(2u * 9u);
+                ws.push_back(2u * (uint32_t)s0);
+                ws.push_back(SARC_SPECIAL | 2u * (uint32_t)s0);
+            }
+            seen[w][s0] = 1;
+            prog[w].insert(prog[w].end(), ws.begin(), ws.end());
+        }
+        for (int w = 0; w < kScalarWaves; ++w) {
+            out.words += (double)prog[w].size();
+            while (b.size() % 16) b.push_back(0);
+            while (prog[w].size() % 16) prog[w].push_back(SARC_SPECIAL | 2u * 9u);
+            b[8 + w] = (uint32_t)b.size();
+            b[12 + w] = (uint32_t)(prog[w].size() / 16);
+            b.insert(b.end(), prog[w].begin(), prog[w].end());
+        }
+        out.leaves = leaves;
+        out.rows = next;
+        return 0;
+    }
+    return 2;
+}
+
 }  // namespace qiwi

@@ -213,9 +213,9 @@ int load_scalar_op(qiw_ctx *c, const qiw_sbm &in, const std::vector<int> &dims, 
 // ---------------------------------------------------------------------------------------
 enum NodeKind { N_PAIR_HEAD, N_PAIR_TAIL, N_IDENTITY, N_OPERATOR };
 
-// Program formats: the scalar structured walk, the LDS block walk, the vector walk, the arc
-// walk (sector blocks).
-enum ProgFormat { FMT_SCALAR = 0, FMT_BLOCK = 1, FMT_VEC = 2, FMT_ARC = 3 };
+// Program formats: the walks of the assignment tries (scalar, LDS block, vector), and the arc
+// walks (sector blocks, scalar).
+enum ProgFormat { FMT_SCALAR = 0, FMT_BLOCK = 1, FMT_VEC = 2, FMT_ARC = 3, FMT_SARC = 4 };
 
 // Format of the assignment tries.  Vector programs also drive the matrix-core walk of wide
 // blocks (float32 chain products).
@@ -226,11 +226,11 @@ int program_format(const HostModel &m, int max_order, int precision) {
     return FMT_BLOCK;
 }
 
-// Models with sector blocks run the arc walk wherever its states fit a CU's LDS
-// (compile_group), and the assignment tries otherwise.
+// Models run the arc walks wherever the states of their groups fit (a CU's LDS; the slots
+// and rows of the scalar walk; compile_group), and the assignment tries otherwise.
 int eval_format(const HostModel &m, int max_order, int precision) {
     const int fmt = program_format(m, max_order, precision);
-    return fmt == FMT_SCALAR || m.ns > 255 ? fmt : FMT_ARC;
+    return fmt == FMT_SCALAR ? FMT_SARC : m.ns > 255 ? fmt : FMT_ARC;
 }
 
 // Stride of the W slots: the table count of the register walk instantiation that runs the
@@ -258,6 +258,7 @@ struct Compiled {
     // arc programs: initial-sector segments, wavefronts and LDS bytes of a workgroup
     int n_segments = 0, waves = 1;
     size_t lds_bytes = 0;
+    int rows = 0;  // scalar arc programs: rows of the LDS table
     int replica_of = -1;  // randomized qMC: another sequence of group `replica_of` (no program of its own)
 };
 
@@ -676,6 +677,28 @@ double sample_flops(const Compiled &cg) {
     return 2.0 * cg.edges_per_sample + 2.0 * cg.leaves_per_sample;
 }
 
+// The group record and program of an arc-compiled group.
+void set_arc_group(const HostModel &m, int kind, int order, int n_after, std::vector<uint32_t> &blob, Compiled &out) {
+    const int d_after = (kind == QIW_G_BARE) ? 2 * order : (kind == QIW_G_SIGMA) ? 0 : n_after;
+    out.n_top = (int)((kind == QIW_G_BARE)    ? topologies_at_order(order, -1, false)
+                      : (kind == QIW_G_SIGMA) ? topologies_at_order(order, 1, false)
+                                              : topologies_at_order(order, n_after, false))
+                    .size();
+    if (blob.size() % 2) blob.push_back(0);
+    out.prog.resize(blob.size() / 2);
+    std::memcpy(out.prog.data(), blob.data(), blob.size() * 4);
+    QiwGroup &g = out.g;
+    g.kind = kind;
+    g.order = order;
+    g.n_after = d_after;
+    g.n_nodes = kind == QIW_G_BARE ? 2 * order + 2 : 2 * order + 3;
+    g.d_before = 2 * order - d_after;
+    g.d_after = d_after;
+    g.pos_w = kind == QIW_G_BARE ? 0 : g.d_before + 2;
+    g.n_pslots = (g.n_nodes - 1) * m.ns;
+    g.n_wslots = order * qiw_vec_tm(m.ntab);
+}
+
 // Compiles a group as an arc program.  Returns 0, 1 when a diagram ends outside its initial
 // sector, 2 when the states do not fit.
 int compile_arcs(const HostModel &m, int kind, int order, int n_after, int corr, int precision, Compiled &out) {
@@ -707,37 +730,44 @@ int compile_arcs(const HostModel &m, int kind, int order, int n_after, int corr,
             if (rc != 2) break;
         }
     if (rc) return rc;
-    const int d_after = (kind == QIW_G_BARE) ? 2 * order : (kind == QIW_G_SIGMA) ? 0 : n_after;
-    out.n_top = (int)((kind == QIW_G_BARE)    ? topologies_at_order(order, -1, false)
-                      : (kind == QIW_G_SIGMA) ? topologies_at_order(order, 1, false)
-                                              : topologies_at_order(order, n_after, false))
-                    .size();
-    if (pg.blob.size() % 2) pg.blob.push_back(0);
-    out.prog.resize(pg.blob.size() / 2);
-    std::memcpy(out.prog.data(), pg.blob.data(), pg.blob.size() * 4);
+    set_arc_group(m, kind, order, n_after, pg.blob, out);
     out.n_segments = pg.n_segments;
     out.waves = l.waves;
     out.lds_bytes = pg.lds;
     out.leaves_per_sample = (int64_t)pg.leaves;
     out.edges_per_sample = (int64_t)pg.joins;
     out.flops_per_sample = pg.flops;
-    QiwGroup &g = out.g;
-    g.kind = kind;
-    g.order = order;
-    g.n_after = d_after;
-    g.n_nodes = kind == QIW_G_BARE ? 2 * order + 2 : 2 * order + 3;
-    g.d_before = 2 * order - d_after;
-    g.d_after = d_after;
-    g.pos_w = kind == QIW_G_BARE ? 0 : g.d_before + 2;
-    g.n_pslots = (g.n_nodes - 1) * m.ns;
-    g.n_wslots = order * qiw_vec_tm(m.ntab);
     return 0;
 }
 
-// LDS doubles of one evaluator wavefront.  Scalar programs keep their state in registers;
+// Compiles a group of a scalar model as an arc program.  Returns as compile_arcs.
+int compile_scalar_arcs(const HostModel &m, int kind, int order, int n_after, int corr, int max_words, Compiled &out) {
+    ArcValues v;
+    for (int p = 0; p < m.np; ++p) {
+        v.head.push_back(m.op_i[p].val);
+        v.tail.push_back(m.op_f[p].val);
+    }
+    if (corr >= 0) {
+        v.a = m.corr_A[corr].val;
+        v.b = m.corr_B[corr].val;
+    }
+    ScalarProgram sp;
+    const int rc = arc_compile_scalar(arc_model(m, corr), v, kind, order, n_after, max_words, sp);
+    if (rc) return rc;
+    set_arc_group(m, kind, order, n_after, sp.blob, out);
+    out.rows = sp.rows;
+    out.leaves_per_sample = (int64_t)sp.leaves;
+    out.edges_per_sample = (int64_t)sp.words;
+    out.flops_per_sample = 2.0 * sp.words;
+    return 0;
+}
+
+// LDS doubles of one evaluator workgroup or wavefront.  Scalar trie programs keep their state in registers;
 // block programs hold per-sample state shared by the lanes (iP slots, W slots, stack, X,
 // acc, out).
-int lds_slots(const QiwGroup &g, const HostModel &m, int fmt) {
+int lds_slots(const Compiled &cg, const HostModel &m, int fmt) {
+    const QiwGroup &g = cg.g;
+    if (fmt == FMT_SARC) return std::max(cg.rows, 32) * QIW_WAVE;  // at least the results of the wavefronts
     if (fmt != FMT_BLOCK) return 0;  // register-resident walks
     int mm = m.mmax * m.mmax;
     return (g.n_nodes - 1) * m.bt + g.n_wslots + 1 + (g.n_nodes + 1) * mm + 2 * mm + m.bt;
@@ -815,7 +845,7 @@ int upload(qiw_ctx *c, const std::string &tag, Batch &b, int64_t N, DevBatch &d,
     std::vector<QiwGroup> gs;
     // END words between and after the programs (never executed: prefetch and alignment)
     const uint64_t end_fl = (uint64_t)QIW_FL_OP_END << 28;
-    const uint64_t pad = b.fmt == FMT_ARC      ? 0ull
+    const uint64_t pad = b.fmt >= FMT_ARC      ? 0ull
                          : b.fmt == FMT_SCALAR ? (end_fl | (end_fl << 32))
                                                : (uint64_t)QIW_OP_END << 48;
     int64_t ut_total = 0, ps_total = 0;
@@ -1282,7 +1312,7 @@ static int ystack_rows(const HostModel &m, int levels) {
 // tasks are cut smaller until a launch holds at least 4 tasks per SIMD of the device.
 // The arc walk takes a workgroup per sample: its tasks are cut until a launch holds 4096.
 int samples_per_task(const qiw_ctx *c, const HostModel &m, int fmt, int64_t total_samples) {
-    if (fmt == FMT_SCALAR || (fmt == FMT_VEC && m.mmax <= 6)) return QIW_WAVE;
+    if (fmt == FMT_SCALAR || fmt == FMT_SARC || (fmt == FMT_VEC && m.mmax <= 6)) return QIW_WAVE;
     if (c->tune.samples_per_task > 0) return c->tune.samples_per_task;
     int spt = QIW_WAVE;
     while (spt > 1 && total_samples / spt < 4096) spt /= 2;
@@ -1326,6 +1356,10 @@ int compile_group(qiw_ctx *c, const Batch &b, int kind, int order, int n_after, 
                   int64_t chunk_cost, Compiled &cg) {
     if (b.fmt == FMT_ARC) {
         const int rc = compile_arcs(c->m, kind, order, n_after, corr, b.precision, cg);
+        return rc == 1 ? fail(c, QIW_E_OFFDIAG, kOffDiagonal) : rc == 2 ? kArcNoFit : 0;
+    }
+    if (b.fmt == FMT_SARC) {
+        const int rc = compile_scalar_arcs(c->m, kind, order, n_after, corr, c->tune.chunk_words, cg);
         return rc == 1 ? fail(c, QIW_E_OFFDIAG, kOffDiagonal) : rc == 2 ? kArcNoFit : 0;
     }
     Compiler comp(c->m, kind, order, n_after, corr, b.fmt, b.max_order);
@@ -1395,7 +1429,7 @@ int build_step_batch_as(qiw_ctx *c, const qiw_run *run, bool bare, const std::ve
             if (cg.n_top == 0) continue;
             if (cg.g.n_wslots > 255 || m.ns > 255)
                 return fail(c, QIW_E_LIMIT, "too many slots");
-            b.lds = std::max(b.lds, lds_slots(cg.g, m, b.fmt));
+            b.lds = std::max(b.lds, lds_slots(cg, m, b.fmt));
             int slot = (int)(std::find(oall.begin(), oall.end(), order) - oall.begin());
             int64_t N = order > 0 ? run->N_samples : 1;
             const auto parts = task_parts(b, cg, split && total / b.spt < 2048);
@@ -1661,6 +1695,10 @@ int launch_eval(qiw_ctx *c, const EvalArgs &a, const Batch &batch) {
     }
     const size_t lds_bytes = (size_t)a.lds_slots * sizeof(double);
     if (lds_bytes > 160 * 1024) return fail(c, QIW_E_LIMIT, "evaluator state exceeds the 160 KiB of LDS of a CU");
+    if (fmt == FMT_SARC) {
+        HIPCHK(c, qiw_launch_eval_sarcs(c->stream, a, n_tasks));
+        return 0;
+    }
     if (fmt == FMT_SCALAR) {
         HIPCHK(c, qiw_launch_eval_flat(c->stream, a, n_tasks, a.max_order, m.ns, m.ntab));
         return 0;
@@ -2365,7 +2403,7 @@ int run_inchworm(qiw_ctx *c, const qiw_run *run, bool do_bare, int first_w, int 
             ArcArgs aa{};
             if ((rc = stage_arcs(c, bold_b.precision, &aa))) return rc;
         }
-        const bool staged = bold_b.fmt == FMT_SCALAR || bold_b.fmt == FMT_ARC ||
+        const bool staged = bold_b.fmt == FMT_SCALAR || bold_b.fmt == FMT_ARC || bold_b.fmt == FMT_SARC ||
                             (bold_b.fmt == FMT_VEC && (m.mmax > 6 ? c->mfma_staged : c->vec_staged));
         bool graph = c->graphs && staged && !warped && !c->no_alloc && !rq.given;
         const int n_known_start = n_known;
@@ -2591,7 +2629,7 @@ int build_diff_batch_as(qiw_ctx *c, const qiw_run *run, Batch &b, bool arcs) {
         if (rc) return rc;
         if (cg.n_top == 0) continue;
         if (cg.g.n_wslots > 255 || m.ns > 255) return fail(c, QIW_E_LIMIT, "too many slots");
-        b.lds = std::max(b.lds, lds_slots(cg.g, m, b.fmt));
+        b.lds = std::max(b.lds, lds_slots(cg, m, b.fmt));
         const int64_t N = order == 1 ? 1 : run->N_samples;
         const auto parts = task_parts(b, cg, total / b.spt < 2048);
         const double flops = (double)N * sample_flops(cg);
@@ -2906,7 +2944,7 @@ int build_corr_groups_as(qiw_ctx *c, const qiw_run *run, int ci, Batch &b, bool 
             if (rc) return rc;
             if (cg.n_top == 0) continue;
             if (b.groups.empty() && order == 0) *first_is_order0 = true;
-            b.lds = std::max(b.lds, lds_slots(cg.g, m, b.fmt));
+            b.lds = std::max(b.lds, lds_slots(cg, m, b.fmt));
             push_sequences(b, std::move(cg), b.n_eval, [](int) {});
         }
     }
@@ -3369,7 +3407,7 @@ static int qiw_autotune_impl(qiw_ctx *c, const qiw_run *run, qiw_tuning *out) {
     for (int i = 0; i < run->n_orders; ++i) max_order = std::max(max_order, (int)run->orders[i]);
     const int fmt = eval_format(m, max_order, run->precision);
     std::vector<qiw_tuning> cand;
-    if (fmt == FMT_SCALAR) {
+    if (fmt == FMT_SCALAR || fmt == FMT_SARC) {
         for (int w : {256, 384, 512, 640, 896, 1024, 2048}) cand.push_back(qiw_tuning{w, 0, 0, 0, 0, 0.0});
     } else if (fmt == FMT_VEC && m.mmax <= 6) {
         for (int e = 16; e <= 20; ++e) cand.push_back(qiw_tuning{0, 0, (int64_t)1 << e, 0, 0, 0.0});

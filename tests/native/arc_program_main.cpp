@@ -2,7 +2,8 @@
 // reads them, with every access checked, against the plain sum over topologies and pair
 // assignments.  Arguments: kind order n_after n_fixed waves cap_bytes elem modes seed [largest block, 5].
 // The model: `modes` fermionic modes, one sector per particle number with random dimensions,
-// random operator blocks, propagators and arc values.  Prints the largest deviation relative
+// random operator blocks, propagators and arc values.  elem 0: the scalar program (blocks 1x1;
+// n_fixed > 0: cut into as many segments as it can be).  Prints the largest deviation relative
 // to the largest element, and the count of diagrams of the program and of the plain sum.
 #include <cmath>
 #include <cstdio>
@@ -125,8 +126,84 @@ int main(int argc, char **argv) {
         return it->second;
     };
 
-    // ---- the program ----
+    std::vector<double> res(l.bt, 0.0), ref(l.bt, 0.0);
     ArcGroupProgram pg;
+    if (elem == 0) {  // the scalar program (all blocks 1x1), read as the scalar walk reads it
+        ArcValues val;
+        auto pick = [&](const std::vector<uint32_t> &v) {
+            std::vector<double> x;
+            for (uint32_t b : v) x.push_back(b == ARC_NONE ? 0.0 : blocks[b][0]);
+            return x;
+        };
+        for (int p = 0; p < m.np; ++p) {
+            val.head.push_back(pick(ob.head[p]));
+            val.tail.push_back(pick(ob.tail[p]));
+        }
+        val.a = pick(ob.a);
+        val.b = pick(ob.b);
+        ScalarProgram sp;
+        const int rc = arc_compile_scalar(m, val, kind, order, n_after, n_fixed ? 1 : 0, sp);
+        if (rc) {
+            std::printf("rc %d\n", rc);
+            return 0;
+        }
+        const std::vector<uint32_t> &b = sp.blob;
+        auto at = [&](size_t i) -> uint32_t {
+            if (i >= b.size()) die("word out of the program");
+            return b[i];
+        };
+        if (sp.rows > 300) die("rows");
+        std::vector<double> tab(sp.rows, NAN);
+        auto set = [&](uint32_t r, double v) {
+            if (r >= tab.size() || !std::isnan(tab[r])) die("row");
+            tab[r] = v;
+        };
+        for (uint32_t i = 0; i < at(0); ++i) {
+            const uint32_t w[2] = {at(at(1) + 2 * i), at(at(1) + 2 * i + 1)};
+            double v;
+            std::memcpy(&v, w, 8);
+            set(i, v);
+        }
+        for (uint32_t i = 0; i < at(2); ++i)
+            for (int q = 0; q < 4; ++q) {
+                const uint32_t r = (at(at(3) + 3 * i + 1 + q / 2) >> (16 * (q & 1))) & 0xFFFF;
+                const uint32_t e = at(at(3) + 3 * i);
+                if (r != 0xFFFF) set(r, arc(e & 255, e >> 8, q));
+            }
+        for (uint32_t i = 0; i < at(4); ++i)
+            for (int s = 0; s < m.ns; ++s) {
+                const uint32_t L = at(at(5) + 3 * i + 1), L2 = at(at(5) + 3 * i + 2);
+                if (L < 2 || L > (uint32_t)n || L2 > (uint32_t)n) die("segment");
+                set(at(at(5) + 3 * i) + s, prop[L][s] * (L2 ? prop[L2][s] : 1.0));
+            }
+        for (uint32_t i = 0; i < at(6); ++i)
+            set(at(at(7) + 3 * i), tab.at(at(at(7) + 3 * i + 1)) * tab.at(at(at(7) + 3 * i + 2)));
+        for (int w = 0; w < kScalarWaves; ++w) {
+            if (at(8 + w) % 16 && at(12 + w)) die("program alignment");
+            std::vector<double> slot(kScalarSlots, NAN);
+            for (int s = 0; s < 8; ++s) slot[s] = 0.0;
+            slot[8] = 1.0;
+            slot[9] = 0.0;
+            double acc = 0.0;
+            for (uint32_t i = 0; i < 16 * at(12 + w); ++i) {
+                const uint32_t x = at(at(8 + w) + i), sl = (x & 255) / 2, r = (x >> 9) & 511;
+                if ((x & 1) || (x & 256) || sl >= (uint32_t)kScalarSlots || r >= tab.size() || std::isnan(tab[r])) die("word");
+                if ((x & SARC_SPECIAL) && !(x & SARC_MINUS)) {
+                    if (sl == 8) die("the constant slot is written");
+                    slot[sl] = acc * tab[r];
+                    acc = 0.0;
+                } else {
+                    if (std::isnan(slot[sl])) die("slot read before it is written");
+                    acc += (x & SARC_SPECIAL ? -1.0 : 1.0) * slot[sl] * tab[r];
+                }
+            }
+            for (int s = 0; s < m.ns; ++s) res[s] += slot[s];
+        }
+        pg.leaves = sp.leaves;
+        pg.n_segments = (int)sp.words;
+        pg.lds = (size_t)sp.rows * 512;
+    } else {
+    // ---- the program ----
     const int rc = arc_compile(m, l, ob, kind, order, n_after, n_fixed, pg);
     if (rc) {
         std::printf("rc %d\n", rc);
@@ -161,7 +238,6 @@ int main(int argc, char **argv) {
                         v += prop[at(2) + 1][off[s] + i + q * m.dims[s]] * prop[at(2)][off[s] + q + j * m.dims[s]];
                     pl[(size_t)(n - 2) * l.bt + off[s] + i + j * m.dims[s]] = v;
                 }
-    std::vector<double> res(l.bt, 0.0), ref(l.bt, 0.0);
     for (uint32_t sg = 0; sg < at(0); ++sg) {
         const size_t h = at(kArcGroupHead + sg);
         const int s0 = at(h) & 255, m0 = (at(h) >> 8) & 255, lg = at(h) >> 16, cg = 1 << lg;
@@ -261,6 +337,8 @@ int main(int argc, char **argv) {
                         res[off[s0] + i + (c0 + col) * m0] += prop[n][off[s0] + i + q * m0] * x[q];
             }
         }
+    }
+
     }
 
     // ---- the plain sum ----

@@ -63,3 +63,28 @@ def test_arc_walk(n_modes, key, order, log2n, precision):
         g_g = qiw.correlator_2p(eg, eg.grid, orders, N, precision=precision)[0]
         g_c = O.correlator_2p(ec, orders, N)[0]
         assert rel(g_g, g_c) < tol
+
+
+@pytest.mark.parametrize("log2n", [0, 6, 7])
+@pytest.mark.parametrize("which,order", [("level", 6), ("orbital", 4), ("orbital", 1)])
+def test_scalar_arc_walk(which, order, log2n):
+    """The scalar arc walk (k_eval_sarcs_t) at its largest and smallest programs, one lane,
+    one block and two blocks of samples, programs in few and in many segments."""
+    make = (lambda: model.bethe_single_level(6)) if which == "level" else \
+        (lambda: model.anderson_single_orbital(n_tau=6, with_correlators=True))
+    eg, ec = make(), make()
+    orders, N = range(0, order + 1), 2 ** log2n
+    for words in (0, 64):
+        qiw.set_tuning(chunk_words=words)
+        try:
+            b_g, _ = qiw.inchworm_step_bare(eg, range(0, min(order, 4) + 1), N)
+            v_g, p_g = qiw.inchworm_step(eg, 2, orders, N)
+            g_g = qiw.correlator_2p(eg, eg.grid, range(0, min(order, 3) + 1), N)
+        finally:
+            qiw.set_tuning()
+        b_c, _ = O.inchworm_step_bare(ec, range(0, min(order, 4) + 1), N)
+        v_c, p_c = O.inchworm_step(ec, orders, N, 2)
+        assert rel(b_g, b_c) < 1e-10 and rel(v_g, v_c) < 1e-10
+        assert np.abs(p_g - p_c).max() < 1e-10 * np.abs(v_c).max()
+        for x, y in zip(g_g, O.correlator_2p(ec, range(0, min(order, 3) + 1), N)):
+            assert rel(x, y) < 1e-10
