@@ -260,20 +260,37 @@ inline bool arc_graph(const ArcModel &m, int kind, int order, int n_after, int s
 //            3 offset of the arc list, 4-7 byte offsets in LDS of the closed state's columns,
 //            the arc values, the propagators and the states, 8.. offsets of the segments
 //   arc      head position | tail position << 8 | table << 16
-//   segment  0 s0 | m0 << 8 | lg << 16, 1 stages, 2 root sector dimension | stride << 8,
-//            3 root operator block (offset, ARC_NONE: identity), 4 root propagator offset,
-//            5 root state offset, 6 parts of the closed state, 7 offset of their list,
-//            8.. per stage: tiles, offset of the tile records
-//   tile     0 operators | rows << 8 | states << 16 | stride << 24, 1 state offset,
-//            2 propagator offset (ARC_NONE: none), 3 offset of the operator records
-//   operator 0 block (offset, ARC_NONE: identity), 1 rows of the source | stride << 8 |
-//            joins per state << 16, 2 offset of the join words
-//   join     source state offset | index of the arc value << 20
+//   segment  0 s0 | m0 << 8 | lg << 16, 1 root sector dimension | stride << 8, 2 root operator
+//            block (offset, ARC_NONE: identity), 3 root propagator offset (ARC_NONE: none),
+//            4 root state offset, 5 parts of the closed state, 6 offset of their list,
+//            8.. of each wavefront the offsets of its records and of its joins
+// A wavefront reads two streams without a gap, in packets of ArcLayout::slots slots, so that
+// all a packet needs is read while the one before it is at work.  A slot is one or two steps
+// of joins, and what its flags say after them; the slots of a tile follow each other.
+// Records, 8 words per slot:
+//   0 flags, 1 rows | stride << 8 | stride of the source << 16 (a stride is the number of rows
+//   that a product computes),
+//   2 operator block (offset), 3 state offset, 4 propagator offset (ARC_NONE: none), 5 states,
+//   6 (first slot of a packet) set when the packet has a second block of joins
+// Joins: blocks of slots x (64 >> lg) words, the slots of a state side by side, one block per
+// packet for the first steps and one for the second steps where a slot has one:
+//   word     LDS byte address of the source state / 4 | index of the arc value << 20
 // Offsets of states and propagators are in elements of the value type.  The arc values are
-// 0: 0, 1: 1, then +v, -v of each arc in turn.  Joins are stored [join][state of the tile];
-// a state with fewer joins than its tile is filled up with value 0.
+// 0: 0, 1: 1, then +v, -v of each arc in turn.  A state with fewer joins than its tile is
+// filled up with value 0.
 constexpr uint32_t ARC_NONE = 0xFFFFFFFFu;
-constexpr int kArcGroupHead = 8, kArcSegHead = 8;
+// Flags of a slot: a barrier before it; the end of the segment; no joins; a second step; the
+// product of the sum of joins with the block; the tile's end: propagator, store.  Without a
+// product the next slot's joins continue the sum.
+enum : uint32_t { ARC_BARRIER = 1, ARC_END = 2, ARC_IDLE = 4, ARC_SECOND = 8, ARC_TIMES = 16, ARC_STORE = 32 };
+constexpr size_t kArcValuesAt = 128;  // LDS offset of the arc values, past 16 times
+constexpr int kArcGroupHead = 8, kArcSegHead = 8, kArcSlotWords = 8;
+constexpr int kArcTileOps = 28;          // most operators of a tile
+constexpr int kArcReadAhead = 6 * 256;   // words a wavefront may read past its streams
+
+// Slots of a packet of the walk whose lanes hold vectors of `rows` values: as many as their
+// blocks fit in registers twice.
+constexpr int arc_slots(int rows, bool fp32) { return fp32 && rows <= 8 ? 4 : rows <= 8 || (fp32 && rows <= 20) ? 2 : 1; }
 
 struct ArcLayout {
     int elem = 4;             // bytes of the value type
@@ -281,6 +298,7 @@ struct ArcLayout {
     int bt = 0;               // elements of one segment's propagator blocks
     std::vector<int> bt_off;  // [ns]
     int waves = 1;            // wavefronts of the workgroup
+    int slots = 4;            // slots of a packet
     size_t cap = 0;           // LDS bytes of the workgroup
 };
 
@@ -291,17 +309,17 @@ inline int arc_stride(int m, int mmax) {
     return mmax > 8 || m > 6 ? (m + 3) & ~3 : m == 1 ? 1 : (m + 1) & ~1;
 }
 
-// LDS of a group in bytes: the times of the positions, the closed state's columns, the arc
-// values, the propagators of n - 2 segments and one product, then the states.
+// LDS of a group in bytes: the times of the positions, the arc values, the closed state's
+// columns, the propagators of n - 2 segments and one product, then the states.
 struct ArcLds {
     size_t fin, arcs, prop, states;
 };
 inline ArcLds arc_lds(const ArcLayout &l, int n, int n_arcs, int m0) {
     auto up = [](size_t b) { return (b + 15) & ~(size_t)15; };
     ArcLds r;
-    r.fin = 16 * 8;
-    r.arcs = r.fin + up((size_t)m0 * m0 * 8);
-    r.prop = r.arcs + up((size_t)(2 + 2 * n_arcs) * l.elem);
+    r.arcs = kArcValuesAt;
+    r.fin = r.arcs + up((size_t)(2 + 2 * n_arcs) * l.elem);
+    r.prop = r.fin + up((size_t)m0 * m0 * 8);
     r.states = r.prop + up((size_t)(n - 1) * l.bt * l.elem);
     return r;
 }
@@ -319,6 +337,7 @@ struct ArcGroupProgram {
 struct ArcBlocks {
     std::vector<std::vector<uint32_t>> head, tail;  // [np][ns]
     std::vector<uint32_t> a, b;                     // [ns]
+    uint32_t id = 0;                                // the identity
 };
 
 struct ArcPacker {
@@ -341,21 +360,59 @@ struct ArcPacker {
 
     struct Tile {
         int sector;
-        std::vector<int> states;  // indices in the level
+        std::vector<int> states;  // indices in the level (one state `spread` times over)
+        int spread = 1;           // the joins of a state are dealt over this many lanes
         std::vector<int> ops;     // keys (op << 16 | pair) this tile sums
+        std::vector<int> steps;   // of each operator
     };
 
-    // states of a level in tiles, with the offsets of every state's parts
+    struct Slot {
+        std::array<uint32_t, kArcSlotWords> head{};
+        std::vector<uint32_t> first, second;  // join words, one per state of the tile
+        static Slot idle(uint32_t flags, int per) {
+            Slot s;
+            s.head[0] = flags;
+            s.first.assign(per, 0u);
+            return s;
+        }
+    };
+
+    // States of a level in tiles, with the offsets of every state's parts.
     struct Placed {
         std::vector<Tile> tiles;
+        std::vector<int> slots;  // of each tile
         std::vector<size_t> tile_off;
         std::vector<std::vector<size_t>> parts;  // [state] offsets
         size_t size = 0;
-    };
 
-    Placed place(const std::vector<ArcState> &lev, const ArcStage &st, int lg) const {
-        const int per = 64 >> lg, cg = 1 << lg;
-        std::vector<std::vector<int>> ops_of(lev.size());
+        std::vector<int> part_counts() const {
+            std::vector<int> n;
+            for (const auto &v : parts) n.push_back((int)v.size());
+            return n;
+        }
+        // wavefronts of the tiles, longest first to the least loaded; returns the largest load
+        double deal(int waves, std::vector<int> *wave) const {
+            std::vector<int> ord(tiles.size());
+            for (size_t i = 0; i < ord.size(); ++i) ord[i] = (int)i;
+            std::stable_sort(ord.begin(), ord.end(), [&](int x, int y) { return slots[x] > slots[y]; });
+            std::vector<double> load(waves, 0.0);
+            if (wave) wave->assign(tiles.size(), 0);
+            for (int i : ord) {
+                const int w = (int)(std::min_element(load.begin(), load.end()) - load.begin());
+                load[w] += kTileCost + slots[i];
+                if (wave) (*wave)[i] = w;
+            }
+            return *std::max_element(load.begin(), load.end());
+        }
+    };
+    static constexpr double kTileCost = 0.5, kStageCost = 2.0;  // propagator and store, barrier; in slots
+
+    // The tiles of a stage before their operators are cut: n_src parts of each source state;
+    // spread: deal the joins of the closed state over lanes.
+    std::vector<Tile> tiles_of(const std::vector<ArcState> &lev, const ArcStage &st, int lg, const std::vector<int> &n_src,
+                               bool spread, std::vector<std::vector<int>> &ops_of) const {
+        const int per = 64 >> lg;
+        ops_of.assign(lev.size(), {});
         for (const ArcJoin &x : st.joins) {
             const int key = (x.op << 16) | x.pair;
             auto &v = ops_of[x.dst];
@@ -375,7 +432,7 @@ struct ArcPacker {
             if (hx != hy) return hx < hy;
             return lev[x] < lev[y];
         });
-        Placed p;
+        std::vector<Tile> tiles;
         for (size_t i = 0; i < ord.size();) {
             Tile t;
             t.sector = lev[ord[i]].sector;
@@ -387,25 +444,61 @@ struct ArcPacker {
                 for (int key : ops_of[s])
                     if (std::find(t.ops.begin(), t.ops.end(), key) == t.ops.end()) t.ops.push_back(key);
             std::sort(t.ops.begin(), t.ops.end());
-            p.tiles.push_back(t);
+            tiles.push_back(t);
         }
-        // a stage with fewer tiles than wavefronts: cut the tiles' operator sums into parts,
-        // each a tile of its own with its own copy of the states
-        const int nt = (int)p.tiles.size();
-        if (nt > 0 && nt < l.waves) {
-            const int share = l.waves / nt;
-            std::vector<Tile> cutted;
-            for (const Tile &t : p.tiles) {
-                const int k = std::max(1, std::min<int>(share, (int)t.ops.size()));
-                for (int q = 0; q < k; ++q) {
-                    Tile c = t;
-                    c.ops.assign(t.ops.begin() + t.ops.size() * q / k, t.ops.begin() + t.ops.size() * (q + 1) / k);
-                    cutted.push_back(c);
+        // joins of each state by operator: the steps of a tile's operator are the most of any
+        std::vector<std::vector<int>> n_joins(lev.size());
+        for (size_t i = 0; i < lev.size(); ++i) n_joins[i].assign(ops_of[i].size(), 0);
+        for (const ArcJoin &x : st.joins) {
+            const auto &v = ops_of[x.dst];
+            const int key = (x.op << 16) | x.pair;
+            n_joins[x.dst][std::lower_bound(v.begin(), v.end(), key) - v.begin()] += n_src[x.src];
+        }
+        for (Tile &t : tiles) {
+            t.steps.assign(t.ops.size(), 0);
+            for (int s : t.states)
+                for (size_t k = 0; k < ops_of[s].size(); ++k) {
+                    const size_t q = std::lower_bound(t.ops.begin(), t.ops.end(), ops_of[s][k]) - t.ops.begin();
+                    t.steps[q] = std::max(t.steps[q], n_joins[s][k]);
                 }
-            }
-            p.tiles.swap(cutted);
         }
-        p.parts.assign(lev.size(), {});
+        // the closed state alone leaves most lanes idle: deal its joins over lanes, each a part
+        if (spread && lev.size() == 1)
+            for (Tile &t : tiles) {
+                const int most = *std::max_element(t.steps.begin(), t.steps.end());
+                t.spread = std::min(std::min(per, 8), std::max(1, most / 3));
+                t.states.assign(t.spread, 0);
+                for (int &n : t.steps) n = (n + t.spread - 1) / t.spread;
+            }
+        return tiles;
+    }
+
+    // Cuts the operator sums of tiles longer than `target` slots (0: only those of too many
+    // operators) into parts, each a tile of its own with its own copy of the states.
+    Placed cut(const std::vector<Tile> &tiles, const std::vector<std::vector<int>> &ops_of, int lg, int target) const {
+        Placed p;
+        const int cg = 1 << lg;
+        for (const Tile &t : tiles) {
+            const int no = (int)t.ops.size();
+            std::vector<int> upto(no + 1, 0);  // slots before an operator
+            for (int i = 0; i < no; ++i) upto[i + 1] = upto[i] + (t.steps[i] + 1) / 2;
+            const int k = std::min(no, std::max(target > 0 ? (upto[no] + target - 1) / target : 1,
+                                                (no + kArcTileOps - 1) / kArcTileOps));
+            for (int q = 0, from = 0; q < k; ++q) {
+                int to = from + 1;  // an even share of the slots, an operator at least for each part left
+                while (to < no - (k - 1 - q) && to - from < kArcTileOps &&
+                       (q == k - 1 || 2 * (long long)upto[to] * k + (upto[to + 1] - upto[to]) * k <= 2LL * upto[no] * (q + 1)))
+                    ++to;
+                Tile c = t;
+                c.ops.assign(t.ops.begin() + from, t.ops.begin() + to);
+                c.steps.assign(t.steps.begin() + from, t.steps.begin() + to);
+                p.slots.push_back(upto[to] - upto[from]);
+                p.tiles.push_back(std::move(c));
+                from = to;
+                if (q == k - 1 && from < no) --q;  // what the operators' limit left over
+            }
+        }
+        p.parts.assign(ops_of.size(), {});
         for (const Tile &t : p.tiles) {
             const size_t step = (size_t)arc_stride(m.dims[t.sector], l.mmax) * cg;
             p.size = (p.size + 3) & ~(size_t)3;
@@ -422,19 +515,72 @@ struct ArcPacker {
         return p;
     }
 
-    // Elements of the state region and wavefront passes of a graph at 1 << lg columns.
-    void measure(const ArcGraph &g, int lg, size_t *region, double *cost) const {
-        const int cg = 1 << lg, m0 = m.dims[g.s0];
-        size_t prev = (size_t)arc_stride(m.dims[g.levels[0][0].sector], l.mmax) * cg, reg = (prev + 3) & ~(size_t)3;
-        double c = 0;
+    struct Plan {
+        std::vector<Placed> placed;  // [stage]
+        size_t region = 0;           // elements of the state region, the closed state at its end
+        size_t closed = 0;           // elements of the closed state
+        double cost = 0;             // slots on the longest wavefronts, over all column passes
+    };
+
+    // Places the states of a graph at 1 << lg columns within `room` elements.  A stage lasts as
+    // long as its longest wavefront: tiles are cut towards an even share as far as the parts
+    // fit and the steps that they add to the next stage do not cost more.
+    bool plan(const ArcGraph &g, int lg, size_t room, Plan &out) const {
+        const int cg = 1 << lg, m0 = m.dims[g.s0], per = 64 >> lg;
+        out = Plan{};
+        size_t prev = ((size_t)arc_stride(m.dims[g.levels[0][0].sector], l.mmax) * cg + 3) & ~(size_t)3, reg = prev;
+        out.closed = prev;
+        double c = kStageCost;
+        std::vector<int> n_src{1};
+        const size_t spare = 8 * (((size_t)arc_stride(m0, l.mmax) * cg + 3) & ~(size_t)3);
         for (size_t s = 0; s < g.stages.size(); ++s) {
-            const Placed p = place(g.levels[s + 1], g.stages[s], lg);
-            reg = std::max(reg, ((prev + 3) & ~(size_t)3) + p.size);
-            prev = p.size;
-            c += 1.0 + (double)((p.tiles.size() + l.waves - 1) / l.waves);
+            const bool last = s + 1 == g.stages.size();
+            std::vector<double> uses(g.levels[s + 1].size(), 0.0);  // lanes' steps that read a state
+            if (!last)
+                for (const ArcJoin &x : g.stages[s + 1].joins) uses[x.src] += 1.0;
+            Placed best;
+            double best_cost = -1;
+            for (int spread = 1; spread >= (last ? 0 : 1); --spread) {
+                std::vector<std::vector<int>> ops_of;
+                const std::vector<Tile> tiles = tiles_of(g.levels[s + 1], g.stages[s], lg, n_src, spread != 0, ops_of);
+                int longest = 0, sum = 0;
+                for (const Tile &t : tiles) {
+                    int n = 0;
+                    for (int k : t.steps) n += (k + 1) / 2;
+                    longest = std::max(longest, n);
+                    sum += n;
+                }
+                for (int target = std::max(1, sum / l.waves);; target += (target + 1) / 2) {
+                    const bool uncut = target >= longest;
+                    Placed p = cut(tiles, ops_of, lg, uncut ? 0 : target);
+                    double cost = p.deal(l.waves, nullptr);
+                    if (last)  // the parts are read one by one
+                        cost += 0.05 * (double)p.parts[0].size();
+                    else
+                        for (size_t i = 0; i < uses.size(); ++i)
+                            cost += ((double)p.parts[i].size() - 1.0) * uses[i] / (2.0 * per * l.waves);
+                    const bool fits = last ? reg + p.size <= room : prev + p.size + spare <= room;
+                    if (fits && (best_cost < 0 || cost < best_cost)) {
+                        best_cost = cost;
+                        best = std::move(p);
+                    }
+                    if (uncut) break;
+                }
+                if (best_cost >= 0 && spread) break;
+            }
+            if (best_cost < 0) return false;
+            n_src = best.part_counts();
+            if (last)
+                out.closed = best.size;
+            else
+                reg = std::max(reg, prev + best.size);
+            prev = best.size;
+            c += kStageCost + best.deal(l.waves, nullptr);
+            out.placed.push_back(std::move(best));
         }
-        *region = reg;
-        *cost = c * ((m0 + cg - 1) / cg);
+        out.region = reg + out.closed;
+        out.cost = c * ((m0 + cg - 1) / cg);
+        return out.region <= room;
     }
 
     double graph_flops(const ArcGraph &g) const {
@@ -466,54 +612,46 @@ struct ArcPacker {
         return f;
     }
 
-    void emit(const ArcGraph &g, int lg, size_t region, ArcGroupProgram &out) {
+    void emit(const ArcGraph &g, int lg, const Plan &pn, size_t states_at, ArcGroupProgram &out) {
         std::vector<uint32_t> &b = out.blob;
-        while (b.size() % 4) b.push_back(0);
+        while (b.size() % 64) b.push_back(0);
         out.blob[kArcGroupHead + out.n_segments] = (uint32_t)b.size();
         const size_t seg = b.size();
-        const int m0 = m.dims[g.s0], s1 = g.levels[0][0].sector;
-        b.resize(seg + kArcSegHead + 2 * g.stages.size(), 0u);
+        const int m0 = m.dims[g.s0], s1 = g.levels[0][0].sector, per = 64 >> lg;
+        const size_t n_st = g.stages.size();
+        b.resize(seg + kArcSegHead + 2 * l.waves, 0u);
         b[seg] = (uint32_t)g.s0 | ((uint32_t)m0 << 8) | ((uint32_t)lg << 16);
-        b[seg + 1] = (uint32_t)g.stages.size();
-        b[seg + 2] = (uint32_t)m.dims[s1] | ((uint32_t)arc_stride(m.dims[s1], l.mmax) << 8);
-        b[seg + 3] = kind == ARC_CORR ? ob.b[g.s0] : ARC_NONE;
+        b[seg + 1] = (uint32_t)m.dims[s1] | ((uint32_t)arc_stride(m.dims[s1], l.mmax) << 8);
+        b[seg + 2] = kind == ARC_CORR ? ob.b[g.s0] : ARC_NONE;
         // with no stage after it the root is the closed state, and its propagator the last one
-        b[seg + 4] = g.stages.empty() ? ARC_NONE : (uint32_t)(slot_after(1) * l.bt + l.bt_off[s1]);
-        b[seg + 5] = 0;
+        b[seg + 3] = n_st == 0 ? ARC_NONE : (uint32_t)(slot_after(1) * l.bt + l.bt_off[s1]);
         std::vector<std::vector<size_t>> src{{0}};
-        for (size_t s = 0; s < g.stages.size(); ++s) {
+        std::vector<std::vector<Slot>> stream(l.waves);
+        const size_t levels = pn.region - pn.closed;  // elements of the alternating levels
+        for (size_t s = 0; s < n_st; ++s) {
             const ArcStage &st = g.stages[s];
-            const bool last = s + 1 == g.stages.size();
-            const Placed p = place(g.levels[s + 1], st, lg);
-            const size_t base = s % 2 == 0 ? region - p.size : 0;  // the levels alternate between the ends
+            const bool last = s + 1 == n_st;
+            const Placed &p = pn.placed[s];
+            // the levels alternate between the ends of their region, the closed state follows
+            const size_t base = last ? levels : s % 2 == 0 ? levels - p.size : 0;
             std::vector<std::vector<size_t>> dst = p.parts;
             for (auto &v : dst)
                 for (size_t &o : v) o += base;
-            // joins by destination and operator
-            std::vector<std::vector<int>> by(g.levels[s + 1].size());
+            std::vector<std::vector<int>> by(g.levels[s + 1].size());  // joins by destination
             for (size_t i = 0; i < st.joins.size(); ++i) by[st.joins[i].dst].push_back((int)i);
-            while (b.size() % 4) b.push_back(0);
-            const size_t tiles = b.size();
-            b[seg + kArcSegHead + 2 * s] = (uint32_t)p.tiles.size();
-            b[seg + kArcSegHead + 2 * s + 1] = (uint32_t)tiles;
-            b.resize(tiles + 4 * p.tiles.size(), 0u);
+            // records of the tiles
+            std::vector<std::vector<Slot>> recs;
             for (size_t ti = 0; ti < p.tiles.size(); ++ti) {
                 const Tile &t = p.tiles[ti];
                 const int md = m.dims[t.sector], ns = (int)t.states.size();
-                while (b.size() % 4) b.push_back(0);
-                const size_t ops = b.size();
-                b.resize(ops + 4 * t.ops.size(), 0u);
-                b[tiles + 4 * ti] = (uint32_t)t.ops.size() | ((uint32_t)md << 8) | ((uint32_t)ns << 16) |
-                                    ((uint32_t)arc_stride(md, l.mmax) << 24);
-                b[tiles + 4 * ti + 1] = (uint32_t)(base + p.tile_off[ti]);
-                b[tiles + 4 * ti + 2] = last ? ARC_NONE : (uint32_t)(slot_after(st.position) * l.bt + l.bt_off[t.sector]);
-                b[tiles + 4 * ti + 3] = (uint32_t)ops;
+                std::vector<Slot> r;
                 for (size_t oi = 0; oi < t.ops.size(); ++oi) {
                     const int op = t.ops[oi] >> 16, pair = t.ops[oi] & 0xFFFF;
                     std::vector<std::vector<uint32_t>> words(ns);
                     int ssec = t.sector;
                     size_t most = 0;
                     for (int i = 0; i < ns; ++i) {
+                        int dealt = 0;
                         for (int ji : by[t.states[i]]) {
                             const ArcJoin &x = st.joins[ji];
                             if (x.op != op || x.pair != pair) continue;
@@ -521,31 +659,88 @@ struct ArcPacker {
                             const uint32_t v = op == ARC_TAIL
                                                    ? arc_value(x.head, st.position, m.table[pair], x.sign)
                                                    : 1u;
-                            for (size_t off : src[x.src]) words[i].push_back((uint32_t)off | (v << 20));
+                            for (size_t off : src[x.src])
+                                if (t.spread == 1 || dealt++ % t.spread == i)
+                                    words[i].push_back((uint32_t)((states_at + off * l.elem) / 4) | (v << 20));
                         }
                         most = std::max(most, words[i].size());
                     }
-                    uint32_t blk = ARC_NONE;
+                    uint32_t blk = ob.id;
                     if (op == ARC_HEAD) blk = ob.head[pair][ssec];
                     if (op == ARC_TAIL) blk = ob.tail[pair][ssec];
                     if (op == ARC_A) blk = ob.a[ssec];
                     const int ms = m.dims[ssec];
-                    b[ops + 4 * oi] = blk;
-                    b[ops + 4 * oi + 1] = (uint32_t)ms | ((uint32_t)arc_stride(ms, l.mmax) << 8) | ((uint32_t)most << 16);
-                    b[ops + 4 * oi + 2] = (uint32_t)b.size();
                     uint32_t any = 0;  // a source of the tile, for the fill words
                     for (int i = 0; i < ns; ++i)
                         if (!words[i].empty()) any = words[i][0] & 0xFFFFFu;
-                    for (size_t e = 0; e < most; ++e)
-                        for (int i = 0; i < ns; ++i) b.push_back(e < words[i].size() ? words[i][e] : any);
+                    for (size_t e = 0; e < most; e += 2) {
+                        Slot q;
+                        q.head[1] = (uint32_t)md | ((uint32_t)arc_stride(md, l.mmax) << 8) |
+                                    ((uint32_t)arc_stride(ms, l.mmax) << 16);
+                        for (int i = 0; i < per; ++i)
+                            q.first.push_back(i < ns && e < words[i].size() ? words[i][e] : any);
+                        if (e + 1 < most) {
+                            q.head[0] |= ARC_SECOND;
+                            for (int i = 0; i < per; ++i)
+                                q.second.push_back(i < ns && e + 1 < words[i].size() ? words[i][e + 1] : any);
+                        }
+                        if (e + 2 >= most) {
+                            q.head[0] |= ARC_TIMES;
+                            q.head[2] = blk;
+                        }
+                        r.push_back(std::move(q));
+                    }
                     out.joins += (double)most * ns;
                 }
+                r.back().head[0] |= ARC_STORE;
+                r.back().head[3] = (uint32_t)(base + p.tile_off[ti]);
+                r.back().head[4] = last ? ARC_NONE : (uint32_t)(slot_after(st.position) * l.bt + l.bt_off[t.sector]);
+                r.back().head[5] = (uint32_t)ns;
+                recs.push_back(std::move(r));
             }
+            // each wavefront's first slot of a stage waits for the barrier
+            std::vector<int> wave;
+            p.deal(l.waves, &wave);
+            std::vector<char> begun(l.waves, 0);
+            auto append = [&](int w, std::vector<Slot> r) {
+                if (!begun[w]) r[0].head[0] |= ARC_BARRIER;
+                begun[w] = 1;
+                stream[w].insert(stream[w].end(), r.begin(), r.end());
+            };
+            for (size_t i = 0; i < recs.size(); ++i) append(wave[i], recs[i]);
+            for (int w = 0; w < l.waves; ++w)
+                if (!begun[w]) append(w, {Slot::idle(ARC_IDLE, per)});  // nothing to do in this stage
             src.swap(dst);
         }
-        // the parts of the closed state
-        b[seg + 6] = (uint32_t)src[0].size();
-        b[seg + 7] = (uint32_t)b.size();
+        for (int w = 0; w < l.waves; ++w) {
+            std::vector<Slot> &q = stream[w];
+            const size_t at_end = q.size() / l.slots * l.slots;  // first slot of the last packet
+            q.push_back(Slot::idle(ARC_BARRIER | ARC_END | ARC_IDLE, per));
+            // a wavefront fetches the operator blocks of one packet more
+            do q.push_back(Slot::idle(ARC_IDLE, per));
+            while (q.size() % l.slots || (int)(q.size() - at_end) <= l.slots);
+            std::vector<uint32_t> joins;
+            while (b.size() % 64) b.push_back(0);
+            b[seg + kArcSegHead + 2 * w] = (uint32_t)b.size();
+            for (size_t i = 0; i < q.size(); i += l.slots) {
+                bool second = false;
+                for (int o = 0; o < l.slots; ++o) second = second || (q[i + o].head[0] & ARC_SECOND);
+                q[i].head[6] = second;
+                for (int o = 0; o < l.slots; ++o) b.insert(b.end(), q[i + o].head.begin(), q[i + o].head.end());
+                for (int sl = 0; sl < per; ++sl)
+                    for (int o = 0; o < l.slots; ++o) joins.push_back(q[i + o].first[sl]);
+                for (int sl = 0; second && sl < per; ++sl)
+                    for (int o = 0; o < l.slots; ++o)
+                        joins.push_back(q[i + o].second.empty() ? 0u : q[i + o].second[sl]);
+            }
+            while (b.size() % 64) b.push_back(0);
+            b[seg + kArcSegHead + 2 * w + 1] = (uint32_t)b.size();
+            b.insert(b.end(), joins.begin(), joins.end());
+        }
+        if (n_st == 0) src[0][0] = levels;
+        b[seg + 4] = n_st == 0 ? (uint32_t)levels : 0u;
+        b[seg + 5] = (uint32_t)src[0].size();  // the parts of the closed state
+        b[seg + 6] = (uint32_t)b.size();
         for (size_t off : src[0]) b.push_back((uint32_t)off);
         out.n_segments++;
         const double f = graph_flops(g);
@@ -590,23 +785,18 @@ inline int arc_compile(const ArcModel &m, const ArcLayout &l, const ArcBlocks &o
     out.lds = at.states;
     for (const ArcGraph &g : graphs) {
         int best = -1;
-        size_t best_region = 0;
-        double best_cost = 0;
+        ArcPacker::Plan plan, best_plan;
         for (int lg = 0; lg <= 5; ++lg) {
             if (lg > 0 && (1 << (lg - 1)) >= m.dims[g.s0]) break;
-            size_t region;
-            double cost;
-            pk.measure(g, lg, &region, &cost);
-            if (region > room || region >= (1u << 20)) break;
-            if (best < 0 || cost < best_cost) {
+            if (!pk.plan(g, lg, room, plan)) break;
+            if (best < 0 || plan.cost < best_plan.cost) {
                 best = lg;
-                best_region = region;
-                best_cost = cost;
+                best_plan = std::move(plan);
             }
         }
         if (best < 0) return 2;
-        pk.emit(g, best, best_region, out);
-        out.lds = std::max(out.lds, at.states + best_region * l.elem);
+        pk.emit(g, best, best_plan, at.states, out);
+        out.lds = std::max(out.lds, at.states + best_plan.region * l.elem);
     }
     while (out.blob.size() % 4) out.blob.push_back(0);
     out.blob[0] = (uint32_t)out.n_segments;
@@ -619,6 +809,7 @@ inline int arc_compile(const ArcModel &m, const ArcLayout &l, const ArcBlocks &o
     out.blob[7] = (uint32_t)at.states;
     out.n_arcs = (int)pk.arcs.size();
     out.blob.insert(out.blob.end(), pk.arcs.begin(), pk.arcs.end());
+    out.blob.resize(out.blob.size() + kArcReadAhead, 0u);
     return 0;
 }
 

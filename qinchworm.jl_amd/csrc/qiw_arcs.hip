@@ -5,8 +5,11 @@
 
 #include <utility>
 
+#include "qiw_arcs.h"
 #include "qiw_device.h"
 #include "qiw_lookup.h"
+
+using namespace qiwi;
 
 namespace {
 
@@ -20,9 +23,26 @@ __device__ __forceinline__ ConstP<T> as_constp(const T *p) {
     return (ConstP<T>)p;
 }
 
-constexpr uint32_t kNone = 0xFFFFFFFFu;
+constexpr uint32_t kNone = ARC_NONE;
+__device__ __forceinline__ uint32_t rlane(uint32_t v, int l) { return __builtin_amdgcn_readlane(v, l); }
+// the word at a byte offset of a uniform base (one load with a 32-bit vector offset)
+__device__ __forceinline__ uint32_t word_at(const uint32_t *base, uint32_t byte) {
+    return *reinterpret_cast<const uint32_t *>(reinterpret_cast<const char *>(base) + byte);
+}
+// source state (column offset coff) and arc value of a join word
+template <typename V>
+__device__ __forceinline__ const V *state_at(const char *lds, uint32_t q, uint32_t coff) {
+    return reinterpret_cast<const V *>(lds + ((q & 0xFFFFu) * 4u + coff));
+}
+template <typename V>
+__device__ __forceinline__ V value_at(const char *lds, uint32_t q) {  // bits 16-19 are clear
+    return *reinterpret_cast<const V *>(lds + kArcValuesAt + (q >> (sizeof(V) == 4 ? 18 : 17)));
+}
 
 // A lane's vector of up to MB values and its products with a block shared by the wavefront.
+// The walk of a slot branches once on the stride C of its source and once on the stride R of
+// its states; all below is straight code for them (branches on every row and column took two
+// thirds of the time).
 //
 // float: a block times the 64 lanes' vectors runs on v_mfma_f32_4x4x1_16b_f32 (16 independent
 // 4x4 outer products).  Its B operand is one vector element of every lane and its result four
@@ -30,103 +50,69 @@ constexpr uint32_t kNone = 0xFFFFFFFFu;
 // operand of one (4 rows, column) slice is broadcast to all 16 products from the four lanes
 // that hold it (CBSZ = 4, ABID = the slice).  A register therefore carries 16 slices of a
 // block, read with one 64-lane load.
-template <typename V, int MB>
-struct LaneVec;
-
-template <int MB>
-struct LaneVec<float, MB> {
-    static constexpr int RG = MB / 4, NV = (RG * MB + 15) / 16;
-    float x[MB];
-    __device__ __forceinline__ void zero() {
-#pragma unroll
-        for (int k = 0; k < MB; ++k) x[k] = 0.f;
-    }
-};
-
-// slice s = row group * MB + column, in register s / 16 of a block, lanes 4 (s % 16) ..
-template <int MB, int R, int K, int... G>
-__device__ __forceinline__ void mfma_column(f4 (&acc)[MB / 4], const float *A, float y, std::integer_sequence<int, G...>) {
-    ((acc[G] = __builtin_amdgcn_mfma_f32_4x4x1f32(A[(G * MB + K) / 16], y, acc[G], 4, (G * MB + K) % 16, 0)), ...);
-}
-// R row groups, columns below cols (uniform) in steps of KS; the columns past cols are zero
-template <int MB, int R, int KS, int... K>
-__device__ __forceinline__ void mfma_rows(f4 (&acc)[MB / 4], const float *A, const float *y, int cols,
-                                          std::integer_sequence<int, K...>) {
-    auto step = [&](auto kc) {
-        constexpr int k0 = decltype(kc)::value * KS;
-        if (k0 < cols) {
-            mfma_column<MB, R, k0>(acc, A, y[k0], std::make_integer_sequence<int, R>{});
-            if constexpr (KS > 1) mfma_column<MB, R, k0 + 1>(acc, A, y[k0 + 1], std::make_integer_sequence<int, R>{});
-            if constexpr (KS > 2) {
-                mfma_column<MB, R, k0 + 2>(acc, A, y[k0 + 2], std::make_integer_sequence<int, R>{});
-                mfma_column<MB, R, k0 + 3>(acc, A, y[k0 + 3], std::make_integer_sequence<int, R>{});
-            }
-        }
-    };
-    (step(std::integral_constant<int, K>{}), ...);
-}
-template <int MB, int R = 1>
-__device__ __forceinline__ void mfma_block(f4 (&acc)[MB / 4], const float *A, const float *y, int rows, int cols) {
-    constexpr int KS = MB <= 8 ? 2 : 4;
-    if constexpr (R < MB / 4) {
-        if (rows > 4 * R) {
-            mfma_block<MB, R + 1>(acc, A, y, rows, cols);
-            return;
-        }
-    }
-    mfma_rows<MB, R, KS>(acc, A, y, cols, std::make_integer_sequence<int, MB / KS>{});
-}
-
-// Joins: y (+)= w * state, the state's rows read from LDS in pairs (narrow) or fours.
-template <int MB, bool FIRST>
-__device__ __forceinline__ void join(float *y, float w, const float *s, int stride) {
-    if (MB <= 8 && stride <= 6) {
-        if (stride == 1) {
-            y[0] = FIRST ? w * s[0] : fmaf(w, s[0], y[0]);
-            return;
-        }
-#pragma unroll
-        for (int k = 0; k < 6; k += 2)
-            if (k < stride) {
-                const f2 v = *(const f2 *)(s + k);
-                y[k] = FIRST ? w * v[0] : fmaf(w, v[0], y[k]);
-                y[k + 1] = FIRST ? w * v[1] : fmaf(w, v[1], y[k + 1]);
-            }
-        return;
-    }
-#pragma unroll
-    for (int k = 0; k < MB; k += 4)
-        if (k < stride) {
-            const f4 v = *(const f4 *)(s + k);
-#pragma unroll
-            for (int q = 0; q < 4; ++q) y[k + q] = FIRST ? w * v[q] : fmaf(w, v[q], y[k + q]);
-        }
-}
-template <int MB, bool FIRST>
-__device__ __forceinline__ void join(double *y, double w, const double *s, int stride) {
-    if (stride == 1) {
-        y[0] = FIRST ? w * s[0] : fma(w, s[0], y[0]);
-        return;
-    }
-#pragma unroll
-    for (int k = 0; k < MB; k += 2)
-        if (k < stride) {
-            const d2 v = *(const d2 *)(s + k);
-            y[k] = FIRST ? w * v[0] : fma(w, v[0], y[k]);
-            y[k + 1] = FIRST ? w * v[1] : fma(w, v[1], y[k + 1]);
-        }
-}
-
+//
+// double: multiply-adds whose block element is broadcast from its lane by the instruction
+// itself (v_fmac_f64 with DPP row_newbcast; every row of 16 lanes holds the same 16
+// elements), so a register pair carries 16 elements.  The float64 matrix instructions have
+// no more rate than the vector units.
 template <typename V, int MB>
 struct Walk;
 
+// y += w s, s a state of C elements in LDS (a stride of arc_stride: 16-byte aligned from 4
+// floats on, but for 6)
+template <int C>
+__device__ __forceinline__ void join(float *y, float w, const float *s) {
+    if constexpr (C == 1) {
+        y[0] = fma(w, s[0], y[0]);
+    } else if constexpr (C % 4 == 0) {
+#pragma unroll
+        for (int k = 0; k < C; k += 4) {
+            const f4 v = *(const f4 *)(s + k);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) y[k + q] = fma(w, v[q], y[k + q]);
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < C; k += 2) {
+            const f2 v = *(const f2 *)(s + k);
+            y[k] = fma(w, v[0], y[k]);
+            y[k + 1] = fma(w, v[1], y[k + 1]);
+        }
+    }
+}
+template <int C>
+__device__ __forceinline__ void join(double *y, double w, const double *s) {
+    if constexpr (C == 1) {
+        y[0] = fma(w, s[0], y[0]);
+    } else {
+#pragma unroll
+        for (int k = 0; k < C; k += 2) {
+            const d2 v = *(const d2 *)(s + k);
+            y[k] = fma(w, v[0], y[k]);
+            y[k + 1] = fma(w, v[1], y[k + 1]);
+        }
+    }
+}
+
+// slice s = row group * MB + column, in register s / 16 of a block, lanes 4 (s % 16) ..
+template <int MB, int G, int K, int... R>
+__device__ __forceinline__ void mfma_column(f4 (&acc)[MB / 4], const float *A, float y, std::integer_sequence<int, R...>) {
+    ((acc[R] = __builtin_amdgcn_mfma_f32_4x4x1f32(A[(R * MB + K) / 16], y, acc[R], 4, (R * MB + K) % 16, 0)), ...);
+}
+// G row groups, the columns K
+template <int MB, int G, int... K>
+__device__ __forceinline__ void mfma_block(f4 (&acc)[MB / 4], const float *A, const float *y,
+                                           std::integer_sequence<int, K...>) {
+    (mfma_column<MB, G, K>(acc, A, y[K], std::make_integer_sequence<int, G>{}), ...);
+}
+
 template <int MB>
 struct Walk<float, MB> {
-    using L = LaneVec<float, MB>;
-    static constexpr int NV = L::NV;
-    f4 acc[MB / 4], out[MB / 4];
-    float y[MB];
-    int rk[NV];  // row | column << 8 of this lane's element of slice register v
+    static constexpr int NV = (MB / 4 * MB + 15) / 16;  // slice registers of a block
+    static constexpr int SL = arc_slots(MB, true);
+    f4 acc[MB / 4];
+    float y[MB], A[SL][NV], next[SL][NV];  // blocks of the packet and of the next one
+    int rk[NV];                            // row | column << 8 of this lane's element of slice register v
     int lane;
 
     __device__ __forceinline__ void init(int lane_) {
@@ -135,133 +121,341 @@ struct Walk<float, MB> {
         for (int v = 0; v < NV; ++v) {
             const int s = 16 * v + (lane >> 2), k = s % MB, row = 4 * (s / MB) + (lane & 3);
             rk[v] = row | (k << 8);
+#pragma unroll
+            for (int o = 0; o < SL; ++o) A[o][v] = next[o][v] = 0.f;
         }
+#pragma unroll
+        for (int k = 0; k < MB; ++k) y[k] = 0.f;
+        clear();
     }
     __device__ __forceinline__ void clear() {
 #pragma unroll
         for (int g = 0; g < MB / 4; ++g) acc[g] = f4{0.f, 0.f, 0.f, 0.f};
     }
-    __device__ __forceinline__ void clear_y() {
+    // blocks in slice registers in memory; str: rows that are computed, ss: columns
+    template <int O>
+    __device__ __forceinline__ void fetch_op(const float *ops, uint32_t off, int str, int ss) {
+        const int last = ((str + 3) / 4 - 1) * MB + ss;  // slices in use
 #pragma unroll
-        for (int k = 0; k < MB; ++k) y[k] = 0.f;
+        for (int v = 0; v < NV; ++v)
+            if (NV == 1 || 16 * v < last) next[O][v] = ops[off + 64 * v + lane];
     }
-    // acc += O y, O in slice registers in memory
-    __device__ __forceinline__ void apply_op(const float *ops, uint32_t off, int rows, int cols) {
-        const int last = ((rows + 3) / 4 - 1) * MB + cols;  // slices in use
-        float A[NV];
+    __device__ __forceinline__ void rotate() {
 #pragma unroll
-        for (int v = 0; v < NV; ++v) A[v] = 16 * v < last ? ops[off + 64 * v + lane] : 0.f;
-        mfma_block<MB>(acc, A, y, rows, cols);
+        for (int o = 0; o < SL; ++o)
+#pragma unroll
+            for (int v = 0; v < NV; ++v) A[o][v] = next[o][v];
     }
-    __device__ __forceinline__ void add_y(int rows) {
+    // acc += O y, y = 0
+    template <int O, int C>
+    __device__ __forceinline__ void product(const float *, uint32_t, int str) {
+        rows<C, 1>(A[O], str);
 #pragma unroll
-        for (int k = 0; k < MB; ++k)
-            if (k < rows) acc[k / 4][k % 4] += y[k];
+        for (int k = 0; k < C; ++k) y[k] = 0.f;
     }
-    // out = P acc, P column-major m x m in LDS
-    __device__ __forceinline__ void apply_prop(const float *P, int m) {
-        const int last = ((m + 3) / 4 - 1) * MB + m;
-        float A[NV];
+    template <int C, int G>
+    __device__ __forceinline__ void rows(const float *a, int str) {
+        if constexpr (G < MB / 4) {
+            if (str > 4 * G) {
+                rows<C, G + 1>(a, str);
+                return;
+            }
+        }
+        mfma_block<MB, G>(acc, a, y, std::make_integer_sequence<int, C>{});
+    }
+    // acc = P acc, P column-major m x m in LDS, C its padded size
+    template <int C>
+    __device__ __forceinline__ void propagate(const float *pl, int m) {
+        constexpr int last = ((C + 3) / 4 - 1) * MB + C;
+        float P[NV], x[C];
 #pragma unroll
-        for (int v = 0; v < NV; ++v) {
-            A[v] = 0.f;
+        for (int v = 0; v < NV; ++v)
             if (16 * v < last) {
                 const int row = rk[v] & 255, k = rk[v] >> 8;
                 const bool in = row < m && k < m;
-                const float p = P[in ? row + k * m : 0];
-                A[v] = in ? p : 0.f;
-            }
-        }
-        float x[MB];
-#pragma unroll
-        for (int k = 0; k < MB; ++k) x[k] = acc[k / 4][k % 4];
-#pragma unroll
-        for (int g = 0; g < MB / 4; ++g) out[g] = f4{0.f, 0.f, 0.f, 0.f};
-        mfma_block<MB>(out, A, x, m, m);
-    }
-    __device__ __forceinline__ void keep() {
-#pragma unroll
-        for (int g = 0; g < MB / 4; ++g) out[g] = acc[g];
-    }
-    __device__ __forceinline__ void store(float *d, int stride) const {
-        if (MB <= 8 && stride <= 6) {
-            if (stride == 1) {
-                d[0] = out[0][0];
-                return;
+                const float p = pl[in ? row + k * m : 0];
+                P[v] = in ? p : 0.f;
             }
 #pragma unroll
-            for (int k = 0; k < 6; k += 2)
-                if (k < stride) *(f2 *)(d + k) = f2{out[k / 4][k % 4], out[(k + 1) / 4][(k + 1) % 4]};
-            return;
-        }
+        for (int k = 0; k < C; ++k) x[k] = acc[k / 4][k % 4];
+        clear();
+        mfma_block<MB, (C + 3) / 4>(acc, P, x, std::make_integer_sequence<int, C>{});
+    }
+    template <int C>
+    __device__ __forceinline__ void store(float *d) const {
+        if constexpr (C == 1) {
+            d[0] = acc[0][0];
+        } else if constexpr (C % 4 == 0) {
 #pragma unroll
-        for (int g = 0; g < MB / 4; ++g)
-            if (4 * g < stride) *(f4 *)(d + 4 * g) = out[g];
+            for (int g = 0; g < C / 4; ++g) *(f4 *)(d + 4 * g) = acc[g];
+        } else {
+#pragma unroll
+            for (int k = 0; k < C; k += 2) *(f2 *)(d + k) = f2{acc[k / 4][k % 4], acc[(k + 1) / 4][(k + 1) % 4]};
+        }
     }
 };
 
-// double: the block's elements are wavefront-uniform multiplicands (operators through the
-// scalar cache, propagators as LDS broadcasts) of ordinary multiply-adds; the matrix cores
-// have no more float64 rate than the vector units.
+// c[0 .. 3] += (elements N .. N + 3 of the 16 in a) * y, and for two and one.  The wait states
+// between a vector write of a and a DPP read of it stand in the block.
+template <int N, int R>
+__device__ __forceinline__ void fmac_bcast(double *c, double a, double y) {
+    if constexpr (R >= 4) {
+        asm("s_nop 1\n"
+            "v_fmac_f64_dpp %0, %4, %5 row_newbcast:%6 row_mask:0xf bank_mask:0xf\n"
+            "v_fmac_f64_dpp %1, %4, %5 row_newbcast:%7 row_mask:0xf bank_mask:0xf\n"
+            "v_fmac_f64_dpp %2, %4, %5 row_newbcast:%8 row_mask:0xf bank_mask:0xf\n"
+            "v_fmac_f64_dpp %3, %4, %5 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n"
+            : "+v"(c[0]), "+v"(c[1]), "+v"(c[2]), "+v"(c[3])
+            : "v"(a), "v"(y), "n"(N), "n"(N + 1), "n"(N + 2), "n"(N + 3));
+    } else if constexpr (R == 2) {
+        asm("s_nop 1\n"
+            "v_fmac_f64_dpp %0, %2, %3 row_newbcast:%4 row_mask:0xf bank_mask:0xf\n"
+            "v_fmac_f64_dpp %1, %2, %3 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n"
+            : "+v"(c[0]), "+v"(c[1])
+            : "v"(a), "v"(y), "n"(N), "n"(N + 1));
+    } else {
+        asm("s_nop 1\n"
+            "v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf\n"
+            : "+v"(c[0])
+            : "v"(a), "v"(y), "n"(N));
+    }
+}
+// R rows of one column, element E of the chunk onwards
+template <int E, int R>
+__device__ __forceinline__ void fmac_rows(double *c, const double *a, double y) {
+    fmac_bcast<E % 16, R>(c, a[E / 16], y);
+    if constexpr (R > 4) fmac_rows<E + 4, R - 4>(c + 4, a, y);
+}
+// rows I .. I + R - 1 of the chunk's columns K
+template <int MB, int I, int R, int... K>
+__device__ __forceinline__ void fmac_block(double *acc, const double *a, const double *y, std::integer_sequence<int, K...>) {
+    (fmac_rows<K * MB + I, R>(acc + I, a, y[K]), ...);
+}
+
 template <int MB>
 struct Walk<double, MB> {
-    double acc[MB], out[MB], y[MB];
+    static constexpr int CH = MB <= 8 ? 8 : 4;  // columns of a chunk
+    static constexpr int NV = CH * MB / 16;     // register pairs of a chunk
+    static constexpr int SL = arc_slots(MB, false);
+    double acc[MB], y[MB], A[SL][NV], next[SL][NV];  // first chunks of the packet and of the next one
+    int rk[NV];  // row | column of the chunk << 8 of this lane's element of register pair v
     int lane;
-    __device__ __forceinline__ void init(int lane_) { lane = lane_; }
+    __device__ __forceinline__ void init(int lane_) {
+        lane = lane_;
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            const int e = 16 * v + (lane & 15);
+            rk[v] = (e % MB) | ((e / MB) << 8);
+#pragma unroll
+            for (int o = 0; o < SL; ++o) A[o][v] = next[o][v] = 0.0;
+        }
+#pragma unroll
+        for (int k = 0; k < MB; ++k) y[k] = 0.0;
+        clear();
+    }
     __device__ __forceinline__ void clear() {
 #pragma unroll
         for (int k = 0; k < MB; ++k) acc[k] = 0.0;
     }
-    __device__ __forceinline__ void clear_y() {
+    // operator blocks: MB x MB column-major, zeros past the block; columns c0 .. of it into a
+    __device__ __forceinline__ void read_op(double (&a)[NV], const double *ops, uint32_t off, int c0, int cols) const {
 #pragma unroll
-        for (int k = 0; k < MB; ++k) y[k] = 0.0;
+        for (int v = 0; v < NV; ++v)
+            if (c0 + 16 * v / MB < cols) a[v] = ops[off + c0 * MB + 16 * v + (lane & 15)];
     }
-    __device__ __forceinline__ void apply_op(const double *ops, uint32_t off, int rows, int cols) {
-        const ConstP<double> O = as_constp(ops) + off;  // column-major, padded past the end
+    template <int O>
+    __device__ __forceinline__ void fetch_op(const double *ops, uint32_t off, int, int ss) {
+        read_op(next[O], ops, off, 0, ss);
+    }
+    __device__ __forceinline__ void rotate() {
 #pragma unroll
-        for (int k = 0; k < MB; ++k)
-            if (k < cols) {
+        for (int o = 0; o < SL; ++o)
 #pragma unroll
-                for (int i = 0; i < MB; i += 2)
-                    if (i < rows) {
-                        acc[i] = fma(O[k * rows + i], y[k], acc[i]);
-                        acc[i + 1] = fma(i + 1 < rows ? O[k * rows + i + 1] : 0.0, y[k], acc[i + 1]);
-                    }
+            for (int v = 0; v < NV; ++v) A[o][v] = next[o][v];
+    }
+    // acc += (C columns of the chunk in a) x
+    template <int C, int R>
+    __device__ __forceinline__ void rows(const double (&a)[NV], const double *x, int str) {
+        constexpr auto columns = std::make_integer_sequence<int, C>{};
+        if constexpr (MB <= 8) {
+            if (str == 4)
+                fmac_block<MB, 0, 4>(acc, a, x, columns);
+            else if (str == 6)
+                fmac_block<MB, 0, 6>(acc, a, x, columns);
+            else if (str == 1)
+                fmac_block<MB, 0, 1>(acc, a, x, columns);
+            else if (str == 2)
+                fmac_block<MB, 0, 2>(acc, a, x, columns);
+            else
+                fmac_block<MB, 0, 8>(acc, a, x, columns);
+        } else if constexpr (R < MB) {  // rows in fours
+            if (R < str) {
+                fmac_block<MB, R, 4>(acc, a, x, columns);
+                rows<C, R + 4>(a, x, str);
             }
-    }
-    __device__ __forceinline__ void add_y(int rows) {
-#pragma unroll
-        for (int k = 0; k < MB; ++k)
-            if (k < rows) acc[k] += y[k];
-    }
-    __device__ __forceinline__ void apply_prop(const double *P, int m) {
-#pragma unroll
-        for (int k = 0; k < MB; ++k) out[k] = 0.0;
-#pragma unroll
-        for (int k = 0; k < MB; ++k)
-            if (k < m) {
-#pragma unroll
-                for (int i = 0; i < MB; i += 2)
-                    if (i < m) {
-                        out[i] = fma(P[k * m + i], acc[k], out[i]);
-                        out[i + 1] = fma(i + 1 < m ? P[k * m + i + 1] : 0.0, acc[k], out[i + 1]);
-                    }
-            }
-    }
-    __device__ __forceinline__ void keep() {
-#pragma unroll
-        for (int k = 0; k < MB; ++k) out[k] = acc[k];
-    }
-    __device__ __forceinline__ void store(double *d, int stride) const {
-        if (stride == 1) {
-            d[0] = out[0];
-            return;
         }
+    }
+    template <int O, int C, int K = 0>
+    __device__ __forceinline__ void product(const double *ops, uint32_t off, int str) {
+        if constexpr (K < C) {
+            if constexpr (K > 0) read_op(A[O], ops, off, K, C);
+            rows<(C < CH ? C : CH), 0>(A[O], y + K, str);
+            product<O, C, K + CH>(ops, off, str);
+        } else {
 #pragma unroll
-        for (int k = 0; k < MB; k += 2)
-            if (k < stride) *(d2 *)(d + k) = d2{out[k], out[k + 1]};
+            for (int k = 0; k < C; ++k) y[k] = 0.0;
+        }
+    }
+    template <int C>
+    __device__ __forceinline__ void propagate(const double *pl, int m) {
+        double x[C];
+#pragma unroll
+        for (int k = 0; k < C; ++k) x[k] = acc[k];
+        clear();
+        prop_chunks<C, 0>(pl, x, m);
+    }
+    template <int C, int K>
+    __device__ __forceinline__ void prop_chunks(const double *pl, const double *x, int m) {
+        if constexpr (K < C) {
+            double P[NV];
+#pragma unroll
+            for (int v = 0; v < NV; ++v)
+                if (K + 16 * v / MB < C) {
+                    const int row = rk[v] & 255, k = K + (rk[v] >> 8);
+                    const bool in = row < m && k < m;
+                    const double p = pl[in ? row + k * m : 0];
+                    P[v] = in ? p : 0.0;
+                }
+            if constexpr (MB <= 8)
+                fmac_block<MB, 0, C>(acc, P, x, std::make_integer_sequence<int, C>{});
+            else
+                rows<CH, 0>(P, x + K, C);
+            prop_chunks<C, K + CH>(pl, x, m);
+        }
+    }
+    template <int C>
+    __device__ __forceinline__ void store(double *d) const {
+        if constexpr (C == 1) {
+            d[0] = acc[0];
+        } else {
+#pragma unroll
+            for (int k = 0; k < C; k += 2) *(d2 *)(d + k) = d2{acc[k], acc[k + 1]};
+        }
     }
 };
+
+// Join words of a packet: first and second steps of its slots.
+template <int SL>
+struct Joins {
+    uint32_t first[SL], second[SL];
+    // byte: of the lane's first word; step: from one block of joins to the next
+    __device__ __forceinline__ void load(const uint32_t *words, uint32_t byte, uint32_t step, bool two) {
+#pragma unroll
+        for (int o = 0; o < SL; ++o) first[o] = word_at(words, byte + 4u * o);
+        if (two) {
+#pragma unroll
+            for (int o = 0; o < SL; ++o) second[o] = word_at(words, byte + step + 4u * o);
+        }
+    }
+};
+
+// The blocks of the packet whose records are in hd, into next (one register: read without
+// asking whether the slot has a block, the first one then).
+template <typename W, typename V, int O>
+__device__ __forceinline__ void fetch_ops(W &w, const V *ops, uint32_t hd) {
+    if constexpr (O < W::SL) {
+        const uint32_t shape = rlane(hd, 8 * O + 1);
+        if (W::NV == 1 || (rlane(hd, 8 * O) & ARC_TIMES))
+            w.template fetch_op<O>(ops, rlane(hd, 8 * O + 2), (int)((shape >> 8) & 255), (int)(shape >> 16));
+        fetch_ops<W, V, O + 1>(w, ops, hd);
+    }
+}
+
+// What a slot needs besides its record.
+template <typename V>
+struct SlotArgs {
+    const char *lds;
+    V *st;
+    const V *pl, *ops;
+    int col, lg;
+};
+
+// Joins and product of slot O, sources of stride C.
+template <typename V, int MB, int O, int C>
+__device__ __forceinline__ void slot_joins(Walk<V, MB> &w, const Joins<Walk<V, MB>::SL> &jw, const SlotArgs<V> &x,
+                                           uint32_t fl, uint32_t blk, int str) {
+    const uint32_t coff = (uint32_t)(x.col * C) * (uint32_t)sizeof(V), q = jw.first[O];
+    join<C>(w.y, value_at<V>(x.lds, q), state_at<V>(x.lds, q, coff));
+    if (fl & ARC_SECOND) {
+        const uint32_t r = jw.second[O];
+        join<C>(w.y, value_at<V>(x.lds, r), state_at<V>(x.lds, r, coff));
+    }
+    if (fl & ARC_TIMES) w.template product<O, C>(x.ops, blk, str);
+}
+// The end of a tile of stride C: propagator and store.
+template <typename V, int MB, int C>
+__device__ __forceinline__ void slot_store(Walk<V, MB> &w, const SlotArgs<V> &x, uint32_t prop, int rows, uint32_t to,
+                                           int lanes) {
+    if (prop != kNone) w.template propagate<C>(x.pl + prop, rows);
+    const int lane = threadIdx.x & 63;
+    if (lane < lanes) w.template store<C>(x.st + to + lane * C);
+    w.clear();
+}
+
+// Slots O .. of a packet; false after the segment's last one.
+template <typename V, int MB, int O>
+__device__ __forceinline__ bool run_slots(Walk<V, MB> &w, const Joins<Walk<V, MB>::SL> &jw, uint32_t hd,
+                                          const SlotArgs<V> &x) {
+    if constexpr (O < Walk<V, MB>::SL) {
+        const uint32_t fl = rlane(hd, 8 * O), shape = rlane(hd, 8 * O + 1), blk = rlane(hd, 8 * O + 2);
+        const int str = (int)((shape >> 8) & 255), ss = (int)(shape >> 16);
+        if (fl & (ARC_BARRIER | ARC_END | ARC_IDLE)) {
+            if (fl & ARC_BARRIER) __syncthreads();
+            if (fl & ARC_END) return false;
+        }
+#define QIW_STRIDE(S, CALL)                     \
+  {                                             \
+    if constexpr (MB <= 8) {                    \
+        if (S == 4) CALL(4);                    \
+        else if (S == 6) CALL(6);               \
+        else if (S == 1) CALL(1);               \
+        else if (S == 2) CALL(2);               \
+        else CALL(8);                           \
+    } else if constexpr (MB <= 20) {            \
+        if (S == 20) CALL(20);                  \
+        else if (S == 16) CALL(16);             \
+        else if (S == 8) CALL(8);               \
+        else if (S == 4) CALL(4);               \
+        else CALL(12);                          \
+    } else {                                    \
+        if (S <= 8) {                           \
+            if (S == 4) CALL(4);                \
+            else CALL(8);                       \
+        } else if (S <= 16) {                   \
+            if (S == 12) CALL(12);              \
+            else CALL(16);                      \
+        } else if (S <= 24) {                   \
+            if (S == 20) CALL(20);              \
+            else CALL(24);                      \
+        } else if (S == 28) CALL(28);           \
+        else CALL(32);                          \
+    }                                           \
+  }
+#define QIW_JOINS(C) slot_joins<V, MB, O, C>(w, jw, x, fl, blk, str)
+        if (!(fl & ARC_IDLE)) QIW_STRIDE(ss, QIW_JOINS)
+        if (fl & ARC_STORE) {
+            const uint32_t to = rlane(hd, 8 * O + 3), prop = rlane(hd, 8 * O + 4);
+            const int rows = (int)(shape & 255), lanes = (int)(rlane(hd, 8 * O + 5) << x.lg);
+#define QIW_STORE(C) slot_store<V, MB, C>(w, x, prop, rows, to, lanes)
+            QIW_STRIDE(str, QIW_STORE)
+        }
+#undef QIW_JOINS
+#undef QIW_STORE
+#undef QIW_STRIDE
+        return run_slots<V, MB, O + 1>(w, jw, hd, x);
+    }
+    return true;
+}
 
 // i*P element e of the cell c from the float64 table.
 __device__ __forceinline__ double prop_element(const double *ptab, int bt, const GridCell &c, int e) {
@@ -269,22 +463,29 @@ __device__ __forceinline__ double prop_element(const double *ptab, int bt, const
     return cell_value(c, c.d > 0 ? r0[e - bt] : 0.0, r0[e], r0[e + bt]);
 }
 
-// The arc walk.  What bounds it: the products with the operator blocks (two thirds of the
-// floating-point work) and the LDS gathers that feed them; a stage's tiles are spread over
-// the workgroup's wavefronts, with one barrier per stage.  Why a workgroup per sample: the
-// states of one sample and column take up to 100 KB (order 4, blocks 1 4 6 4 1, float32), so
-// a lane cannot own a sample; states of one sector share operator and propagator, so both
-// are wavefront-uniform.  Measured against the walk of the assignment tries (one pass per
-// diagram): two-orbital step orders 0:4 at N = 2^11, float32 639 -> 43.6 ms; orders 0:3 at
-// N = 2^12, float64 144 -> 18.2 ms; three-orbital step orders 0:3 at N = 2^9, float32
-// 399 -> 54.8 ms.
+// The arc walk.  What bounds it: issue of the products (vector units 50 % busy, matrix cores
+// 30 to 40 % for float32), the LDS gathers that feed them (20 %) and the stages' barriers.  Why
+// a workgroup per sample: the states of one sample and column take up to 100 KB (order 4,
+// blocks 1 4 6 4 1, float32), so a lane cannot own a sample; states of one sector share
+// operator and propagator, so both are wavefront-uniform.  Measured against the walk of the
+// assignment tries (one pass per diagram): two-orbital solve on 50 points, orders 0:2 at
+// N = 2^10, float64 452 -> 24.5 ms; two-orbital step, orders 0:4 at N = 2^11, float32 636 -> 24.2
+// ms; orders 0:3 at N = 2^12, float64 142 -> 9.9 ms; three-orbital step, orders 0:3 at N =
+// 2^9, float32 402 -> 36.9 ms; orders 0:2 at N = 2^8, float64 63.7 -> 9.3 ms.  Of these the
+// first form of the walk reached 29.9, 43.6, 18.2, 54.8 and 28.8 ms: what it lost were branches
+// on every row and column (one in five instructions), operator blocks and joins read when they
+// were wanted (a load's whole latency each), stages waiting for one wavefront with a tile of
+// many operators, and for float64 operator elements through the scalar cache.
 //
 // One workgroup: the samples of a task one after the other; per sample the times, arc values
 // and propagators go to LDS once, then every segment (initial sector) of the task is walked
 // level by level.  The wavefronts share the tiles of a stage; a lane holds one column of one
 // state.  The closed state's columns are multiplied by the last propagator in float64.
+// Wavefronts per SIMD: float64 at MB = 8 takes three (168 registers, what spills is outside the
+// slots; 11.7 -> 9.9 ms against two), float32 of wide blocks two (no spills; 43.3 -> 37.2 ms
+// against four).
 template <typename V, int MB, int NT>
-__global__ __launch_bounds__(NT) void k_eval_arcs_t(ArcArgs aa) {
+__global__ __launch_bounds__(NT, MB == 8 && sizeof(V) == 8 ? 3 : 2) void k_eval_arcs_t(ArcArgs aa) {
     extern __shared__ __attribute__((aligned(16))) char lds[];
     const EvalArgs &a = aa.e;
     const int tid = threadIdx.x, nt = blockDim.x;
@@ -297,7 +498,7 @@ __global__ __launch_bounds__(NT) void k_eval_arcs_t(ArcArgs aa) {
     const uint32_t *words = reinterpret_cast<const uint32_t *>(a.prog + g.prog_off);
     double *tl = reinterpret_cast<double *>(lds);
     double *fin = reinterpret_cast<double *>(lds + b[4]);
-    V *dv = reinterpret_cast<V *>(lds + b[5]);
+    V *dv = reinterpret_cast<V *>(lds + kArcValuesAt);
     V *pl = reinterpret_cast<V *>(lds + b[6]);
     V *st = reinterpret_cast<V *>(lds + b[7]);
     const V *ops = reinterpret_cast<const V *>(aa.ops);
@@ -309,8 +510,6 @@ __global__ __launch_bounds__(NT) void k_eval_arcs_t(ArcArgs aa) {
     const int skip_w = (int)b[2];
     for (int e = tid; e < bt; e += nt) prow[e] = 0.0;
 
-    Walk<V, MB> w;
-    w.init(lane);
     const int n_here = g.sampled ? min(a.spt, g.n_samples - task.first_sample) : 1;
     for (int sr = 0; sr < n_here; ++sr) {
         const int64_t sample = (int64_t)task.first_sample + sr;
@@ -349,15 +548,14 @@ __global__ __launch_bounds__(NT) void k_eval_arcs_t(ArcArgs aa) {
             dv[2 + 2 * i] = v;
             dv[3 + 2 * i] = -v;
         }
-        for (int L = 2; L < n; ++L) {
-            V *dst = pl + (L - 2) * bt;
+        for (int i = tid; i < (n - 2) * bt; i += nt) {
+            const int L = 2 + i / bt, e = i - (L - 2) * bt;
             if (bare) {
                 double dt = tl[L] - tl[L - 1];
                 dt = dt > 0.0 ? dt : 0.0;
-                for (int e = tid; e < bt; e += nt) dst[e] = aa.emask[e] ? (V)exp(-dt * aa.ediag[e]) : (V)0;
+                pl[i] = aa.emask[e] ? (V)exp(-dt * aa.ediag[e]) : (V)0;
             } else {
-                const GridCell c = grid_cell(tl[L], tl[L - 1], inv_h, a.n_tau);
-                for (int e = tid; e < bt; e += nt) dst[e] = (V)prop_element(a.ptab, bt, c, e);
+                pl[i] = (V)prop_element(a.ptab, bt, grid_cell(tl[L], tl[L - 1], inv_h, a.n_tau), e);
             }
         }
         __syncthreads();
@@ -377,80 +575,68 @@ __global__ __launch_bounds__(NT) void k_eval_arcs_t(ArcArgs aa) {
             const ConstP<uint32_t> h = b + b[8 + sg];
             const uint32_t h0 = h[0];
             const int s0 = (int)(h0 & 255), m0 = (int)((h0 >> 8) & 255), lg = (int)(h0 >> 16), cg = 1 << lg;
-            const int n_stages = (int)h[1], m1 = (int)(h[2] & 255), str1 = (int)(h[2] >> 8);
-            const uint32_t rblk = h[3], rprop = h[4];
-            const int col = lane & (cg - 1), sl = lane >> lg;
+            const int m1 = (int)(h[1] & 255), str1 = (int)(h[1] >> 8);
+            const uint32_t rblk = h[2], rprop = h[3];
+            constexpr int SL = Walk<V, MB>::SL;
+            const int col = lane & (cg - 1);
+            const uint32_t jstep = 4u * (SL * (64u >> lg));  // bytes of a block of joins
             for (int c0 = 0; c0 < m0; c0 += cg) {
-                if (wave == 0) {  // position 1: unit columns, or columns of the operator B
-                    w.clear();
-                    w.clear_y();
-                    const int c = c0 + col;
-#pragma unroll
-                    for (int k = 0; k < MB; ++k) {
-                        V v = (V)0;
-                        if (k < m1 && c < m0) v = rblk == kNone ? (k == c ? (V)1 : (V)0) : ops_cm[rblk + c * m1 + k];
-                        w.y[k] = v;
-                    }
-                    w.add_y(MB);
-                    if (rprop != kNone)
-                        w.apply_prop(pl + rprop, m1);
-                    else
-                        w.keep();
-                    if (lane < cg) w.store(st + h[5] + lane * str1, str1);
-                }
-                __syncthreads();
-                for (int s = 0; s < n_stages; ++s) {
-                    const int n_tiles = (int)h[8 + 2 * s];
-                    const ConstP<uint32_t> tiles = b + h[8 + 2 * s + 1];
-                    for (int ti = wave; ti < n_tiles; ti += nw) {
-                        const uint32_t t0 = tiles[4 * ti], t1 = tiles[4 * ti + 1], t2 = tiles[4 * ti + 2];
-                        const ConstP<uint32_t> op = b + tiles[4 * ti + 3];
-                        const int n_ops = (int)(t0 & 255), rows = (int)((t0 >> 8) & 255), ns = (int)((t0 >> 16) & 255);
-                        const int str = (int)(t0 >> 24);
-                        const int sq = sl < ns ? sl : ns - 1;
-                        w.clear();
-                        w.clear_y();
-                        for (int oi = 0; oi < n_ops; ++oi) {
-                            const uint32_t blk = op[4 * oi], o1 = op[4 * oi + 1], wo = op[4 * oi + 2];
-                            const int ms = (int)(o1 & 255), ss = (int)((o1 >> 8) & 255), ne = (int)(o1 >> 16);
-                            const uint32_t *jw = words + wo + sq;
-                            uint32_t q = jw[0];
-                            for (int e = 0; e < ne; ++e) {
-                                const uint32_t qn = e + 1 < ne ? jw[(e + 1) * ns] : 0u;
-                                const V dvv = dv[q >> 20];
-                                const V *src = st + (q & 0xFFFFFu) + col * ss;
-                                if (e == 0)
-                                    join<MB, true>(w.y, dvv, src, ss);
-                                else
-                                    join<MB, false>(w.y, dvv, src, ss);
-                                q = qn;
-                            }
-                            if (blk == kNone)
-                                w.add_y(ms);
-                            else
-                                w.apply_op(ops, blk, rows, ms);
-                        }
-                        if (t2 != kNone)
-                            w.apply_prop(pl + t2, rows);
+                // the first packet and the second one's records, read ahead of the root
+                uint32_t rec = 4u * h[8 + 2 * wave] + 4u * lane;  // byte offsets in the program
+                uint32_t jat = 4u * h[9 + 2 * wave] + 4u * (SL * ((uint32_t)lane >> lg));
+                uint32_t hd = word_at(words, rec), hn = word_at(words, rec + 32u * SL);
+                const uint32_t part = lane < (int)h[5] ? words[h[6] + lane] : 0u;
+                Joins<SL> jw, jn;
+                bool two = rlane(hd, 6) != 0;
+                jw.load(words, jat, jstep, two);
+                Walk<V, MB> w;
+                w.init(lane);
+                fetch_ops<Walk<V, MB>, V, 0>(w, ops, hd);
+                w.rotate();
+                const SlotArgs<V> sa{lds, st, pl, ops, col, lg};
+                // position 1: unit columns, or columns of the operator B, times the propagator
+                // that follows
+                for (int i = tid; i < cg * str1; i += nt) {
+                    const int cc = i / str1, k = i - cc * str1, c = c0 + cc;
+                    V v = (V)0;
+                    if (k < m1 && c < m0) {
+                        if (rblk == kNone)
+                            v = rprop == kNone ? (k == c ? (V)1 : (V)0) : pl[rprop + k + c * m1];
+                        else if (rprop == kNone)
+                            v = ops_cm[rblk + c * m1 + k];
                         else
-                            w.keep();
-                        if (lane < ns * cg) w.store(st + t1 + lane * str, str);
+                            for (int j = 0; j < m1; ++j) v = fma(pl[rprop + k + j * m1], ops_cm[rblk + c * m1 + j], v);
                     }
-                    __syncthreads();
+                    st[h[4] + i] = v;
                 }
-                // the closed state's columns, its parts added in float64
-                const int np = (int)h[6];
-                const ConstP<uint32_t> parts = b + h[7];
-                const int stf = n_stages == 0 ? str1 : aa.stride[s0];
-                for (int i = tid; i < m0 * cg; i += nt) {
+                for (;;) {
+                    // the next packet, and the records of the one after it
+                    rec += 32u * SL;
+                    jat += two ? 2u * jstep : jstep;
+                    two = rlane(hn, 6) != 0;
+                    const uint32_t h2 = word_at(words, rec + 32u * SL);
+                    jn.load(words, jat, jstep, two);
+                    fetch_ops<Walk<V, MB>, V, 0>(w, ops, hn);
+                    if (!run_slots<V, MB, 0>(w, jw, hd, sa)) break;
+                    hd = hn;
+                    hn = h2;
+                    jw = jn;
+                    w.rotate();
+                }
+                // the closed state's columns, its parts (one per lane) added in float64; no other
+                // state lies where the closed ones do, so the next pass may start
+                const int np = (int)h[5], stf = aa.stride[s0];
+                for (int i = wave; i < m0 * cg; i += nw) {
                     const int c = i / m0, r = i - c * m0;
-                    if (c0 + c >= m0) continue;
-                    double v = 0.0;
-                    for (int p = 0; p < np; ++p) v += (double)st[parts[p] + c * stf + r];
-                    fin[(c0 + c) * m0 + r] = v;
+                    if (c0 + c >= m0) break;
+                    double v = lane < np ? (double)st[part + c * stf + r] : 0.0;
+                    for (int p = lane + 64; p < np; p += 64) v += (double)st[words[h[6] + p] + c * stf + r];
+#pragma unroll
+                    for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d, 64);
+                    if (lane == 0) fin[(c0 + c) * m0 + r] = v;
                 }
-                __syncthreads();
             }
+            __syncthreads();
             // out[s0] += weight * iP_n[s0] * closed state, in float64
             const int o = aa.bt_off[s0];
             const GridCell cn = grid_cell(tl[n], tl[n - 1], inv_h, a.n_tau);
@@ -468,8 +654,9 @@ __global__ __launch_bounds__(NT) void k_eval_arcs_t(ArcArgs aa) {
                 mag += fabs(v);
                 prow[o + i] += wt * v;
             }
-            __syncthreads();
+            // fin is written again only after the next segment's first barrier
         }
+        __syncthreads();
         if (a.per_sample) {
 #pragma unroll
             for (int d = 32; d > 0; d >>= 1) mag += __shfl_xor(mag, d, 64);
@@ -720,12 +907,12 @@ __global__ __launch_bounds__(256, 3) void k_eval_sarcs_t(EvalArgs a) {
 // Vector length of the instantiation for blocks up to mb, and the most wavefronts a
 // workgroup of it can have (its registers).
 int qiw_arc_rows(int mb) { return mb <= 8 ? 8 : mb <= 20 ? 20 : 32; }
-int qiw_arc_waves(int mb, int fp32) { return mb <= 8 ? 16 : (mb <= 20 && fp32) ? 16 : 8; }
+int qiw_arc_waves(int mb, int fp32) { return mb <= 8 && fp32 ? 16 : 8; }
 
 hipError_t qiw_launch_eval_arcs(hipStream_t st, const ArcArgs &a, int n_tasks, int mb, int fp32, int waves, size_t lds) {
     if (n_tasks < 1 || mb > 32 || a.e.n_tau < 2) return hipErrorInvalidValue;
-    if (mb <= 8) return fp32 ? launch<float, 8, 1024>(st, a, n_tasks, waves, lds) : launch<double, 8, 1024>(st, a, n_tasks, waves, lds);
-    if (mb <= 20) return fp32 ? launch<float, 20, 1024>(st, a, n_tasks, waves, lds) : launch<double, 20, 512>(st, a, n_tasks, waves, lds);
+    if (mb <= 8) return fp32 ? launch<float, 8, 1024>(st, a, n_tasks, waves, lds) : launch<double, 8, 512>(st, a, n_tasks, waves, lds);
+    if (mb <= 20) return fp32 ? launch<float, 20, 512>(st, a, n_tasks, waves, lds) : launch<double, 20, 512>(st, a, n_tasks, waves, lds);
     return fp32 ? launch<float, 32, 512>(st, a, n_tasks, waves, lds) : launch<double, 32, 512>(st, a, n_tasks, waves, lds);
 }
 

@@ -631,22 +631,21 @@ ArcModel arc_model(const HostModel &m, int corr) {
     return a;
 }
 
-// Slice registers of the float32 operator blocks (64 floats each) in the instantiation for
-// the model's blocks.
-int arc_slice_regs(const HostModel &m) {
+// Elements of a stored operator block in the instantiation for the model's blocks: float32
+// slice registers (64 floats each), or float64 blocks padded to its size.
+uint32_t arc_block_size(const HostModel &m, bool fp32) {
     const int mb = qiw_arc_rows(m.mmax);
-    return (mb / 4 * mb + 15) / 16;
+    return fp32 ? 64u * (uint32_t)((mb / 4 * mb + 15) / 16) : (uint32_t)(mb * mb);
 }
 
 ArcBlocks arc_blocks(const HostModel &m, int corr, int precision) {
     ArcBlocks o;
-    const uint32_t per = 64u * (uint32_t)arc_slice_regs(m);
+    const uint32_t per = arc_block_size(m, precision == QIW_PREC_FP32);
     auto offsets = [&](const ScalarOp &op, bool column_major) {
         std::vector<uint32_t> v(m.ns, ARC_NONE);
         for (int s = 0; s < m.ns; ++s)
             if (op.blk[s] >= 0)
-                v[s] = column_major || precision == QIW_PREC_FP64 ? (uint32_t)m.op_desc[3 * op.blk[s]]
-                                                                  : per * (uint32_t)op.blk[s];
+                v[s] = column_major ? (uint32_t)m.op_desc[3 * op.blk[s]] : per * (uint32_t)op.blk[s];
         return v;
     };
     for (int p = 0; p < m.np; ++p) {
@@ -657,6 +656,7 @@ ArcBlocks arc_blocks(const HostModel &m, int corr, int precision) {
         o.a = offsets(m.corr_A[corr], false);
         o.b = offsets(m.corr_B[corr], true);  // the root reads columns of B
     }
+    o.id = per * (uint32_t)(m.op_desc.size() / 3);  // past the operators' blocks
     return o;
 }
 
@@ -669,6 +669,7 @@ struct ArcShape {
     int tiles;
 };
 constexpr ArcShape kArcShapes[] = {{1, 20 << 10, 2}, {4, 53 << 10, 12}, {8, 80 << 10, 32}, {16, 160 << 10, 1 << 30}};
+constexpr ArcShape kArcShapesWide[] = {{4, 53 << 10, 3}, {8, 80 << 10, 12}, {8, 160 << 10, 1 << 30}};  // mmax > 8
 
 // Algorithmic real FLOPs of one sample of a compiled group: the scalar walk's multiply per
 // trie edge and leaf, or the block programs' chain products.
@@ -709,6 +710,7 @@ int compile_arcs(const HostModel &m, int kind, int order, int n_after, int corr,
     const int max_waves = qiw_arc_waves(m.mmax, fp32 ? 1 : 0);
     ArcLayout l;
     l.elem = fp32 ? 4 : 8;
+    l.slots = arc_slots(qiw_arc_rows(m.mmax), fp32);
     l.mmax = m.mmax;
     l.bt = m.bt;
     l.bt_off.assign(m.bt_off.begin(), m.bt_off.end());
@@ -719,10 +721,14 @@ int compile_arcs(const HostModel &m, int kind, int order, int n_after, int corr,
         if (!arc_graph(am, kind, order, n_after, s0, {}, kind == QIW_G_BOLD && order > 0, g)) return 1;
         for (const auto &lev : g.levels) widest = std::max(widest, lev.size());
     }
+    const bool wide = m.mmax > 8;
+    const ArcShape *shapes = wide ? kArcShapesWide : kArcShapes;
+    const int n_shapes = wide ? 3 : 4;
     ArcGroupProgram pg;
     int rc = 2;
     for (int n_fixed = 0; n_fixed <= order && rc == 2; ++n_fixed)
-        for (const ArcShape &sh : kArcShapes) {
+        for (int i = 0; i < n_shapes; ++i) {
+            const ArcShape &sh = shapes[i];
             if (n_fixed == 0 && (widest + 63) / 64 > (size_t)sh.tiles) continue;
             l.waves = std::min(sh.waves, max_waves);
             l.cap = sh.cap;
@@ -1608,62 +1614,64 @@ int ensure_model_buffers(qiw_ctx *c, double **dcoef, int32_t **dkind, double **e
     return 0;
 }
 
-// Device tables of the arc walk: the operator blocks (float32: column-major and as slice
-// registers; float64: column-major, padded past the end), E + lambda and the layout of the
-// blocks.  Staged once per model and precision (synchronous copies).
+// Device tables of the arc walk: the operator blocks (as the products read them, and
+// column-major), E + lambda and the layout of the blocks.  Staged once per model and
+// precision (synchronous copies).
 int stage_arcs(qiw_ctx *c, int precision, ArcArgs *aa) {
     const HostModel &m = c->m;
     const bool fp32 = precision == QIW_PREC_FP32;
-    const size_t pad = 64, nb = m.op_desc.size() / 3, regs = (size_t)arc_slice_regs(m);
+    const size_t pad = 64, nb = m.op_desc.size() / 3, per = arc_block_size(m, fp32), el = fp32 ? 4 : 8;
     int rc = 0;
-    float *sl = fp32 ? (float *)dev(c, "arc.slices", std::max<size_t>(nb, 1) * regs * 64 * 4, &rc) : nullptr;
-    float *cm32 = fp32 ? (float *)dev(c, "arc.ops32", (m.op_data.size() + pad) * 4, &rc) : nullptr;
-    double *cm64 = fp32 ? nullptr : (double *)dev(c, "arc.ops", (m.op_data.size() + pad) * 8, &rc);
+    void *blocks = dev(c, fp32 ? "arc.slices" : "arc.blocks", (nb + 1) * per * el, &rc);
+    void *cm = dev(c, fp32 ? "arc.ops32" : "arc.ops", (m.op_data.size() + pad) * el, &rc);
     double *ediag = (double *)dev(c, "arc.ediag", (size_t)m.bt * 8, &rc);
     uint8_t *emask = (uint8_t *)dev(c, "arc.emask", (size_t)m.bt, &rc);
     int32_t *lay = (int32_t *)dev(c, "arc.layout", ((size_t)m.bt + 3 * m.ns) * 4, &rc);
     if (rc) return rc;
     if (!(c->arc_staged & (fp32 ? 2 : 1))) {
         HIPCHK(c, hipStreamSynchronize(c->stream));
-        std::vector<double> o(m.op_data);
+        const int mb = qiw_arc_rows(m.mmax);
+        std::vector<double> o(m.op_data), s((nb + 1) * per, 0.0);
         o.resize(m.op_data.size() + pad, 0.0);
+        auto at = [&](size_t b, int i, int k) -> double & {  // element (i, k) of a block
+            const int slice = (i / 4) * mb + k;              // float32: slice registers
+            return s[b * per + (fp32 ? (size_t)(slice / 16) * 64 + 4 * (slice % 16) + i % 4 : (size_t)k * mb + i)];
+        };
+        for (size_t b = 0; b < nb; ++b) {
+            const int off = m.op_desc[3 * b], mf = m.op_desc[3 * b + 1], mi = m.op_desc[3 * b + 2];
+            for (int i = 0; i < mf; ++i)
+                for (int k = 0; k < mi; ++k) at(b, i, k) = m.op_data[off + i + k * mf];
+        }
+        for (int i = 0; i < mb; ++i) at(nb, i, i) = 1.0;
         if (fp32) {
-            const int mb = qiw_arc_rows(m.mmax);
-            std::vector<float> o32(o.begin(), o.end()), s((size_t)std::max<size_t>(nb, 1) * regs * 64, 0.f);
-            for (size_t b = 0; b < nb; ++b) {
-                const int off = m.op_desc[3 * b], mf = m.op_desc[3 * b + 1], mi = m.op_desc[3 * b + 2];
-                for (int i = 0; i < mf; ++i)
-                    for (int k = 0; k < mi; ++k) {
-                        const int slice = (i / 4) * mb + k;
-                        s[(b * regs + slice / 16) * 64 + 4 * (slice % 16) + i % 4] = (float)m.op_data[off + i + k * mf];
-                    }
-            }
-            HIPCHK(c, hipMemcpy(sl, s.data(), s.size() * 4, hipMemcpyHostToDevice));
-            HIPCHK(c, hipMemcpy(cm32, o32.data(), o32.size() * 4, hipMemcpyHostToDevice));
+            const std::vector<float> s32(s.begin(), s.end()), o32(o.begin(), o.end());
+            HIPCHK(c, hipMemcpy(blocks, s32.data(), s32.size() * 4, hipMemcpyHostToDevice));
+            HIPCHK(c, hipMemcpy(cm, o32.data(), o32.size() * 4, hipMemcpyHostToDevice));
         } else {
-            HIPCHK(c, hipMemcpy(cm64, o.data(), o.size() * 8, hipMemcpyHostToDevice));
+            HIPCHK(c, hipMemcpy(blocks, s.data(), s.size() * 8, hipMemcpyHostToDevice));
+            HIPCHK(c, hipMemcpy(cm, o.data(), o.size() * 8, hipMemcpyHostToDevice));
         }
         std::vector<double> ed((size_t)m.bt, 0.0);
         std::vector<uint8_t> mk((size_t)m.bt, 0);
         std::vector<int32_t> l((size_t)m.bt + 3 * m.ns);
-        for (int s = 0; s < m.ns; ++s) {
-            const int d = m.dims[s];
-            for (int e = 0; e < d * d; ++e) l[m.bt_off[s] + e] = s;
+        for (int q = 0; q < m.ns; ++q) {
+            const int d = m.dims[q];
+            for (int e = 0; e < d * d; ++e) l[m.bt_off[q] + e] = q;
             for (int i = 0; i < d; ++i) {
-                ed[m.bt_off[s] + i + i * d] = m.E[s][i] + m.lambda0;
-                mk[m.bt_off[s] + i + i * d] = 1;
+                ed[m.bt_off[q] + i + i * d] = m.E[q][i] + m.lambda0;
+                mk[m.bt_off[q] + i + i * d] = 1;
             }
-            l[m.bt + s] = d;
-            l[m.bt + m.ns + s] = m.bt_off[s];
-            l[m.bt + 2 * m.ns + s] = arc_stride(d, m.mmax);
+            l[m.bt + q] = d;
+            l[m.bt + m.ns + q] = m.bt_off[q];
+            l[m.bt + 2 * m.ns + q] = arc_stride(d, m.mmax);
         }
         HIPCHK(c, hipMemcpy(ediag, ed.data(), ed.size() * 8, hipMemcpyHostToDevice));
         HIPCHK(c, hipMemcpy(emask, mk.data(), mk.size(), hipMemcpyHostToDevice));
         HIPCHK(c, hipMemcpy(lay, l.data(), l.size() * 4, hipMemcpyHostToDevice));
         c->arc_staged |= fp32 ? 2 : 1;
     }
-    aa->ops = fp32 ? (const void *)sl : (const void *)cm64;
-    aa->ops_cm = fp32 ? (const void *)cm32 : (const void *)cm64;
+    aa->ops = blocks;
+    aa->ops_cm = cm;
     aa->ediag = ediag;
     aa->emask = emask;
     aa->sector_of = lay;

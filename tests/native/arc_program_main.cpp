@@ -80,6 +80,7 @@ int main(int argc, char **argv) {
     l.bt = off[m.ns];
     l.bt_off.assign(off.begin(), off.end() - 1);
     l.waves = waves;
+    l.slots = arc_slots(l.mmax <= 8 ? 8 : l.mmax <= 20 ? 20 : 32, elem == 4);
     l.cap = cap;
     std::vector<std::vector<double>> blocks;  // operator blocks, named by index
     std::vector<std::pair<int, int>> shape;
@@ -92,6 +93,7 @@ int main(int argc, char **argv) {
         shape.push_back({m.dims[to], m.dims[from]});
         return (uint32_t)blocks.size() - 1;
     };
+    ob.id = 1u << 30;
     for (int p = 0; p < m.np; ++p) {
         std::vector<int> h, t;
         std::vector<uint32_t> hb, tb;
@@ -216,8 +218,8 @@ int main(int argc, char **argv) {
     };
     const size_t region = (pg.lds - at(7)) / elem;
     if (pg.lds > l.cap) die("more LDS than the cap");
-    if (at(4) != 128 || at(5) % 16 || at(6) % 16 || at(7) % 16) die("alignment");
-    const size_t dv_size = (at(6) - at(5)) / elem, prop_size = (at(7) - at(6)) / elem;
+    if (at(5) != kArcValuesAt || at(4) % 16 || at(6) % 16 || at(7) % 16) die("alignment");
+    const size_t dv_size = (at(4) - at(5)) / elem, prop_size = (at(7) - at(6)) / elem;
     std::vector<double> dv(2 + 2 * at(1));
     if (dv.size() > dv_size) die("arc values");
     dv[1] = 1.0;
@@ -261,52 +263,105 @@ int main(int argc, char **argv) {
                     }
                 return y;
             };
-            const int m1 = at(h + 2) & 255, str1 = at(h + 2) >> 8;
+            const int m1 = at(h + 1) & 255, str1 = at(h + 1) >> 8, per = 64 >> lg;
             for (int col = 0; col < cg; ++col) {
                 std::vector<double> x(m1, 0.0);
                 for (int k = 0; k < m1; ++k)
                     if (c0 + col < m0)
-                        x[k] = at(h + 3) == ARC_NONE ? (k == c0 + col) : blocks.at(at(h + 3)).at((c0 + col) * m1 + k);
-                if (at(h + 4) != ARC_NONE) x = times(at(h + 4), m1, x);
-                for (int k = 0; k < m1; ++k) put(at(h + 5) + col * str1 + k, x[k]);
+                        x[k] = at(h + 2) == ARC_NONE ? (k == c0 + col) : blocks.at(at(h + 2)).at((c0 + col) * m1 + k);
+                if (at(h + 3) != ARC_NONE) x = times(at(h + 3), m1, x);
+                for (int k = 0; k < str1; ++k) put(at(h + 4) + col * str1 + k, k < m1 ? x[k] : 0.0);
             }
             int stf = str1;
-            for (uint32_t s = 0; s < at(h + 1); ++s) {
-                const uint32_t n_tiles = at(h + kArcSegHead + 2 * s);
-                const size_t tiles = at(h + kArcSegHead + 2 * s + 1);
+            // of each wavefront: slot and block of joins it has come to
+            std::vector<size_t> pos(waves, 0), joins(waves), packet(waves, ~(size_t)0), second(waves, 0);
+            std::vector<std::vector<std::vector<double>>> acc(waves), y(waves);  // per lane
+            for (int w = 0; w < waves; ++w) {
+                joins[w] = at(h + kArcSegHead + 2 * w + 1);
+                if (at(h + kArcSegHead + 2 * w) % 64 || joins[w] % 64) die("stream alignment");
+                acc[w].assign(64, {});
+                y[w].assign(64, {});
+            }
+            const size_t block = (size_t)l.slots * per;  // words of a block of joins
+            for (bool more = true; more;) {  // a stage: every wavefront's slots up to its next barrier
                 std::vector<std::pair<size_t, double>> writes;
-                for (uint32_t ti = 0; ti < n_tiles; ++ti) {
-                    const uint32_t t0 = at(tiles + 4 * ti);
-                    const int n_ops = t0 & 255, rows = (t0 >> 8) & 255, ns = (t0 >> 16) & 255, str = t0 >> 24;
-                    if (ns < 1 || ns > (64 >> lg) || str != arc_stride(rows, l.mmax)) die("tile");
-                    for (int lane = 0; lane < ns * cg; ++lane) {
-                        const int col = lane & (cg - 1), sl = lane >> lg;
-                        std::vector<double> acc(rows, 0.0);
-                        for (int oi = 0; oi < n_ops; ++oi) {
-                            const size_t o = at(tiles + 4 * ti + 3) + 4 * oi;
-                            const int ms = at(o + 1) & 255, ss = (at(o + 1) >> 8) & 255, ne = at(o + 1) >> 16;
-                            std::vector<double> y(ms, 0.0);
-                            for (int e = 0; e < ne; ++e) {
-                                const uint32_t q = at(at(o + 2) + e * ns + sl);
-                                for (int k = 0; k < ms; ++k) {
-                                    const double v = get((q & 0xFFFFF) + col * ss + k);
-                                    if (std::isnan(v)) die("state read before it is written");
-                                    y[k] += dv.at(q >> 20) * v;
+                std::vector<std::pair<size_t, int>> reads;
+                for (int w = 0; w < waves; ++w) {
+                    for (bool first = true;; first = false) {
+                        const size_t rec = at(h + kArcSegHead + 2 * w), pk = pos[w] / l.slots, o = pos[w] % l.slots;
+                        const size_t r = rec + kArcSlotWords * pos[w];
+                        if (packet[w] != pk) {
+                            if (packet[w] != ~(size_t)0) joins[w] += (1 + second[w]) * block;
+                            packet[w] = pk;
+                            second[w] = at(rec + kArcSlotWords * l.slots * pk + 6);
+                            if (second[w] > 1) die("packet");
+                        }
+                        const uint32_t fl = at(r);
+                        if (first != ((fl & ARC_BARRIER) != 0)) {
+                            if (first) die("no barrier at a stage");
+                            break;
+                        }
+                        if (fl & ARC_END) {
+                            if (w > 0 && more) die("wavefronts end apart");
+                            more = false;
+                            // what the wavefront reads ahead: two packets of records, one of joins
+                            (void)at(rec + kArcSlotWords * l.slots * (pk + 2) + 63);
+                            for (int i = 0; i < l.slots; ++i)  // blocks are fetched one packet ahead
+                                if (at(rec + kArcSlotWords * (l.slots * (pk + 1) + i)) & ARC_TIMES) die("block past the end");
+                            (void)at(joins[w] + 4 * block - 1);
+                            break;
+                        }
+                        if (!more) die("wavefronts end apart");
+                        pos[w]++;
+                        if (fl & ARC_IDLE) continue;
+                        const int rows = at(r + 1) & 255, str = (at(r + 1) >> 8) & 255, ss = at(r + 1) >> 16;
+                        const int ns = at(r + 5);
+                        if (str != arc_stride(rows, l.mmax)) die("stride");
+                        if ((fl & ARC_SECOND) && !second[w]) die("no second steps");
+                        if ((fl & ARC_STORE) && !(fl & ARC_TIMES)) die("sum left over");
+                        for (int lane = 0; lane < 64; ++lane) {
+                            const int col = lane & (cg - 1), sl = lane >> lg;
+                            std::vector<double> &v = y[w][lane], &x = acc[w][lane];
+                            if (v.empty()) v.assign(ss, 0.0);
+                            if ((int)v.size() != ss) die("continued sum");
+                            for (int e = 0; e < (fl & ARC_SECOND ? 2 : 1); ++e) {
+                                const uint32_t q = at(joins[w] + e * block + sl * l.slots + o);
+                                for (int k = 0; k < ss; ++k) {  // the walk reads whole strides
+                                    const size_t byte = (q & 0xFFFF) * 4;
+                                    if ((q & 0xF0000) || byte < at(7) || (byte - at(7)) % elem) die("state address");
+                                    const size_t i = (byte - at(7)) / elem + col * ss + k;
+                                    const double sv = get(i);
+                                    if (std::isnan(sv)) die("state read before it is written");
+                                    reads.push_back({i, 0});
+                                    v[k] += dv.at(q >> 20) * sv;
                                 }
                             }
-                            const uint32_t blk = at(o);
-                            if (blk == ARC_NONE) {
-                                for (int k = 0; k < ms; ++k) acc[k] += y[k];
-                            } else {
-                                if (shape.at(blk) != std::make_pair(rows, ms)) die("operator shape");
-                                for (int k = 0; k < ms; ++k)
-                                    for (int i = 0; i < rows; ++i) acc[i] += blocks[blk][i + k * rows] * y[k];
+                            if (x.empty()) x.assign(rows, 0.0);
+                            if ((int)x.size() != rows) die("rows of a tile");
+                            if (fl & ARC_TIMES) {
+                                const uint32_t blk = at(r + 2);
+                                if (blk == ob.id) {
+                                    if (ss != str) die("identity");
+                                    for (int k = 0; k < ss; ++k)
+                                        if (k < rows) x[k] += v[k];
+                                } else {
+                                    const int ms = shape.at(blk).second;
+                                    if (shape[blk].first != rows || arc_stride(ms, l.mmax) != ss) die("operator shape");
+                                    for (int k = 0; k < ms; ++k)
+                                        for (int i = 0; i < rows; ++i) x[i] += blocks[blk][i + k * rows] * v[k];
+                                }
+                                v.clear();
                             }
+                            if (!(fl & ARC_STORE)) continue;
+                            if (ns < 1 || ns > per) die("tile");
+                            if (lane < (ns << lg)) {
+                                std::vector<double> d = at(r + 4) != ARC_NONE ? times(at(r + 4), rows, x) : x;
+                                for (int k = 0; k < str; ++k)
+                                    writes.push_back({at(r + 3) + lane * str + k, k < rows ? d[k] : 0.0});
+                            }
+                            x.clear();
+                            stf = str;
                         }
-                        if (at(tiles + 4 * ti + 2) != ARC_NONE) acc = times(at(tiles + 4 * ti + 2), rows, acc);
-                        for (int k = 0; k < str; ++k)
-                            writes.push_back({at(tiles + 4 * ti + 1) + lane * str + k, k < rows ? acc[k] : 0.0});
-                        stf = str;
                     }
                 }
                 // a stage may not write what it reads: the new states are stored after all reads
@@ -315,23 +370,14 @@ int main(int argc, char **argv) {
                     if (w.first >= region || hit[w.first]) die("two states in one place");
                     hit[w.first] = 1;
                 }
-                for (uint32_t ti = 0; ti < n_tiles; ++ti) {
-                    const uint32_t t0 = at(tiles + 4 * ti);
-                    for (uint32_t oi = 0; oi < (t0 & 255); ++oi) {
-                        const size_t o = at(tiles + 4 * ti + 3) + 4 * oi;
-                        const int ms = at(o + 1) & 255, ss = (at(o + 1) >> 8) & 255, ne = at(o + 1) >> 16;
-                        for (uint32_t i = 0; i < ne * ((t0 >> 16) & 255); ++i)
-                            for (int col = 0; col < cg; ++col)
-                                for (int k = 0; k < ms; ++k)
-                                    if (hit[(at(at(o + 2) + i) & 0xFFFFF) + col * ss + k]) die("a stage overwrites its source");
-                    }
-                }
+                for (auto &q : reads)
+                    if (hit[q.first]) die("a stage overwrites its source");
                 for (auto &w : writes) put(w.first, w.second);
             }
             for (int col = 0; col < cg && c0 + col < m0; ++col) {
                 std::vector<double> x(m0, 0.0);
-                for (uint32_t p = 0; p < at(h + 6); ++p)
-                    for (int k = 0; k < m0; ++k) x[k] += get(at(at(h + 7) + p) + col * stf + k);
+                for (uint32_t p = 0; p < at(h + 5); ++p)
+                    for (int k = 0; k < m0; ++k) x[k] += get(at(at(h + 6) + p) + col * stf + k);
                 for (int i = 0; i < m0; ++i)
                     for (int q = 0; q < m0; ++q)
                         res[off[s0] + i + (c0 + col) * m0] += prop[n][off[s0] + i + q * m0] * x[q];
