@@ -179,6 +179,7 @@ struct FinalizeArgs {
     int n_order_slots;
     const double *partial;             // [rows][bt]
     int bt;                            // outputs per row (sum m^2)
+    int most_rows;                     // most rows of a group
     const int32_t *diag_idx;           // [n_diag] BT indices of diagonal elements
     int n_diag;
     double *ptab;                      // [n_tau][bt] i*P (differential step: the self-energy table)
@@ -192,7 +193,7 @@ struct FinalizeArgs {
     double tau_w, tau_f;               // step times (tau_i = 0)
     int bare;                          // RootTransform Jacobian (initial step)
     int normalize;                     // apply normalize!(P, tau_f)
-    double *scratch;                   // [n_order_slots][bt]
+    double *scratch;                   // [n_real][2][bt] randomized qMC: mean and deviation of each group
     double *gsum;                      // [n_groups][bt] per-group sums of the partial rows
     unsigned *done;                    // blocks of the step launch that have finished (0 between launches)
     // randomized qMC (k_step_reduce_finalize_rqmc): the groups above are the sequences of

@@ -824,6 +824,9 @@ inline bool tasks_fit(Batch &b, int64_t more) {
     return !b.overflow;
 }
 
+// Most task rows of a group (the reduction's block is sized by it).
+int most_rows(const Batch &b) { return b.g_count.empty() ? 0 : *std::max_element(b.g_count.begin(), b.g_count.end()); }
+
 struct DevBatch {
     QiwGroup *groups = nullptr;
     QiwTask *tasks = nullptr;
@@ -2291,7 +2294,8 @@ int run_inchworm(qiw_ctx *c, const qiw_run *run, bool do_bare, int first_w, int 
     double *ptab = (double *)dev(c, "ptab", (size_t)m.ntau * m.bt * 8, &rc);
     double *porders = (double *)dev(c, "porders", (size_t)n_slots * m.ntau * m.bt * 8, &rc);
     double *lam = (double *)dev(c, "lambda", (size_t)m.ntau * 8, &rc);
-    double *scratch = (double *)dev(c, "fin.scratch", (size_t)n_slots * m.bt * 8, &rc);
+    double *scratch = (double *)dev(c, "fin.scratch",
+                                    std::max(bare_b.r_first.size(), bold_b.r_first.size()) * 2 * m.bt * 8 + 8, &rc);
     double *gsum = (double *)dev(c, "fin.gsum",
                                  (size_t)std::max(bare_b.groups.size(), bold_b.groups.size()) * m.bt * 8 + 8, &rc);
     int32_t *diag = (int32_t *)dev(c, "diag", (size_t)m.bt * 4, &rc);
@@ -2367,6 +2371,7 @@ int run_inchworm(qiw_ctx *c, const qiw_run *run, bool do_bare, int first_w, int 
         fa.groups = bare_d.groups;
         fa.group_task_first = bare_d.g_first;
         fa.group_task_count = bare_d.g_count;
+        fa.most_rows = most_rows(bare_b);
         fa.group_order_slot = bare_d.g_slot;
         fa.n_groups = (int)bare_b.groups.size();
         fa.jf = fa.jt = 1;
@@ -2389,6 +2394,7 @@ int run_inchworm(qiw_ctx *c, const qiw_run *run, bool do_bare, int first_w, int 
         fa.groups = bold_d.groups;
         fa.group_task_first = bold_d.g_first;
         fa.group_task_count = bold_d.g_count;
+        fa.most_rows = most_rows(bold_b);
         fa.group_order_slot = bold_d.g_slot;
         fa.n_groups = (int)bold_b.groups.size();
         fa.bare = 0;
@@ -2725,7 +2731,7 @@ int run_diff(qiw_ctx *c, const qiw_run *run, double *S_out, double *S_std_out) {
     double *sig = (double *)dev(c, "diff.sigma", tab * 8, &rc);
     double *porders = (double *)dev(c, "porders", (size_t)n_slots * tab * 8, &rc);
     double *pstd = rqmc ? (double *)dev(c, "porders_std", (size_t)n_slots * tab * 8, &rc) : nullptr;
-    double *scratch = (double *)dev(c, "fin.scratch", (size_t)n_slots * m.bt * 8, &rc);
+    double *scratch = (double *)dev(c, "fin.scratch", b.r_first.size() * 2 * m.bt * 8 + 8, &rc);
     double *gsum = (double *)dev(c, "fin.gsum", std::max<size_t>(b.groups.size(), 1) * m.bt * 8, &rc);
     double *hdiag = (double *)dev(c, "diff.hdiag", (size_t)m.bt * 8, &rc);
     int32_t *ddims = (int32_t *)dev(c, "diff.dims", (size_t)m.ns * 4, &rc);
@@ -2751,6 +2757,7 @@ int run_diff(qiw_ctx *c, const qiw_run *run, double *S_out, double *S_std_out) {
     fa.groups = d.groups;
     fa.group_task_first = d.g_first;
     fa.group_task_count = d.g_count;
+    fa.most_rows = most_rows(b);
     fa.group_order_slot = d.g_slot;
     fa.n_groups = (int)b.groups.size();
     fa.n_order_slots = n_slots;

@@ -1486,57 +1486,76 @@ struct KahanSum {
     }
 };
 
-// Sum over the task rows of each group, one block per group (and per 256 elements when
-// bt > 256).  The rows of a group are contiguous, so the block reads them as one
-// contiguous range: thread t covers element t % bt of rows t / bt, t / bt + R, ... with R
-// = 256 / bt rows per pass, and the R partial sums of each element are then added in a
-// fixed order, so the result does not depend on scheduling.  Both stages are compensated.
-__device__ void reduce_rows_block(const int32_t *__restrict__ first, const int32_t *__restrict__ count,
-                                  const double *__restrict__ partial, int bt, double *__restrict__ gsum) {
-    __shared__ double red[256], cmp[256];
-    const int g = blockIdx.x, t = threadIdx.x;
-    const int f0 = first[g], nr = count[g];
-    const int R = bt <= 256 ? 256 / bt : 1;     // rows per pass
-    const int e = bt <= 256 ? t % bt : blockIdx.y * 256 + t;
-    const int r0 = bt <= 256 ? t / bt : 0;
-    // four independent compensated sums over rows r0, r0 + R, ... (round robin), so four
-    // loads are in flight at a time; combined in a fixed order
-    KahanSum k4[4];
-    if (r0 < R && e < bt) {
-        const double *p = partial + (int64_t)(f0 + r0) * bt + e;
-        const int64_t step = (int64_t)R * bt;
-        int r = r0;
-        for (; r + 3 * R < nr; r += 4 * R, p += 4 * step) {
-            const double x0 = p[0], x1 = p[step], x2 = p[2 * step], x3 = p[3 * step];
-            k4[0].add(x0);
-            k4[1].add(x1);
-            k4[2].add(x2);
-            k4[3].add(x3);
-        }
-        for (int q = 0; r < nr; r += R, p += step, ++q) k4[q].add(p[0]);
-    }
-    KahanSum k;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        k.add(k4[q].s);
-        k.add(-k4[q].c);
-    }
-    red[t] = k.s;
-    cmp[t] = k.c;
-    __syncthreads();
-    if (t < (bt <= 256 ? bt : 256) && e < bt) {
-        KahanSum v;
-        for (int q = 0; q < R; ++q) {
-            const int i = q * (bt <= 256 ? bt : 0) + t;
-            v.add(red[i]);
-            v.add(-cmp[i]);
-        }
-        gsum[(int64_t)g * bt + e] = v.s;
-    }
+// Adds two compensated sums (each s - c), with the rounding error of the addition in c.
+__device__ __forceinline__ void add_sums(double &s, double &c, double s2, double c2) {
+    const double t = s + s2, b = t - s;
+    c = c + c2 - ((s - (t - b)) + (s2 - b));
+    s = t;
 }
 
-// Step bookkeeping on the per-group sums gsum, run by one block of 256 threads.  gsum is
-// read through a volatile pointer: other blocks of the same launch wrote it.  The group
+// Sum over the task rows of each group, one block per group (and per 256 elements when
+// bt > 256).  The rows of a group are contiguous, so the block reads them as one
+// contiguous range: thread t covers element t % E of rows t / E, t / E + R, ... with E
+// elements per block and R = threads / E rows per pass; eight compensated sums per thread, so
+// that eight loads are in flight.  The sums of an element are then added pairwise in a fixed
+// order, so the result does not depend on scheduling.  What bounds it: the latency of the
+// passes, so a launch of many rows takes 1024 threads (reduce_threads).
+constexpr int kReduceMax = 1024, kReduceLoads = 8;
+__device__ void reduce_rows_block(const int32_t *__restrict__ first, const int32_t *__restrict__ count,
+                                  const double *__restrict__ partial, int bt, double *__restrict__ gsum) {
+    __shared__ double red[kReduceMax], cmp[kReduceMax];
+    const int g = blockIdx.x, t = threadIdx.x;
+    const int f0 = first[g], nr = count[g];
+    const int e0 = blockIdx.y * 256, E = min(bt - e0, 256);
+    const int R = (int)blockDim.x / E;  // rows per pass
+    const int e = t % E, r0 = t / E;
+    KahanSum k[kReduceLoads];
+    if (r0 < R) {
+        const double *p = partial + (int64_t)f0 * bt + e0 + e;
+        for (int r = r0; r < nr; r += kReduceLoads * R) {
+            double x[kReduceLoads];
+#pragma unroll
+            for (int q = 0; q < kReduceLoads; ++q) x[q] = r + q * R < nr ? p[(int64_t)(r + q * R) * bt] : 0.0;
+#pragma unroll
+            for (int q = 0; q < kReduceLoads; ++q) k[q].add(x[q]);
+        }
+    }
+#pragma unroll
+    for (int w = kReduceLoads / 2; w > 0; w /= 2)
+#pragma unroll
+        for (int q = 0; q < w; ++q) add_sums(k[q].s, k[q].c, k[q + w].s, k[q + w].c);
+    red[t] = k[0].s;
+    cmp[t] = k[0].c;
+    __syncthreads();
+    for (int n = R; n > 1;) {
+        const int h = (n + 1) / 2;
+        if (r0 < n - h) {
+            double s = red[t], c = cmp[t];
+            add_sums(s, c, red[t + h * E], cmp[t + h * E]);
+            red[t] = s;
+            cmp[t] = c;
+        }
+        n = h;
+        __syncthreads();
+    }
+    if (t < E) gsum[(int64_t)g * bt + e0 + t] = red[t] - cmp[t];
+}
+
+// The last block of a launch to get here (a counter every block increments after its sums are
+// visible); it resets the counter for the next launch and sees the sums of all blocks.
+__device__ __forceinline__ bool last_block(unsigned *done) {
+    __threadfence();
+    __syncthreads();
+    __shared__ int last;
+    if (threadIdx.x == 0) last = atomicAdd(done, 1u) == gridDim.x * gridDim.y - 1;
+    __syncthreads();
+    if (!last) return false;
+    if (threadIdx.x == 0) *done = 0u;
+    __threadfence();
+    return true;
+}
+
+// Step bookkeeping on the per-group sums gsum, run by the last block (last_block).  The group
 // prefactors are computed once per group (in parallel), each thread then sums its
 // elements over the groups in group order, per order slot in registers.
 constexpr int kFinMaxGroups = 64;
@@ -1557,29 +1576,44 @@ __device__ double step_group_factor(const QiwGroup &g, const FinalizeArgs &a) {
 
 // normalize!(P, tau_f) after row jf was stored (src/ppgf.jl:646-668): lambda from the
 // largest diagonal element of row jf, then every known row j scaled by exp(-tau_j lambda)
-// (one exp per row).
+// (one exp per row, kept in LDS for 256 rows at a time).
 __device__ void step_normalize(const FinalizeArgs &a) {
     const int tid = threadIdx.x, jf = a.jf;
     __threadfence_block();
     __syncthreads();
-    __shared__ double lam_sh;
-    if (tid == 0) {
+    __shared__ double lam_sh, scale[256];
+    if (tid < 64) {
         double pmax = -INFINITY;
-        for (int i = 0; i < a.n_diag; ++i) pmax = fmax(pmax, a.ptab[(int64_t)jf * a.bt + a.diag_idx[i]]);
-        lam_sh = log(pmax) / a.tau_f;
-        a.lambda_out[jf] = lam_sh;
+        for (int i = tid; i < a.n_diag; i += 64) pmax = fmax(pmax, a.ptab[(int64_t)jf * a.bt + a.diag_idx[i]]);
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) pmax = fmax(pmax, __shfl_xor(pmax, o, 64));
+        if (tid == 0) {
+            lam_sh = log(pmax) / a.tau_f;
+            a.lambda_out[jf] = lam_sh;
+        }
     }
     __syncthreads();
     const double lam = lam_sh;
-    for (int j = tid; j < a.n_known; j += blockDim.x) {
-        const double f = exp(-(j * a.h) * lam);
-        double *row = a.ptab + (int64_t)j * a.bt;
-        for (int e = 0; e < a.bt; ++e) row[e] *= f;
+    for (int j0 = 0; j0 < a.n_known; j0 += 256) {
+        const int nj = min(256, a.n_known - j0);
+        if (tid < nj) scale[tid] = exp(-((j0 + tid) * a.h) * lam);
+        __syncthreads();
+        double *rows = a.ptab + (int64_t)j0 * a.bt;
+        const int nv = nj * a.bt, nt = (int)blockDim.x;
+        for (int i = tid; i < nv; i += 4 * nt) {  // four loads in flight
+            double v[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) v[q] = i + q * nt < nv ? rows[i + q * nt] : 0.0;
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (i + q * nt < nv) rows[i + q * nt] = v[q] * scale[(i + q * nt) / a.bt];
+        }
+        __syncthreads();
     }
 }
 
 __device__ void finalize_step_body(const FinalizeArgs &a) {
-    const volatile double *gsum = a.gsum;
+    const double *gsum = a.gsum;
     const int tid = threadIdx.x;
     const int jf = a.jf;
     __shared__ double fac_sh[kFinMaxGroups];
@@ -1593,6 +1627,7 @@ __device__ void finalize_step_body(const FinalizeArgs &a) {
         double acc[kFinMaxSlots];
 #pragma unroll
         for (int o = 0; o < kFinMaxSlots; ++o) acc[o] = 0.0;
+#pragma unroll 8
         for (int gi = 0; gi < a.n_groups; ++gi) {
             const double v = fac_sh[gi] * gsum[(int64_t)gi * a.bt + e];
             const int sl = slot_sh[gi];
@@ -1612,19 +1647,13 @@ __device__ void finalize_step_body(const FinalizeArgs &a) {
     if (a.normalize) step_normalize(a);
 }
 
-// One launch per step: every block reduces its group's rows; the last block to finish
-// (a counter every block increments after its sums are visible) runs the bookkeeping and
-// resets the counter for the next step.  This saves a launch and its gap per step.
-__global__ __launch_bounds__(256) void k_step_reduce_finalize(FinalizeArgs a) {
+// One launch per step: every block reduces its group's rows; the last block to finish runs
+// the bookkeeping.  This saves a launch and its gap per step.  What bounds it: latency (a pass
+// of row loads, the counter, the groups' sums, the table's rows): 10.7 us for 256 rows of 4 in each
+// of 17 groups and 200 propagator rows (13.9 with volatile reads of the sums, one at a time).
+__global__ __launch_bounds__(kReduceMax) void k_step_reduce_finalize(FinalizeArgs a) {
     reduce_rows_block(a.group_task_first, a.group_task_count, a.partial, a.bt, a.gsum);
-    __threadfence();
-    __syncthreads();
-    __shared__ int last;
-    if (threadIdx.x == 0) last = atomicAdd(a.done, 1u) == gridDim.x * gridDim.y - 1;
-    __syncthreads();
-    if (!last) return;
-    if (threadIdx.x == 0) *a.done = 0u;
-    finalize_step_body(a);
+    if (last_block(a.done)) finalize_step_body(a);
 }
 
 // Correlator bookkeeping (src/inchworm.jl:825-889): per (pair, tau) row, sum the groups'
@@ -1817,77 +1846,143 @@ __global__ __launch_bounds__(256) void k_points_coords(const QiwGroup *__restric
     for (int k = 0; k < d; ++k) out[(int64_t)k * ng + r] = u[k];
 }
 
-// Step bookkeeping with randomized qMC (inchworm_step, src/inchworm.jl:172-195), one
-// block of 256 threads after all per-sequence sums are in gsum.  For each (order,
-// n_pts_after) group, the prefactor-scaled sums of its sequences are the samples; the
-// sequences are taken in order until, from the second on, the largest element of their
-// standard deviation is <= target_std.  The group adds the mean (sum * (1/n), as
-// SectorBlockMatrix / n) and the deviation over the sequences taken to its order's rows.
-// Thread t owns elements t, t + 256, ... throughout, so each element's sums run in group
-// order.
-__device__ void finalize_step_rqmc_body(const FinalizeArgs &a) {
-    const volatile double *gsum = a.gsum;
-    const int tid = threadIdx.x, jf = a.jf, bt = a.bt;
-    __shared__ double red[256];
-    for (int o = 0; o < a.n_order_slots; ++o)
-        for (int e = tid; e < bt; e += blockDim.x) {
-            a.porders[((int64_t)o * a.n_tau + jf) * bt + e] = 0.0;
-            a.porders_std[((int64_t)o * a.n_tau + jf) * bt + e] = 0.0;
-        }
-    for (int r = 0; r < a.n_real; ++r) {
-        const int base = a.real_first[r], cnt = a.real_count[r];
-        const QiwGroup g = a.groups[base];
-        const double fac = step_group_factor(g, a);
-        const int slot = a.group_order_slot[base];
-        const bool exact = qiw_group_exact(g);
-        const int nmax = exact ? 1 : a.n_seqs;
-        int nuse = nmax;
-        for (int n = 2; n <= nmax; ++n) {
-            double loc = 0.0;
-            for (int e = tid; e < bt; e += blockDim.x) {
-                auto x = [&](int s) { return __dmul_rn(fac, gsum[(int64_t)(base + (cnt > 1 ? s : 0)) * bt + e]); };
-                loc = fmax(loc, seq_std(x, n));
-            }
-            red[tid] = loc;
-            __syncthreads();
-            for (int w = 128; w > 0; w >>= 1) {
-                if (tid < w) red[tid] = fmax(red[tid], red[tid + w]);
-                __syncthreads();
-            }
-            const bool stop = red[0] <= a.target_std;
-            __syncthreads();
-            if (stop) {
-                nuse = n;
-                break;
-            }
-        }
-        if (a.nuse_out && tid == 0) a.nuse_out[(int64_t)jf * a.n_real + r] = nuse;
-        for (int e = tid; e < bt; e += blockDim.x) {
-            auto x = [&](int s) { return __dmul_rn(fac, gsum[(int64_t)(base + (cnt > 1 ? s : 0)) * bt + e]); };
-            const double mean = __dmul_rn(seq_sum(x, nuse), 1.0 / nuse);
-            const double sd = exact ? 0.0 : (nuse > 1 ? seq_std(x, nuse) : __builtin_nan(""));
-            a.porders[((int64_t)slot * a.n_tau + jf) * bt + e] += mean;  // after the group's mean is rounded
-            a.porders_std[((int64_t)slot * a.n_tau + jf) * bt + e] += sd;
-        }
+// Values of sequences 0 .. NS - 1 of one element in registers (n of them used), and the
+// statistics of seq_sum and seq_std on them with loops that unroll.
+template <int NS>
+struct SeqValues {
+    double v[NS];
+    __device__ __forceinline__ void load(const double *gsum, int64_t step, double fac, int n) {
+#pragma unroll
+        for (int s = 0; s < NS; ++s) v[s] = s < n ? __dmul_rn(fac, gsum[s * step]) : 0.0;
     }
-    for (int e = tid; e < bt; e += blockDim.x) {
+    __device__ __forceinline__ double sum(int n) const {
+#pragma clang fp contract(off)
+        double s = 0.0;
+#pragma unroll
+        for (int i = 0; i < NS; ++i) s = i < n ? s + v[i] : s;
+        return s;
+    }
+    __device__ __forceinline__ double std(int n) const {
+#pragma clang fp contract(off)
+        const double mean = sum(n) / n;
+        double q = 0.0;
+#pragma unroll
+        for (int i = 0; i < NS; ++i) {
+            const double d = v[i] - mean;
+            q = i < n ? q + d * d : q;
+        }
+        return sqrt(q / (n - 1));
+    }
+};
+// The same on values in memory, for more sequences than a thread keeps.
+template <>
+struct SeqValues<0> {
+    const double *p;
+    int64_t step;
+    double fac;
+    __device__ __forceinline__ void load(const double *gsum, int64_t step_, double fac_, int) {
+        p = gsum;
+        step = step_;
+        fac = fac_;
+    }
+    __device__ __forceinline__ double operator()(int s) const { return __dmul_rn(fac, p[s * step]); }
+    __device__ __forceinline__ double sum(int n) const { return seq_sum(*this, n); }
+    __device__ __forceinline__ double std(int n) const { return seq_std(*this, n); }
+};
+
+// Step bookkeeping with randomized qMC (inchworm_step, src/inchworm.jl:172-195), one
+// block after all per-sequence sums are in gsum.  For each (order, n_pts_after) group, the
+// prefactor-scaled sums of its sequences are the samples; the sequences are taken in order
+// until, from the second on, the largest element of their standard deviation is <=
+// target_std.  The group adds the mean (sum * (1/n), as SectorBlockMatrix / n) and the
+// deviation over the sequences taken to its order's rows, in group order.
+//
+// A thread takes one element of one group at a time, 64 groups side by side: first the
+// sequence counts whose deviation is above the target (one bit each; the element-wise
+// maximum is above it when any element's is), then mean and deviation into scratch
+// ([n_real][2][bt]), then the sums over the groups.  Group after group with a tree per
+// sequence count, as before, the launch took 280 us for 16 groups, eight sequences and two
+// elements (dependent loads and barriers); now 22 us.
+template <int NS>
+__device__ void finalize_step_rqmc_body(const FinalizeArgs &a) {
+    const int tid = threadIdx.x, nt = blockDim.x, jf = a.jf, bt = a.bt;
+    constexpr int NR = 64;
+    __shared__ unsigned long long above[NR];  // bit n - 1: n sequences deviate by more than the target
+    __shared__ double fac_sh[NR];
+    __shared__ int base_sh[NR], seqs_sh[NR];  // group, its sequences (1: exact)
+    __shared__ int64_t step_sh[NR];           // from one sequence to the next in gsum
+    double *stat = a.scratch;
+    for (int r0 = 0; r0 < a.n_real; r0 += NR) {
+        const int nr = min(NR, a.n_real - r0);
+        if (tid < nr) {
+            const int base = a.real_first[r0 + tid];
+            const QiwGroup g = a.groups[base];
+            above[tid] = 0ull;
+            fac_sh[tid] = step_group_factor(g, a);
+            base_sh[tid] = base;
+            seqs_sh[tid] = qiw_group_exact(g) ? 1 : a.n_seqs;
+            step_sh[tid] = a.real_count[r0 + tid] > 1 ? bt : 0;
+        }
+        __syncthreads();
+        for (int i = tid; i < nr * bt; i += nt) {
+            const int r = i / bt, e = i - r * bt, nmax = seqs_sh[r];
+            SeqValues<NS> x;
+            x.load(a.gsum + (int64_t)base_sh[r] * bt + e, step_sh[r], fac_sh[r], nmax);
+            unsigned long long over = 0ull;
+            for (int n = 2; n <= nmax; ++n)
+                if (x.std(n) > a.target_std) over |= 1ull << (n - 1);
+            if (over) atomicOr(&above[r], over);
+        }
+        __syncthreads();
+        for (int i = tid; i < nr * bt; i += nt) {
+            const int r = i / bt, e = i - r * bt, nmax = seqs_sh[r];
+            int nuse = nmax;
+            if (0.0 <= a.target_std)
+                for (int n = nmax; n >= 2; --n)
+                    if (!((above[r] >> (n - 1)) & 1ull)) nuse = n;
+            if (a.nuse_out && e == 0) a.nuse_out[(int64_t)jf * a.n_real + r0 + r] = nuse;
+            SeqValues<NS> x;
+            x.load(a.gsum + (int64_t)base_sh[r] * bt + e, step_sh[r], fac_sh[r], nuse);
+            const bool exact = qiw_group_exact(a.groups[base_sh[r]]);
+            double *s = stat + (int64_t)(r0 + r) * 2 * bt + e;
+            s[0] = __dmul_rn(x.sum(nuse), 1.0 / nuse);
+            s[bt] = exact ? 0.0 : (nuse > 1 ? x.std(nuse) : __builtin_nan(""));
+        }
+        __threadfence_block();
+        __syncthreads();
+    }
+    for (int i = tid; i < a.n_order_slots * bt; i += nt) {
+        const int o = i / bt, e = i - o * bt;
+        double mean = 0.0, sd = 0.0;
+#pragma unroll 8
+        for (int r = 0; r < a.n_real; ++r) {
+            const bool mine = a.group_order_slot[a.real_first[r]] == o;
+            const double v = stat[(int64_t)r * 2 * bt + e], w = stat[(int64_t)(2 * r + 1) * bt + e];
+            mean = mine ? mean + v : mean;
+            sd = mine ? sd + w : sd;
+        }
+        a.porders[((int64_t)o * a.n_tau + jf) * bt + e] = mean;
+        a.porders_std[((int64_t)o * a.n_tau + jf) * bt + e] = sd;
+    }
+    __threadfence_block();
+    __syncthreads();
+    for (int e = tid; e < bt; e += nt) {
         double tot = 0.0;
         for (int o = 0; o < a.n_order_slots; ++o) tot += a.porders[((int64_t)o * a.n_tau + jf) * bt + e];
         a.ptab[(int64_t)a.jt * bt + e] = tot;
     }
     if (a.normalize) step_normalize(a);
 }
+__device__ void finalize_step_rqmc(const FinalizeArgs &a) {
+    if (a.n_seqs <= 8)
+        finalize_step_rqmc_body<8>(a);
+    else
+        finalize_step_rqmc_body<0>(a);
+}
 
-__global__ __launch_bounds__(256) void k_step_reduce_finalize_rqmc(FinalizeArgs a) {
+__global__ __launch_bounds__(kReduceMax) void k_step_reduce_finalize_rqmc(FinalizeArgs a) {
     reduce_rows_block(a.group_task_first, a.group_task_count, a.partial, a.bt, a.gsum);
-    __threadfence();
-    __syncthreads();
-    __shared__ int last;
-    if (threadIdx.x == 0) last = atomicAdd(a.done, 1u) == gridDim.x * gridDim.y - 1;
-    __syncthreads();
-    if (!last) return;
-    if (threadIdx.x == 0) *a.done = 0u;
-    finalize_step_rqmc_body(a);
+    if (last_block(a.done)) finalize_step_rqmc(a);
 }
 
 // Euler step of diff_inchworm_step! (src/inchworm.jl:603-635) after the self-energy row
@@ -1895,42 +1990,54 @@ __global__ __launch_bounds__(256) void k_step_reduce_finalize_rqmc(FinalizeArgs 
 //   p(tau_{a+1}) = p(tau_a) + h (sum_j w_j sigma(tau_a - tau_j) p(tau_j) - H p(tau_a)),
 // w the trapezoid weights of kd.integrate over grid[0..a] (the contour measure -i dtau
 // turns Σ P into sigma p), H = diag(E + lambda).  Per element of each sector block.
+// The terms of the convolution are spread over the block (element after element, then the
+// next term) and added pairwise.
 __device__ void diff_euler(const FinalizeArgs &a) {
+    __shared__ double part[kReduceMax];
     __threadfence_block();
     __syncthreads();
-    const int A = a.a, bt = a.bt;
-    for (int e = threadIdx.x; e < bt; e += blockDim.x) {
+    const int A = a.a, bt = a.bt, t = threadIdx.x;
+    for (int e0 = 0; e0 < bt; e0 += 256) {
+        const int E = min(bt - e0, 256), parts = (int)blockDim.x / E, q = t / E, e = e0 + t % E;
         int s = 0;
         while (s + 1 < a.ns && a.bt_off[s + 1] <= e) ++s;
         const int m = a.dims[s], o = a.bt_off[s], r = (e - o) % m, c = (e - o) / m;
         double conv = 0.0;
-        for (int j = 0; j <= A && A > 0; ++j) {
-            const double w = (j == 0 || j == A) ? 0.5 * a.h : a.h;
-            const double *S = a.ptab + (int64_t)(A - j) * bt + o;
-            const double *Pj = a.P + (int64_t)j * bt + o;
-            double t = 0.0;
-            for (int l = 0; l < m; ++l) t += S[r + l * m] * Pj[l + c * m];
-            conv += w * t;
+        if (q < parts && A > 0) {
+#pragma unroll 4
+            for (int j = q; j <= A; j += parts) {
+                const double w = (j == 0 || j == A) ? 0.5 * a.h : a.h;
+                const double *S = a.ptab + (int64_t)(A - j) * bt + o;
+                const double *Pj = a.P + (int64_t)j * bt + o;
+                double v = 0.0;
+                for (int l = 0; l < m; ++l) v += S[r + l * m] * Pj[l + c * m];
+                conv += w * v;
+            }
         }
-        const double pp = a.P[(int64_t)A * bt + e];
-        a.P[(int64_t)(A + 1) * bt + e] = pp + a.h * (conv - a.hdiag[o + r * (m + 1)] * pp);
+        part[t] = conv;
+        __syncthreads();
+        for (int n = parts; n > 1;) {
+            const int h = (n + 1) / 2;
+            if (q < n - h) part[t] += part[t + h * E];
+            n = h;
+            __syncthreads();
+        }
+        if (t < E) {
+            const double pp = a.P[(int64_t)A * bt + e];
+            a.P[(int64_t)(A + 1) * bt + e] = pp + a.h * (part[t] - a.hdiag[o + r * (m + 1)] * pp);
+        }
+        __syncthreads();
     }
 }
 
 // One launch per differential step: per-group row sums, then (last workgroup) the
 // self-energy bookkeeping as for an inchworm step (ptab = sigma table, no normalization)
 // and the Euler step.
-__global__ __launch_bounds__(256) void k_diff_reduce_finalize(FinalizeArgs a, int rqmc) {
+__global__ __launch_bounds__(kReduceMax) void k_diff_reduce_finalize(FinalizeArgs a, int rqmc) {
     reduce_rows_block(a.group_task_first, a.group_task_count, a.partial, a.bt, a.gsum);
-    __threadfence();
-    __syncthreads();
-    __shared__ int last;
-    if (threadIdx.x == 0) last = atomicAdd(a.done, 1u) == gridDim.x * gridDim.y - 1;
-    __syncthreads();
-    if (!last) return;
-    if (threadIdx.x == 0) *a.done = 0u;
+    if (!last_block(a.done)) return;
     if (rqmc)
-        finalize_step_rqmc_body(a);
+        finalize_step_rqmc(a);
     else
         finalize_step_body(a);
     diff_euler(a);
@@ -2120,9 +2227,17 @@ hipError_t qiw_launch_eval_block(hipStream_t st, const BlockArgs &b, int n_tasks
     return hipGetLastError();
 }
 
+// Grid and threads of a launch that reduces task rows.  256 threads take 2048 values in one
+// pass of loads; above that the passes are what takes time and 1024 threads take a quarter of
+// them (9 groups of 1024 rows of 70 elements: 55 -> 25 us; below, the wider block only adds to
+// the last block's barriers).
+static dim3 reduce_grid(const FinalizeArgs &a) { return dim3(a.n_groups, (a.bt + 255) / 256); }
+static dim3 reduce_threads(const FinalizeArgs &a) {
+    return dim3((int64_t)a.most_rows * (a.bt < 256 ? a.bt : 256) > 256 * kReduceLoads ? kReduceMax : 256);
+}
+
 hipError_t qiw_launch_finalize_step(hipStream_t st, const FinalizeArgs &a) {
-    hipLaunchKernelGGL(k_step_reduce_finalize, dim3(a.n_groups, a.bt <= 256 ? 1 : (a.bt + 255) / 256), dim3(256), 0,
-                       st, a);
+    hipLaunchKernelGGL(k_step_reduce_finalize, reduce_grid(a), reduce_threads(a), 0, st, a);
     return hipGetLastError();
 }
 
@@ -2133,15 +2248,13 @@ hipError_t qiw_launch_finalize_corr(hipStream_t st, const CorrFinalizeArgs &a) {
 
 hipError_t qiw_launch_finalize_step_rqmc(hipStream_t st, const FinalizeArgs &a) {
     if (a.n_seqs < 1 || a.n_seqs > QIW_MAX_SEQS) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_step_reduce_finalize_rqmc, dim3(a.n_groups, a.bt <= 256 ? 1 : (a.bt + 255) / 256),
-                       dim3(256), 0, st, a);
+    hipLaunchKernelGGL(k_step_reduce_finalize_rqmc, reduce_grid(a), reduce_threads(a), 0, st, a);
     return hipGetLastError();
 }
 
 hipError_t qiw_launch_finalize_diff(hipStream_t st, const FinalizeArgs &a, int rqmc) {
     if (a.n_seqs < 1 || a.n_seqs > QIW_MAX_SEQS || a.normalize) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_diff_reduce_finalize, dim3(a.n_groups, a.bt <= 256 ? 1 : (a.bt + 255) / 256), dim3(256), 0,
-                       st, a, rqmc);
+    hipLaunchKernelGGL(k_diff_reduce_finalize, reduce_grid(a), reduce_threads(a), 0, st, a, rqmc);
     return hipGetLastError();
 }
 

@@ -1,0 +1,61 @@
+"""Step bookkeeping (row sums, order sums, sequence statistics, normalization, Euler step) at
+the edges of its work mapping, against the float64 oracle: sequence counts kept in registers
+(8) and read from memory (9, 17), reductions of 256 and of 1024 threads, blocks of 2, 4 and 70
+elements, more than 256 propagator rows.  Tolerance 1e-10 relative, as for every float64 path;
+a deviation's error is bounded by 1e-10 of the samples' scale."""
+import numpy as np
+import pytest
+
+import oracle_lib as O
+import qiw
+from qiw import model
+
+pytestmark = pytest.mark.gpu
+RTOL = 1e-10
+MODELS = {"level": lambda n_tau: model.bethe_single_level(n_tau, 10.0),
+          "orbital": lambda n_tau: model.anderson_single_orbital(n_tau=n_tau),
+          "blocks": lambda n_tau: model.kanamori(2, 2.0, 0.2, -1.0, 10.0, n_tau, 0.5)}
+
+
+def rel(a, b):
+    return np.linalg.norm((np.asarray(a) - np.asarray(b)).ravel()) / np.linalg.norm(np.asarray(b).ravel())
+
+
+def std_close(s_gpu, s_cpu, mean_cpu):
+    scale = np.abs(mean_cpu).max() + np.abs(s_cpu).max()
+    return np.abs(np.asarray(s_gpu) - np.asarray(s_cpu)).max() <= RTOL * scale
+
+
+@pytest.mark.parametrize("which,order,log2n,n_seqs,target", [
+    ("level", 3, 5, 8, 0.0), ("level", 3, 5, 9, 0.0), ("orbital", 2, 6, 17, 1e-3), ("orbital", 3, 4, 8, 1e-3),
+    ("blocks", 2, 2, 8, 1e-2), ("blocks", 1, 3, 9, 1e-3)])
+def test_sequences(which, order, log2n, n_seqs, target):
+    eg, ec = MODELS[which](8), MODELS[which](8)
+    orders, N = range(0, order + 1), 2 ** log2n
+    Po_g, Ps_g = qiw.inchworm(eg, eg.grid, orders, orders, N, rand_params=qiw.RandomizationParams(7, n_seqs, target))
+    P_c, Po_c, Ps_c = O.inchworm(ec, orders, orders, N, rand=(n_seqs, 1, 7, target))
+    assert rel(eg.P, P_c) < RTOL
+    for o in orders:
+        assert np.abs(Po_g[o] - Po_c[o]).max() < RTOL * np.abs(P_c).max()
+        assert std_close(Ps_g[o], Ps_c[o], Po_c[o])
+
+
+@pytest.mark.parametrize("which,n_tau,order,log2n", [("level", 4, 2, 16), ("orbital", 4, 1, 16), ("blocks", 4, 1, 9)])
+def test_many_rows(which, n_tau, order, log2n):
+    eg, ec = MODELS[which](n_tau), MODELS[which](n_tau)
+    orders = range(0, order + 1)
+    qiw.inchworm(eg, eg.grid, orders, orders, 2 ** log2n)
+    P_c, Po_c, _ = O.inchworm(ec, orders, orders, 2 ** log2n)
+    assert rel(eg.P, P_c) < RTOL
+
+
+@pytest.mark.parametrize("which,n_tau", [("level", 300), ("blocks", 40)])
+def test_many_times(which, n_tau):
+    eg, ec = MODELS[which](n_tau), MODELS[which](n_tau)
+    qiw.inchworm(eg, eg.grid, range(0, 2), range(0, 2), 4)
+    P_c, _, _ = O.inchworm(ec, range(0, 2), range(0, 2), 4)
+    assert rel(eg.P, P_c) < RTOL
+    eg, ec = MODELS[which](n_tau), MODELS[which](n_tau)
+    S_g, _ = qiw.diff_inchworm(eg, eg.grid, range(1, 3), 4)
+    P_c, S_c = O.diff_inchworm(ec, range(1, 3), 4)[:2]
+    assert rel(eg.P, P_c) < RTOL
