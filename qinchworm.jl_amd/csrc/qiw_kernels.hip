@@ -20,16 +20,18 @@
 // Sobol points (ScrambledSobolSeq next!, src/scrambled_sobol.jl:158-173) in closed form:
 // x_i = x_0 xor (xor over the set bits j of gray(i) of m[:, j]), then ldexp(x, -32).
 // ---------------------------------------------------------------------------------------
-__device__ __forceinline__ uint32_t sobol_word(const uint32_t *__restrict__ m, uint32_t x0, int d,
-                                                uint64_t i) {
-    uint64_t g = i ^ (i >> 1);
+// bits: the words of i's Gray code that can be set (i < 2^bits, at most 32).
+__device__ __forceinline__ uint32_t sobol_word(const uint32_t *__restrict__ m, uint32_t x0, int d, uint64_t i,
+                                                int bits = 32) {
+    const uint32_t g = (uint32_t)(i ^ (i >> 1));
     uint32_t x = x0;
     const uint32_t *md = m + d * 32;
 #pragma unroll 4
-    for (int j = 0; j < 32; ++j)
-        if ((g >> j) & 1ull) x ^= md[j];
+    for (int j = 0; j < bits; ++j) x ^= md[j] & (uint32_t)__builtin_amdgcn_sbfe((int)g, (unsigned)j, 1u);
     return x;
 }
+// Bits of the indices below n (n >= 1).
+__device__ __forceinline__ int index_bits(int64_t n) { return n > 1 ? min(32, 64 - __clzll(n - 1)) : 0; }
 
 __global__ void k_sobol_points(const uint32_t *__restrict__ m, const uint32_t *__restrict__ x0, int dim,
                                int64_t first, int64_t n, double *__restrict__ out) {
@@ -39,6 +41,31 @@ __global__ void k_sobol_points(const uint32_t *__restrict__ m, const uint32_t *_
         out[r * dim + d] = ldexp((double)sobol_word(m, x0[d], d, (uint64_t)(first + r)), -32);
 }
 
+// x^(1/n) for a uniform n.  pow takes some 150 instructions, and the coordinates of a randomized
+// step are 100 roots per sample; here r = x^(-1/n) starts from the float32 exponential of the
+// float32 logarithm (error 2^-20) and takes two Newton steps r += r (1 - x r^n) / n (error
+// squared each time), then y = x r^(n-1) one on y itself, so its rounding errors do not add up:
+// y += (x - y^n) r^(n-1) / n.  Outside the float32 range (0 among it) pow.
+__device__ __forceinline__ double int_pow(double y, int n) {
+    double p = n & 1 ? y : 1.0;
+    for (n >>= 1; n; n >>= 1) {
+        y *= y;
+        if (n & 1) p *= y;
+    }
+    return p;
+}
+__device__ __forceinline__ double root_n(double x, int n) {
+    if (n == 1) return x;
+    if (n == 2) return sqrt(x);
+    const double inv = 1.0 / n;
+    if (!(x >= 0x1p-100 && x <= 0x1p100)) return pow(x, inv);
+    double r = (double)exp2f(-log2f((float)x) * (float)inv);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) r = fma(r * inv, fma(-x, int_pow(r, n), 1.0), r);
+    const double q = int_pow(r, n - 1), y = x * q;
+    return fma(q * inv, x - int_pow(y, n), y);
+}
+
 // Unscaled double-simplex coordinates u~ of DoubleSimplexRootTransform
 // (src/qmc_integrate.jl:425-449): the first d_after coordinates form the simplex after
 // tau_w, the remaining d_before the one before it.  RootTransform is d_before = 0.
@@ -46,12 +73,12 @@ __global__ void k_sobol_points(const uint32_t *__restrict__ m, const uint32_t *_
 __device__ __forceinline__ void root_map(const double *x, int d_after, int d_before, double *u) {
     int d = d_after + d_before;
     if (d_after > 0) {
-        u[0] = pow(x[0], 1.0 / d_after);
-        for (int i = 1; i < d_after; ++i) u[i] = u[i - 1] * pow(x[i], 1.0 / (d_after - i));
+        u[0] = root_n(x[0], d_after);
+        for (int i = 1; i < d_after; ++i) u[i] = u[i - 1] * root_n(x[i], d_after - i);
     }
     if (d_before > 0) {
-        u[d_after] = pow(x[d_after], 1.0 / d_before);
-        for (int i = d_after + 1; i < d; ++i) u[i] = u[i - 1] * pow(x[i], 1.0 / (d - i));
+        u[d_after] = root_n(x[d_after], d_before);
+        for (int i = d_after + 1; i < d; ++i) u[i] = u[i - 1] * root_n(x[i], d - i);
     }
 }
 
@@ -1733,6 +1760,10 @@ __device__ double seq_std(X x, int n) {
 // row p of the lower-triangular matrix holds entries (p, q < p) in bits 31 - q and 1 on
 // the diagonal; bit 31 - p of a scrambled direction number is the parity of row p AND the
 // plain one), then maps its samples as k_simplex_coords does.
+// What bounds it: the roots' float64 multiplies.  A block takes kRqmcSamples samples, so that
+// its scramble costs less than they do: 100 roots of eight times 2^12 samples take 23 us (52 with
+// pow, all 32 bits of every index, and 256 samples per block).
+constexpr int kRqmcSamples = 512;
 __global__ __launch_bounds__(256) void k_rqmc_coords(const QiwGroup *__restrict__ groups, const uint32_t *__restrict__ m,
                                                      int64_t n, uint64_t seed, uint64_t domain, uint64_t key,
                                                      double *__restrict__ ut) {
@@ -1763,19 +1794,25 @@ __global__ __launch_bounds__(256) void k_rqmc_coords(const QiwGroup *__restrict_
         ms[k * 32 + j] = v;
     }
     __syncthreads();
-    const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t ng = g.n_samples;  // <= n
-    if (r >= ng) return;
-    double x[2 * QIW_KMAX], u[2 * QIW_KMAX];
-    for (int k = 0; k < d; ++k) x[k] = ldexp((double)sobol_word(ms, rows[k][0], k, (uint64_t)r), -32);
+    const int bits = index_bits(ng);
     double *out = ut + g.ut_off;
-    if (sigma) {
-        sigma_row_values(x, g.order, u);
-        for (int k = 0; k < 2 * g.order; ++k) out[(int64_t)k * ng + r] = u[k];
-        return;
+    // the coordinates one after the other: u of the simplex, after tau_w and before it
+    for (int64_t r = (int64_t)blockIdx.x * kRqmcSamples + threadIdx.x; r < min(ng, (int64_t)(blockIdx.x + 1) * kRqmcSamples);
+         r += blockDim.x) {
+        const int after = sigma ? 0 : g.d_after, row0 = sigma ? 1 : 0;
+        double u = 1.0;
+        for (int k = 0; k < d; ++k) {
+            const double x = ldexp((double)sobol_word(ms, rows[k][0], k, (uint64_t)r, bits), -32);
+            const double y = root_n(x, k < after ? after - k : d - k);
+            u = k == 0 || k == after ? y : u * y;
+            out[(int64_t)(row0 + k) * ng + r] = u;
+        }
+        if (sigma) {  // pinned to tau_f_prev and tau_i (sigma_row_values)
+            out[r] = 1.0;
+            out[(int64_t)(d + 1) * ng + r] = 0.0;
+        }
     }
-    root_map(x, g.d_after, g.d_before, u);
-    for (int k = 0; k < d; ++k) out[(int64_t)k * ng + r] = u[k];
 }
 
 // Simplex coordinates from caller-drawn sequences (the states of the ScrambledSobolSeq
@@ -2289,7 +2326,7 @@ hipError_t qiw_launch_given_coords(hipStream_t st, const QiwGroup *groups, int n
 hipError_t qiw_launch_rqmc_coords(hipStream_t st, const QiwGroup *groups, int n_groups, int max_dim, int64_t n,
                                   const uint32_t *m, uint64_t seed, int domain, int64_t key, double *ut) {
     if (max_dim > 2 * QIW_KMAX || n_groups < 1 || n < 1) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_rqmc_coords, dim3((unsigned)((n + 255) / 256), (unsigned)n_groups), dim3(256), 0, st,
+    hipLaunchKernelGGL(k_rqmc_coords, dim3((unsigned)((n + kRqmcSamples - 1) / kRqmcSamples), (unsigned)n_groups), dim3(256), 0, st,
                        groups, m, n, seed, (uint64_t)domain, (uint64_t)key, ut);
     return hipGetLastError();
 }

@@ -3,12 +3,15 @@ the edges of its work mapping, against the float64 oracle: sequence counts kept 
 (8) and read from memory (9, 17), reductions of 256 and of 1024 threads, blocks of 2, 4 and 70
 elements, more than 256 propagator rows.  Tolerance 1e-10 relative, as for every float64 path;
 a deviation's error is bounded by 1e-10 of the samples' scale."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 import oracle_lib as O
 import qiw
-from qiw import model
+from qiw import abi, model
+from qiw.sobol import ScrambledSobolSeq
 
 pytestmark = pytest.mark.gpu
 RTOL = 1e-10
@@ -59,3 +62,17 @@ def test_many_times(which, n_tau):
     S_g, _ = qiw.diff_inchworm(eg, eg.grid, range(1, 3), 4)
     P_c, S_c = O.diff_inchworm(ec, range(1, 3), 4)[:2]
     assert rel(eg.P, P_c) < RTOL
+
+
+@pytest.mark.parametrize("n", range(1, 13))
+def test_roots(n):
+    """First simplex coordinate x^(1/n): half an ulp of the last rounding and up to one of the
+    correction before it, against extended precision (0 and 1 ulp at x = 0)."""
+    ctx, seq, N = qiw.context(), ScrambledSobolSeq(n), 4096
+    ctx.check(ctx.lib.qiw_set_sobol(ctx.h, n, abi.ptr(np.ascontiguousarray(seq.m), C.c_uint32),
+                                    abi.ptr(np.ascontiguousarray(seq.x0), C.c_uint32)))
+    out = np.zeros((N, n))
+    ctx.check(ctx.lib.qiw_simplex_points(ctx.h, 0, n, 0.0, 0.0, 1.0, N, out.ctypes.data_as(abi._f64p)))
+    x = np.asarray(seq.points(N))[:, 0].astype(np.longdouble)
+    y = np.where(x > 0, np.exp(np.log(np.where(x > 0, x, 1)) / n), 0)
+    assert np.all(np.abs(out[:, 0] - y) <= 1.5 * np.spacing(np.maximum(out[:, 0], 2.0 ** -40)))
