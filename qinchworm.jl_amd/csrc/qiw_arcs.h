@@ -832,9 +832,17 @@ inline int arc_compile(const ArcModel &m, const ArcLayout &l, const ArcBlocks &o
 //   4 propagators, 5 their offset, 6 scaled rows, 7 their offset, 8-11 program offsets of the
 //   wavefronts, 12-15 their lengths in blocks of 16 words
 //   arc      head | tail << 8, then the rows of tables 0, 1 and 2, 3 (16 bits each, 0xFFFF none)
-//   prop     first row (one per sector), segment, second segment of a product (0: none)
+//   prop     a pair of sectors s, s + 1 (s even; those with no state in either are left out):
+//            row of s | s << 16 | 1 << 24 if s + 1 is a sector (the next row), segment | second
+//            segment of a product << 8 (0: none)
 //   scaled   row, source row, constant row
+// A wavefront reads eight words past its program (zeros).
 constexpr int kScalarWaves = 4, kScalarSlots = 64, kScalarFree = 10, kScalarRows = 300;
+// Results that a wavefront stores, at least one per sector; rows of LDS before the times (the
+// results take the place of the first rows), and with the times of the positions 0 .. n.
+constexpr int scalar_out_rows(int ns) { return ns <= 2 ? 2 : ns <= 4 ? 4 : 8; }
+inline int scalar_table_rows(int rows, int ns) { return std::max(rows, kScalarWaves * scalar_out_rows(ns)); }
+inline int scalar_lds_rows(int rows, int ns, int n) { return scalar_table_rows(rows, ns) + std::max(n + 1, ns); }
 constexpr uint32_t SARC_SPECIAL = 1u << 31, SARC_MINUS = 1u << 30;
 
 // Operator matrix elements of a scalar model.
@@ -846,7 +854,7 @@ struct ArcValues {
 struct ScalarProgram {
     std::vector<uint32_t> blob;
     double leaves = 0, words = 0;
-    int rows = 0;
+    int rows = 0, slots = 0;  // LDS rows and register slots it needs
 };
 
 struct ScalarPacker {
@@ -1065,8 +1073,9 @@ inline int arc_compile_scalar(const ArcModel &m, const ArcValues &val, int kind,
             if (longest > (size_t)max_words) continue;
         }
         if (pk.rows.size() + m.ns > (size_t)kScalarRows) return 2;
-        // rows: constants, arcs, scaled rows, then one run of sectors per propagator segment
-        std::vector<int> at(pk.rows.size(), -1), prop_row(n + 1, -1);
+        // rows: constants, arcs, scaled rows, then the propagators by pairs of sectors
+        std::vector<int> at(pk.rows.size(), -1);
+        std::vector<std::array<int, 4>> prop_row(n + 1, std::array<int, 4>{-1, -1, -1, -1});
         int next = (int)pk.consts.size();
         for (size_t i = 0; i < pk.rows.size(); ++i) {
             const auto &r = pk.rows[i];
@@ -1077,11 +1086,12 @@ inline int arc_compile_scalar(const ArcModel &m, const ArcValues &val, int kind,
         for (size_t i = 0; i < pk.rows.size(); ++i) {
             const auto &r = pk.rows[i];
             if (r.kind != ScalarPacker::R_PROP) continue;
-            if (prop_row[r.a] < 0) {
-                prop_row[r.a] = next;
-                next += m.ns;
+            int &pair = prop_row[r.a][r.b / 2];
+            if (pair < 0) {
+                pair = next;
+                next += std::min(2, m.ns - r.b / 2 * 2);
             }
-            at[i] = prop_row[r.a] + r.b;
+            at[i] = pair + r.b % 2;
         }
         if (next > kScalarRows) return 2;
         std::vector<uint32_t> &b = out.blob;
@@ -1104,12 +1114,14 @@ inline int arc_compile_scalar(const ArcModel &m, const ArcValues &val, int kind,
         }
         b[5] = (uint32_t)b.size();
         for (int q = 0; q < n; ++q)
-            if (prop_row[q] >= 0) {
-                b[4]++;
-                b.push_back((uint32_t)prop_row[q]);
-                b.push_back((uint32_t)(q == n - 2 ? pos_w : q == n - 1 ? n : q + 2));
-                b.push_back((uint32_t)(q == n - 2 ? pos_w + 1 : 0));
-            }
+            for (int pair = 0; pair < 4; ++pair)
+                if (prop_row[q][pair] >= 0) {
+                    b[4]++;
+                    b.push_back((uint32_t)prop_row[q][pair] | (uint32_t)(2 * pair) << 16 |
+                                (2 * pair + 1 < m.ns ? 1u << 24 : 0u));
+                    b.push_back((uint32_t)(q == n - 2 ? pos_w | (pos_w + 1) << 8 : q == n - 1 ? n : q + 2));
+                }
+        if (b[4] > 64) return 2;  // one record per lane
         b[6] = (uint32_t)pk.scaled.size();
         b[7] = (uint32_t)b.size();
         for (const auto &sc : pk.scaled) {
@@ -1146,7 +1158,9 @@ inline int arc_compile_scalar(const ArcModel &m, const ArcValues &val, int kind,
             b[8 + w] = (uint32_t)b.size();
             b[12 + w] = (uint32_t)(prog[w].size() / 16);
             b.insert(b.end(), prog[w].begin(), prog[w].end());
+            for (uint32_t x : prog[w]) out.slots = std::max(out.slots, (int)(x & 255u) / 2 + 1);
         }
+        b.resize(b.size() + 16, 0u);  // zeros behind the last program; the others run into words or zeros
         out.leaves = leaves;
         out.rows = next;
         return 0;

@@ -683,25 +683,39 @@ hipError_t launch(hipStream_t st, const ArcArgs &a, int n_tasks, int waves, size
 // ---------------------------------------------------------------------------------------
 // The scalar arc walk (all sectors 1x1; programs of ScalarPacker, qiw_arcs.h)
 //
-// What bounds it: per program word one 512-byte LDS row read (4 cycles of the CU's LDS) and
-// three to four scalar instructions (one scalar unit per CU); the arithmetic is one float64
-// multiply-add per word.  Why states in registers read through the VGPR index mode: the
-// order-4 states of 64 samples (47 at a time) would fill 24 KB of LDS per wavefront and
-// double the LDS reads; an indexed multiply-add takes its source slot without a move.  The
-// compiler has no register array of 64 float64 values with a run-time index (its tuples end
-// at 16), so the loop is one assembly block on fixed registers:
-//   v[32:159] slots, v[14:15] accumulator, v[16:31] the rows of eight words, v10 v13 row
-//   addresses, v11 lane offset, v12 row mask; s[40:47] s[48:55] two half blocks of words.
-// Every load's wait is inside the block.  Measured against the walk of the assignment tries:
-// single-orbital solve (199 steps, orders 0:4, N = 2^14) 64.9 -> 20.0 ms, its evaluator 0.31
-// -> 0.08 ms per step; single-level step of orders 0:5 at N = 2^15 7.39 -> 0.68 ms.
+// What bounds it: for the order-4 programs of the single orbital (1900 words) the issue of six
+// to ten instructions per word, two of them scalar; for all smaller programs (16 to 400 words)
+// the set-up of the rows, whose gathers keep the address unit of the CU half busy.  Why states
+// in registers read through the VGPR index mode: the order-4 states of 64 samples (47 at a
+// time) would fill 24 KB of LDS per wavefront and double the LDS reads; an indexed multiply-add
+// takes its source slot without a move.  The compiler has no register array of 64 float64
+// values with a run-time index (its tuples end at 16), so the loop is one assembly block on
+// fixed registers:
+//   v[32:] slots, v[14:15] accumulator, v[16:23] v[24:31] the rows of four words each, v10 v13
+//   row addresses, v11 lane offset, v12 row mask; s[40:55] a ring of four times four words.
+// Rows and words of the next fours are read while four words are at work; every load's wait is
+// inside the block.
+//
+// SLOTS: programs of up to 24 slots (all but order 4 of the single orbital and order 6 of the
+// single level) run in 80 registers, six wavefronts per SIMD, the others in 168, three.
+// Measured against the walk of the assignment tries: single-orbital solve (199 steps, orders
+// 0:4, N = 2^14) 64.9 -> 18.0 ms, its evaluator 0.31 -> 0.078 ms per step; single-level step of
+// orders 0:5 at N = 2^15 7.4 -> 0.61 ms.  Of these the walk with one register count, rows and
+// gathers one after the other took 0.084 ms; three correlators of orders 0:3 on 200 points at
+// N = 2^14 went from 10.3 to 7.1 ms with both, a randomized step of the single level (orders
+// 0:4, eight times 2^12) from 67 to 39 us.  A launch takes one instantiation for all its groups:
+// with two launches of a step the small programs' own launch cost more than it gained (single
+// orbital 85 instead of 78 us per step).
 // ---------------------------------------------------------------------------------------
-#define QIW_SARC_VGPRS                                                                                              \
+constexpr int kScalarFew = 24;
+#define QIW_SARC_FEW                                                                                                \
     "v10", "v11", "v12", "v13", "v14", "v15", "v16", "v17", "v18", "v19", "v20", "v21", "v22", "v23", "v24", \
     "v25", "v26", "v27", "v28", "v29", "v30", "v31", "v32", "v33", "v34", "v35", "v36", "v37", "v38", "v39", \
     "v40", "v41", "v42", "v43", "v44", "v45", "v46", "v47", "v48", "v49", "v50", "v51", "v52", "v53", "v54", \
     "v55", "v56", "v57", "v58", "v59", "v60", "v61", "v62", "v63", "v64", "v65", "v66", "v67", "v68", "v69", \
-    "v70", "v71", "v72", "v73", "v74", "v75", "v76", "v77", "v78", "v79", "v80", "v81", "v82", "v83", "v84", \
+    "v70", "v71", "v72", "v73", "v74", "v75", "v76", "v77", "v78", "v79"
+#define QIW_SARC_MANY                                                                                               \
+    QIW_SARC_FEW, "v80", "v81", "v82", "v83", "v84",                                                          \
     "v85", "v86", "v87", "v88", "v89", "v90", "v91", "v92", "v93", "v94", "v95", "v96", "v97", "v98", "v99", \
     "v100", "v101", "v102", "v103", "v104", "v105", "v106", "v107", "v108", "v109", "v110", "v111", "v112", \
     "v113", "v114", "v115", "v116", "v117", "v118", "v119", "v120", "v121", "v122", "v123", "v124", "v125", \
@@ -711,161 +725,302 @@ hipError_t launch(hipStream_t st, const ArcArgs &a, int n_tasks, int waves, size
 #define QIW_ROW(w, a, lo, hi)                            \
     "v_and_or_b32 v" #a ", s" #w ", v12, v11\n"          \
     "ds_read_b64 v[" #lo ":" #hi "], v" #a "\n"
-#define QIW_ROWS(w0, w1, w2, w3, w4, w5, w6, w7)                                                                  \
-    QIW_ROW(w0, 10, 16, 17) QIW_ROW(w1, 13, 18, 19) QIW_ROW(w2, 10, 20, 21) QIW_ROW(w3, 13, 22, 23)               \
-    QIW_ROW(w4, 10, 24, 25) QIW_ROW(w5, 13, 26, 27) QIW_ROW(w6, 10, 28, 29) QIW_ROW(w7, 13, 30, 31)
-// a positive TERM falls through; the others run out of line and come back
+#define QIW_ROWS_A(w0, w1, w2, w3) \
+    QIW_ROW(w0, 10, 16, 17) QIW_ROW(w1, 13, 18, 19) QIW_ROW(w2, 10, 20, 21) QIW_ROW(w3, 13, 22, 23)
+#define QIW_ROWS_B(w0, w1, w2, w3) \
+    QIW_ROW(w0, 10, 24, 25) QIW_ROW(w1, 13, 26, 27) QIW_ROW(w2, 10, 28, 29) QIW_ROW(w3, 13, 30, 31)
+// a positive TERM falls through; the others run out of line and come back.  The index mode
+// stays on for first sources, which are slots only in the terms.
 #define QIW_WORD(w, lo, hi)                                       \
     "s_bitcmp1_b32 s" #w ", 31\n"                                 \
     "s_cbranch_scc1 .Lsp" #w "_%=\n"                              \
-    "s_set_gpr_idx_on s" #w ", gpr_idx(SRC0)\n"                   \
+    "s_set_gpr_idx_idx s" #w "\n"                                 \
     "v_fma_f64 v[14:15], v[32:33], v[" #lo ":" #hi "], v[14:15]\n" \
-    "s_set_gpr_idx_off\n"                                         \
     ".Lnx" #w "_%=:\n"
-#define QIW_WORDS(w0, w1, w2, w3, w4, w5, w6, w7)                                                       \
-    QIW_WORD(w0, 16, 17) QIW_WORD(w1, 18, 19) QIW_WORD(w2, 20, 21) QIW_WORD(w3, 22, 23)                 \
-    QIW_WORD(w4, 24, 25) QIW_WORD(w5, 26, 27) QIW_WORD(w6, 28, 29) QIW_WORD(w7, 30, 31)
+#define QIW_WORDS_A(w0, w1, w2, w3) QIW_WORD(w0, 16, 17) QIW_WORD(w1, 18, 19) QIW_WORD(w2, 20, 21) QIW_WORD(w3, 22, 23)
+#define QIW_WORDS_B(w0, w1, w2, w3) QIW_WORD(w0, 24, 25) QIW_WORD(w1, 26, 27) QIW_WORD(w2, 28, 29) QIW_WORD(w3, 30, 31)
 #define QIW_SPECIAL(w, lo, hi)                                    \
     ".Lsp" #w "_%=:\n"                                            \
     "s_bitcmp1_b32 s" #w ", 30\n"                                 \
     "s_cbranch_scc1 .Lmi" #w "_%=\n"                              \
     "s_set_gpr_idx_on s" #w ", gpr_idx(DST)\n"                    \
     "v_mul_f64 v[32:33], v[14:15], v[" #lo ":" #hi "]\n"          \
-    "s_set_gpr_idx_off\n"                                         \
+    "s_set_gpr_idx_on s" #w ", gpr_idx(SRC0)\n"                   \
     "v_mov_b32 v14, 0\n"                                          \
     "v_mov_b32 v15, 0\n"                                          \
     "s_branch .Lnx" #w "_%=\n"                                    \
     ".Lmi" #w "_%=:\n"                                            \
-    "s_set_gpr_idx_on s" #w ", gpr_idx(SRC0)\n"                   \
+    "s_set_gpr_idx_idx s" #w "\n"                                 \
     "v_fma_f64 v[14:15], v[32:33], -v[" #lo ":" #hi "], v[14:15]\n" \
-    "s_set_gpr_idx_off\n"                                         \
     "s_branch .Lnx" #w "_%=\n"
-#define QIW_SPECIALS(w0, w1, w2, w3, w4, w5, w6, w7)                                                    \
-    QIW_SPECIAL(w0, 16, 17) QIW_SPECIAL(w1, 18, 19) QIW_SPECIAL(w2, 20, 21) QIW_SPECIAL(w3, 22, 23)     \
-    QIW_SPECIAL(w4, 24, 25) QIW_SPECIAL(w5, 26, 27) QIW_SPECIAL(w6, 28, 29) QIW_SPECIAL(w7, 30, 31)
+#define QIW_SPECIALS_A(w0, w1, w2, w3) \
+    QIW_SPECIAL(w0, 16, 17) QIW_SPECIAL(w1, 18, 19) QIW_SPECIAL(w2, 20, 21) QIW_SPECIAL(w3, 22, 23)
+#define QIW_SPECIALS_B(w0, w1, w2, w3) \
+    QIW_SPECIAL(w0, 24, 25) QIW_SPECIAL(w1, 26, 27) QIW_SPECIAL(w2, 28, 29) QIW_SPECIAL(w3, 30, 31)
 #define QIW_ZERO(r) "v_mov_b32 v" #r ", 0\n"
 #define QIW_OUT(lo, hi, off) "ds_write_b64 v11, v[" #lo ":" #hi "] offset:" #off "\n"
+#define QIW_SARC_WORDS                                                                                        \
+    "s_mov_b32 s59, m0\n"                                                                                     \
+    QIW_ZERO(14) QIW_ZERO(15) QIW_ZERO(32) QIW_ZERO(33) QIW_ZERO(34) QIW_ZERO(35) QIW_ZERO(36) QIW_ZERO(37)   \
+    QIW_ZERO(38) QIW_ZERO(39) QIW_ZERO(40) QIW_ZERO(41) QIW_ZERO(42) QIW_ZERO(43) QIW_ZERO(44) QIW_ZERO(45)   \
+    QIW_ZERO(46) QIW_ZERO(47) QIW_ZERO(48) QIW_ZERO(50) QIW_ZERO(51)                                          \
+    "v_mov_b32 v49, 0x3ff00000\n"                                                                             \
+    "v_mov_b32 v11, %2\n"                                                                                     \
+    "v_mov_b32 v12, 0x3fe00\n"                                                                                \
+    "s_mov_b64 s[56:57], %0\n"                                                                                \
+    "s_mov_b32 s58, %1\n"                                                                                     \
+    "s_cmp_eq_u32 s58, 0\n"                                                                                   \
+    "s_cbranch_scc1 .Lend_%=\n"                                                                               \
+    "s_load_dwordx8 s[40:47], s[56:57], 0x0\n"                                                                \
+    "s_waitcnt lgkmcnt(0)\n"                                                                                  \
+    QIW_ROWS_A(40, 41, 42, 43)                                                                                \
+    "s_set_gpr_idx_on s40, gpr_idx(SRC0)\n"                                                                   \
+    ".Lloop_%=:\n"                                                                                            \
+    "s_waitcnt lgkmcnt(0)\n"                                                                                  \
+    "s_load_dwordx4 s[48:51], s[56:57], 0x20\n"                                                               \
+    QIW_ROWS_B(44, 45, 46, 47)                                                                                \
+    QIW_WORDS_A(40, 41, 42, 43)                                                                               \
+    "s_waitcnt lgkmcnt(0)\n"                                                                                  \
+    "s_load_dwordx4 s[52:55], s[56:57], 0x30\n"                                                               \
+    QIW_ROWS_A(48, 49, 50, 51)                                                                                \
+    QIW_WORDS_B(44, 45, 46, 47)                                                                               \
+    "s_waitcnt lgkmcnt(0)\n"                                                                                  \
+    "s_load_dwordx4 s[40:43], s[56:57], 0x40\n"                                                               \
+    QIW_ROWS_B(52, 53, 54, 55)                                                                                \
+    QIW_WORDS_A(48, 49, 50, 51)                                                                               \
+    "s_waitcnt lgkmcnt(0)\n"                                                                                  \
+    "s_load_dwordx4 s[44:47], s[56:57], 0x50\n"                                                               \
+    QIW_ROWS_A(40, 41, 42, 43)                                                                                \
+    QIW_WORDS_B(52, 53, 54, 55)                                                                               \
+    "s_add_u32 s56, s56, 64\n"                                                                                \
+    "s_addc_u32 s57, s57, 0\n"                                                                                \
+    "s_sub_u32 s58, s58, 1\n"                                                                                 \
+    "s_cmp_lg_u32 s58, 0\n"                                                                                   \
+    "s_cbranch_scc1 .Lloop_%=\n"                                                                              \
+    "s_set_gpr_idx_off\n"                                                                                     \
+    "s_branch .Lend_%=\n"                                                                                     \
+    QIW_SPECIALS_A(40, 41, 42, 43) QIW_SPECIALS_B(44, 45, 46, 47)                                             \
+    QIW_SPECIALS_A(48, 49, 50, 51) QIW_SPECIALS_B(52, 53, 54, 55)                                             \
+    ".Lend_%=:\n"                                                                                             \
+    "s_waitcnt vmcnt(0) lgkmcnt(0)\n"                                                                         \
+    "s_barrier\n"                                                                                             \
+    "v_add_u32 v11, %3, v11\n"                                                                                \
+    QIW_OUT(32, 33, 0) QIW_OUT(34, 35, 512)                                                                   \
+    "s_cmp_lt_u32 %4, 4\n"                                                                                    \
+    "s_cbranch_scc1 .Lout_%=\n"                                                                               \
+    QIW_OUT(36, 37, 1024) QIW_OUT(38, 39, 1536)                                                               \
+    "s_cmp_lt_u32 %4, 8\n"                                                                                    \
+    "s_cbranch_scc1 .Lout_%=\n"                                                                               \
+    QIW_OUT(40, 41, 2048) QIW_OUT(42, 43, 2560) QIW_OUT(44, 45, 3072) QIW_OUT(46, 47, 3584)                   \
+    ".Lout_%=:\n"                                                                                             \
+    "s_mov_b32 m0, s59\n"                                                                                     \
+    "s_waitcnt lgkmcnt(0)\n"
 
-// Runs `blocks` blocks of 16 words from `prog` (the read-ahead passes the end by half a
-// block) on the rows at LDS address 0, lane_off = 8 * lane; then, after a workgroup barrier,
-// stores the results of the sectors at out_off + 512 s.
-__device__ __forceinline__ void sarc_words(const uint32_t *prog, int blocks, uint32_t lane_off, uint32_t out_off) {
-    asm volatile(
-        "s_mov_b32 s59, m0\n"
-        QIW_ZERO(14) QIW_ZERO(15) QIW_ZERO(32) QIW_ZERO(33) QIW_ZERO(34) QIW_ZERO(35) QIW_ZERO(36) QIW_ZERO(37)
-        QIW_ZERO(38) QIW_ZERO(39) QIW_ZERO(40) QIW_ZERO(41) QIW_ZERO(42) QIW_ZERO(43) QIW_ZERO(44) QIW_ZERO(45)
-        QIW_ZERO(46) QIW_ZERO(47) QIW_ZERO(48) QIW_ZERO(50) QIW_ZERO(51)
-        "v_mov_b32 v49, 0x3ff00000\n"
-        "v_mov_b32 v11, %2\n"
-        "v_mov_b32 v12, 0x3fe00\n"
-        "s_mov_b64 s[56:57], %0\n"
-        "s_mov_b32 s58, %1\n"
-        "s_cmp_eq_u32 s58, 0\n"
-        "s_cbranch_scc1 .Lend_%=\n"
-        "s_load_dwordx8 s[40:47], s[56:57], 0x0\n"
-        "s_waitcnt lgkmcnt(0)\n"
-        ".Lloop_%=:\n"
-        QIW_ROWS(40, 41, 42, 43, 44, 45, 46, 47)
-        "s_load_dwordx8 s[48:55], s[56:57], 0x20\n"
-        "s_waitcnt lgkmcnt(0)\n"
-        QIW_WORDS(40, 41, 42, 43, 44, 45, 46, 47)
-        QIW_ROWS(48, 49, 50, 51, 52, 53, 54, 55)
-        "s_add_u32 s56, s56, 64\n"
-        "s_addc_u32 s57, s57, 0\n"
-        "s_load_dwordx8 s[40:47], s[56:57], 0x0\n"
-        "s_waitcnt lgkmcnt(0)\n"
-        QIW_WORDS(48, 49, 50, 51, 52, 53, 54, 55)
-        "s_sub_u32 s58, s58, 1\n"
-        "s_cmp_lg_u32 s58, 0\n"
-        "s_cbranch_scc1 .Lloop_%=\n"
-        "s_branch .Lend_%=\n"
-        QIW_SPECIALS(40, 41, 42, 43, 44, 45, 46, 47)
-        QIW_SPECIALS(48, 49, 50, 51, 52, 53, 54, 55)
-        ".Lend_%=:\n"
-        "s_waitcnt vmcnt(0) lgkmcnt(0)\n"
-        "s_barrier\n"
-        "v_add_u32 v11, %3, v11\n"
-        QIW_OUT(32, 33, 0) QIW_OUT(34, 35, 512) QIW_OUT(36, 37, 1024) QIW_OUT(38, 39, 1536)
-        QIW_OUT(40, 41, 2048) QIW_OUT(42, 43, 2560) QIW_OUT(44, 45, 3072) QIW_OUT(46, 47, 3584)
-        "s_mov_b32 m0, s59\n"
-        "s_waitcnt lgkmcnt(0)\n"
-        :
-        : "s"(prog), "s"(blocks), "v"(lane_off), "s"(out_off)
-        : "memory", "scc", "s40", "s41", "s42", "s43", "s44", "s45", "s46", "s47", "s48", "s49", "s50", "s51",
-          "s52", "s53", "s54", "s55", "s56", "s57", "s58", "s59", QIW_SARC_VGPRS);
+// Runs `blocks` blocks of 16 words from `prog` (eight words and the rows of four past the end
+// are read too) on the rows at LDS address 0, lane_off = 8 * lane; then, after a workgroup
+// barrier, stores the results of sectors 0 .. n_out - 1 (2, 4 or 8) at out_off + 512 s.
+template <int SLOTS>
+__device__ __forceinline__ void sarc_words(const uint32_t *prog, int blocks, uint32_t lane_off, uint32_t out_off, int n_out) {
+    if constexpr (SLOTS <= kScalarFew)
+        asm volatile(QIW_SARC_WORDS
+                     :
+                     : "s"(prog), "s"(blocks), "v"(lane_off), "s"(out_off), "s"(n_out)
+                     : "memory", "scc", "s40", "s41", "s42", "s43", "s44", "s45", "s46", "s47", "s48", "s49", "s50", "s51",
+                       "s52", "s53", "s54", "s55", "s56", "s57", "s58", "s59", QIW_SARC_FEW);
+    else
+        asm volatile(QIW_SARC_WORDS
+                     :
+                     : "s"(prog), "s"(blocks), "v"(lane_off), "s"(out_off), "s"(n_out)
+                     : "memory", "scc", "s40", "s41", "s42", "s43", "s44", "s45", "s46", "s47", "s48", "s49", "s50", "s51",
+                       "s52", "s53", "s54", "s55", "s56", "s57", "s58", "s59", QIW_SARC_MANY);
 }
 
-template <bool DLR>
-__global__ __launch_bounds__(256, 3) void k_eval_sarcs_t(EvalArgs a) {
+// The sum over the wavefront, in lane 63.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double add_dpp(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xf, false);
+    return v + __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double wave_sum(double v) {
+    v = add_dpp<0x111, 0xf>(v);  // row_shr 1, 2, 4, 8
+    v = add_dpp<0x112, 0xf>(v);
+    v = add_dpp<0x114, 0xf>(v);
+    v = add_dpp<0x118, 0xf>(v);
+    v = add_dpp<0x142, 0xa>(v);  // row_bcast 15, 31
+    return add_dpp<0x143, 0xc>(v);
+}
+
+// Sectors s and s + 1 (one of them if !two) of the propagator table at a cell: three loads.
+typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
+struct PairLoad {
+    d2u gm, g0, gp;
+    __device__ __forceinline__ void load(const double *ptab, int ns, const GridCell &c, int s, bool two) {
+        const uint32_t at = (uint32_t)(c.d * ns + s), back = c.d > 0 ? at - (uint32_t)ns : at;
+        if (two) {
+            gm = *reinterpret_cast<const d2u *>(ptab + back);
+            g0 = *reinterpret_cast<const d2u *>(ptab + at);
+            gp = *reinterpret_cast<const d2u *>(ptab + at + ns);
+        } else {
+            gm = d2u{ptab[back], 0.0};
+            g0 = d2u{ptab[at], 0.0};
+            gp = d2u{ptab[at + ns], 0.0};
+        }
+    }
+    __device__ __forceinline__ d2u value(const GridCell &c) const {
+        return d2u{cell_value(c, gm[0], g0[0], gp[0]), cell_value(c, gm[1], g0[1], gp[1])};
+    }
+};
+
+// GRID: every table is a grid container.  The set-up reads all records with the first loads,
+// one per lane, and gathers for UA arcs and UP propagators at a time: with one after the other
+// a wavefront waited for nine tenths of its time.
+template <bool GRID, bool DLR, int SLOTS>
+__global__ __launch_bounds__(256, SLOTS > kScalarFew ? 3 : DLR ? 4 : 6) void k_eval_sarcs_t(EvalArgs a) {
     extern __shared__ __attribute__((aligned(16))) char lds[];
+    constexpr int UA = GRID ? 3 : SLOTS <= kScalarFew ? 1 : 2, UP = 2;
     double *tab = reinterpret_cast<double *>(lds);  // rows, LDS address 0
-    double *tl = tab + a.lds_slots;                 // times of the positions
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const QiwTask task = a.tasks[blockIdx.x];
     const QiwGroup g = a.groups[task.group];
     const int n = g.n_nodes, ns = a.ns;
+    double *tl = tab + g.n_pslots * 64;  // times of the positions
     const double inv_h = 1.0 / a.h;
     const uint32_t *words = reinterpret_cast<const uint32_t *>(a.prog + g.prog_off);
     const ConstP<uint32_t> b = as_constp(words);
     const StepTimes T = step_times(a, g, task.tau_index);
     const bool bare = g.kind == QIW_G_BARE;
-    const int64_t sample = (int64_t)task.first_sample + lane;
-    const bool active = sample < g.n_samples;
-    const double *u = a.ut + g.ut_off + (int64_t)task.tau_index * a.ut_row_stride + (active ? sample : 0);
-    // ---- times of the configuration positions ----
-    for (int p = wave; p <= n; p += 4) {
-        double t = 0.0;
-        if (p == n) {
-            t = T.tau_f;
-        } else if (!bare && p == g.pos_w) {
-            t = T.tau_w;
-        } else if (p > 1 && g.sampled) {
+    const int na = (int)b[2], np = (int)b[4];
+    // ---- times of the configuration positions, and the records of the rows ----
+    {
+        const int64_t sample = (int64_t)task.first_sample + lane;
+        const double *u = a.ut + g.ut_off + (int64_t)task.tau_index * a.ut_row_stride + (sample < g.n_samples ? sample : 0);
+        double v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int p = wave + 4 * i;
             const bool after = bare || p > g.pos_w;
             const int j = after ? n - 1 - p : g.d_after + g.pos_w - 1 - p;
-            const double v = u[(int64_t)j * g.n_samples];
-            t = after ? v * (T.tau_f - T.tau_w) + T.tau_w : v * T.tau_w;
+            v[i] = 0.0;
+            if (p > 1 && p < n && g.sampled && (bare || p != g.pos_w)) v[i] = u[(int64_t)j * g.n_samples];
         }
-        tl[p * 64 + lane] = t;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int p = wave + 4 * i;
+            if (p > n) break;
+            double t = 0.0;
+            if (p == n)
+                t = T.tau_f;
+            else if (!bare && p == g.pos_w)
+                t = T.tau_w;
+            else if (p > 1 && g.sampled)
+                t = bare || p > g.pos_w ? v[i] * (T.tau_f - T.tau_w) + T.tau_w : v[i] * T.tau_w;
+            tl[p * 64 + lane] = t;
+        }
     }
+    const ConstP<uint32_t> arc = b + b[3];
+    uint32_t rec[3] = {0u, 0u, 0u}, prec[2] = {0u, 0u};
+    if (lane < na) {
+        const uint32_t *r = words + b[3] + 3 * lane;
+        rec[0] = r[0];
+        rec[1] = r[1];
+        rec[2] = r[2];
+    }
+    if (lane < np) {
+        const uint32_t *r = words + b[5] + 2 * lane;
+        prec[0] = r[0];
+        prec[1] = r[1];
+    }
+    auto arc_word = [&](int i, int w) { return i < 64 ? rlane(rec[w], i) : arc[3 * i + w]; };
     __syncthreads();
     // ---- rows: constants, arc values, propagators ----
     {
         const ConstP<uint32_t> c = b + b[1];
         for (int i = wave; i < (int)b[0]; i += 4)
             tab[i * 64 + lane] = __hiloint2double((int)c[2 * i + 1], (int)c[2 * i]);
-        const ConstP<uint32_t> arc = b + b[3];
-        for (int i = wave; i < (int)b[2]; i += 4) {
-            const uint32_t ends = arc[3 * i];
-            const ArcPos ap = arc_pos(tl[(ends >> 8) * 64 + lane], tl[(ends & 255) * 64 + lane], inv_h, a.n_tau);
+    }
+    for (int i0 = wave; i0 < na; i0 += 4 * UA) {
+        ArcPos ap[UA];
 #pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                const int r = (int)((arc[3 * i + 1 + t / 2] >> (16 * (t & 1))) & 0xFFFFu);
-                if (r != 0xFFFF) tab[r * 64 + lane] = delta_value<DLR>(a.dtab, t, ap);
-            }
+        for (int q = 0; q < UA; ++q) {  // past the last arc: the last one again
+            const uint32_t ends = arc_word(min(i0 + 4 * q, na - 1), 0);
+            const double t1 = tl[(ends >> 8) * 64 + lane], t0 = tl[(ends & 255) * 64 + lane];
+            if constexpr (GRID)
+                ap[q].c = grid_cell(t1, t0, inv_h, a.n_tau);
+            else
+                ap[q] = arc_pos(t1, t0, inv_h, a.n_tau);
         }
-        const ConstP<uint32_t> pr = b + b[5];
-        for (int i = wave; i < (int)b[4]; i += 4) {
-            const int r = (int)pr[3 * i], L = (int)pr[3 * i + 1], L2 = (int)pr[3 * i + 2];
-            const double t1 = tl[L * 64 + lane], t0 = tl[(L - 1) * 64 + lane], t2 = L2 ? tl[L2 * 64 + lane] : 0.0;
-            if (bare) {
-                double dt = t1 - t0;
-                dt = dt > 0.0 ? dt : 0.0;
-                for (int s = 0; s < ns; ++s) tab[(r + s) * 64 + lane] = exp(-dt * a.e_shift[s]);
-            } else {
-                const GridCell c1 = grid_cell(t1, t0, inv_h, a.n_tau);
-                const double *q1 = a.ptab + (int64_t)c1.d * ns;
-                const int m1 = c1.d > 0 ? ns : 0;
-                if (L2) {
-                    const GridCell c2 = grid_cell(t2, t1, inv_h, a.n_tau);
-                    const double *q2 = a.ptab + (int64_t)c2.d * ns;
-                    const int m2 = c2.d > 0 ? ns : 0;
-                    for (int s = 0; s < ns; ++s)
-                        tab[(r + s) * 64 + lane] = cell_value(c1, q1[s - m1], q1[s], q1[s + ns]) *
-                                                   cell_value(c2, q2[s - m2], q2[s], q2[s + ns]);
-                } else {
-                    for (int s = 0; s < ns; ++s)
-                        tab[(r + s) * 64 + lane] = cell_value(c1, q1[s - m1], q1[s], q1[s + ns]);
+        for (int tb = 0; tb < a.dtab.n_tables; tb += 2) {
+            double c[UA][2][GRID ? 3 : 4];
+            uint32_t rows[UA];
+#pragma unroll
+            for (int q = 0; q < UA; ++q) {
+                rows[q] = i0 + 4 * q < na ? arc_word(i0 + 4 * q, 1 + tb / 2) : 0xFFFFFFFFu;
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    if (((rows[q] >> (16 * t)) & 0xFFFFu) == 0xFFFFu) continue;
+                    if (DLR && ((a.dtab.dlr_mask >> (tb + t)) & 1)) continue;
+                    const double *co = a.dtab.coef + (int64_t)(tb + t) * (a.n_tau - 1) * 4;
+                    const uint32_t at = 4u * (uint32_t)(GRID || ((a.dtab.grid_mask >> (tb + t)) & 1) ? ap[q].c.d : ap[q].j);
+#pragma unroll
+                    for (int k = 0; k < (GRID ? 3 : 4); ++k) c[q][t][k] = co[at + k];
                 }
+            }
+#pragma unroll
+            for (int q = 0; q < UA; ++q)
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    const uint32_t r = (rows[q] >> (16 * t)) & 0xFFFFu;
+                    if (r == 0xFFFFu) continue;
+                    double v;
+                    if (DLR && ((a.dtab.dlr_mask >> (tb + t)) & 1))
+                        v = delta_value<DLR>(a.dtab, tb + t, ap[q]);
+                    else if (GRID || ((a.dtab.grid_mask >> (tb + t)) & 1))
+                        v = c[q][t][0] + ap[q].c.wp * c[q][t][1] - ap[q].c.wm * c[q][t][2];
+                    else
+                        v = c[q][t][0] + ap[q].u * (c[q][t][1] + ap[q].u * (c[q][t][2] + ap[q].u * c[q][t][GRID ? 2 : 3]));
+                    tab[r * 64 + lane] = v;
+                }
+        }
+    }
+    if (bare) {
+        for (int i = wave; i < np; i += 4) {
+            const uint32_t w = rlane(prec[0], i), seg = rlane(prec[1], i);
+            const int r = (int)(w & 0xFFFFu), s = (int)((w >> 16) & 255u), L = (int)(seg & 255u);
+            double dt = tl[L * 64 + lane] - tl[(L - 1) * 64 + lane];
+            dt = dt > 0.0 ? dt : 0.0;
+            tab[r * 64 + lane] = exp(-dt * a.e_shift[s]);
+            if (w >> 24) tab[(r + 1) * 64 + lane] = exp(-dt * a.e_shift[s + 1]);
+        }
+    } else {
+        for (int i0 = wave; i0 < np; i0 += 4 * UP) {
+            GridCell c[UP];
+            PairLoad x[UP];
+#pragma unroll
+            for (int q = 0; q < UP; ++q) {
+                const int i = min(i0 + 4 * q, np - 1), L = (int)(rlane(prec[1], i) & 255u);
+                c[q] = grid_cell(tl[L * 64 + lane], tl[(L - 1) * 64 + lane], inv_h, a.n_tau);
+            }
+#pragma unroll
+            for (int q = 0; q < UP; ++q) {
+                const uint32_t w = rlane(prec[0], min(i0 + 4 * q, np - 1));
+                x[q].load(a.ptab, ns, c[q], (int)((w >> 16) & 255u), (w >> 24) != 0);
+            }
+#pragma unroll
+            for (int q = 0; q < UP; ++q) {
+                const int i = i0 + 4 * q;
+                if (i >= np) break;
+                const uint32_t w = rlane(prec[0], i), seg = rlane(prec[1], i);
+                const int r = (int)(w & 0xFFFFu), s = (int)((w >> 16) & 255u), L = (int)(seg & 255u), L2 = (int)(seg >> 8);
+                d2u v = x[q].value(c[q]);
+                if (L2) {  // times the propagator after the left-out node at tau_w
+                    const GridCell c2 = grid_cell(tl[L2 * 64 + lane], tl[L * 64 + lane], inv_h, a.n_tau);
+                    PairLoad y;
+                    y.load(a.ptab, ns, c2, s, (w >> 24) != 0);
+                    v *= y.value(c2);
+                }
+                tab[r * 64 + lane] = v[0];
+                if (w >> 24) tab[(r + 1) * 64 + lane] = v[1];
             }
         }
     }
@@ -876,21 +1031,27 @@ __global__ __launch_bounds__(256, 3) void k_eval_sarcs_t(EvalArgs a) {
             tab[sc[3 * i] * 64 + lane] = tab[sc[3 * i + 1] * 64 + lane] * tab[sc[3 * i + 2] * 64 + lane];
         __syncthreads();
     }
-    // ---- each wavefront's program; results in row 8 * wave + s ----
-    sarc_words(words + b[8 + wave], (int)b[12 + wave], (uint32_t)lane * 8u, (uint32_t)wave * 4096u);
+    // ---- each wavefront's program; results in row n_out * wave + s ----
+    const int n_out = scalar_out_rows(ns);
+    sarc_words<SLOTS>(words + b[8 + wave], (int)b[12 + wave], (uint32_t)lane * 8u, (uint32_t)(wave * n_out) * 512u, n_out);
     __syncthreads();
     // the leaves' sign (-1)^order, and (-1)^n_after for the external arc of a correlator
+    // (src/diagrammatics.jl:288-303)
+    const int64_t sample = (int64_t)task.first_sample + lane;
+    const bool active = sample < g.n_samples;
     const bool odd = (g.order + (g.kind == QIW_G_CORR ? g.n_after : 0)) & 1;
-    const double wt = (odd ? -1.0 : 1.0) * (g.weighted ? u[(int64_t)(g.d_before + g.d_after) * g.n_samples] : 1.0);
+    double wt = odd ? -1.0 : 1.0;
+    if (g.weighted) {
+        const double *u = a.ut + g.ut_off + (int64_t)task.tau_index * a.ut_row_stride + (active ? sample : 0);
+        wt *= u[(int64_t)(g.d_before + g.d_after) * g.n_samples];
+    }
     for (int s = wave; s < ns; s += 4) {
         double v = 0.0;
 #pragma unroll
-        for (int w = 0; w < 4; ++w) v += tab[(8 * w + s) * 64 + lane];
+        for (int w = 0; w < 4; ++w) v += tab[(n_out * w + s) * 64 + lane];
         if (a.per_sample) tl[s * 64 + lane] = fabs(v);
-        v = active ? v * wt : 0.0;
-#pragma unroll
-        for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d, 64);
-        if (lane == 0) a.partial[(int64_t)task.out_index * ns + s] = v;
+        v = wave_sum(active ? v * wt : 0.0);
+        if (lane == 63) a.partial[(int64_t)task.out_index * ns + s] = v;
     }
     if (a.per_sample) {
         __syncthreads();
@@ -900,6 +1061,17 @@ __global__ __launch_bounds__(256, 3) void k_eval_sarcs_t(EvalArgs a) {
             a.per_sample[g.ps_off + sample] = m;
         }
     }
+}
+
+template <int SLOTS>
+void launch_sarcs(hipStream_t st, const EvalArgs &a, int n_tasks, size_t lds) {
+    const dim3 grid(n_tasks), block(256);
+    if (a.dtab.dlr_mask)
+        hipLaunchKernelGGL((k_eval_sarcs_t<false, true, SLOTS>), grid, block, lds, st, a);
+    else if (a.dtab.grid_mask == (1 << a.dtab.n_tables) - 1)
+        hipLaunchKernelGGL((k_eval_sarcs_t<true, false, SLOTS>), grid, block, lds, st, a);
+    else
+        hipLaunchKernelGGL((k_eval_sarcs_t<false, false, SLOTS>), grid, block, lds, st, a);
 }
 
 }  // namespace
@@ -916,13 +1088,13 @@ hipError_t qiw_launch_eval_arcs(hipStream_t st, const ArcArgs &a, int n_tasks, i
     return fp32 ? launch<float, 32, 512>(st, a, n_tasks, waves, lds) : launch<double, 32, 512>(st, a, n_tasks, waves, lds);
 }
 
-// lds_slots: float64 values of the rows (64 per row); the times of 16 positions follow.
-hipError_t qiw_launch_eval_sarcs(hipStream_t st, const EvalArgs &a, int n_tasks) {
-    if (n_tasks < 1 || a.ns > 8 || a.dtab.n_tables > 4 || a.lds_slots < 32 * 64) return hipErrorInvalidValue;
-    const size_t lds = ((size_t)a.lds_slots + 16 * 64) * 8;
-    if (a.dtab.dlr_mask)
-        hipLaunchKernelGGL((k_eval_sarcs_t<true>), dim3(n_tasks), dim3(256), lds, st, a);
+// slots: register slots of the programs; lds: scalar_lds_rows of the largest group, 512 bytes each.
+hipError_t qiw_launch_eval_sarcs(hipStream_t st, const EvalArgs &a, int n_tasks, int slots, size_t lds) {
+    if (n_tasks < 1 || a.ns > 8 || a.dtab.n_tables > 4 || slots > kScalarSlots) return hipErrorInvalidValue;
+    if (slots <= kScalarFew)
+        launch_sarcs<kScalarFew>(st, a, n_tasks, lds);
     else
-        hipLaunchKernelGGL((k_eval_sarcs_t<false>), dim3(n_tasks), dim3(256), lds, st, a);
+        launch_sarcs<kScalarSlots>(st, a, n_tasks, lds);
     return hipGetLastError();
 }
+int qiw_sarc_slots(int slots) { return slots <= kScalarFew ? kScalarFew : kScalarSlots; }

@@ -103,7 +103,7 @@ struct QiwGroup {
     int32_t n_nodes;       // configuration positions
     int32_t d_before, d_after;
     int32_t pos_w;         // position of the inch / A operator node (0 for bare)
-    int32_t n_pslots, n_wslots;
+    int32_t n_pslots, n_wslots;  // (scalar arc programs: n_pslots the rows before the times)
     int32_t prog_off;      // offset into the program word array
     int32_t topo_off;      // offset into the topology table: [n_top][2] words of head/tail nibbles
     int32_t coef_off;      // offset into the leaf coefficient table (scalar programs)
@@ -327,7 +327,8 @@ hipError_t qiw_launch_eval_flat(hipStream_t st, const EvalArgs &a, int n_tasks, 
 hipError_t qiw_launch_eval_block(hipStream_t st, const BlockArgs &b, int n_tasks, size_t lds_bytes);
 hipError_t qiw_launch_eval_mfma(hipStream_t st, const MfmaArgs &m, int n_tasks, int km, int tm, size_t lds_bytes);
 hipError_t qiw_launch_eval_arcs(hipStream_t st, const ArcArgs &a, int n_tasks, int mb, int fp32, int waves, size_t lds);
-hipError_t qiw_launch_eval_sarcs(hipStream_t st, const EvalArgs &a, int n_tasks);
+hipError_t qiw_launch_eval_sarcs(hipStream_t st, const EvalArgs &a, int n_tasks, int slots, size_t lds);
+int qiw_sarc_slots(int slots);  // slots of the instantiation that runs a program of `slots`
 int qiw_arc_rows(int mb);
 int qiw_arc_waves(int mb, int fp32);
 hipError_t qiw_launch_eval_vec(hipStream_t st, const VecArgs &v, int n_tasks, int mb, int km, int tm, int fp32);

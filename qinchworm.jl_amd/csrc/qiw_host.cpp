@@ -255,10 +255,10 @@ struct Compiled {
     // operator block per edge, the leaf accumulation)
     double flops_per_sample = 0;
     int n_top = 0;
-    // arc programs: initial-sector segments, wavefronts and LDS bytes of a workgroup
-    int n_segments = 0, waves = 1;
+    // arc programs: initial-sector segments, shape (wavefronts of a workgroup; scalar: register
+    // slots) and LDS bytes of a workgroup
+    int n_segments = 0, shape = 1;
     size_t lds_bytes = 0;
-    int rows = 0;  // scalar arc programs: rows of the LDS table
     int replica_of = -1;  // randomized qMC: another sequence of group `replica_of` (no program of its own)
 };
 
@@ -738,7 +738,7 @@ int compile_arcs(const HostModel &m, int kind, int order, int n_after, int corr,
     if (rc) return rc;
     set_arc_group(m, kind, order, n_after, pg.blob, out);
     out.n_segments = pg.n_segments;
-    out.waves = l.waves;
+    out.shape = l.waves;
     out.lds_bytes = pg.lds;
     out.leaves_per_sample = (int64_t)pg.leaves;
     out.edges_per_sample = (int64_t)pg.joins;
@@ -761,20 +761,21 @@ int compile_scalar_arcs(const HostModel &m, int kind, int order, int n_after, in
     const int rc = arc_compile_scalar(arc_model(m, corr), v, kind, order, n_after, max_words, sp);
     if (rc) return rc;
     set_arc_group(m, kind, order, n_after, sp.blob, out);
-    out.rows = sp.rows;
+    out.g.n_pslots = scalar_table_rows(sp.rows, m.ns);
+    out.shape = qiw_sarc_slots(sp.slots);
+    out.lds_bytes = (size_t)scalar_lds_rows(sp.rows, m.ns, out.g.n_nodes) * QIW_WAVE * 8;
     out.leaves_per_sample = (int64_t)sp.leaves;
     out.edges_per_sample = (int64_t)sp.words;
     out.flops_per_sample = 2.0 * sp.words;
     return 0;
 }
 
-// LDS doubles of one evaluator workgroup or wavefront.  Scalar trie programs keep their state in registers;
+// LDS doubles of one evaluator wavefront.  Scalar trie programs keep their state in registers;
 // block programs hold per-sample state shared by the lanes (iP slots, W slots, stack, X,
 // acc, out).
 int lds_slots(const Compiled &cg, const HostModel &m, int fmt) {
     const QiwGroup &g = cg.g;
-    if (fmt == FMT_SARC) return std::max(cg.rows, 32) * QIW_WAVE;  // at least the results of the wavefronts
-    if (fmt != FMT_BLOCK) return 0;  // register-resident walks
+    if (fmt != FMT_BLOCK) return 0;  // register-resident walks, and the arc walks (Compiled::lds_bytes)
     int mm = m.mmax * m.mmax;
     return (g.n_nodes - 1) * m.bt + g.n_wslots + 1 + (g.n_nodes + 1) * mm + 2 * mm + m.bt;
 }
@@ -799,8 +800,8 @@ struct Batch {
     double flops_per_launch = 0;  // algorithmic FLOPs of one launch
     int64_t leaves_per_launch = 0, diagram_evals_per_launch = 0;
     bool overflow = false;  // the launch would exceed kMaxTasks workgroups
-    struct Launch {         // arc walk: one launch per workgroup shape
-        int first, count, waves;
+    struct Launch {         // arc walks: one launch per workgroup shape
+        int first, count, shape;
         size_t lds;
     };
     std::vector<Launch> launches;
@@ -1057,7 +1058,7 @@ void push_sequences(Batch &b, Compiled &&cg, int n_eval, AddTasks add_tasks) {
         rep.flops_per_sample = cg.flops_per_sample;
         rep.n_top = cg.n_top;
         rep.n_segments = cg.n_segments;
-        rep.waves = cg.waves;
+        rep.shape = cg.shape;
         rep.lds_bytes = cg.lds_bytes;
         rep.replica_of = first;
     }
@@ -1214,10 +1215,15 @@ void order_tasks(Batch &b) {
     const size_t ng = b.groups.size();
     std::vector<int> go(ng);
     for (size_t i = 0; i < ng; ++i) go[i] = (int)i;
-    if (b.fmt == FMT_ARC) {  // one launch per workgroup shape, heaviest groups first in each
+    if (b.fmt == FMT_SARC) {  // one launch for all: the small groups fill the large ones' tail
+        int shape = 0;
+        for (const Compiled &cg : b.groups) shape = std::max(shape, cg.shape);
+        for (Compiled &cg : b.groups) cg.shape = shape;
+    }
+    if (b.fmt >= FMT_ARC) {  // one launch per workgroup shape, heaviest groups first in each
         std::stable_sort(go.begin(), go.end(), [&](int x, int y) {
             const Compiled &p = b.groups[x], &q = b.groups[y];
-            return p.waves != q.waves ? p.waves > q.waves : p.flops_per_sample > q.flops_per_sample;
+            return p.shape != q.shape ? p.shape > q.shape : p.flops_per_sample > q.flops_per_sample;
         });
         std::vector<std::vector<QiwTask>> of(ng);
         for (const QiwTask &t : b.tasks) of[t.group].push_back(t);
@@ -1225,8 +1231,8 @@ void order_tasks(Batch &b) {
         for (int gi : go) {
             const Compiled &cg = b.groups[gi];
             if (of[gi].empty()) continue;
-            if (b.launches.empty() || b.launches.back().waves != cg.waves)
-                b.launches.push_back({(int)b.tasks.size(), 0, cg.waves, 0});
+            if (b.launches.empty() || b.launches.back().shape != cg.shape)
+                b.launches.push_back({(int)b.tasks.size(), 0, cg.shape, 0});
             Batch::Launch &ln = b.launches.back();
             ln.count += (int)of[gi].size();
             ln.lds = std::max(ln.lds, cg.lds_bytes);
@@ -1699,7 +1705,7 @@ int launch_eval(qiw_ctx *c, const EvalArgs &a, const Batch &batch) {
         aa.e = a;
         for (const Batch::Launch &ln : batch.launches) {
             aa.e.tasks = a.tasks + ln.first;
-            HIPCHK(c, qiw_launch_eval_arcs(c->stream, aa, ln.count, m.mmax, precision == QIW_PREC_FP32 ? 1 : 0, ln.waves,
+            HIPCHK(c, qiw_launch_eval_arcs(c->stream, aa, ln.count, m.mmax, precision == QIW_PREC_FP32 ? 1 : 0, ln.shape,
                                            ln.lds));
         }
         return 0;
@@ -1707,7 +1713,11 @@ int launch_eval(qiw_ctx *c, const EvalArgs &a, const Batch &batch) {
     const size_t lds_bytes = (size_t)a.lds_slots * sizeof(double);
     if (lds_bytes > 160 * 1024) return fail(c, QIW_E_LIMIT, "evaluator state exceeds the 160 KiB of LDS of a CU");
     if (fmt == FMT_SARC) {
-        HIPCHK(c, qiw_launch_eval_sarcs(c->stream, a, n_tasks));
+        EvalArgs e = a;
+        for (const Batch::Launch &ln : batch.launches) {
+            e.tasks = a.tasks + ln.first;
+            HIPCHK(c, qiw_launch_eval_sarcs(c->stream, e, ln.count, ln.shape, ln.lds));
+        }
         return 0;
     }
     if (fmt == FMT_SCALAR) {

@@ -172,12 +172,12 @@ int main(int argc, char **argv) {
                 const uint32_t e = at(at(3) + 3 * i);
                 if (r != 0xFFFF) set(r, arc(e & 255, e >> 8, q));
             }
-        for (uint32_t i = 0; i < at(4); ++i)
-            for (int s = 0; s < m.ns; ++s) {
-                const uint32_t L = at(at(5) + 3 * i + 1), L2 = at(at(5) + 3 * i + 2);
-                if (L < 2 || L > (uint32_t)n || L2 > (uint32_t)n) die("segment");
-                set(at(at(5) + 3 * i) + s, prop[L][s] * (L2 ? prop[L2][s] : 1.0));
-            }
+        for (uint32_t i = 0; i < at(4); ++i) {
+            const uint32_t r = at(at(5) + 2 * i), seg = at(at(5) + 2 * i + 1), L = seg & 255, L2 = seg >> 8;
+            const int s = (int)((r >> 16) & 255);
+            if (L < 2 || L > (uint32_t)n || L2 > (uint32_t)n || s % 2 || s + (int)(r >> 24) >= m.ns || i >= 64) die("segment");
+            for (int q = 0; q <= (int)(r >> 24); ++q) set((r & 0xFFFF) + q, prop[L][s + q] * (L2 ? prop[L2][s + q] : 1.0));
+        }
         for (uint32_t i = 0; i < at(6); ++i)
             set(at(at(7) + 3 * i), tab.at(at(at(7) + 3 * i + 1)) * tab.at(at(at(7) + 3 * i + 2)));
         for (int w = 0; w < kScalarWaves; ++w) {
@@ -189,7 +189,7 @@ int main(int argc, char **argv) {
             double acc = 0.0;
             for (uint32_t i = 0; i < 16 * at(12 + w); ++i) {
                 const uint32_t x = at(at(8 + w) + i), sl = (x & 255) / 2, r = (x >> 9) & 511;
-                if ((x & 1) || (x & 256) || sl >= (uint32_t)kScalarSlots || r >= tab.size() || std::isnan(tab[r])) die("word");
+                if ((x & 1) || (x & 256) || sl >= (uint32_t)sp.slots || sp.slots > kScalarSlots || r >= tab.size() || std::isnan(tab[r])) die("word");
                 if ((x & SARC_SPECIAL) && !(x & SARC_MINUS)) {
                     if (sl == 8) die("the constant slot is written");
                     slot[sl] = acc * tab[r];
@@ -200,6 +200,8 @@ int main(int argc, char **argv) {
                 }
             }
             for (int s = 0; s < m.ns; ++s) res[s] += slot[s];
+            for (uint32_t i = 0; i < 8; ++i)  // words read ahead, the rows of the first four too
+                if (((at(at(8 + w) + 16 * at(12 + w) + i) >> 9) & 511) >= tab.size()) die("row read ahead");
         }
         pg.leaves = sp.leaves;
         pg.n_segments = (int)sp.words;
