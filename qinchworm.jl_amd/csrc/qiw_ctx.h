@@ -125,6 +125,10 @@ struct qiw_ctx {
     qiw_tuning tune{};                 // work mapping (qiw_set_tuning / qiw_autotune); 0 = default
     bool graphs = true;                // replay the bold-step loop from a hipGraph (qiw_set_graphs)
     qiwi::StepGraph *graph = nullptr;  // the captured loop and the launch arguments it holds
+    void *pin = nullptr;               // pinned host memory of the calls' transfers (Stage)
+    size_t pin_bytes = 0;
+    bool pin_busy = false;             // the stream may still read or write it
+    std::vector<double> es;            // E + lambda per eigenvalue, for the next transfer
     std::vector<hipEvent_t> evpool;    // timing events of the eager launches, reused
     // qiw_inchworm_step_noalloc: this device's static scratch array (its device address),
     // the bytes handed out during the current call, and the flag that makes dev() serve

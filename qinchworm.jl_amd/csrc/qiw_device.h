@@ -311,7 +311,20 @@ __host__ __device__ static inline uint32_t qiw_rq_word(uint64_t seed, uint64_t s
     return (uint32_t)qiw_mix64(qiw_mix64(seed ^ qiw_mix64(stream)) + (uint64_t)(33 * d + w));
 }
 
+// Copies of 32-bit words between device and pinned host memory (null source: zeros).
+struct StageOp {
+    uint32_t *dst;
+    const uint32_t *src;
+    int64_t words;
+};
+constexpr int kStageOps = 16;
+struct StageArgs {
+    int n;
+    StageOp op[kStageOps];
+};
+
 // Launch wrappers (qiw_kernels.hip)
+hipError_t qiw_launch_stage(hipStream_t st, const StageArgs &a);
 hipError_t qiw_launch_zero(hipStream_t st, void *p, size_t bytes);  // bytes: a multiple of 4
 hipError_t qiw_launch_sobol_points(hipStream_t st, const uint32_t *m, const uint32_t *x0, int dim, int64_t first,
                                    int64_t n, double *out);

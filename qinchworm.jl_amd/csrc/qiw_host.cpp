@@ -1603,24 +1603,143 @@ int step_plan(qiw_ctx *c, const qiw_run *run, const std::vector<int> &oall, bool
     return 0;
 }
 
-int ensure_model_buffers(qiw_ctx *c, double **dcoef, int32_t **dkind, double **eshift) {
+// Transfers of a call through the context's pinned buffer: what a call hands over (tables,
+// zeros) goes to the device in one kernel that reads the buffer, and its results come back in
+// one that writes it.  Nine synchronous copies and three fills took 130 us of a small step.
+// Pieces of more than kStageDirect bytes are copied on the stream, where a copy engine is
+// faster than loads over the bus.  Without a buffer (no-alloc calls that need more than there
+// is) every piece is copied by itself.
+constexpr size_t kStageDirect = 64 << 10;
+struct Stage {
+    qiw_ctx *c;
+    struct Piece {
+        void *to;
+        const void *from;  // null: zeros
+        size_t bytes;
+    };
+    std::vector<Piece> pieces;
+    explicit Stage(qiw_ctx *c_) : c(c_) {}
+    void add(void *to, const void *from, size_t bytes) {
+        if (bytes) pieces.push_back({to, from, bytes});
+    }
+    template <class T>
+    void add(void *to, const std::vector<T> &v) {
+        add(to, v.data(), v.size() * sizeof(T));
+    }
+    static size_t up(size_t b) { return (b + 15) & ~(size_t)15; }
+    char *pinned(size_t bytes) {
+        if (c->pin_busy) {  // a call that failed may have left work that reads it
+            if (hipStreamSynchronize(c->stream) != hipSuccess) return nullptr;
+            c->pin_busy = false;
+        }
+        if (c->pin_bytes >= bytes) return (char *)c->pin;
+        if (c->no_alloc) return nullptr;
+        if (c->pin) (void)hipHostFree(c->pin);
+        c->pin = nullptr;
+        c->pin_bytes = 0;
+        const size_t n = std::max<size_t>(bytes, 256 << 10);
+        if (hipHostMalloc(&c->pin, n, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            c->pin = nullptr;
+            return nullptr;
+        }
+        c->pin_bytes = n;
+        return (char *)c->pin;
+    }
+    hipError_t launch(const std::vector<StageOp> &ops) {
+        hipError_t e = hipSuccess;
+        for (size_t i = 0; i < ops.size() && e == hipSuccess; i += kStageOps) {
+            StageArgs a{};
+            a.n = (int)std::min<size_t>(kStageOps, ops.size() - i);
+            std::copy(ops.begin() + i, ops.begin() + i + a.n, a.op);
+            e = qiw_launch_stage(c->stream, a);
+        }
+        return e;
+    }
+    // To the device, in stream order.
+    int upload() {
+        size_t total = 0;
+        for (const Piece &p : pieces)
+            if (p.from) total += up(p.bytes);
+        char *pin = pinned(total);
+        std::vector<StageOp> ops;
+        size_t at = 0;
+        if (pin) c->pin_busy = true;
+        for (const Piece &p : pieces) {
+            if (p.from && !pin) {
+                HIPCHK(c, hipMemcpy(p.to, p.from, p.bytes, hipMemcpyHostToDevice));
+                continue;
+            }
+            if (p.from) {
+                std::memcpy(pin + at, p.from, p.bytes);
+                if (p.bytes > kStageDirect) {
+                    HIPCHK(c, hipMemcpyAsync(p.to, pin + at, p.bytes, hipMemcpyHostToDevice, c->stream));
+                    at += up(p.bytes);
+                    continue;
+                }
+            }
+            ops.push_back(StageOp{(uint32_t *)p.to, p.from ? (const uint32_t *)(pin + at) : nullptr, (int64_t)(p.bytes / 4)});
+            if (p.from) at += up(p.bytes);
+        }
+        HIPCHK(c, launch(ops));
+        pieces.clear();
+        return 0;
+    }
+    // Back to the host; the stream is idle afterwards.
+    int download() {
+        size_t total = 0;
+        for (const Piece &p : pieces) total += up(p.bytes);
+        if (c->pin_busy && c->pin_bytes < total) {
+            HIPCHK(c, hipStreamSynchronize(c->stream));
+            c->pin_busy = false;
+        }
+        // what the upload left in the buffer has been read when the kernels below run
+        char *pin = c->pin_bytes >= total ? (char *)c->pin : pinned(total);
+        std::vector<StageOp> ops;
+        size_t at = 0;
+        for (const Piece &p : pieces) {
+            if (!pin) break;
+            if (p.bytes > kStageDirect)
+                HIPCHK(c, hipMemcpyAsync(pin + at, p.from, p.bytes, hipMemcpyDeviceToHost, c->stream));
+            else
+                ops.push_back(StageOp{(uint32_t *)(pin + at), (const uint32_t *)p.from, (int64_t)(p.bytes / 4)});
+            at += up(p.bytes);
+        }
+        HIPCHK(c, launch(ops));
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        c->pin_busy = false;
+        at = 0;
+        for (const Piece &p : pieces) {
+            if (pin)
+                std::memcpy(p.to, pin + at, p.bytes);
+            else
+                HIPCHK(c, hipMemcpy(p.to, p.from, p.bytes, hipMemcpyDeviceToHost));
+            at += up(p.bytes);
+        }
+        pieces.clear();
+        return 0;
+    }
+};
+
+int ensure_model_buffers(qiw_ctx *c, double **dcoef, int32_t **dkind, double **eshift, Stage *stage = nullptr) {
     int rc = 0;
     const HostModel &m = c->m;
     *dcoef = (double *)dev(c, "delta.coef", std::max<size_t>(m.dcoef.size(), 1) * 8, &rc);
     *dkind = (int32_t *)dev(c, "delta.kind", std::max<size_t>(m.dkind.size(), 1) * 4, &rc);
     double *ddlr = (double *)dev(c, "delta.dlr", std::max<size_t>(m.dlr.size(), 1) * 8, &rc);
-    if (!rc && !m.dlr.empty()) HIPCHK(c, hipMemcpy(ddlr, m.dlr.data(), m.dlr.size() * 8, hipMemcpyHostToDevice));
     size_t n_eig = 0;
     for (int s = 0; s < m.ns; ++s) n_eig += m.dims[s];
     *eshift = (double *)dev(c, "eshift", n_eig * 8, &rc);
     if (rc) return rc;
-    if (!m.dcoef.empty()) HIPCHK(c, hipMemcpy(*dcoef, m.dcoef.data(), m.dcoef.size() * 8, hipMemcpyHostToDevice));
-    if (!m.dkind.empty()) HIPCHK(c, hipMemcpy(*dkind, m.dkind.data(), m.dkind.size() * 4, hipMemcpyHostToDevice));
-    std::vector<double> es;  // E + lambda per eigenvalue, sector-major
+    c->es.clear();  // E + lambda per eigenvalue, sector-major
     for (int s = 0; s < m.ns; ++s)
-        for (double e : m.E[s]) es.push_back(e + m.lambda0);
-    HIPCHK(c, hipMemcpy(*eshift, es.data(), es.size() * 8, hipMemcpyHostToDevice));
-    return 0;
+        for (double e : m.E[s]) c->es.push_back(e + m.lambda0);
+    Stage own(c), &st = stage ? *stage : own;
+    st.add(ddlr, m.dlr);
+    st.add(*dcoef, m.dcoef);
+    st.add(*dkind, m.dkind);
+    st.add(*eshift, c->es);
+    return stage ? 0 : own.upload();
 }
 
 // Device tables of the arc walk: the operator blocks (as the products read them, and
@@ -1985,6 +2104,7 @@ static void qiw_destroy_impl(qiw_ctx *c) {
     warp_destroy(c->warp);
     plans_destroy(c->plans);
     step_graph_destroy(c->graph);
+    if (c->pin) (void)hipHostFree(c->pin);
     for (auto e : c->evpool) (void)hipEventDestroy(e);
     for (auto &kv : c->bufs)
         if (kv.second.p) (void)hipFree(kv.second.p);
@@ -2116,20 +2236,20 @@ static int qiw_set_model_impl(qiw_ctx *c, const qiw_model *mi) {
     if (m.mmax > 6) wide_layout(m);
     m.mfma_ok = !m.scalar_kernel && m.mmax <= 32 && m.ntab <= 2 && m.ns <= 255 && m.bt < 4096 &&
                 m.op_data.size() < 0xFFFF - 64 && m.ops_rm.size() < 0xFFFF && m.btp < 4096;
-    c->m = m;
+    c->m = std::move(m);
     c->has_model = true;
-    std::string fp = model_fingerprint(m);
+    std::string fp = model_fingerprint(c->m);
     if (fp != c->model_fp) c->tune = qiw_tuning{};  // the work mapping was chosen for another model
     c->model_fp = fp;
     c->vec_staged = false;
     c->mfma_staged = false;
     c->arc_staged = 0;
     atomic_ip(c->m, c->ip);
-    c->n_known = (m.ppgf_kind == QIW_GF_INC_SPLINE) ? 1 : m.ntau;
-    c->der0.assign(m.bt, cd(0.0));  // initial_ppgf_derivative: -i diag(-E - lambda), src/ppgf.jl:710-720
-    for (int s = 0; s < m.ns; ++s)
-        for (int i = 0; i < m.dims[s]; ++i) c->der0[m.bt_off[s] + i + i * m.dims[s]] = cd(0.0, m.E[s][i] + m.lambda0);
-    c->lambdas.assign(m.ntau, 0.0);
+    c->n_known = (c->m.ppgf_kind == QIW_GF_INC_SPLINE) ? 1 : c->m.ntau;
+    c->der0.assign(c->m.bt, cd(0.0));  // initial_ppgf_derivative: -i diag(-E - lambda), src/ppgf.jl:710-720
+    for (int s = 0; s < c->m.ns; ++s)
+        for (int i = 0; i < c->m.dims[s]; ++i) c->der0[c->m.bt_off[s] + i + i * c->m.dims[s]] = cd(0.0, c->m.E[s][i] + c->m.lambda0);
+    c->lambdas.assign(c->m.ntau, 0.0);
     return QIW_OK;
 }
 
@@ -2230,6 +2350,7 @@ namespace {
 
 // Runs the initial step and then bold steps jw = first_w .. last_w on the device; the
 // device tables are initialized from the host mirror and copied back at the end.
+constexpr int kGraphSteps = 4;
 int run_inchworm(qiw_ctx *c, const qiw_run *run, bool do_bare, int first_w, int last_w, bool normalize,
                  bool store_host_P, double *P_orders_out, double *P_orders_std_out, std::vector<double> *step_value,
                  std::vector<double> *step_orders) {
@@ -2298,7 +2419,8 @@ int run_inchworm(qiw_ctx *c, const qiw_run *run, bool do_bare, int first_w, int 
     }
     double *dcoef, *eshift;
     int32_t *dkind;
-    if ((rc = ensure_model_buffers(c, &dcoef, &dkind, &eshift))) return rc;
+    Stage stage(c);
+    if ((rc = ensure_model_buffers(c, &dcoef, &dkind, &eshift, &stage))) return rc;
     size_t rows = std::max(bare_b.tasks.size(), bold_b.tasks.size());
     double *partial = (double *)dev(c, "partial", std::max<size_t>(rows, 1) * m.bt * 8, &rc);
     double *ptab = (double *)dev(c, "ptab", (size_t)m.ntau * m.bt * 8, &rc);
@@ -2313,16 +2435,17 @@ int run_inchworm(qiw_ctx *c, const qiw_run *run, bool do_bare, int first_w, int 
     double *pstd = rqmc ? (double *)dev(c, "porders_std", (size_t)n_slots * m.ntau * m.bt * 8, &rc) : nullptr;
     uint32_t *sobm = rq.scrambled ? (uint32_t *)dev(c, "sobol.m", c->sob_m.size() * 4, &rc) : nullptr;
     if (rc) return rc;
-    HIPCHK(c, qiw_launch_zero(c->stream, done, 4));
-    if (pstd) HIPCHK(c, qiw_launch_zero(c->stream, pstd, (size_t)n_slots * m.ntau * m.bt * 8));
-    if (sobm) HIPCHK(c, hipMemcpy(sobm, c->sob_m.data(), c->sob_m.size() * 4, hipMemcpyHostToDevice));
     std::vector<int32_t> dg;
     for (int s = 0; s < m.ns; ++s)
         for (int i = 0; i < m.dims[s]; ++i) dg.push_back(m.bt_off[s] + i + i * m.dims[s]);
-    HIPCHK(c, hipMemcpy(diag, dg.data(), dg.size() * 4, hipMemcpyHostToDevice));
-    HIPCHK(c, hipMemcpy(ptab, c->ip.data(), c->ip.size() * 8, hipMemcpyHostToDevice));
-    HIPCHK(c, qiw_launch_zero(c->stream, porders, (size_t)n_slots * m.ntau * m.bt * 8));
-    HIPCHK(c, qiw_launch_zero(c->stream, lam, (size_t)m.ntau * 8));
+    if (sobm) stage.add(sobm, c->sob_m);
+    stage.add(diag, dg);
+    stage.add(ptab, c->ip);
+    stage.add(done, nullptr, 4);
+    stage.add(porders, nullptr, (size_t)n_slots * m.ntau * m.bt * 8);
+    stage.add(lam, nullptr, (size_t)m.ntau * 8);
+    if (pstd) stage.add(pstd, nullptr, (size_t)n_slots * m.ntau * m.bt * 8);
+    if ((rc = stage.upload())) return rc;
 
     FinalizeArgs fa{};
     fa.partial = partial;
@@ -2429,7 +2552,8 @@ int run_inchworm(qiw_ctx *c, const qiw_run *run, bool do_bare, int first_w, int 
         }
         const bool staged = bold_b.fmt == FMT_SCALAR || bold_b.fmt == FMT_ARC || bold_b.fmt == FMT_SARC ||
                             (bold_b.fmt == FMT_VEC && (m.mmax > 6 ? c->mfma_staged : c->vec_staged));
-        bool graph = c->graphs && staged && !warped && !c->no_alloc && !rq.given;
+        // a few steps launch faster one by one than a graph is replayed, or captured for new times
+        bool graph = c->graphs && staged && !warped && !c->no_alloc && !rq.given && last_w - first_w >= kGraphSteps;
         const int n_known_start = n_known;
         if (graph) {
             if (!c->graph) c->graph = new StepGraph;
@@ -2532,7 +2656,20 @@ int run_inchworm(qiw_ctx *c, const qiw_run *run, bool do_bare, int first_w, int 
             c->stats.diagram_evals += bold_b.diagram_evals_per_launch;
         }
     }
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    // a step returns its own row, the other calls all rows
+    const bool one_row = step_value && !store_host_P && !P_orders_out && !P_orders_std_out;
+    const int row0 = one_row ? (do_bare ? 1 : first_w + 1) : 0, n_rows = one_row ? 1 : m.ntau;
+    std::vector<double> ptab_h((size_t)n_rows * m.bt), por((size_t)n_slots * n_rows * m.bt), lam_h(one_row ? 0 : m.ntau);
+    std::vector<double> pstd_h(pstd && !one_row ? por.size() : 0);
+    stage.add(ptab_h.data(), ptab + (size_t)row0 * m.bt, ptab_h.size() * 8);
+    if (one_row)
+        for (int o = 0; o < n_slots; ++o)
+            stage.add(por.data() + (size_t)o * m.bt, porders + ((size_t)o * m.ntau + row0) * m.bt, (size_t)m.bt * 8);
+    else
+        stage.add(por.data(), porders, por.size() * 8);
+    stage.add(lam_h.data(), lam, lam_h.size() * 8);
+    stage.add(pstd_h.data(), pstd, pstd_h.size() * 8);
+    if ((rc = stage.download())) return rc;
     for (size_t i = 0; i + 1 < n_ev; i += 2) {
         float ms = 0;
         HIPCHK(c, hipEventElapsedTime(&ms, c->evpool[i], c->evpool[i + 1]));
@@ -2547,12 +2684,6 @@ int run_inchworm(qiw_ctx *c, const qiw_run *run, bool do_bare, int first_w, int 
     if ((rc = check_given_use(c, bare_b, use_bare, nuse_bare, rows_bare))) return rc;
     if ((rc = check_given_use(c, bold_b, use_bold, nuse_bold, rows_bold))) return rc;
 
-    std::vector<double> ptab_h((size_t)m.ntau * m.bt), por((size_t)n_slots * m.ntau * m.bt), lam_h(m.ntau);
-    std::vector<double> pstd_h(pstd ? por.size() : 0);
-    if (pstd) HIPCHK(c, hipMemcpy(pstd_h.data(), pstd, pstd_h.size() * 8, hipMemcpyDeviceToHost));
-    HIPCHK(c, hipMemcpy(ptab_h.data(), ptab, ptab_h.size() * 8, hipMemcpyDeviceToHost));
-    HIPCHK(c, hipMemcpy(por.data(), porders, por.size() * 8, hipMemcpyDeviceToHost));
-    HIPCHK(c, hipMemcpy(lam_h.data(), lam, lam_h.size() * 8, hipMemcpyDeviceToHost));
     if (store_host_P) {
         c->ip = ptab_h;
         c->n_known = (m.ppgf_kind == QIW_GF_INC_SPLINE) ? n_known : m.ntau;
@@ -2581,12 +2712,12 @@ int run_inchworm(qiw_ctx *c, const qiw_run *run, bool do_bare, int first_w, int 
         }
     }
     if (step_value) {
-        int jf = do_bare ? 1 : first_w + 1;
+        const int jf = (do_bare ? 1 : first_w + 1) - row0;
         step_value->assign(ptab_h.begin() + (size_t)jf * m.bt, ptab_h.begin() + (size_t)(jf + 1) * m.bt);
         step_orders->clear();
         for (int o = 0; o < n_slots; ++o)
-            step_orders->insert(step_orders->end(), por.begin() + ((size_t)o * m.ntau + jf) * m.bt,
-                                por.begin() + ((size_t)o * m.ntau + jf + 1) * m.bt);
+            step_orders->insert(step_orders->end(), por.begin() + ((size_t)o * n_rows + jf) * m.bt,
+                                por.begin() + ((size_t)o * n_rows + jf + 1) * m.bt);
     }
     c->stats.wall_s += std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
     return 0;

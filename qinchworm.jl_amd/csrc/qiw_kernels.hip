@@ -2140,6 +2140,21 @@ __global__ __launch_bounds__(256) void k_finalize_corr_rqmc(CorrFinalizeArgs a) 
     }
 }
 
+// The transfers of a call (StageArgs), one row of blocks per piece.  What bounds it: the bus's
+// latency; four loads in flight per thread.
+__global__ __launch_bounds__(256) void k_stage(StageArgs a) {
+    const StageOp o = a.op[blockIdx.y];
+    const int64_t step = (int64_t)gridDim.x * 256;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < o.words; i += 4 * step) {
+        uint32_t v[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[q] = o.src && i + q * step < o.words ? o.src[i + q * step] : 0u;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (i + q * step < o.words) o.dst[i + q * step] = v[q];
+    }
+}
+
 // Zero n 32-bit words (clears counters and output tables with a kernel instead of a memset
 // node, so the stream work stays capturable).
 __global__ void k_zero_words(uint32_t *__restrict__ p, int64_t n) {
@@ -2275,6 +2290,15 @@ static dim3 reduce_threads(const FinalizeArgs &a) {
 
 hipError_t qiw_launch_finalize_step(hipStream_t st, const FinalizeArgs &a) {
     hipLaunchKernelGGL(k_step_reduce_finalize, reduce_grid(a), reduce_threads(a), 0, st, a);
+    return hipGetLastError();
+}
+
+hipError_t qiw_launch_stage(hipStream_t st, const StageArgs &a) {
+    int64_t most = 0;
+    for (int i = 0; i < a.n; ++i) most = a.op[i].words > most ? a.op[i].words : most;
+    if (a.n < 1 || a.n > kStageOps || most < 1) return hipErrorInvalidValue;
+    const unsigned blocks = (unsigned)((most + 1023) / 1024 < 64 ? (most + 1023) / 1024 : 64);
+    hipLaunchKernelGGL(k_stage, dim3(blocks, a.n), dim3(256), 0, st, a);
     return hipGetLastError();
 }
 

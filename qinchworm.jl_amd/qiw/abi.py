@@ -114,13 +114,18 @@ class ModelStruct:
     def _sbm(self, blocks):
         """blocks: dict s_i -> (s_f, complex matrix)."""
         keys = sorted(blocks)
-        s_i = np.array(keys, dtype=np.int32)
-        s_f = np.array([blocks[k][0] for k in keys], dtype=np.int32)
-        data = [np.asarray(blocks[k][1], dtype=np.complex128).ravel(order="F") for k in keys]
-        data = np.ascontiguousarray(np.concatenate(data) if data else np.zeros(1, np.complex128))
+        n = len(keys)
+        s_i = (C.c_int32 * max(n, 1))(*[int(k) for k in keys])
+        s_f = (C.c_int32 * max(n, 1))(*[int(blocks[k][0]) for k in keys])
+        data = [np.asarray(blocks[k][1]) for k in keys]
+        if all(d.size == 1 for d in data):  # ctypes arrays cost less than numpy's for a few values
+            v = [complex(d.flat[0]) for d in data]
+            data = (C.c_double * max(2 * n, 2))(*[x for z in v for x in (z.real, z.imag)])
+            self._keep += [s_i, s_f, data]
+            return qiw_sbm(n_blocks=n, s_i=s_i, s_f=s_f, data=data)
+        data = np.concatenate([d.ravel(order="F") for d in data]).astype(np.complex128, copy=False)
         self._keep += [s_i, s_f, data]
-        return qiw_sbm(n_blocks=len(keys), s_i=ptr(s_i, C.c_int32), s_f=ptr(s_f, C.c_int32),
-                       data=data.ctypes.data_as(_f64p))
+        return qiw_sbm(n_blocks=n, s_i=s_i, s_f=s_f, data=data.ctypes.data_as(_f64p))
 
     def ref(self):
         return C.byref(self.struct)

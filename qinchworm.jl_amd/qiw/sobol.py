@@ -3,6 +3,7 @@
 Mirrors the constructor of ScrambledSobolSeq (src/scrambled_sobol.jl:66-143), whose state
 (m, x) is what the C ABI takes (qiw_set_sobol); point generation itself runs on the GPU.
 """
+import functools
 import json
 import os
 
@@ -21,6 +22,13 @@ def _table():
 
 
 def direction_numbers(D):
+    """m[d, j] of the reference after src/scrambled_sobol.jl:78-100 (unscrambled), shape (D, 32),
+    uint32: a copy of a table that depends on D alone."""
+    return _direction_numbers(D).copy()
+
+
+@functools.lru_cache(maxsize=16)
+def _direction_numbers(D):
     """m[d, j] of the reference after :78-100 (unscrambled), shape (D, 32), uint32.
 
     Dimension 1 is van der Corput (all initial m = 1); dimension d >= 2 uses primitive
