@@ -283,7 +283,8 @@ constexpr uint32_t ARC_NONE = 0xFFFFFFFFu;
 // product of the sum of joins with the block; the tile's end: propagator, store.  Without a
 // product the next slot's joins continue the sum.
 enum : uint32_t { ARC_BARRIER = 1, ARC_END = 2, ARC_IDLE = 4, ARC_SECOND = 8, ARC_TIMES = 16, ARC_STORE = 32 };
-constexpr size_t kArcValuesAt = 128;  // LDS offset of the arc values, past 16 times
+// LDS offsets: 16 times, the grid cells of 16 segments (24 bytes each), the arc values.
+constexpr size_t kArcCellsAt = 128, kArcValuesAt = 512;
 constexpr int kArcGroupHead = 8, kArcSegHead = 8, kArcSlotWords = 8;
 constexpr int kArcTileOps = 28;          // most operators of a tile
 constexpr int kArcReadAhead = 6 * 256;   // words a wavefront may read past its streams
@@ -309,17 +310,18 @@ inline int arc_stride(int m, int mmax) {
     return mmax > 8 || m > 6 ? (m + 3) & ~3 : m == 1 ? 1 : (m + 1) & ~1;
 }
 
-// LDS of a group in bytes: the times of the positions, the arc values, the closed state's
-// columns, the propagators of n - 2 segments and one product, then the states.
+// LDS of a group in bytes: the times of the positions and cells of the segments, the arc
+// values, the closed states of all sectors, the propagators of n - 2 segments and one product,
+// then the states (and at the end, in their place, the last propagator).
 struct ArcLds {
     size_t fin, arcs, prop, states;
 };
-inline ArcLds arc_lds(const ArcLayout &l, int n, int n_arcs, int m0) {
+inline ArcLds arc_lds(const ArcLayout &l, int n, int n_arcs) {
     auto up = [](size_t b) { return (b + 15) & ~(size_t)15; };
     ArcLds r;
     r.arcs = kArcValuesAt;
     r.fin = r.arcs + up((size_t)(2 + 2 * n_arcs) * l.elem);
-    r.prop = r.fin + up((size_t)m0 * m0 * 8);
+    r.prop = r.fin + up((size_t)l.bt * 8);
     r.states = r.prop + up((size_t)(n - 1) * l.bt * l.elem);
     return r;
 }
@@ -775,14 +777,12 @@ inline int arc_compile(const ArcModel &m, const ArcLayout &l, const ArcBlocks &o
             if (!arc_graph(m, kind, order, n_after, s0, fix, skip_w, g)) return 1;
             if (!g.levels.empty()) graphs.push_back(std::move(g));
         }
-    int m0 = 1;
-    for (const ArcGraph &g : graphs) m0 = std::max(m0, m.dims[g.s0]);
     const int most_arcs = order * (2 * order - 1) * (1 + *std::max_element(m.table.begin(), m.table.end()));
-    const ArcLds at = arc_lds(l, n, order > 0 ? most_arcs : 0, m0);
-    if (at.states >= l.cap || 2 + 2 * most_arcs >= 4096) return 2;
+    const ArcLds at = arc_lds(l, n, order > 0 ? most_arcs : 0);
+    if (at.states + (size_t)l.bt * 8 > l.cap || 2 + 2 * most_arcs >= 4096) return 2;
     const size_t room = (l.cap - at.states) / l.elem;
     out.blob.assign(kArcGroupHead + graphs.size(), 0u);
-    out.lds = at.states;
+    out.lds = at.states + (size_t)l.bt * 8;
     for (const ArcGraph &g : graphs) {
         int best = -1;
         ArcPacker::Plan plan, best_plan;

@@ -457,6 +457,13 @@ __device__ __forceinline__ bool run_slots(Walk<V, MB> &w, const Joins<Walk<V, MB
     return true;
 }
 
+// Grid cell of a segment in LDS.
+struct ArcCell {
+    double wp, wm;
+    int d, pad_;
+};
+static_assert(kArcCellsAt + 16 * sizeof(ArcCell) <= kArcValuesAt, "LDS of the cells");
+
 // i*P element e of the cell c from the float64 table.
 __device__ __forceinline__ double prop_element(const double *ptab, int bt, const GridCell &c, int e) {
     const double *r0 = ptab + (int64_t)c.d * bt;
@@ -469,18 +476,20 @@ __device__ __forceinline__ double prop_element(const double *ptab, int bt, const
 // blocks 1 4 6 4 1, float32), so a lane cannot own a sample; states of one sector share
 // operator and propagator, so both are wavefront-uniform.  Measured against the walk of the
 // assignment tries (one pass per diagram): two-orbital solve on 50 points, orders 0:2 at
-// N = 2^10, float64 452 -> 24.5 ms; two-orbital step, orders 0:4 at N = 2^11, float32 636 -> 24.2
-// ms; orders 0:3 at N = 2^12, float64 142 -> 9.9 ms; three-orbital step, orders 0:3 at N =
-// 2^9, float32 402 -> 36.9 ms; orders 0:2 at N = 2^8, float64 63.7 -> 9.3 ms.  Of these the
+// N = 2^10, float64 451 -> 15.7 ms; two-orbital step, orders 0:4 at N = 2^11, float32 643 -> 22.5
+// ms; orders 0:3 at N = 2^12, float64 144 -> 8.8 ms; three-orbital step, orders 0:3 at N =
+// 2^9, float32 399 -> 33.9 ms; orders 0:2 at N = 2^8, float64 63.8 -> 3.2 ms.  Of these the
 // first form of the walk reached 29.9, 43.6, 18.2, 54.8 and 28.8 ms: what it lost were branches
 // on every row and column (one in five instructions), operator blocks and joins read when they
 // were wanted (a load's whole latency each), stages waiting for one wavefront with a tile of
-// many operators, and for float64 operator elements through the scalar cache.
+// many operators, for float64 operator elements through the scalar cache, the last propagator's
+// gathers in every segment, and the workgroup shapes.
 //
 // One workgroup: the samples of a task one after the other; per sample the times, arc values
 // and propagators go to LDS once, then every segment (initial sector) of the task is walked
 // level by level.  The wavefronts share the tiles of a stage; a lane holds one column of one
-// state.  The closed state's columns are multiplied by the last propagator in float64.
+// state.  The closed states of all segments are multiplied by the last propagator in float64
+// at the end (segment by segment its gathers and the sums in memory were waited for each time).
 // Wavefronts per SIMD: float64 at MB = 8 takes three (168 registers, what spills is outside the
 // slots; 11.7 -> 9.9 ms against two), float32 of wide blocks two (no spills; 43.3 -> 37.2 ms
 // against four).
@@ -508,7 +517,7 @@ __global__ __launch_bounds__(NT, MB == 8 && sizeof(V) == 8 ? 3 : 2) void k_eval_
     const int seg0 = task.chunk < 0 ? 0 : task.chunk, seg1 = task.chunk < 0 ? (int)b[0] : seg0 + task.pad_;
     const bool bare = g.kind == QIW_G_BARE;
     const int skip_w = (int)b[2];
-    for (int e = tid; e < bt; e += nt) prow[e] = 0.0;
+    ArcCell *cells = reinterpret_cast<ArcCell *>(lds + kArcCellsAt);
 
     const int n_here = g.sampled ? min(a.spt, g.n_samples - task.first_sample) : 1;
     for (int sr = 0; sr < n_here; ++sr) {
@@ -529,12 +538,13 @@ __global__ __launch_bounds__(NT, MB == 8 && sizeof(V) == 8 ? 3 : 2) void k_eval_
             }
             tl[tid] = t;
         }
+        for (int e = tid; e < bt; e += nt) fin[e] = 0.0;
         // the leaves' sign (-1)^order, and (-1)^n_after for the external arc of a correlator
         // (src/diagrammatics.jl:288-303)
         const bool odd = (g.order + (g.kind == QIW_G_CORR ? g.n_after : 0)) & 1;
         const double wt = (odd ? -1.0 : 1.0) * (g.weighted ? u[(int64_t)(g.d_before + g.d_after) * g.n_samples] : 1.0);
         __syncthreads();
-        // ---- arc values +-i*Delta and propagators i*P of segments 2 .. n - 1 ----
+        // ---- arc values +-i*Delta, and the grid cells of the segments ----
         const int na = (int)b[1];
         for (int i = tid; i < na + 1; i += nt) {
             if (i == na) {
@@ -548,14 +558,24 @@ __global__ __launch_bounds__(NT, MB == 8 && sizeof(V) == 8 ? 3 : 2) void k_eval_
             dv[2 + 2 * i] = v;
             dv[3 + 2 * i] = -v;
         }
-        for (int i = tid; i < (n - 2) * bt; i += nt) {
-            const int L = 2 + i / bt, e = i - (L - 2) * bt;
+        if (tid >= nt - 16 && !bare) {  // (the last threads: the first ones have the arcs)
+            const int L = 2 + tid - (nt - 16);
+            if (L <= n) {
+                const GridCell c = grid_cell(tl[L], tl[L - 1], inv_h, a.n_tau);
+                cells[L - 2] = ArcCell{c.wp, c.wm, c.d, 0};
+            }
+        }
+        __syncthreads();
+        // ---- propagators i*P of segments 2 .. n - 1 ----
+        for (int L = 2; L < n; ++L) {
+            V *p = pl + (L - 2) * bt;
             if (bare) {
                 double dt = tl[L] - tl[L - 1];
                 dt = dt > 0.0 ? dt : 0.0;
-                pl[i] = aa.emask[e] ? (V)exp(-dt * aa.ediag[e]) : (V)0;
+                for (int e = tid; e < bt; e += nt) p[e] = aa.emask[e] ? (V)exp(-dt * aa.ediag[e]) : (V)0;
             } else {
-                pl[i] = (V)prop_element(a.ptab, bt, grid_cell(tl[L], tl[L - 1], inv_h, a.n_tau), e);
+                const GridCell c{cells[L - 2].d, cells[L - 2].wp, cells[L - 2].wm};
+                for (int e = tid; e < bt; e += nt) p[e] = (V)prop_element(a.ptab, bt, c, e);
             }
         }
         __syncthreads();
@@ -563,7 +583,8 @@ __global__ __launch_bounds__(NT, MB == 8 && sizeof(V) == 8 ? 3 : 2) void k_eval_
             const V *Pa = pl + (skip_w - 2) * bt, *Pb = pl + (skip_w - 1) * bt;
             V *dst = pl + (n - 2) * bt;
             for (int e = tid; e < bt; e += nt) {
-                const int s = aa.sector_of[e], m = aa.dims[s], o = aa.bt_off[s], i = (e - o) % m, j = (e - o) / m;
+                const uint32_t at = aa.element[e];
+                const int o = (int)(at & 0xFFFFu), i = (int)((at >> 16) & 31u), j = (int)((at >> 21) & 31u), m = 1 + (int)(at >> 26);
                 V v = (V)0;
                 for (int q = 0; q < m; ++q) v = fma(Pb[o + i + q * m], Pa[o + q + j * m], v);
                 dst[e] = v;
@@ -577,6 +598,7 @@ __global__ __launch_bounds__(NT, MB == 8 && sizeof(V) == 8 ? 3 : 2) void k_eval_
             const int s0 = (int)(h0 & 255), m0 = (int)((h0 >> 8) & 255), lg = (int)(h0 >> 16), cg = 1 << lg;
             const int m1 = (int)(h[1] & 255), str1 = (int)(h[1] >> 8);
             const uint32_t rblk = h[2], rprop = h[3];
+            const int o = aa.bt_off[s0];
             constexpr int SL = Walk<V, MB>::SL;
             const int col = lane & (cg - 1);
             const uint32_t jstep = 4u * (SL * (64u >> lg));  // bytes of a block of joins
@@ -633,28 +655,31 @@ __global__ __launch_bounds__(NT, MB == 8 && sizeof(V) == 8 ? 3 : 2) void k_eval_
                     for (int p = lane + 64; p < np; p += 64) v += (double)st[words[h[6] + p] + c * stf + r];
 #pragma unroll
                     for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d, 64);
-                    if (lane == 0) fin[(c0 + c) * m0 + r] = v;
+                    if (lane == 0) fin[o + (c0 + c) * m0 + r] += v;
                 }
             }
+            __syncthreads();  // the next segment's states may lie where these closed ones do
+        }
+        // out[s0] = weight * iP_n[s0] * closed state, in float64; iP_n where the states were
+        double *last = reinterpret_cast<double *>(st);
+        if (!bare) {
+            const GridCell c{cells[n - 2].d, cells[n - 2].wp, cells[n - 2].wm};
+            for (int e = tid; e < bt; e += nt) last[e] = prop_element(a.ptab, bt, c, e);
             __syncthreads();
-            // out[s0] += weight * iP_n[s0] * closed state, in float64
-            const int o = aa.bt_off[s0];
-            const GridCell cn = grid_cell(tl[n], tl[n - 1], inv_h, a.n_tau);
-            double dtn = tl[n] - tl[n - 1];
-            dtn = dtn > 0.0 ? dtn : 0.0;
-            for (int i = tid; i < m0 * m0; i += nt) {
-                const int c = i / m0, r = i - c * m0;
-                double v = 0.0;
-                if (bare) {
-                    v = exp(-dtn * aa.ediag[o + r * (m0 + 1)]) * fin[i];
-                } else {
-                    for (int q = 0; q < m0; ++q)
-                        v = fma(prop_element(a.ptab, bt, cn, o + r + q * m0), fin[c * m0 + q], v);
-                }
-                mag += fabs(v);
-                prow[o + i] += wt * v;
+        }
+        double dtn = tl[n] - tl[n - 1];
+        dtn = dtn > 0.0 ? dtn : 0.0;
+        for (int e = tid; e < bt; e += nt) {
+            const uint32_t at = aa.element[e];
+            const int o = (int)(at & 0xFFFFu), r = (int)((at >> 16) & 31u), c = (int)((at >> 21) & 31u), m = 1 + (int)(at >> 26);
+            double v = 0.0;
+            if (bare) {
+                v = exp(-dtn * aa.ediag[o + r * (m + 1)]) * fin[e];
+            } else {
+                for (int q = 0; q < m; ++q) v = fma(last[o + r + q * m], fin[o + c * m + q], v);
             }
-            // fin is written again only after the next segment's first barrier
+            mag += fabs(v);
+            prow[e] = sr == 0 ? wt * v : prow[e] + wt * v;
         }
         __syncthreads();
         if (a.per_sample) {

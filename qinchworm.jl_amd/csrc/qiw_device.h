@@ -281,8 +281,8 @@ struct ArcArgs {
     const void *ops_cm;        // the same column-major in the value type
     const double *ediag;       // [bt] E + lambda on the diagonal positions (bare groups)
     const uint8_t *emask;      // [bt] 1 on the diagonal positions
-    const int32_t *sector_of;  // [bt]
-    const int32_t *dims, *bt_off, *stride;  // [ns]
+    const uint32_t *element;   // [bt] offset of its block | row << 16 | column << 21 | (size - 1) << 26
+    const int32_t *bt_off, *stride;  // [ns]
     int bt;
 };
 // Wavefronts per workgroup of k_eval_mfma_t (tasks come in units of this many)

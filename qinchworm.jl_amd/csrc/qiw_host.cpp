@@ -660,16 +660,23 @@ ArcBlocks arc_blocks(const HostModel &m, int corr, int precision) {
     return o;
 }
 
-// Workgroup shapes of the arc walk, narrowest first: wavefronts and the LDS they may take
-// (eight, three, two and one workgroup per CU), and the widest level, in 64-state tiles,
-// that the shape is for.
+// Workgroup shapes of the arc walk, narrowest first: wavefronts, the LDS they may take, and
+// the widest level, in 64-state tiles, that the shape is for.  Small levels take two
+// wavefronts: one (20 KB) leaves the set-up of a sample to 64 lanes, four meet at more barriers
+// than their tiles are worth (two-orbital solve of orders 0:2, N = 2^10: 21.9, 16.6, 20.5 ms
+// with one, two, four).  Order 3 of the same model takes four in 53 KB (8.9 ms a step at N =
+// 2^12; 11.1 in 40 KB, 11.2 with eight in 80 KB, 13.7 with two).  Wide blocks take all of a
+// CU's LDS: the more columns fit beside each other, the fewer lanes idle in the tiles of one
+// operator (three-orbital step of orders 0:2, N = 2^8, float64: 8.6 ms with two workgroups of
+// 80 KB per CU, which left seven in a hundred lanes at work, 3.1 with one of 160 KB; orders 0:3,
+// N = 2^9, float32: 35.3 and 33.5 ms).
 struct ArcShape {
     int waves;
     size_t cap;
     int tiles;
 };
-constexpr ArcShape kArcShapes[] = {{1, 20 << 10, 2}, {4, 53 << 10, 12}, {8, 80 << 10, 32}, {16, 160 << 10, 1 << 30}};
-constexpr ArcShape kArcShapesWide[] = {{4, 53 << 10, 3}, {8, 80 << 10, 12}, {8, 160 << 10, 1 << 30}};  // mmax > 8
+constexpr ArcShape kArcShapes[] = {{2, 40 << 10, 2}, {4, 53 << 10, 12}, {8, 80 << 10, 32}, {16, 160 << 10, 1 << 30}};
+constexpr ArcShape kArcShapesWide[] = {{8, 160 << 10, 1 << 30}};  // mmax > 8
 
 // Algorithmic real FLOPs of one sample of a compiled group: the scalar walk's multiply per
 // trie edge and leaf, or the block programs' chain products.
@@ -723,7 +730,7 @@ int compile_arcs(const HostModel &m, int kind, int order, int n_after, int corr,
     }
     const bool wide = m.mmax > 8;
     const ArcShape *shapes = wide ? kArcShapesWide : kArcShapes;
-    const int n_shapes = wide ? 3 : 4;
+    const int n_shapes = wide ? 1 : 4;
     ArcGroupProgram pg;
     int rc = 2;
     for (int n_fixed = 0; n_fixed <= order && rc == 2; ++n_fixed)
@@ -1754,7 +1761,7 @@ int stage_arcs(qiw_ctx *c, int precision, ArcArgs *aa) {
     void *cm = dev(c, fp32 ? "arc.ops32" : "arc.ops", (m.op_data.size() + pad) * el, &rc);
     double *ediag = (double *)dev(c, "arc.ediag", (size_t)m.bt * 8, &rc);
     uint8_t *emask = (uint8_t *)dev(c, "arc.emask", (size_t)m.bt, &rc);
-    int32_t *lay = (int32_t *)dev(c, "arc.layout", ((size_t)m.bt + 3 * m.ns) * 4, &rc);
+    int32_t *lay = (int32_t *)dev(c, "arc.layout", ((size_t)m.bt + 2 * m.ns) * 4, &rc);
     if (rc) return rc;
     if (!(c->arc_staged & (fp32 ? 2 : 1))) {
         HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -1781,17 +1788,18 @@ int stage_arcs(qiw_ctx *c, int precision, ArcArgs *aa) {
         }
         std::vector<double> ed((size_t)m.bt, 0.0);
         std::vector<uint8_t> mk((size_t)m.bt, 0);
-        std::vector<int32_t> l((size_t)m.bt + 3 * m.ns);
+        std::vector<int32_t> l((size_t)m.bt + 2 * m.ns);
         for (int q = 0; q < m.ns; ++q) {
             const int d = m.dims[q];
-            for (int e = 0; e < d * d; ++e) l[m.bt_off[q] + e] = q;
+            for (int e = 0; e < d * d; ++e)  // bt < 2^16 where the propagators fit in LDS
+                l[m.bt_off[q] + e] = (int32_t)((uint32_t)m.bt_off[q] | (uint32_t)(e % d) << 16 | (uint32_t)(e / d) << 21 |
+                                               (uint32_t)(d - 1) << 26);
             for (int i = 0; i < d; ++i) {
                 ed[m.bt_off[q] + i + i * d] = m.E[q][i] + m.lambda0;
                 mk[m.bt_off[q] + i + i * d] = 1;
             }
-            l[m.bt + q] = d;
-            l[m.bt + m.ns + q] = m.bt_off[q];
-            l[m.bt + 2 * m.ns + q] = arc_stride(d, m.mmax);
+            l[m.bt + q] = m.bt_off[q];
+            l[m.bt + m.ns + q] = arc_stride(d, m.mmax);
         }
         HIPCHK(c, hipMemcpy(ediag, ed.data(), ed.size() * 8, hipMemcpyHostToDevice));
         HIPCHK(c, hipMemcpy(emask, mk.data(), mk.size(), hipMemcpyHostToDevice));
@@ -1802,10 +1810,9 @@ int stage_arcs(qiw_ctx *c, int precision, ArcArgs *aa) {
     aa->ops_cm = cm;
     aa->ediag = ediag;
     aa->emask = emask;
-    aa->sector_of = lay;
-    aa->dims = lay + m.bt;
-    aa->bt_off = lay + m.bt + m.ns;
-    aa->stride = lay + m.bt + 2 * m.ns;
+    aa->element = (const uint32_t *)lay;
+    aa->bt_off = lay + m.bt;
+    aa->stride = lay + m.bt + m.ns;
     aa->bt = m.bt;
     return 0;
 }
