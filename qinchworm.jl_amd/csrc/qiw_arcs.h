@@ -826,7 +826,7 @@ inline int arc_compile(const ArcModel &m, const ArcLayout &l, const ArcBlocks &o
 // 47 slots where its two widest neighbouring levels hold 120 states.
 //   word     bits 0-7 twice the slot, 9-17 row, 31 set for all but a positive TERM, 30 set
 //            for a negative TERM (clear: STORE)
-// Slots 0-7 are the results of initial sectors 0-7, slot 8 holds 1, slot 9 takes the padding.
+// Slots 0-7 are the results (of initial sectors 0-7), slot 8 holds 1, slot 9 takes the padding.
 // The program of a group is a blob of 32-bit words, offsets relative to its start:
 //   0 constants, 1 their offset (float64 pairs; rows 0 ..), 2 arcs, 3 their offset,
 //   4 propagators, 5 their offset, 6 scaled rows, 7 their offset, 8-11 program offsets of the
@@ -838,11 +838,11 @@ inline int arc_compile(const ArcModel &m, const ArcLayout &l, const ArcBlocks &o
 //   scaled   row, source row, constant row
 // A wavefront reads eight words past its program (zeros).
 constexpr int kScalarWaves = 4, kScalarSlots = 64, kScalarFree = 10, kScalarRows = 300;
-// Results that a wavefront stores, at least one per sector; rows of LDS before the times (the
+// Results that a wavefront stores, for n_out in use; rows of LDS before the times (the
 // results take the place of the first rows), and with the times of the positions 0 .. n.
-constexpr int scalar_out_rows(int ns) { return ns <= 2 ? 2 : ns <= 4 ? 4 : 8; }
-inline int scalar_table_rows(int rows, int ns) { return std::max(rows, kScalarWaves * scalar_out_rows(ns)); }
-inline int scalar_lds_rows(int rows, int ns, int n) { return scalar_table_rows(rows, ns) + std::max(n + 1, ns); }
+constexpr int scalar_out_rows(int n_out) { return n_out <= 2 ? 2 : n_out <= 4 ? 4 : 8; }
+inline int scalar_table_rows(int rows, int n_out) { return std::max(rows, kScalarWaves * scalar_out_rows(n_out)); }
+inline int scalar_lds_rows(int rows, int n_out, int n) { return scalar_table_rows(rows, n_out) + std::max(n + 1, n_out); }
 constexpr uint32_t SARC_SPECIAL = 1u << 31, SARC_MINUS = 1u << 30;
 
 // Operator matrix elements of a scalar model.
@@ -858,8 +858,6 @@ struct ScalarProgram {
 };
 
 struct ScalarPacker {
-    const ArcModel &m;
-    const ArcValues &val;
     int kind, n, w_skipped;
     std::vector<double> consts{1.0};
     struct Arc {
@@ -907,12 +905,12 @@ struct ScalarPacker {
     };
     struct Segment {
         std::vector<uint32_t> words;  // rows by id in bits 9..
-        int s0;
+        int result;                   // slot it adds to
     };
 
     // One initial sector: states in the greedy order, slots from the free list.  Returns
     // false when the states need more slots than there are.
-    bool segment(const ArcGraph &g, Segment &out) {
+    bool segment(const ArcModel &m, const ArcValues &val, const ArcGraph &g, int result, Segment &out) {
         std::vector<Node> node;
         std::vector<std::vector<int>> id(g.levels.size());
         for (size_t l = 0; l < g.levels.size(); ++l)
@@ -974,8 +972,8 @@ struct ScalarPacker {
             return r;
         };
         auto store = [&](int i) {
-            if (i + 1 == N) {  // the closed state: the result of s0
-                slot[i] = g.s0;
+            if (i + 1 == N) {  // the closed state
+                slot[i] = result;
             } else {
                 if (pool.empty()) return false;
                 slot[i] = pool.back();
@@ -1022,17 +1020,22 @@ struct ScalarPacker {
             if (!store(i)) return false;
             done(i);
         }
-        out.s0 = g.s0;
+        out.result = result;
         return true;
     }
 };
 
-// Compiles a scalar group.  max_words: cut the graphs by the pairs of their first arcs until
+// Compiles a scalar group.  models: one, whose results are its initial sectors, or several
+// that differ in A and B alone (and their values), with one result each, the sum over the
+// initial sectors (the trace): what they share is computed once.  max_words: cut the graphs by the pairs of their first arcs until
 // a segment holds at most this many words (0: as few segments as fit).  Returns 0, 1 when a diagram ends outside its initial sector, or
 // 2 when the program does not fit the slots, the rows or the tables of the walk.
-inline int arc_compile_scalar(const ArcModel &m, const ArcValues &val, int kind, int order, int n_after, int max_words,
-                              ScalarProgram &out) {
+inline int arc_compile_scalar(const std::vector<ArcModel> &models, const std::vector<ArcValues> &values, int kind, int order,
+                              int n_after, int max_words, ScalarProgram &out) {
     out = ScalarProgram{};
+    const ArcModel &m = models[0];
+    const int n_models = (int)models.size();
+    if (n_models > 8) return 2;
     const int n = kind == ARC_BARE ? 2 * order + 2 : 2 * order + 3;
     const bool skip_w = kind == ARC_BOLD && order > 0;
     const int pos_w = kind == ARC_BARE ? 0 : 2 * order - n_after + 2;
@@ -1040,28 +1043,29 @@ inline int arc_compile_scalar(const ArcModel &m, const ArcValues &val, int kind,
     for (int t : m.table)
         if (t > 3) return 2;
     for (int n_fixed = 0; n_fixed <= order; ++n_fixed) {
-        ScalarPacker pk{m, val, kind, n, skip_w ? pos_w : 0};
+        ScalarPacker pk{kind, n, skip_w ? pos_w : 0};
         pk.const_row(1.0);
         std::vector<ScalarPacker::Segment> segs;
         double leaves = 0, total = 1;
         std::vector<int> fix(n_fixed, 0);
         for (int i = 0; i < n_fixed; ++i) total *= m.np;
         bool fits = total <= 4096;
-        for (int s0 = 0; s0 < m.ns && fits; ++s0)
+        for (int ms = 0; ms < n_models * m.ns && fits; ++ms)
             for (double c = 0; c < total && fits; ++c) {
+                const int im = ms / m.ns, s0 = ms % m.ns;
                 long long r = (long long)c;
                 for (int i = 0; i < n_fixed; ++i) {
                     fix[i] = (int)(r % m.np);
                     r /= m.np;
                 }
                 ArcGraph g;
-                if (!arc_graph(m, kind, order, n_after, s0, fix, skip_w, g)) return 1;
+                if (!arc_graph(models[im], kind, order, n_after, s0, fix, skip_w, g)) return 1;
                 if (g.levels.empty()) continue;
                 leaves += g.leaves;
                 size_t states = 0;
                 for (const auto &l : g.levels) states += l.size();
                 ScalarPacker::Segment sg;
-                if (states > 20000 || !pk.segment(g, sg))
+                if (states > 20000 || !pk.segment(models[im], values[im], g, n_models > 1 ? im : s0, sg))
                     fits = false;
                 else
                     segs.push_back(std::move(sg));
@@ -1141,8 +1145,8 @@ inline int arc_compile_scalar(const ArcModel &m, const ArcValues &val, int kind,
                 if (prog[q].size() < prog[w].size()) w = q;
             std::vector<uint32_t> ws = segs[i].words;
             for (uint32_t &x : ws) x = (x & ~(0x1FFu << 9)) | ((uint32_t)at[(x >> 9) & 0x1FFu] << 9);
-            const int s0 = segs[i].s0;
-            if (seen[w][s0]) {  // add to the sector's result of this wavefront
+            const int s0 = segs[i].result;
+            if (seen[w][s0]) {  // add to the result of this wavefront
                 ws.back() = (ws.back() & ~0xFFu) | (2u * 9u);
                 ws.push_back(2u * 9u);
                 ws.push_back(2u * (uint32_t)s0);
@@ -1166,6 +1170,11 @@ inline int arc_compile_scalar(const ArcModel &m, const ArcValues &val, int kind,
         return 0;
     }
     return 2;
+}
+
+inline int arc_compile_scalar(const ArcModel &m, const ArcValues &val, int kind, int order, int n_after, int max_words,
+                              ScalarProgram &out) {
+    return arc_compile_scalar(std::vector<ArcModel>{m}, std::vector<ArcValues>{val}, kind, order, n_after, max_words, out);
 }
 
 }  // namespace qiwi

@@ -1057,7 +1057,7 @@ __global__ __launch_bounds__(256, SLOTS > kScalarFew ? 3 : DLR ? 4 : 6) void k_e
         __syncthreads();
     }
     // ---- each wavefront's program; results in row n_out * wave + s ----
-    const int n_out = scalar_out_rows(ns);
+    const int n_res = a.n_out, n_out = scalar_out_rows(n_res);
     sarc_words<SLOTS>(words + b[8 + wave], (int)b[12 + wave], (uint32_t)lane * 8u, (uint32_t)(wave * n_out) * 512u, n_out);
     __syncthreads();
     // the leaves' sign (-1)^order, and (-1)^n_after for the external arc of a correlator
@@ -1070,19 +1070,19 @@ __global__ __launch_bounds__(256, SLOTS > kScalarFew ? 3 : DLR ? 4 : 6) void k_e
         const double *u = a.ut + g.ut_off + (int64_t)task.tau_index * a.ut_row_stride + (active ? sample : 0);
         wt *= u[(int64_t)(g.d_before + g.d_after) * g.n_samples];
     }
-    for (int s = wave; s < ns; s += 4) {
+    for (int s = wave; s < n_res; s += 4) {
         double v = 0.0;
 #pragma unroll
         for (int w = 0; w < 4; ++w) v += tab[(n_out * w + s) * 64 + lane];
         if (a.per_sample) tl[s * 64 + lane] = fabs(v);
         v = wave_sum(active ? v * wt : 0.0);
-        if (lane == 63) a.partial[(int64_t)task.out_index * ns + s] = v;
+        if (lane == 63) a.partial[(int64_t)task.out_index * n_res + s] = v;
     }
     if (a.per_sample) {
         __syncthreads();
         if (wave == 0 && active) {
             double m = 0.0;
-            for (int s = 0; s < ns; ++s) m += tl[s * 64 + lane];
+            for (int s = 0; s < n_res; ++s) m += tl[s * 64 + lane];
             a.per_sample[g.ps_off + sample] = m;
         }
     }
@@ -1115,7 +1115,7 @@ hipError_t qiw_launch_eval_arcs(hipStream_t st, const ArcArgs &a, int n_tasks, i
 
 // slots: register slots of the programs; lds: scalar_lds_rows of the largest group, 512 bytes each.
 hipError_t qiw_launch_eval_sarcs(hipStream_t st, const EvalArgs &a, int n_tasks, int slots, size_t lds) {
-    if (n_tasks < 1 || a.ns > 8 || a.dtab.n_tables > 4 || slots > kScalarSlots) return hipErrorInvalidValue;
+    if (n_tasks < 1 || a.ns > 8 || a.n_out < 1 || a.n_out > 8 || a.dtab.n_tables > 4 || slots > kScalarSlots) return hipErrorInvalidValue;
     if (slots <= kScalarFew)
         launch_sarcs<kScalarFew>(st, a, n_tasks, lds);
     else

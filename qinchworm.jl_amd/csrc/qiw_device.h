@@ -162,6 +162,7 @@ struct EvalArgs {
     int n_tau;
     double h, beta;
     int lds_slots;             // LDS doubles per wavefront
+    int n_out;                 // scalar arc walk: outputs per task (ns, or the pairs of a correlator launch)
     int step_w;                // tau_w index of a bold step
     int max_order;             // largest order of the launch's groups
     double *partial;           // [n_out][ns]
@@ -225,10 +226,10 @@ struct CorrFinalizeArgs {
     int n_tau;
     const double *partial;           // [tasks][bt] per-task block sums
     int bt;
-    const int32_t *diag_idx;         // BT indices of the diagonal elements (the trace)
-    int n_diag;
+    const int32_t *diag_idx;         // [n_pairs][n_diag] elements of a row summed for each pair (the trace)
+    int n_diag, n_pairs;
     double h, beta;
-    double *out;                     // [n_rows]
+    double *out;                     // [n_pairs][n_rows]
     // randomized qMC (k_finalize_corr_rqmc): real groups as in FinalizeArgs
     int n_real;
     const int32_t *real_first;

@@ -754,23 +754,32 @@ int compile_arcs(const HostModel &m, int kind, int order, int n_after, int corr,
 }
 
 // Compiles a group of a scalar model as an arc program.  Returns as compile_arcs.
-int compile_scalar_arcs(const HostModel &m, int kind, int order, int n_after, int corr, int max_words, Compiled &out) {
-    ArcValues v;
-    for (int p = 0; p < m.np; ++p) {
-        v.head.push_back(m.op_i[p].val);
-        v.tail.push_back(m.op_f[p].val);
+// corrs: the operator pair (-1: none), or several pairs for the traces of all.
+int compile_scalar_arcs(const HostModel &m, int kind, int order, int n_after, const std::vector<int> &corrs, int max_words,
+                        Compiled &out) {
+    std::vector<ArcModel> models;
+    std::vector<ArcValues> values;
+    for (int corr : corrs) {
+        ArcValues v;
+        for (int p = 0; p < m.np; ++p) {
+            v.head.push_back(m.op_i[p].val);
+            v.tail.push_back(m.op_f[p].val);
+        }
+        if (corr >= 0) {
+            v.a = m.corr_A[corr].val;
+            v.b = m.corr_B[corr].val;
+        }
+        models.push_back(arc_model(m, corr));
+        values.push_back(std::move(v));
     }
-    if (corr >= 0) {
-        v.a = m.corr_A[corr].val;
-        v.b = m.corr_B[corr].val;
-    }
+    const int n_out = corrs.size() > 1 ? (int)corrs.size() : m.ns;
     ScalarProgram sp;
-    const int rc = arc_compile_scalar(arc_model(m, corr), v, kind, order, n_after, max_words, sp);
+    const int rc = arc_compile_scalar(models, values, kind, order, n_after, max_words, sp);
     if (rc) return rc;
     set_arc_group(m, kind, order, n_after, sp.blob, out);
-    out.g.n_pslots = scalar_table_rows(sp.rows, m.ns);
+    out.g.n_pslots = scalar_table_rows(sp.rows, n_out);
     out.shape = qiw_sarc_slots(sp.slots);
-    out.lds_bytes = (size_t)scalar_lds_rows(sp.rows, m.ns, out.g.n_nodes) * QIW_WAVE * 8;
+    out.lds_bytes = (size_t)scalar_lds_rows(sp.rows, n_out, out.g.n_nodes) * QIW_WAVE * 8;
     out.leaves_per_sample = (int64_t)sp.leaves;
     out.edges_per_sample = (int64_t)sp.words;
     out.flops_per_sample = 2.0 * sp.words;
@@ -807,6 +816,7 @@ struct Batch {
     double flops_per_launch = 0;  // algorithmic FLOPs of one launch
     int64_t leaves_per_launch = 0, diagram_evals_per_launch = 0;
     bool overflow = false;  // the launch would exceed kMaxTasks workgroups
+    int n_out = 0;          // scalar arc walk: outputs per task (0: the sectors)
     struct Launch {         // arc walks: one launch per workgroup shape
         int first, count, shape;
         size_t lds;
@@ -1381,7 +1391,7 @@ int compile_group(qiw_ctx *c, const Batch &b, int kind, int order, int n_after, 
         return rc == 1 ? fail(c, QIW_E_OFFDIAG, kOffDiagonal) : rc == 2 ? kArcNoFit : 0;
     }
     if (b.fmt == FMT_SARC) {
-        const int rc = compile_scalar_arcs(c->m, kind, order, n_after, corr, c->tune.chunk_words, cg);
+        const int rc = compile_scalar_arcs(c->m, kind, order, n_after, {corr}, c->tune.chunk_words, cg);
         return rc == 1 ? fail(c, QIW_E_OFFDIAG, kOffDiagonal) : rc == 2 ? kArcNoFit : 0;
     }
     Compiler comp(c->m, kind, order, n_after, corr, b.fmt, b.max_order);
@@ -1501,6 +1511,7 @@ struct Plan {
     Batch b;
     DevBatch d;
     bool first_is_order0 = false;  // correlator plans: the leading group is order 0
+    bool fits = false;             // plan of all pairs: its groups fit the scalar arc walk
     int32_t *rf = nullptr, *rcnt = nullptr;  // correlator plans: per (tau row, group) task ranges
 };
 struct PlanStore {
@@ -1999,6 +2010,7 @@ EvalArgs make_eval_args(qiw_ctx *c, const Batch &bt, const DevBatch &d, double *
     a.h = m.h;
     a.beta = m.beta;
     a.lds_slots = lds;
+    a.n_out = bt.n_out ? bt.n_out : m.ns;
     a.step_w = 0;
     a.partial = partial;
     a.spt = bt.spt;
@@ -3123,6 +3135,39 @@ int build_corr_groups(qiw_ctx *c, const qiw_run *run, int ci, Batch &b, bool *fi
     return build_corr_groups_as(c, run, ci, b, first_is_order0, false);
 }
 
+// The groups of all operator pairs in one batch, one output per pair: a scalar model's pairs
+// on the same points share times, arc values and propagators, which is what a correlator of
+// low order spends its time on (three pairs of orders 0:3 on 200 points, N = 2^14: 6.9 ms one
+// after the other, 3.5 ms together).  Returns kArcNoFit when a group does not fit the walk.
+bool corr_together(const HostModel &m, const RandPlan &rq) {
+    return m.scalar_kernel && m.ncorr > 1 && m.ncorr <= 8 && !rq.scrambled && !rq.given && rq.n_seqs == 1;
+}
+int build_corr_all(qiw_ctx *c, const qiw_run *run, Batch &b, bool *first_is_order0) {
+    const HostModel &m = c->m;
+    std::vector<int> all;
+    for (int ci = 0; ci < m.ncorr; ++ci) all.push_back(ci);
+    for (int oi = 0; oi < run->n_orders; ++oi) b.max_order = std::max(b.max_order, (int)run->orders[oi]);
+    b.precision = run->precision;
+    set_format(m, b, true);
+    if (b.fmt != FMT_SARC) return kArcNoFit;
+    b.n_out = m.ncorr;
+    *first_is_order0 = false;
+    for (int oi = 0; oi < run->n_orders; ++oi) {
+        const int order = run->orders[oi];
+        if (order > 0 && run->N_samples <= 0) continue;
+        for (int na = order == 0 ? 0 : 1; na <= (order == 0 ? 0 : 2 * order - 1); ++na) {
+            Compiled cg;
+            const int rc = compile_scalar_arcs(m, QIW_G_CORR, order, na, all, c->tune.chunk_words, cg);
+            if (rc) return rc == 1 ? fail(c, QIW_E_OFFDIAG, kOffDiagonal) : kArcNoFit;
+            if (cg.n_top == 0) continue;
+            if (b.groups.empty() && order == 0) *first_is_order0 = true;
+            push_sequences(b, std::move(cg), 1, [](int) {});
+        }
+    }
+    if (b.r_first.size() > 64) return fail(c, QIW_E_LIMIT, "more than 64 (order, n_pts_after) groups");
+    return 0;
+}
+
 // correlator_2p(expansion, grid, orders, N_samples, RequestStdDev(); rand_params)
 // (src/inchworm.jl:918-1052); corr_std_out may be NULL.
 int run_correlator(qiw_ctx *c, const qiw_run *run, double *corr_out, double *corr_std_out) {
@@ -3151,7 +3196,25 @@ int run_correlator(qiw_ctx *c, const qiw_run *run, double *corr_out, double *cor
     std::vector<int32_t> dg;  // BT indices of the diagonal elements (the trace)
     for (int s = 0; s < m.ns; ++s)
         for (int i = 0; i < m.dims[s]; ++i) dg.push_back(m.bt_off[s] + i + i * m.dims[s]);
-    int32_t *diag = (int32_t *)dev(c, "diag", (size_t)m.bt * 4, &rc);
+    // all pairs in one batch where they can be
+    bool together = corr_together(m, rq);
+    if (together) {
+        Plan &p = plan_slot(c, "corr.all");
+        const std::string key = plan_key(c, run, oall, "corr.all");
+        if (p.key != key) {
+            p = Plan{};
+            rc = build_corr_all(c, run, p.b, &p.first_is_order0);
+            if (rc && rc != kArcNoFit) return rc;
+            p.fits = rc == 0;
+            rc = 0;
+        }
+        together = p.fits;
+        if (!together) p.key = key;
+    }
+    if (together)
+        for (int ci = 0; ci < m.ncorr; ++ci) dg.push_back(ci);  // behind the trace: each pair's output
+    const int dg_trace = (int)dg.size() - (together ? m.ncorr : 0);
+    int32_t *diag = (int32_t *)dev(c, "corr.diag", dg.size() * 4, &rc);
     uint32_t *sobm = rq.scrambled ? (uint32_t *)dev(c, "sobol.m", c->sob_m.size() * 4, &rc) : nullptr;
     if (rc) return rc;
     HIPCHK(c, hipMemcpy(diag, dg.data(), dg.size() * 4, hipMemcpyHostToDevice));
@@ -3159,7 +3222,7 @@ int run_correlator(qiw_ctx *c, const qiw_run *run, double *corr_out, double *cor
     // the pairs are queued on the stream back to back; their results are read after one
     // synchronisation
     struct PairOut {
-        int ci;
+        int ci, n;  // pairs ci .. ci + n - 1
         std::vector<double> out, out_std;
         hipEvent_t e0, e1;
         bool any_sampled;
@@ -3167,15 +3230,18 @@ int run_correlator(qiw_ctx *c, const qiw_run *run, double *corr_out, double *cor
     std::vector<PairOut> pending;
     pending.reserve(m.ncorr);
     int64_t given_next = 0;  // caller-drawn sequences taken by the pairs so far
-    for (int ci = 0; ci < m.ncorr; ++ci) {
+    const int n_pairs = together ? m.ncorr : 1;  // of a launch
+    for (int ci = 0; ci < m.ncorr; ci += n_pairs) {
         // groups (src/inchworm.jl:957-981): every n_pts_after of every order
-        const std::string tag = "corr" + std::to_string(ci);
+        const std::string tag = together ? "corr.all" : "corr" + std::to_string(ci);
         Plan &p = plan_slot(c, tag);
         const std::string key = plan_key(c, run, oall, tag);
         if (p.key != key) {
-            p = Plan{};
             Batch &b = p.b;
-            if ((rc = build_corr_groups(c, run, ci, b, &p.first_is_order0))) return rc;
+            if (!together) {
+                p = Plan{};
+                if ((rc = build_corr_groups(c, run, ci, b, &p.first_is_order0))) return rc;
+            }
             if (!b.groups.empty()) {
                 int ng = (int)b.groups.size();
                 const int64_t total = (int64_t)m.ntau * ng * std::max<int64_t>(run->N_samples, 1);
@@ -3198,7 +3264,7 @@ int run_correlator(qiw_ctx *c, const qiw_run *run, double *corr_out, double *cor
                                 b.tasks.push_back({gi, t * b.spt, j, (int32_t)b.tasks.size(), q.first, q.second});
                         b.flops_per_launch += (double)N * sample_flops(b.groups[gi]);
                         b.leaves_per_launch += N * b.groups[gi].leaves_per_sample;
-                        b.diagram_evals_per_launch += N * b.groups[gi].n_top;
+                        b.diagram_evals_per_launch += N * b.groups[gi].n_top * n_pairs;
                     }
                 order_tasks(b);
                 if ((rc = upload(c, tag, b, run->N_samples, p.d))) return rc;
@@ -3216,12 +3282,13 @@ int run_correlator(qiw_ctx *c, const qiw_run *run, double *corr_out, double *cor
         int ng = (int)b.groups.size();
         // the device buffers are reused by the next pair in stream order (its evaluator runs
         // after this pair's bookkeeping and copies); the host results stay per pair
-        const size_t partial_bytes = b.tasks.size() * m.bt * 8;
+        const int n_out = together ? m.ncorr : m.bt;
+        const size_t partial_bytes = b.tasks.size() * n_out * 8;
         if (c->bufs["corr.partial"].n < partial_bytes)  // the buffer grows: let queued pairs finish with it
             HIPCHK(c, hipStreamSynchronize(c->stream));
         double *partial = (double *)dev(c, "corr.partial", partial_bytes, &rc);
         int32_t *drf = p.rf, *drc = p.rcnt;
-        double *dout = (double *)dev(c, "corr.out", (size_t)m.ntau * 8, &rc);
+        double *dout = (double *)dev(c, "corr.out", (size_t)n_pairs * m.ntau * 8, &rc);
         double *dout_std = rqmc ? (double *)dev(c, "corr.out_std", (size_t)m.ntau * 8, &rc) : nullptr;
         if (rc) return rc;
         // caller-drawn sequences: tau rows 1 .. n_tau-1 of every pair in turn, each with its own
@@ -3260,8 +3327,8 @@ int run_correlator(qiw_ctx *c, const qiw_run *run, double *corr_out, double *cor
             HIPCHK(c, qiw_launch_rqmc_coords(c->stream, d.groups, ng, 2 * b.max_order, run->N_samples, sobm, rq.seed,
                                              QIW_RQ_CORR, ci, d.ut));
         }
-        pending.push_back(PairOut{ci, std::vector<double>(m.ntau), std::vector<double>(m.ntau, 0.0), nullptr, nullptr,
-                                  false});
+        pending.push_back(PairOut{ci, n_pairs, std::vector<double>((size_t)n_pairs * m.ntau),
+                                  std::vector<double>(m.ntau, 0.0), nullptr, nullptr, false});
         PairOut &po = pending.back();
         for (auto &cg : b.groups) po.any_sampled = po.any_sampled || cg.g.sampled;
         hipEvent_t &e0 = po.e0, &e1 = po.e1;
@@ -3283,9 +3350,10 @@ int run_correlator(qiw_ctx *c, const qiw_run *run, double *corr_out, double *cor
         fa.n_rows = m.ntau;
         fa.n_tau = m.ntau;
         fa.partial = partial;
-        fa.bt = m.bt;
-        fa.diag_idx = diag;
-        fa.n_diag = (int)dg.size();
+        fa.bt = n_out;
+        fa.diag_idx = together ? diag + dg_trace : diag;
+        fa.n_diag = together ? 1 : dg_trace;
+        fa.n_pairs = n_pairs;
         fa.h = m.h;
         fa.beta = m.beta;
         fa.out = dout;
@@ -3298,7 +3366,7 @@ int run_correlator(qiw_ctx *c, const qiw_run *run, double *corr_out, double *cor
         fa.nuse_out = nuse;
         HIPCHK(c, rqmc ? qiw_launch_finalize_corr_rqmc(c->stream, fa) : qiw_launch_finalize_corr(c->stream, fa));
         if ((rc = check_given_use(c, b, use, nuse, rows))) return rc;
-        HIPCHK(c, hipMemcpyAsync(po.out.data(), dout, m.ntau * 8, hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(c, hipMemcpyAsync(po.out.data(), dout, po.out.size() * 8, hipMemcpyDeviceToHost, c->stream));
         if (dout_std)
             HIPCHK(c, hipMemcpyAsync(po.out_std.data(), dout_std, m.ntau * 8, hipMemcpyDeviceToHost, c->stream));
         c->stats.n_kernel_launches += 1;
@@ -3313,13 +3381,13 @@ int run_correlator(qiw_ctx *c, const qiw_run *run, double *corr_out, double *cor
         (void)hipEventDestroy(po.e0);
         (void)hipEventDestroy(po.e1);
         c->stats.kernel_ms += ms;
-        const int ci = po.ci;
         const std::vector<double> &out = po.out, &out_std = po.out_std;
         const bool any_sampled = po.any_sampled;
-        for (int j = 0; j < m.ntau; ++j) {  // value = -i * out / Z
-            const size_t i = (size_t)ci * m.ntau + j;
+        for (int k = 0; k < po.n * m.ntau; ++k) {  // value = -i * out / Z
+            const int j = k % m.ntau;
+            const size_t i = (size_t)po.ci * m.ntau + k;
             corr_out[2 * i] = 0.0;
-            corr_out[2 * i + 1] = -out[j] / Z;
+            corr_out[2 * i + 1] = -out[k] / Z;
             if (!corr_std_out) continue;
             if (rqmc) {  // sum of the groups' deviations / Z (real)
                 corr_std_out[2 * i] = out_std[j] / Z;

@@ -1687,12 +1687,13 @@ __global__ __launch_bounds__(kReduceMax) void k_step_reduce_finalize(FinalizeArg
 // prefactor-weighted traces.  out[c][j] = sum_g (-1)^k J_g / N_g * R_g (real; the value
 // is -i * out / Z).
 
-// One block per tau row: for each group the block sums the diagonal elements of the
+// One block per tau row and pair: for each group the block sums the diagonal elements of the
 // group's task rows (items spread over the threads, then a fixed-order tree), scaled by
 // the group's sign, simplex volume and 1/N.
 __global__ __launch_bounds__(256) void k_finalize_corr(CorrFinalizeArgs a) {
     __shared__ double red[256];
     const int row = blockIdx.x, t = threadIdx.x;
+    const int32_t *diag_idx = a.diag_idx + (int64_t)blockIdx.y * a.n_diag;
     const int j = row % a.n_tau;
     const double tau_i = 0.0, tau_w = j * a.h, tau_f = a.beta;
     double tot = 0.0;
@@ -1704,7 +1705,7 @@ __global__ __launch_bounds__(256) void k_finalize_corr(CorrFinalizeArgs a) {
         KahanSum s;
         for (int64_t i = t; i < items; i += 256) {
             const int r = (int)(i / a.n_diag), e = (int)(i % a.n_diag);
-            s.add(a.partial[(int64_t)(f0 + r) * a.bt + a.diag_idx[e]]);
+            s.add(a.partial[(int64_t)(f0 + r) * a.bt + diag_idx[e]]);
         }
         red[t] = s.s - s.c;
         __syncthreads();
@@ -1723,7 +1724,7 @@ __global__ __launch_bounds__(256) void k_finalize_corr(CorrFinalizeArgs a) {
         }
         __syncthreads();
     }
-    if (t == 0) a.out[row] = tot;
+    if (t == 0) a.out[(int64_t)blockIdx.y * a.n_rows + row] = tot;
 }
 
 // ---------------------------------------------------------------------------------------
@@ -2303,7 +2304,7 @@ hipError_t qiw_launch_stage(hipStream_t st, const StageArgs &a) {
 }
 
 hipError_t qiw_launch_finalize_corr(hipStream_t st, const CorrFinalizeArgs &a) {
-    hipLaunchKernelGGL(k_finalize_corr, dim3(a.n_rows), dim3(256), 0, st, a);
+    hipLaunchKernelGGL(k_finalize_corr, dim3(a.n_rows, a.n_pairs), dim3(256), 0, st, a);
     return hipGetLastError();
 }
 
@@ -2327,7 +2328,7 @@ hipError_t qiw_launch_sigma_coords(hipStream_t st, const uint32_t *m, const uint
 }
 
 hipError_t qiw_launch_finalize_corr_rqmc(hipStream_t st, const CorrFinalizeArgs &a) {
-    if (a.n_seqs < 1 || a.n_seqs > QIW_MAX_SEQS) return hipErrorInvalidValue;
+    if (a.n_seqs < 1 || a.n_seqs > QIW_MAX_SEQS || a.n_pairs != 1) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_finalize_corr_rqmc, dim3(a.n_rows), dim3(256), 0, st, a);
     return hipGetLastError();
 }

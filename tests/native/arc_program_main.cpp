@@ -149,6 +149,8 @@ int main(int argc, char **argv) {
             std::printf("rc %d\n", rc);
             return 0;
         }
+        auto run = [&](const ScalarProgram &sp) {  // the results of its slots 0 .. 7
+        std::array<double, 8> out{};
         const std::vector<uint32_t> &b = sp.blob;
         auto at = [&](size_t i) -> uint32_t {
             if (i >= b.size()) die("word out of the program");
@@ -199,9 +201,31 @@ int main(int argc, char **argv) {
                     acc += (x & SARC_SPECIAL ? -1.0 : 1.0) * slot[sl] * tab[r];
                 }
             }
-            for (int s = 0; s < m.ns; ++s) res[s] += slot[s];
+            for (int s = 0; s < 8; ++s) out[s] += slot[s];
             for (uint32_t i = 0; i < 8; ++i)  // words read ahead, the rows of the first four too
                 if (((at(at(8 + w) + 16 * at(12 + w) + i) >> 9) & 511) >= tab.size()) die("row read ahead");
+        }
+        return out;
+        };
+        const std::array<double, 8> single = run(sp);
+        for (int s = 0; s < m.ns; ++s) res[s] += single[s];
+        if (kind == ARC_CORR) {  // with the operators' roles exchanged too: both traces in one program
+            std::vector<ArcModel> models{m, m};
+            std::vector<ArcValues> values{val, val};
+            std::swap(models[1].a_sf, models[1].b_sf);
+            std::swap(values[1].a, values[1].b);
+            ScalarProgram both, other;
+            if (arc_compile_scalar(models, values, kind, order, n_after, n_fixed ? 1 : 0, both) ||
+                arc_compile_scalar(models[1], values[1], kind, order, n_after, n_fixed ? 1 : 0, other))
+                die("programs of two pairs");
+            const std::array<double, 8> o = run(other), t = run(both);
+            double t0 = 0, t1 = 0, size = 1e-300;
+            for (int s = 0; s < m.ns; ++s) {
+                t0 += single[s];
+                t1 += o[s];
+                size += std::fabs(single[s]) + std::fabs(o[s]);
+            }
+            if (!(std::fabs(t0 - t[0]) < 1e-9 * size && std::fabs(t1 - t[1]) < 1e-9 * size)) die("traces of two pairs");
         }
         pg.leaves = sp.leaves;
         pg.n_segments = (int)sp.words;

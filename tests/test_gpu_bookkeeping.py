@@ -76,3 +76,23 @@ def test_roots(n):
     x = np.asarray(seq.points(N))[:, 0].astype(np.longdouble)
     y = np.where(x > 0, np.exp(np.log(np.where(x > 0, x, 1)) / n), 0)
     assert np.all(np.abs(out[:, 0] - y) <= 1.5 * np.spacing(np.maximum(out[:, 0], 2.0 ** -40)))
+
+
+@pytest.mark.parametrize("order,log2n", [(0, 0), (1, 3), (2, 6), (3, 7), (4, 2)])
+def test_pairs_together(order, log2n):
+    """Correlators of several pairs in one launch (three pairs, and eight: every output of a
+    wavefront in use) against the float64 oracle and against each pair alone."""
+    for copies in (1, 3):
+        e = model.anderson_single_orbital(n_tau=9, with_correlators=True)
+        e = model.Expansion(e.ed, e.grid, e.pairs, (list(e.corr_operators) * copies)[:8])
+        qiw.inchworm(e, e.grid, range(0, 2), range(0, 2), 16)
+        orders, N = range(0, order + 1), 2 ** log2n
+        g = qiw.correlator_2p(e, e.grid, orders, N)
+        c = O.correlator_2p(e, orders, N)
+        for i, x in enumerate(g):
+            one = model.Expansion(e.ed, e.grid, e.pairs, [e.corr_operators[i]])
+            one.P, one.P_n_known, one.P_der0 = e.P, e.P_n_known, e.P_der0
+            alone = qiw.correlator_2p(one, one.grid, orders, N)[0]
+            scale = np.abs(np.asarray(c[i])).max() + 1e-3
+            assert np.abs(x - np.asarray(c[i])).max() < RTOL * scale
+            assert np.abs(x - alone).max() < RTOL * scale
