@@ -345,8 +345,9 @@ typedef struct {
     double wall_s;              /* host wall time of the call                             */
     double kernel_ms;           /* summed device time of the evaluator launches (HIP events
                                    on the launch stream around each launch); a bold-step
-                                   loop replayed from its hipGraph counts as a whole, its
-                                   bookkeeping kernels included (qiw_set_graphs)          */
+                                   loop replayed from its hipGraph (qiw_set_graphs) and the
+                                   loop of qiw_diff_inchworm count as a whole, their
+                                   bookkeeping kernels included                           */
     int64_t n_kernel_launches;  /* evaluator launches                                     */
     int64_t diagram_evals;      /* (topology, sample) pairs evaluated                     */
     int64_t leaves;             /* (topology, sample, initial sector, pair assignment)

@@ -324,6 +324,18 @@ struct StageArgs {
     StageOp op[kStageOps];
 };
 
+// Simplex coordinates of every sampled group's sequence for one step: the staged
+// direction numbers m (dimensions 0..dim_max-1) LMS + shift scrambled with the bits of the
+// group's stream (domain, key, order, n_after, seq).
+struct RqmcCoords {
+    const QiwGroup *groups;
+    const uint32_t *m;
+    int n_groups;
+    int64_t n;               // samples (of the largest group)
+    uint64_t seed, domain, key;
+    double *ut;
+};
+
 // Launch wrappers (qiw_kernels.hip)
 hipError_t qiw_launch_stage(hipStream_t st, const StageArgs &a);
 hipError_t qiw_launch_zero(hipStream_t st, void *p, size_t bytes);  // bytes: a multiple of 4
@@ -350,16 +362,14 @@ hipError_t qiw_launch_ptab_cells(hipStream_t st, const double *T, int n_tau, int
                                  QiwCell32 *out32);
 hipError_t qiw_launch_finalize_step(hipStream_t st, const FinalizeArgs &a);
 hipError_t qiw_launch_finalize_corr(hipStream_t st, const CorrFinalizeArgs &a);
-hipError_t qiw_launch_finalize_step_rqmc(hipStream_t st, const FinalizeArgs &a);
+// next: coordinates to draw beside the bookkeeping (null: none)
+hipError_t qiw_launch_finalize_step_rqmc(hipStream_t st, const FinalizeArgs &a, const RqmcCoords *next);
 hipError_t qiw_launch_finalize_diff(hipStream_t st, const FinalizeArgs &a, int rqmc);
 // Coordinates of a self-energy group: rows 0 and 2k-1 are 1 and 0 (tau_f_prev, tau_i),
 // rows 1..2k-2 the RootTransform of Sobol dimensions 0..2k-3.
 hipError_t qiw_launch_sigma_coords(hipStream_t st, const uint32_t *m, const uint32_t *x0, int order, int64_t n,
                                    double *out);
 hipError_t qiw_launch_finalize_corr_rqmc(hipStream_t st, const CorrFinalizeArgs &a);
-// Simplex coordinates of every sampled group's sequence for one step: the staged
-// direction numbers m (dimensions 0..dim_max-1) LMS + shift scrambled with the bits of the
-// group's stream (domain, key, order, n_after, seq).
 // The caller's sequences of a call: the states of caller-drawn scrambled Sobol sequences
 // (gm: [.][stride][32] direction numbers, gx: [.][stride] shifts), or, with pts set, the
 // points of caller-supplied sequences (pts: [.][npts][stride]).
@@ -373,5 +383,4 @@ struct GivenSrc {
 // r) * row_stride) maps sequence idx[r * n_groups + g] (< 0: none)
 hipError_t qiw_launch_given_coords(hipStream_t st, const QiwGroup *groups, int n_groups, int64_t n, const GivenSrc &src,
                                    const int64_t *idx, int n_rows, int row0, int64_t row_stride, double *ut);
-hipError_t qiw_launch_rqmc_coords(hipStream_t st, const QiwGroup *groups, int n_groups, int max_dim, int64_t n,
-                                  const uint32_t *m, uint64_t seed, int domain, int64_t key, double *ut);
+hipError_t qiw_launch_rqmc_coords(hipStream_t st, const RqmcCoords &a, int max_dim);

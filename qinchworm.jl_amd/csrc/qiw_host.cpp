@@ -2483,11 +2483,17 @@ int run_inchworm(qiw_ctx *c, const qiw_run *run, bool do_bare, int first_w, int 
     fa.n_seqs = rq.n_seqs;
     fa.target_std = rq.target_std;
     fa.porders_std = pstd;
-    auto finalize = [&](const Batch &b, const DevBatch &d) -> hipError_t {
+    auto rqmc_args = [&](const Batch &b, const DevBatch &d, int domain, int key) {
+        return RqmcCoords{d.groups, sobm, (int)b.groups.size(), run->N_samples, rq.seed, (uint64_t)domain, (uint64_t)key, d.ut};
+    };
+    // next_w: the bold step whose coordinates are drawn beside the bookkeeping (-1: none)
+    auto finalize = [&](const Batch &b, const DevBatch &d, int next_w) -> hipError_t {
         fa.n_real = (int)b.r_first.size();
         fa.real_first = d.r_first;
         fa.real_count = d.r_count;
-        return rqmc ? qiw_launch_finalize_step_rqmc(c->stream, fa) : qiw_launch_finalize_step(c->stream, fa);
+        if (!rqmc) return qiw_launch_finalize_step(c->stream, fa);
+        const RqmcCoords next = rqmc_args(b, d, QIW_RQ_BOLD, next_w);
+        return qiw_launch_finalize_step_rqmc(c->stream, fa, next_w >= 0 ? &next : nullptr);
     };
     // per-step scrambled sequences: coordinates of every group's sequences for this step
     auto coords = [&](const Batch &b, const DevBatch &d, int domain, int key, const int64_t *gidx) -> hipError_t {
@@ -2495,9 +2501,11 @@ int run_inchworm(qiw_ctx *c, const qiw_run *run, bool do_bare, int first_w, int 
         if (b.given)
             return qiw_launch_given_coords(c->stream, d.groups, (int)b.groups.size(), run->N_samples, gsrc, gidx, 1, 0, 0,
                                            d.ut);
-        return qiw_launch_rqmc_coords(c->stream, d.groups, (int)b.groups.size(), 2 * b.max_order, run->N_samples,
-                                      sobm, rq.seed, domain, key, d.ut);
+        return qiw_launch_rqmc_coords(c->stream, rqmc_args(b, d, domain, key), 2 * b.max_order);
     };
+    // the bookkeeping of a randomized step draws the next step's coordinates (2^24 samples at most)
+    const bool draws_next = rqmc && bold_b.scrambled && !bold_b.given && run->N_samples > 0 && run->N_samples <= (1 << 24);
+    auto next_of = [&](int jw) { return draws_next && jw < last_w ? jw + 1 : -1; };
 
     // every evaluator launch is bracketed by an event pair on the launch stream
     // timing events from the context's pool (created once, reused by every call)
@@ -2533,7 +2541,7 @@ int run_inchworm(qiw_ctx *c, const qiw_run *run, bool do_bare, int first_w, int 
         fa.normalize = 0;
         fa.n_known = 0;
         fa.nuse_out = nuse_bare;
-        HIPCHK(c, finalize(bare_b, bare_d));
+        HIPCHK(c, finalize(bare_b, bare_d, -1));
         ++launches;
         if (m.ppgf_kind == QIW_GF_INC_SPLINE) n_known = 2;
         c->stats.flops += bare_b.flops_per_launch;
@@ -2613,12 +2621,14 @@ int run_inchworm(qiw_ctx *c, const qiw_run *run, bool do_bare, int first_w, int 
                 hipError_t err = hipSuccess;
                 for (int jw = first_w; jw <= last_w && err == hipSuccess; ++jw) {
                     step_args(jw);
-                    if ((err = coords(bold_b, bold_d, QIW_RQ_BOLD, jw, nullptr)) != hipSuccess) break;  // never given
+                    if ((jw == first_w || !draws_next) &&
+                        (err = coords(bold_b, bold_d, QIW_RQ_BOLD, jw, nullptr)) != hipSuccess)
+                        break;  // never given
                     if (launch_eval(c, a, bold_b) != 0) {
                         err = hipErrorUnknown;
                         break;
                     }
-                    err = finalize(bold_b, bold_d);
+                    err = finalize(bold_b, bold_d, next_of(jw));
                 }
                 hipGraph_t gr = nullptr;
                 const hipError_t e2 = hipStreamEndCapture(c->stream, &gr);
@@ -2657,8 +2667,9 @@ int run_inchworm(qiw_ctx *c, const qiw_run *run, bool do_bare, int first_w, int 
         for (int jw = first_w; jw <= last_w && !graph; ++jw) {
             a.step_w = jw;
             if (warped && (rc = warp_points(c, jw * m.h / m.beta, bold_d.ut))) return rc;
-            HIPCHK(c, coords(bold_b, bold_d, QIW_RQ_BOLD, jw,
-                             gidx_bold ? gidx_bold + (size_t)(jw - first_w) * bold_b.groups.size() : nullptr));
+            if (jw == first_w || !draws_next)
+                HIPCHK(c, coords(bold_b, bold_d, QIW_RQ_BOLD, jw,
+                                 gidx_bold ? gidx_bold + (size_t)(jw - first_w) * bold_b.groups.size() : nullptr));
             HIPCHK(c, mark());
             if ((rc = launch_eval(c, a, bold_b))) return rc;
             HIPCHK(c, mark());
@@ -2668,7 +2679,7 @@ int run_inchworm(qiw_ctx *c, const qiw_run *run, bool do_bare, int first_w, int 
             if (m.ppgf_kind == QIW_GF_INC_SPLINE && normalize) n_known = std::max(n_known, jw + 2);
             fa.n_known = (m.ppgf_kind == QIW_GF_INC_SPLINE) ? n_known : m.ntau;
             fa.normalize = normalize ? 1 : 0;
-            HIPCHK(c, finalize(bold_b, bold_d));
+            HIPCHK(c, finalize(bold_b, bold_d, next_of(jw)));
             ++launches;
             c->stats.flops += bold_b.flops_per_launch;
             c->stats.leaves += bold_b.leaves_per_launch;
@@ -2962,6 +2973,9 @@ int run_diff(qiw_ctx *c, const qiw_run *run, double *S_out, double *S_std_out) {
     };
     EvalArgs a = make_eval_args(c, b, d, ptab, eshift, dcoef, dkind, partial);
     int64_t launches = 0;
+    // the loop is timed as a whole: an event before and after every evaluator kept the GPU waiting
+    // for a third of each step
+    HIPCHK(c, mark());
     for (int st = 0; st + 1 < m.ntau; ++st) {
         fa.a = st;
         fa.jf = st + 1;  // Σ_orders at tau_f (src/inchworm.jl:770-773)
@@ -2972,18 +2986,19 @@ int run_diff(qiw_ctx *c, const qiw_run *run, double *S_out, double *S_std_out) {
             HIPCHK(c, qiw_launch_given_coords(c->stream, d.groups, (int)b.groups.size(), run->N_samples, gsrc,
                                               gidx + (size_t)st * b.groups.size(), 1, 0, 0, d.ut));
         else if (b.scrambled && !b.given)
-            HIPCHK(c, qiw_launch_rqmc_coords(c->stream, d.groups, (int)b.groups.size(), 2 * b.max_order,
-                                             run->N_samples > 0 ? run->N_samples : 1, sobm, rq.seed, QIW_RQ_DIFF, st,
-                                             d.ut));
-        HIPCHK(c, mark());
+            HIPCHK(c, qiw_launch_rqmc_coords(c->stream,
+                                             RqmcCoords{d.groups, sobm, (int)b.groups.size(),
+                                                        run->N_samples > 0 ? run->N_samples : 1, rq.seed, QIW_RQ_DIFF,
+                                                        (uint64_t)st, d.ut},
+                                             2 * b.max_order));
         if ((rc = launch_eval(c, a, b))) return rc;
-        HIPCHK(c, mark());
         HIPCHK(c, qiw_launch_finalize_diff(c->stream, fa, rqmc ? 1 : 0));
         ++launches;
         c->stats.flops += b.flops_per_launch;
         c->stats.leaves += b.leaves_per_launch;
         c->stats.diagram_evals += b.diagram_evals_per_launch;
     }
+    HIPCHK(c, mark());
     HIPCHK(c, hipStreamSynchronize(c->stream));
     for (size_t i = 0; i + 1 < n_ev; i += 2) {
         float ms = 0;
@@ -3324,8 +3339,10 @@ int run_correlator(qiw_ctx *c, const qiw_run *run, double *corr_out, double *cor
             HIPCHK(c, qiw_launch_given_coords(c->stream, d.groups, ng, run->N_samples, gsrc, didx, m.ntau - 1, 1,
                                               b.ut_total, ut_rows));
         } else if (sobm && !b.given && run->N_samples > 0) {  // one set of scrambled sequences for all tau rows
-            HIPCHK(c, qiw_launch_rqmc_coords(c->stream, d.groups, ng, 2 * b.max_order, run->N_samples, sobm, rq.seed,
-                                             QIW_RQ_CORR, ci, d.ut));
+            HIPCHK(c, qiw_launch_rqmc_coords(c->stream,
+                                             RqmcCoords{d.groups, sobm, ng, run->N_samples, rq.seed, QIW_RQ_CORR,
+                                                        (uint64_t)ci, d.ut},
+                                             2 * b.max_order));
         }
         pending.push_back(PairOut{ci, n_pairs, std::vector<double>((size_t)n_pairs * m.ntau),
                                   std::vector<double>(m.ntau, 0.0), nullptr, nullptr, false});

@@ -1520,6 +1520,17 @@ __device__ __forceinline__ void add_sums(double &s, double &c, double s2, double
     s = t;
 }
 
+// The per-group sums, written by one block and read by another of the same launch: device-scope
+// accesses, which are coherent by themselves.  A __threadfence instead writes the whole L2 of
+// the XCD back, the evaluator's and the next coordinates' rows among it (41 instead of 26 us for
+// a randomized step's bookkeeping with coordinates, 10.7 instead of 9.4 for a plain one).
+__device__ __forceinline__ void store_shared(double *p, double v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ double load_shared(const double *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // Sum over the task rows of each group, one block per group (and per 256 elements when
 // bt > 256).  The rows of a group are contiguous, so the block reads them as one
 // contiguous range: thread t covers element t % E of rows t / E, t / E + R, ... with E
@@ -1565,20 +1576,19 @@ __device__ void reduce_rows_block(const int32_t *__restrict__ first, const int32
         n = h;
         __syncthreads();
     }
-    if (t < E) gsum[(int64_t)g * bt + e0 + t] = red[t] - cmp[t];
+    if (t < E) store_shared(gsum + (int64_t)g * bt + e0 + t, red[t] - cmp[t]);
 }
 
-// The last block of a launch to get here (a counter every block increments after its sums are
-// visible); it resets the counter for the next launch and sees the sums of all blocks.
-__device__ __forceinline__ bool last_block(unsigned *done) {
-    __threadfence();
+// The last of a launch's blocks to get here (a counter every block increments after its sums are
+// stored); it resets the counter for the next launch and sees the sums of all blocks.
+__device__ __forceinline__ bool last_block(unsigned *done, unsigned blocks) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's sums have arrived
     __syncthreads();
     __shared__ int last;
-    if (threadIdx.x == 0) last = atomicAdd(done, 1u) == gridDim.x * gridDim.y - 1;
+    if (threadIdx.x == 0) last = atomicAdd(done, 1u) == blocks - 1;
     __syncthreads();
     if (!last) return false;
     if (threadIdx.x == 0) *done = 0u;
-    __threadfence();
     return true;
 }
 
@@ -1656,7 +1666,7 @@ __device__ void finalize_step_body(const FinalizeArgs &a) {
         for (int o = 0; o < kFinMaxSlots; ++o) acc[o] = 0.0;
 #pragma unroll 8
         for (int gi = 0; gi < a.n_groups; ++gi) {
-            const double v = fac_sh[gi] * gsum[(int64_t)gi * a.bt + e];
+            const double v = fac_sh[gi] * load_shared(gsum + (int64_t)gi * a.bt + e);
             const int sl = slot_sh[gi];
 #pragma unroll
             for (int o = 0; o < kFinMaxSlots; ++o) acc[o] += (o == sl) ? v : 0.0;
@@ -1676,11 +1686,11 @@ __device__ void finalize_step_body(const FinalizeArgs &a) {
 
 // One launch per step: every block reduces its group's rows; the last block to finish runs
 // the bookkeeping.  This saves a launch and its gap per step.  What bounds it: latency (a pass
-// of row loads, the counter, the groups' sums, the table's rows): 10.7 us for 256 rows of 4 in each
+// of row loads, the counter, the groups' sums, the table's rows): 9.4 us for 256 rows of 4 in each
 // of 17 groups and 200 propagator rows (13.9 with volatile reads of the sums, one at a time).
 __global__ __launch_bounds__(kReduceMax) void k_step_reduce_finalize(FinalizeArgs a) {
     reduce_rows_block(a.group_task_first, a.group_task_count, a.partial, a.bt, a.gsum);
-    if (last_block(a.done)) finalize_step_body(a);
+    if (last_block(a.done, gridDim.x * gridDim.y)) finalize_step_body(a);
 }
 
 // Correlator bookkeeping (src/inchworm.jl:825-889): per (pair, tau) row, sum the groups'
@@ -1765,20 +1775,20 @@ __device__ double seq_std(X x, int n) {
 // its scramble costs less than they do: 100 roots of eight times 2^12 samples take 23 us (52 with
 // pow, all 32 bits of every index, and 256 samples per block).
 constexpr int kRqmcSamples = 512;
-__global__ __launch_bounds__(256) void k_rqmc_coords(const QiwGroup *__restrict__ groups, const uint32_t *__restrict__ m,
-                                                     int64_t n, uint64_t seed, uint64_t domain, uint64_t key,
-                                                     double *__restrict__ ut) {
-    const QiwGroup g = groups[blockIdx.y];
+__device__ void rqmc_coords(const RqmcCoords &a, int group, int block) {
+    const QiwGroup g = a.groups[group];
+    const uint32_t *m = a.m;
+    double *ut = a.ut;
     if (!g.sampled) return;
     const bool sigma = g.kind == QIW_G_SIGMA;
     const int d = sigma ? 2 * g.order - 2 : g.d_before + g.d_after;  // Sobol dimensions used
     __shared__ uint32_t rows[2 * QIW_KMAX][33];
     __shared__ uint32_t ms[2 * QIW_KMAX * 32];
     // self-energy groups are keyed like the reference's topology data, n_pts_after = 1
-    const uint64_t stream = qiw_rq_stream(domain, key, g.order, sigma ? 1 : g.n_after, g.seq);
+    const uint64_t stream = qiw_rq_stream(a.domain, a.key, g.order, sigma ? 1 : g.n_after, g.seq);
     for (int i = threadIdx.x; i < d * 33; i += blockDim.x) {
         const int k = i / 33, w = i % 33;
-        uint32_t v = qiw_rq_word(seed, stream, k, w);
+        uint32_t v = qiw_rq_word(a.seed, stream, k, w);
         if (w > 0) {
             const int p = w - 1;
             const uint32_t below = p == 0 ? 0u : (0xFFFFFFFFu << (32 - p));
@@ -1799,7 +1809,7 @@ __global__ __launch_bounds__(256) void k_rqmc_coords(const QiwGroup *__restrict_
     const int bits = index_bits(ng);
     double *out = ut + g.ut_off;
     // the coordinates one after the other: u of the simplex, after tau_w and before it
-    for (int64_t r = (int64_t)blockIdx.x * kRqmcSamples + threadIdx.x; r < min(ng, (int64_t)(blockIdx.x + 1) * kRqmcSamples);
+    for (int64_t r = (int64_t)block * kRqmcSamples + threadIdx.x; r < min(ng, (int64_t)(block + 1) * kRqmcSamples);
          r += blockDim.x) {
         const int after = sigma ? 0 : g.d_after, row0 = sigma ? 1 : 0;
         double u = 1.0;
@@ -1815,6 +1825,8 @@ __global__ __launch_bounds__(256) void k_rqmc_coords(const QiwGroup *__restrict_
         }
     }
 }
+
+__global__ __launch_bounds__(256) void k_rqmc_coords(RqmcCoords a) { rqmc_coords(a, blockIdx.y, blockIdx.x); }
 
 // Simplex coordinates from caller-drawn sequences (the states of the ScrambledSobolSeq
 // objects the reference constructs with the caller's RNG, src/randomization.jl:94 and
@@ -1891,7 +1903,7 @@ struct SeqValues {
     double v[NS];
     __device__ __forceinline__ void load(const double *gsum, int64_t step, double fac, int n) {
 #pragma unroll
-        for (int s = 0; s < NS; ++s) v[s] = s < n ? __dmul_rn(fac, gsum[s * step]) : 0.0;
+        for (int s = 0; s < NS; ++s) v[s] = s < n ? __dmul_rn(fac, load_shared(gsum + s * step)) : 0.0;
     }
     __device__ __forceinline__ double sum(int n) const {
 #pragma clang fp contract(off)
@@ -1923,7 +1935,7 @@ struct SeqValues<0> {
         step = step_;
         fac = fac_;
     }
-    __device__ __forceinline__ double operator()(int s) const { return __dmul_rn(fac, p[s * step]); }
+    __device__ __forceinline__ double operator()(int s) const { return __dmul_rn(fac, load_shared(p + s * step)); }
     __device__ __forceinline__ double sum(int n) const { return seq_sum(*this, n); }
     __device__ __forceinline__ double std(int n) const { return seq_std(*this, n); }
 };
@@ -1935,12 +1947,12 @@ struct SeqValues<0> {
 // target_std.  The group adds the mean (sum * (1/n), as SectorBlockMatrix / n) and the
 // deviation over the sequences taken to its order's rows, in group order.
 //
-// A thread takes one element of one group at a time, 64 groups side by side: first the
-// sequence counts whose deviation is above the target (one bit each; the element-wise
-// maximum is above it when any element's is), then mean and deviation into scratch
+// A thread takes one element of one group (and sequence count) at a time, 64 groups side by
+// side: first the sequence counts whose deviation is above the target (one bit each; the
+// element-wise maximum is above it when any element's is), then mean and deviation into scratch
 // ([n_real][2][bt]), then the sums over the groups.  Group after group with a tree per
 // sequence count, as before, the launch took 280 us for 16 groups, eight sequences and two
-// elements (dependent loads and barriers); now 22 us.
+// elements (dependent loads and barriers); now 26 us with the next step's coordinates in it.
 template <int NS>
 __device__ void finalize_step_rqmc_body(const FinalizeArgs &a) {
     const int tid = threadIdx.x, nt = blockDim.x, jf = a.jf, bt = a.bt;
@@ -1962,14 +1974,12 @@ __device__ void finalize_step_rqmc_body(const FinalizeArgs &a) {
             step_sh[tid] = a.real_count[r0 + tid] > 1 ? bt : 0;
         }
         __syncthreads();
-        for (int i = tid; i < nr * bt; i += nt) {
-            const int r = i / bt, e = i - r * bt, nmax = seqs_sh[r];
+        for (int i = tid; i < nr * bt * (a.n_seqs - 1); i += nt) {  // elements of a count side by side
+            const int e = i % bt, r = (i / bt) % nr, n = 2 + i / (bt * nr);
+            if (n > seqs_sh[r]) continue;
             SeqValues<NS> x;
-            x.load(a.gsum + (int64_t)base_sh[r] * bt + e, step_sh[r], fac_sh[r], nmax);
-            unsigned long long over = 0ull;
-            for (int n = 2; n <= nmax; ++n)
-                if (x.std(n) > a.target_std) over |= 1ull << (n - 1);
-            if (over) atomicOr(&above[r], over);
+            x.load(a.gsum + (int64_t)base_sh[r] * bt + e, step_sh[r], fac_sh[r], n);
+            if (x.std(n) > a.target_std) atomicOr(&above[r], 1ull << (n - 1));
         }
         __syncthreads();
         for (int i = tid; i < nr * bt; i += nt) {
@@ -2018,9 +2028,18 @@ __device__ void finalize_step_rqmc(const FinalizeArgs &a) {
         finalize_step_rqmc_body<0>(a);
 }
 
-__global__ __launch_bounds__(kReduceMax) void k_step_reduce_finalize_rqmc(FinalizeArgs a) {
+// next: the coordinates of the following step, drawn by rows of blocks behind those of the
+// reduction: the evaluator has read the present ones, and the bookkeeping's chain of latencies
+// leaves the chip idle (a launch of their own took 23 us per step of 16 groups, eight
+// sequences of 2^12).
+__global__ __launch_bounds__(kReduceMax) void k_step_reduce_finalize_rqmc(FinalizeArgs a, RqmcCoords next) {
+    const int rows = (a.bt + 255) / 256;
+    if ((int)blockIdx.y >= rows) {
+        rqmc_coords(next, blockIdx.x, blockIdx.y - rows);
+        return;
+    }
     reduce_rows_block(a.group_task_first, a.group_task_count, a.partial, a.bt, a.gsum);
-    if (last_block(a.done)) finalize_step_rqmc(a);
+    if (last_block(a.done, gridDim.x * rows)) finalize_step_rqmc(a);
 }
 
 // Euler step of diff_inchworm_step! (src/inchworm.jl:603-635) after the self-energy row
@@ -2073,7 +2092,7 @@ __device__ void diff_euler(const FinalizeArgs &a) {
 // and the Euler step.
 __global__ __launch_bounds__(kReduceMax) void k_diff_reduce_finalize(FinalizeArgs a, int rqmc) {
     reduce_rows_block(a.group_task_first, a.group_task_count, a.partial, a.bt, a.gsum);
-    if (!last_block(a.done)) return;
+    if (!last_block(a.done, gridDim.x * gridDim.y)) return;
     if (rqmc)
         finalize_step_rqmc(a);
     else
@@ -2282,7 +2301,7 @@ hipError_t qiw_launch_eval_block(hipStream_t st, const BlockArgs &b, int n_tasks
 
 // Grid and threads of a launch that reduces task rows.  256 threads take 2048 values in one
 // pass of loads; above that the passes are what takes time and 1024 threads take a quarter of
-// them (9 groups of 1024 rows of 70 elements: 55 -> 25 us; below, the wider block only adds to
+// them (9 groups of 1024 rows of 70 elements: 55 -> 19 us; below, the wider block only adds to
 // the last block's barriers).
 static dim3 reduce_grid(const FinalizeArgs &a) { return dim3(a.n_groups, (a.bt + 255) / 256); }
 static dim3 reduce_threads(const FinalizeArgs &a) {
@@ -2308,9 +2327,15 @@ hipError_t qiw_launch_finalize_corr(hipStream_t st, const CorrFinalizeArgs &a) {
     return hipGetLastError();
 }
 
-hipError_t qiw_launch_finalize_step_rqmc(hipStream_t st, const FinalizeArgs &a) {
+hipError_t qiw_launch_finalize_step_rqmc(hipStream_t st, const FinalizeArgs &a, const RqmcCoords *next) {
     if (a.n_seqs < 1 || a.n_seqs > QIW_MAX_SEQS) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_step_reduce_finalize_rqmc, reduce_grid(a), reduce_threads(a), 0, st, a);
+    dim3 grid = reduce_grid(a);
+    if (next) {
+        if (next->n < 1 || next->n_groups != a.n_groups) return hipErrorInvalidValue;
+        grid.y += (unsigned)((next->n + kRqmcSamples - 1) / kRqmcSamples);
+        if (grid.y > 65535) return hipErrorInvalidValue;
+    }
+    hipLaunchKernelGGL(k_step_reduce_finalize_rqmc, grid, reduce_threads(a), 0, st, a, next ? *next : RqmcCoords{});
     return hipGetLastError();
 }
 
@@ -2348,10 +2373,9 @@ hipError_t qiw_launch_given_coords(hipStream_t st, const QiwGroup *groups, int n
     return hipGetLastError();
 }
 
-hipError_t qiw_launch_rqmc_coords(hipStream_t st, const QiwGroup *groups, int n_groups, int max_dim, int64_t n,
-                                  const uint32_t *m, uint64_t seed, int domain, int64_t key, double *ut) {
-    if (max_dim > 2 * QIW_KMAX || n_groups < 1 || n < 1) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_rqmc_coords, dim3((unsigned)((n + kRqmcSamples - 1) / kRqmcSamples), (unsigned)n_groups), dim3(256), 0, st,
-                       groups, m, n, seed, (uint64_t)domain, (uint64_t)key, ut);
+hipError_t qiw_launch_rqmc_coords(hipStream_t st, const RqmcCoords &a, int max_dim) {
+    if (max_dim > 2 * QIW_KMAX || a.n_groups < 1 || a.n < 1) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_rqmc_coords, dim3((unsigned)((a.n + kRqmcSamples - 1) / kRqmcSamples), (unsigned)a.n_groups),
+                       dim3(256), 0, st, a);
     return hipGetLastError();
 }
