@@ -724,13 +724,14 @@ hipError_t launch(hipStream_t st, const ArcArgs &a, int n_tasks, int waves, size
 // SLOTS: programs of up to 24 slots (all but order 4 of the single orbital and order 6 of the
 // single level) run in 80 registers, six wavefronts per SIMD, the others in 168, three.
 // Measured against the walk of the assignment tries: single-orbital solve (199 steps, orders
-// 0:4, N = 2^14) 64.9 -> 18.0 ms, its evaluator 0.31 -> 0.078 ms per step; single-level step of
-// orders 0:5 at N = 2^15 7.4 -> 0.61 ms.  Of these the walk with one register count, rows and
-// gathers one after the other took 0.084 ms; three correlators of orders 0:3 on 200 points at
-// N = 2^14 went from 10.3 to 7.1 ms with both, a randomized step of the single level (orders
-// 0:4, eight times 2^12) from 67 to 39 us.  A launch takes one instantiation for all its groups:
-// with two launches of a step the small programs' own launch cost more than it gained (single
-// orbital 85 instead of 78 us per step).
+// 0:4, N = 2^14) 64.9 -> 17.0 ms, its evaluator 0.31 -> 0.076 ms per step; single-level step of
+// orders 0:5 at N = 2^15 7.4 -> 0.18 ms, its evaluator 0.10.  Of these the walk with one register
+// count, rows and gathers one after the other took 0.084 and 0.15 ms; three correlators of orders
+// 0:3 on 200 points at N = 2^14 went from 10.3 to 7.1 ms with both (3.3 in one launch), a
+// randomized step of the single level (orders 0:4, eight times 2^12) from 67 to 36 us.  Keeping
+// intervals and fractions of the times instead cost LDS (41 us).  A launch takes one
+// instantiation for all its groups: with two launches of a step the small programs' own launch
+// cost more than it gained (single orbital 85 instead of 78 us per step).
 // ---------------------------------------------------------------------------------------
 constexpr int kScalarFew = 24;
 #define QIW_SARC_FEW                                                                                                \
@@ -897,9 +898,18 @@ struct PairLoad {
     }
 };
 
-// GRID: every table is a grid container.  The set-up reads all records with the first loads,
-// one per lane, and gathers for UA arcs and UP propagators at a time: with one after the other
-// a wavefront waited for nine tenths of its time.
+// grid_cell of two times in units of the grid step.
+__device__ __forceinline__ GridCell cell_between(double x1, double x2, int n_tau) {
+    x1 = x1 > x2 ? x1 : x2;
+    const int i1 = min(max((int)x1, 0), n_tau - 2), i2 = min(max((int)x2, 0), n_tau - 2);
+    const double a = x1 - (double)i1, b = x2 - (double)i2;
+    return GridCell{i1 - i2, a * (1.0 - b), (1.0 - a) * b};
+}
+
+// GRID: every table is a grid container, and no bare group: the times are kept in units of the
+// grid step, which halves the instructions of a cell.  The set-up reads all records with
+// the first loads, one per lane, and gathers for UA arcs and UP propagators at a time: with one
+// after the other a wavefront waited for nine tenths of its time.
 template <bool GRID, bool DLR, int SLOTS>
 __global__ __launch_bounds__(256, SLOTS > kScalarFew ? 3 : DLR ? 4 : 6) void k_eval_sarcs_t(EvalArgs a) {
     extern __shared__ __attribute__((aligned(16))) char lds[];
@@ -909,13 +919,19 @@ __global__ __launch_bounds__(256, SLOTS > kScalarFew ? 3 : DLR ? 4 : 6) void k_e
     const QiwTask task = a.tasks[blockIdx.x];
     const QiwGroup g = a.groups[task.group];
     const int n = g.n_nodes, ns = a.ns;
-    double *tl = tab + g.n_pslots * 64;  // times of the positions
+    double *tl = tab + g.n_pslots * 64;  // times of the positions (GRID: in grid steps)
     const double inv_h = 1.0 / a.h;
     const uint32_t *words = reinterpret_cast<const uint32_t *>(a.prog + g.prog_off);
     const ConstP<uint32_t> b = as_constp(words);
     const StepTimes T = step_times(a, g, task.tau_index);
-    const bool bare = g.kind == QIW_G_BARE;
+    const bool bare = !GRID && g.kind == QIW_G_BARE;
     const int na = (int)b[2], np = (int)b[4];
+    if (!(b[12] | b[13] | b[14] | b[15])) {  // no diagram: zeros
+        if (tid < a.n_out) a.partial[(int64_t)task.out_index * a.n_out + tid] = 0.0;
+        if (a.per_sample && wave == 0 && task.first_sample + lane < g.n_samples)
+            a.per_sample[g.ps_off + task.first_sample + lane] = 0.0;
+        return;
+    }
     // ---- times of the configuration positions, and the records of the rows ----
     {
         const int64_t sample = (int64_t)task.first_sample + lane;
@@ -940,23 +956,30 @@ __global__ __launch_bounds__(256, SLOTS > kScalarFew ? 3 : DLR ? 4 : 6) void k_e
                 t = T.tau_w;
             else if (p > 1 && g.sampled)
                 t = bare || p > g.pos_w ? v[i] * (T.tau_f - T.tau_w) + T.tau_w : v[i] * T.tau_w;
-            tl[p * 64 + lane] = t;
+            tl[p * 64 + lane] = GRID ? t * inv_h : t;
         }
     }
-    const ConstP<uint32_t> arc = b + b[3];
+    auto cell = [&](int later, int earlier) {  // of two positions
+        if constexpr (GRID)
+            return cell_between(tl[later * 64 + lane], tl[earlier * 64 + lane], a.n_tau);
+        else
+            return grid_cell(tl[later * 64 + lane], tl[earlier * 64 + lane], inv_h, a.n_tau);
+    };
     uint32_t rec[3] = {0u, 0u, 0u}, prec[2] = {0u, 0u};
-    if (lane < na) {
-        const uint32_t *r = words + b[3] + 3 * lane;
-        rec[0] = r[0];
-        rec[1] = r[1];
-        rec[2] = r[2];
-    }
+    auto arc_records = [&](int first) {
+        if (first + lane < na) {
+            const uint32_t *r = words + b[3] + 3 * (first + lane);
+            rec[0] = r[0];
+            rec[1] = r[1];
+            rec[2] = r[2];
+        }
+    };
+    arc_records(0);
     if (lane < np) {
         const uint32_t *r = words + b[5] + 2 * lane;
         prec[0] = r[0];
         prec[1] = r[1];
     }
-    auto arc_word = [&](int i, int w) { return i < 64 ? rlane(rec[w], i) : arc[3 * i + w]; };
     __syncthreads();
     // ---- rows: constants, arc values, propagators ----
     {
@@ -964,23 +987,25 @@ __global__ __launch_bounds__(256, SLOTS > kScalarFew ? 3 : DLR ? 4 : 6) void k_e
         for (int i = wave; i < (int)b[0]; i += 4)
             tab[i * 64 + lane] = __hiloint2double((int)c[2 * i + 1], (int)c[2 * i]);
     }
-    for (int i0 = wave; i0 < na; i0 += 4 * UA) {
+    for (int c0 = 0; c0 < na; c0 += 64) {  // records of up to 64 arcs
+    const int nc = min(64, na - c0);
+    if (c0 > 0) arc_records(c0);
+    for (int i0 = wave; i0 < nc; i0 += 4 * UA) {
         ArcPos ap[UA];
 #pragma unroll
         for (int q = 0; q < UA; ++q) {  // past the last arc: the last one again
-            const uint32_t ends = arc_word(min(i0 + 4 * q, na - 1), 0);
-            const double t1 = tl[(ends >> 8) * 64 + lane], t0 = tl[(ends & 255) * 64 + lane];
+            const uint32_t ends = rlane(rec[0], min(i0 + 4 * q, nc - 1));
             if constexpr (GRID)
-                ap[q].c = grid_cell(t1, t0, inv_h, a.n_tau);
+                ap[q].c = cell((int)(ends >> 8), (int)(ends & 255));
             else
-                ap[q] = arc_pos(t1, t0, inv_h, a.n_tau);
+                ap[q] = arc_pos(tl[(ends >> 8) * 64 + lane], tl[(ends & 255) * 64 + lane], inv_h, a.n_tau);
         }
         for (int tb = 0; tb < a.dtab.n_tables; tb += 2) {
             double c[UA][2][GRID ? 3 : 4];
             uint32_t rows[UA];
 #pragma unroll
             for (int q = 0; q < UA; ++q) {
-                rows[q] = i0 + 4 * q < na ? arc_word(i0 + 4 * q, 1 + tb / 2) : 0xFFFFFFFFu;
+                rows[q] = i0 + 4 * q < nc ? rlane(tb ? rec[2] : rec[1], i0 + 4 * q) : 0xFFFFFFFFu;
 #pragma unroll
                 for (int t = 0; t < 2; ++t) {
                     if (((rows[q] >> (16 * t)) & 0xFFFFu) == 0xFFFFu) continue;
@@ -1008,6 +1033,7 @@ __global__ __launch_bounds__(256, SLOTS > kScalarFew ? 3 : DLR ? 4 : 6) void k_e
                 }
         }
     }
+    }
     if (bare) {
         for (int i = wave; i < np; i += 4) {
             const uint32_t w = rlane(prec[0], i), seg = rlane(prec[1], i);
@@ -1024,7 +1050,7 @@ __global__ __launch_bounds__(256, SLOTS > kScalarFew ? 3 : DLR ? 4 : 6) void k_e
 #pragma unroll
             for (int q = 0; q < UP; ++q) {
                 const int i = min(i0 + 4 * q, np - 1), L = (int)(rlane(prec[1], i) & 255u);
-                c[q] = grid_cell(tl[L * 64 + lane], tl[(L - 1) * 64 + lane], inv_h, a.n_tau);
+                c[q] = cell(L, L - 1);
             }
 #pragma unroll
             for (int q = 0; q < UP; ++q) {
@@ -1039,7 +1065,7 @@ __global__ __launch_bounds__(256, SLOTS > kScalarFew ? 3 : DLR ? 4 : 6) void k_e
                 const int r = (int)(w & 0xFFFFu), s = (int)((w >> 16) & 255u), L = (int)(seg & 255u), L2 = (int)(seg >> 8);
                 d2u v = x[q].value(c[q]);
                 if (L2) {  // times the propagator after the left-out node at tau_w
-                    const GridCell c2 = grid_cell(tl[L2 * 64 + lane], tl[L * 64 + lane], inv_h, a.n_tau);
+                    const GridCell c2 = cell(L2, L);
                     PairLoad y;
                     y.load(a.ptab, ns, c2, s, (w >> 24) != 0);
                     v *= y.value(c2);
@@ -1089,11 +1115,11 @@ __global__ __launch_bounds__(256, SLOTS > kScalarFew ? 3 : DLR ? 4 : 6) void k_e
 }
 
 template <int SLOTS>
-void launch_sarcs(hipStream_t st, const EvalArgs &a, int n_tasks, size_t lds) {
+void launch_sarcs(hipStream_t st, const EvalArgs &a, int n_tasks, bool bare, size_t lds) {
     const dim3 grid(n_tasks), block(256);
     if (a.dtab.dlr_mask)
         hipLaunchKernelGGL((k_eval_sarcs_t<false, true, SLOTS>), grid, block, lds, st, a);
-    else if (a.dtab.grid_mask == (1 << a.dtab.n_tables) - 1)
+    else if (!bare && a.dtab.grid_mask == (1 << a.dtab.n_tables) - 1)
         hipLaunchKernelGGL((k_eval_sarcs_t<true, false, SLOTS>), grid, block, lds, st, a);
     else
         hipLaunchKernelGGL((k_eval_sarcs_t<false, false, SLOTS>), grid, block, lds, st, a);
@@ -1113,13 +1139,13 @@ hipError_t qiw_launch_eval_arcs(hipStream_t st, const ArcArgs &a, int n_tasks, i
     return fp32 ? launch<float, 32, 512>(st, a, n_tasks, waves, lds) : launch<double, 32, 512>(st, a, n_tasks, waves, lds);
 }
 
-// slots: register slots of the programs; lds: scalar_lds_rows of the largest group, 512 bytes each.
-hipError_t qiw_launch_eval_sarcs(hipStream_t st, const EvalArgs &a, int n_tasks, int slots, size_t lds) {
+// slots: register slots of the programs; bare: its groups are bare ones; lds: scalar_lds_rows of the largest group, 512 bytes each.
+hipError_t qiw_launch_eval_sarcs(hipStream_t st, const EvalArgs &a, int n_tasks, int slots, bool bare, size_t lds) {
     if (n_tasks < 1 || a.ns > 8 || a.n_out < 1 || a.n_out > 8 || a.dtab.n_tables > 4 || slots > kScalarSlots) return hipErrorInvalidValue;
     if (slots <= kScalarFew)
-        launch_sarcs<kScalarFew>(st, a, n_tasks, lds);
+        launch_sarcs<kScalarFew>(st, a, n_tasks, bare, lds);
     else
-        launch_sarcs<kScalarSlots>(st, a, n_tasks, lds);
+        launch_sarcs<kScalarSlots>(st, a, n_tasks, bare, lds);
     return hipGetLastError();
 }
 int qiw_sarc_slots(int slots) { return slots <= kScalarFew ? kScalarFew : kScalarSlots; }

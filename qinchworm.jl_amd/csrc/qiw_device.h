@@ -353,7 +353,7 @@ hipError_t qiw_launch_eval_flat(hipStream_t st, const EvalArgs &a, int n_tasks, 
 hipError_t qiw_launch_eval_block(hipStream_t st, const BlockArgs &b, int n_tasks, size_t lds_bytes);
 hipError_t qiw_launch_eval_mfma(hipStream_t st, const MfmaArgs &m, int n_tasks, int km, int tm, size_t lds_bytes);
 hipError_t qiw_launch_eval_arcs(hipStream_t st, const ArcArgs &a, int n_tasks, int mb, int fp32, int waves, size_t lds);
-hipError_t qiw_launch_eval_sarcs(hipStream_t st, const EvalArgs &a, int n_tasks, int slots, size_t lds);
+hipError_t qiw_launch_eval_sarcs(hipStream_t st, const EvalArgs &a, int n_tasks, int slots, bool bare, size_t lds);
 int qiw_sarc_slots(int slots);  // slots of the instantiation that runs a program of `slots`
 int qiw_arc_rows(int mb);
 int qiw_arc_waves(int mb, int fp32);

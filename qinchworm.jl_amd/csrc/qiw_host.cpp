@@ -1853,7 +1853,7 @@ int launch_eval(qiw_ctx *c, const EvalArgs &a, const Batch &batch) {
         EvalArgs e = a;
         for (const Batch::Launch &ln : batch.launches) {
             e.tasks = a.tasks + ln.first;
-            HIPCHK(c, qiw_launch_eval_sarcs(c->stream, e, ln.count, ln.shape, ln.lds));
+            HIPCHK(c, qiw_launch_eval_sarcs(c->stream, e, ln.count, ln.shape, batch.groups[0].g.kind == QIW_G_BARE, ln.lds));
         }
         return 0;
     }
