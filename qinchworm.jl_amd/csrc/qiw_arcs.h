@@ -289,9 +289,11 @@ constexpr int kArcGroupHead = 8, kArcSegHead = 8, kArcSlotWords = 8;
 constexpr int kArcTileOps = 28;          // most operators of a tile
 constexpr int kArcReadAhead = 6 * 256;   // words a wavefront may read past its streams
 
-// Slots of a packet of the walk whose lanes hold vectors of `rows` values: as many as their
-// blocks fit in registers twice.
-constexpr int arc_slots(int rows, bool fp32) { return fp32 && rows <= 8 ? 4 : rows <= 8 || (fp32 && rows <= 20) ? 2 : 1; }
+// Slots of a packet of the walk whose lanes hold vectors of `rows` values.  The blocks of a packet
+// and of the next one stay in registers: with more slots what spills costs more than the longer
+// read-ahead saves (two-orbital step of orders 0:4, float32: 22.4, 21.1, 21.1 ms with four, three
+// and two slots; three-orbital step of orders 0:3, float32: 31.7 and 31.1 ms with two and one).
+constexpr int arc_slots(int rows) { return rows <= 8 ? 2 : 1; }
 
 struct ArcLayout {
     int elem = 4;             // bytes of the value type

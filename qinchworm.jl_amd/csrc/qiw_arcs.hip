@@ -109,7 +109,7 @@ __device__ __forceinline__ void mfma_block(f4 (&acc)[MB / 4], const float *A, co
 template <int MB>
 struct Walk<float, MB> {
     static constexpr int NV = (MB / 4 * MB + 15) / 16;  // slice registers of a block
-    static constexpr int SL = arc_slots(MB, true);
+    static constexpr int SL = arc_slots(MB);
     f4 acc[MB / 4];
     float y[MB], A[SL][NV], next[SL][NV];  // blocks of the packet and of the next one
     int rk[NV];                            // row | column << 8 of this lane's element of slice register v
@@ -236,7 +236,7 @@ template <int MB>
 struct Walk<double, MB> {
     static constexpr int CH = MB <= 8 ? 8 : 4;  // columns of a chunk
     static constexpr int NV = CH * MB / 16;     // register pairs of a chunk
-    static constexpr int SL = arc_slots(MB, false);
+    static constexpr int SL = arc_slots(MB);
     double acc[MB], y[MB], A[SL][NV], next[SL][NV];  // first chunks of the packet and of the next one
     int rk[NV];  // row | column of the chunk << 8 of this lane's element of register pair v
     int lane;
@@ -476,9 +476,9 @@ __device__ __forceinline__ double prop_element(const double *ptab, int bt, const
 // blocks 1 4 6 4 1, float32), so a lane cannot own a sample; states of one sector share
 // operator and propagator, so both are wavefront-uniform.  Measured against the walk of the
 // assignment tries (one pass per diagram): two-orbital solve on 50 points, orders 0:2 at
-// N = 2^10, float64 451 -> 15.7 ms; two-orbital step, orders 0:4 at N = 2^11, float32 643 -> 22.5
+// N = 2^10, float64 451 -> 15.4 ms; two-orbital step, orders 0:4 at N = 2^11, float32 643 -> 21.2
 // ms; orders 0:3 at N = 2^12, float64 144 -> 8.8 ms; three-orbital step, orders 0:3 at N =
-// 2^9, float32 399 -> 33.9 ms; orders 0:2 at N = 2^8, float64 63.8 -> 3.2 ms.  Of these the
+// 2^9, float32 399 -> 31.4 ms; orders 0:2 at N = 2^8, float64 63.8 -> 3.2 ms.  Of these the
 // first form of the walk reached 29.9, 43.6, 18.2, 54.8 and 28.8 ms: what it lost were branches
 // on every row and column (one in five instructions), operator blocks and joins read when they
 // were wanted (a load's whole latency each), stages waiting for one wavefront with a tile of
@@ -491,10 +491,10 @@ __device__ __forceinline__ double prop_element(const double *ptab, int bt, const
 // state.  The closed states of all segments are multiplied by the last propagator in float64
 // at the end (segment by segment its gathers and the sums in memory were waited for each time).
 // Wavefronts per SIMD: float64 at MB = 8 takes three (168 registers, what spills is outside the
-// slots; 11.7 -> 9.9 ms against two), float32 of wide blocks two (no spills; 43.3 -> 37.2 ms
-// against four).
+// slots; two-orbital step 8.7 ms, 11.0 with two and 11.1 with four), float32 at MB = 20 three
+// (three-orbital step 31.7 ms; 33.7 with two, 39.2 with four).
 template <typename V, int MB, int NT>
-__global__ __launch_bounds__(NT, MB == 8 && sizeof(V) == 8 ? 3 : 2) void k_eval_arcs_t(ArcArgs aa) {
+__global__ __launch_bounds__(NT, (MB == 8 && sizeof(V) == 8) || NT == 768 ? 3 : 2) void k_eval_arcs_t(ArcArgs aa) {
     extern __shared__ __attribute__((aligned(16))) char lds[];
     const EvalArgs &a = aa.e;
     const int tid = threadIdx.x, nt = blockDim.x;
@@ -1130,12 +1130,12 @@ void launch_sarcs(hipStream_t st, const EvalArgs &a, int n_tasks, bool bare, siz
 // Vector length of the instantiation for blocks up to mb, and the most wavefronts a
 // workgroup of it can have (its registers).
 int qiw_arc_rows(int mb) { return mb <= 8 ? 8 : mb <= 20 ? 20 : 32; }
-int qiw_arc_waves(int mb, int fp32) { return mb <= 8 && fp32 ? 16 : 8; }
+int qiw_arc_waves(int mb, int fp32) { return !fp32 ? 8 : mb <= 8 ? 16 : mb <= 20 ? 12 : 8; }
 
 hipError_t qiw_launch_eval_arcs(hipStream_t st, const ArcArgs &a, int n_tasks, int mb, int fp32, int waves, size_t lds) {
     if (n_tasks < 1 || mb > 32 || a.e.n_tau < 2) return hipErrorInvalidValue;
     if (mb <= 8) return fp32 ? launch<float, 8, 1024>(st, a, n_tasks, waves, lds) : launch<double, 8, 512>(st, a, n_tasks, waves, lds);
-    if (mb <= 20) return fp32 ? launch<float, 20, 512>(st, a, n_tasks, waves, lds) : launch<double, 20, 512>(st, a, n_tasks, waves, lds);
+    if (mb <= 20) return fp32 ? launch<float, 20, 768>(st, a, n_tasks, waves, lds) : launch<double, 20, 512>(st, a, n_tasks, waves, lds);
     return fp32 ? launch<float, 32, 512>(st, a, n_tasks, waves, lds) : launch<double, 32, 512>(st, a, n_tasks, waves, lds);
 }
 

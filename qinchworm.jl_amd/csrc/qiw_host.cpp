@@ -669,14 +669,14 @@ ArcBlocks arc_blocks(const HostModel &m, int corr, int precision) {
 // CU's LDS: the more columns fit beside each other, the fewer lanes idle in the tiles of one
 // operator (three-orbital step of orders 0:2, N = 2^8, float64: 8.6 ms with two workgroups of
 // 80 KB per CU, which left seven in a hundred lanes at work, 3.1 with one of 160 KB; orders 0:3,
-// N = 2^9, float32: 35.3 and 33.5 ms).
+// N = 2^9, float32: 35.3 and 33.5 ms; 31.2 with twelve wavefronts instead of eight).
 struct ArcShape {
     int waves;
     size_t cap;
     int tiles;
 };
 constexpr ArcShape kArcShapes[] = {{2, 40 << 10, 2}, {4, 53 << 10, 12}, {8, 80 << 10, 32}, {16, 160 << 10, 1 << 30}};
-constexpr ArcShape kArcShapesWide[] = {{8, 160 << 10, 1 << 30}};  // mmax > 8
+constexpr ArcShape kArcShapesWide[] = {{12, 160 << 10, 1 << 30}};  // mmax > 8; at most qiw_arc_waves
 
 // Algorithmic real FLOPs of one sample of a compiled group: the scalar walk's multiply per
 // trie edge and leaf, or the block programs' chain products.
@@ -717,7 +717,7 @@ int compile_arcs(const HostModel &m, int kind, int order, int n_after, int corr,
     const int max_waves = qiw_arc_waves(m.mmax, fp32 ? 1 : 0);
     ArcLayout l;
     l.elem = fp32 ? 4 : 8;
-    l.slots = arc_slots(qiw_arc_rows(m.mmax), fp32);
+    l.slots = arc_slots(qiw_arc_rows(m.mmax));
     l.mmax = m.mmax;
     l.bt = m.bt;
     l.bt_off.assign(m.bt_off.begin(), m.bt_off.end());

@@ -80,7 +80,7 @@ int main(int argc, char **argv) {
     l.bt = off[m.ns];
     l.bt_off.assign(off.begin(), off.end() - 1);
     l.waves = waves;
-    l.slots = arc_slots(l.mmax <= 8 ? 8 : l.mmax <= 20 ? 20 : 32, elem == 4);
+    l.slots = arc_slots(l.mmax <= 8 ? 8 : l.mmax <= 20 ? 20 : 32);
     l.cap = cap;
     std::vector<std::vector<double>> blocks;  // operator blocks, named by index
     std::vector<std::pair<int, int>> shape;
