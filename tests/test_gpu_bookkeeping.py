@@ -1,8 +1,9 @@
-"""Step bookkeeping (row sums, order sums, sequence statistics, normalization, Euler step) at
-the edges of its work mapping, against the float64 oracle: sequence counts kept in registers
-(8) and read from memory (9, 17), reductions of 256 and of 1024 threads, blocks of 2, 4 and 70
-elements, more than 256 propagator rows, tables handed over by a kernel and (beyond 64 KB) by a copy.  Tolerance 1e-10 relative, as for every float64 path;
-a deviation's error is bounded by 1e-10 of the samples' scale."""
+"""Step bookkeeping (row sums, order sums, sequence statistics, normalization, Euler step),
+transfers, roots and correlator launches at the edges of their work mapping, against the float64
+oracle: sequence counts kept in registers (8) and read from memory (9, 17), reductions of 256 and
+of 1024 threads, blocks of 2, 4 and 70 elements, more than 256 propagator rows, tables handed over
+by a kernel and (beyond 64 KB) by a copy.  Tolerance 1e-10 relative, as for every float64 path; a
+deviation's error is bounded by 1e-10 of the samples' scale."""
 import ctypes as C
 
 import numpy as np
