@@ -32,8 +32,8 @@ sys.path.insert(0, os.path.join(REPO, "tests"))
 FP64_PEAK_TFLOPS = 78.6   # MI355X dense FP64 (vector and matrix)
 FP32_PEAK_TFLOPS = 157.3  # MI355X dense FP32, published (vector with packed FP32, and matrix)
 FP32_VALU_UNPACKED_TFLOPS = 78.6  # FP32 VALU without packed math (disabled in this build)
-C1_TRAFFIC_PROFILE = os.path.join(REPO, "profiles", "k_eval_flat_c1_hbm_traffic.md")
-C2_TRAFFIC_PROFILE = os.path.join(REPO, "profiles", "k_eval_vec_c2_hbm_traffic.md")
+C1_TRAFFIC_PROFILE = os.path.join(REPO, "profiles", "k_eval_sarcs_c1_hbm_traffic.md")
+C2_TRAFFIC_PROFILE = os.path.join(REPO, "profiles", "k_eval_arcs_c2_hbm_traffic.md")
 
 
 _T0 = time.perf_counter()
@@ -507,10 +507,11 @@ def single_orbital(log2n, steps, warmup, sync, with_cpu):
            "value": g["evals"] / g["dt"], "unit": "diagram evals/s", "ms_per_step": 1e3 * g["dt"] / steps,
            "time_to_solution_s": g["dt"] / steps,
            "eager": {"ms_per_step": 1e3 * e["dt"] / steps, "value": e["evals"] / e["dt"]},
-           "roofline": {"bound": "salu", "achieved": achieved, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
+           "roofline": {"bound": "issue", "achieved": achieved, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
                         "frac": achieved / FP64_PEAK_TFLOPS, "traffic": measured_traffic(C1_TRAFFIC_PROFILE),
-                        "kernel": "k_eval_flat_t<4,4,2,false>", "avg_launch_ms": avg_launch_ms,
-                        "note": "float64 scalar walk: one multiply per trie edge, bound by scalar-unit issue"}}
+                        "kernel": "k_eval_sarcs_t<true,false,64>", "avg_launch_ms": avg_launch_ms,
+                        "note": "float64 open-arc programs: one multiply-add per word, bound by instruction issue; the "
+                                "FLOPs are those of the merged partial diagrams"}}
     if with_cpu:
         out["cpu_baseline"] = cpu_baseline(N)
     return out
@@ -566,15 +567,14 @@ def two_orbital_headline(log2n, steps, warmup, sync, with_cpu, cpu_log2n=8, err_
            "leaves_per_s": acc["leaves"] / dt,
            "fp32_vs_fp64": {"N": ne, "rel_err_step": float(np.linalg.norm(v32 - v64) / np.linalg.norm(v64)),
                             "max_abs_err_step": float(np.abs(v32 - v64).max())},
-           "roofline": {"bound": "valu", "achieved": achieved, "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
+           "roofline": {"bound": "issue", "achieved": achieved, "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
                         "frac": achieved / FP32_PEAK_TFLOPS,
                         "frac_of_unpacked_fp32_valu": achieved / FP32_VALU_UNPACKED_TFLOPS,
-                        "traffic": measured_traffic(C2_TRAFFIC_PROFILE), "kernel": "k_eval_vec_t<float,6,4,2,2>",
+                        "traffic": measured_traffic(C2_TRAFFIC_PROFILE), "kernel": "k_eval_arcs_t<float,8,1024>",
                         "avg_launch_ms": avg_launch_ms, "flops_per_launch": acc["flops"] / max(acc["launches"], 1),
-                        "note": "float32 chain products on the vector ALUs (blocks <= 6 do not fill MFMA tiles); "
-                                "packed FP32 is disabled in this build, so 78.6 TFLOP/s is the reachable ceiling; "
-                                "the busiest unit is the vector-memory address path (per-lane propagator-cell "
-                                "gathers, 79 % busy, profiles/k_eval_vec_c2_counters.md), VALU issue 39 %"}}
+                        "note": "float32 open-arc products on v_mfma_f32_4x4x1 (one lane per column of a state), "
+                                "bound by issue and the stages' barriers; the FLOPs are those of the merged "
+                                "partial diagrams"}}
     if with_cpu:
         import oracle_lib as O
         threads = cpu_threads()
