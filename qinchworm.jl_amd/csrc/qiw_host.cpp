@@ -1522,8 +1522,9 @@ struct PlanStore {
 void plans_destroy(PlanStore *p) { delete p; }
 
 // The bold-step loop of an inchworm run (per step: coordinates when scrambled, the
-// evaluator between two timing events, the bookkeeping kernel) captured once and replayed
-// while every launch argument is the same: `key` holds their bytes.
+// evaluator's launches, the bookkeeping kernel) captured once and replayed while every launch is
+// the same: `key` holds the bytes of their arguments, and of the evaluators' workgroup counts,
+// shapes and LDS (launch_eval), which two programs of one order and sample count need not share.
 struct StepGraph {
     std::string key;
     hipGraph_t graph = nullptr;
@@ -1831,9 +1832,16 @@ int stage_arcs(qiw_ctx *c, int precision, ArcArgs *aa) {
 // Launches the evaluator matching the model's sector structure.  The vector and matrix-core
 // walks stage their operator tables once per model on their first launch (synchronous
 // copies), so a launch can be captured into a hipGraph only after that
-// (c->vec_staged / c->mfma_staged).
-int launch_eval(qiw_ctx *c, const EvalArgs &a, const Batch &batch) {
+// (c->vec_staged / c->mfma_staged).  record: append the bytes of every launch (arguments,
+// workgroups, shape, LDS) instead of launching; two calls of one format and precision with the
+// same bytes launch the same.
+int launch_eval(qiw_ctx *c, const EvalArgs &a, const Batch &batch, std::string *record = nullptr) {
     const HostModel &m = c->m;
+    auto put = [&](const auto &args, int count, int shape, size_t lds) {
+        record->append((const char *)&args, sizeof(args));
+        const int64_t v[4] = {m.mmax, count, shape, (int64_t)lds};
+        record->append((const char *)v, sizeof(v));
+    };
     const int n_tasks = (int)batch.tasks.size(), fmt = batch.fmt, precision = batch.precision;
     if (fmt == FMT_ARC) {
         ArcArgs aa{};
@@ -1842,6 +1850,10 @@ int launch_eval(qiw_ctx *c, const EvalArgs &a, const Batch &batch) {
         aa.e = a;
         for (const Batch::Launch &ln : batch.launches) {
             aa.e.tasks = a.tasks + ln.first;
+            if (record) {
+                put(aa, ln.count, ln.shape, ln.lds);
+                continue;
+            }
             HIPCHK(c, qiw_launch_eval_arcs(c->stream, aa, ln.count, m.mmax, precision == QIW_PREC_FP32 ? 1 : 0, ln.shape,
                                            ln.lds));
         }
@@ -1853,11 +1865,19 @@ int launch_eval(qiw_ctx *c, const EvalArgs &a, const Batch &batch) {
         EvalArgs e = a;
         for (const Batch::Launch &ln : batch.launches) {
             e.tasks = a.tasks + ln.first;
+            if (record) {
+                put(e, ln.count, ln.shape, ln.lds);
+                continue;
+            }
             HIPCHK(c, qiw_launch_eval_sarcs(c->stream, e, ln.count, ln.shape, batch.groups[0].g.kind == QIW_G_BARE, ln.lds));
         }
         return 0;
     }
     if (fmt == FMT_SCALAR) {
+        if (record) {
+            put(a, n_tasks, 0, 0);
+            return 0;
+        }
         HIPCHK(c, qiw_launch_eval_flat(c->stream, a, n_tasks, a.max_order, m.ns, m.ntab));
         return 0;
     }
@@ -1906,6 +1926,10 @@ int launch_eval(qiw_ctx *c, const EvalArgs &a, const Batch &batch) {
         mf.btp = m.btp;
         mf.ops_zero = (int)m.ops_rm.size() - 4;
         mf.wave_lds = (int)wave_lds;
+        if (record) {
+            put(mf, n_tasks, 0, lds);
+            return 0;
+        }
         HIPCHK(c, qiw_launch_eval_mfma(c->stream, mf, n_tasks, a.max_order, m.ntab, lds));
         return 0;
     }
@@ -1936,7 +1960,6 @@ int launch_eval(qiw_ctx *c, const EvalArgs &a, const Batch &batch) {
             HIPCHK(c, hipMemset(pt, 0, ((size_t)(m.ntau - 1) * m.bt + pad) * 16));
             c->vec_staged = true;
         }
-        HIPCHK(c, qiw_launch_ptab_cells(c->stream, a.ptab, m.ntau, m.bt, pt, ptm, pt32));
         VecArgs v{};
         v.e = a;
         v.pt = pt;
@@ -1946,6 +1969,11 @@ int launch_eval(qiw_ctx *c, const EvalArgs &a, const Batch &batch) {
         v.ops = ops;
         v.ops32 = ops32;
         v.bt = m.bt;
+        if (record) {
+            put(v, n_tasks, 0, 0);
+            return 0;
+        }
+        HIPCHK(c, qiw_launch_ptab_cells(c->stream, a.ptab, m.ntau, m.bt, pt, ptm, pt32));
         HIPCHK(c, qiw_launch_eval_vec(c->stream, v, n_tasks, m.mmax, a.max_order, m.ntab,
                                       precision == QIW_PREC_FP32 ? 1 : 0));
         return 0;
@@ -2573,10 +2601,6 @@ int run_inchworm(qiw_ctx *c, const qiw_run *run, bool do_bare, int first_w, int 
         // are unchanged: the flat scalar walk, the arc walk, and the vector and matrix-core walks once their
         // tables are staged (from the second call on); the LDS block walk copies host data per
         // launch and stays eager
-        if (bold_b.fmt == FMT_ARC) {  // stages its tables here, before a capture
-            ArcArgs aa{};
-            if ((rc = stage_arcs(c, bold_b.precision, &aa))) return rc;
-        }
         const bool staged = bold_b.fmt == FMT_SCALAR || bold_b.fmt == FMT_ARC || bold_b.fmt == FMT_SARC ||
                             (bold_b.fmt == FMT_VEC && (m.mmax > 6 ? c->mfma_staged : c->vec_staged));
         // a few steps launch faster one by one than a graph is replayed, or captured for new times
@@ -2588,8 +2612,7 @@ int run_inchworm(qiw_ctx *c, const qiw_run *run, bool do_bare, int first_w, int 
             const int n_known0 = n_known;
             std::string key;
             auto put = [&](const void *p, size_t n) { key.append((const char *)p, n); };
-            const int n_tasks = (int)bold_b.tasks.size();
-            put(&n_tasks, 4);
+            if ((rc = launch_eval(c, a, bold_b, &key))) return rc;  // (stages the arc walk's tables, before a capture)
             put(&bold_b.max_order, 4);
             put(&rq.seed, 8);
             const uint32_t *sm = sobm;
