@@ -779,7 +779,9 @@ inline int arc_compile(const ArcModel &m, const ArcLayout &l, const ArcBlocks &o
             if (!arc_graph(m, kind, order, n_after, s0, fix, skip_w, g)) return 1;
             if (!g.levels.empty()) graphs.push_back(std::move(g));
         }
-    const int most_arcs = order * (2 * order - 1) * (1 + *std::max_element(m.table.begin(), m.table.end()));
+    int n_tables = 0;  // (none in a model without pairs)
+    for (int t : m.table) n_tables = std::max(n_tables, t + 1);
+    const int most_arcs = order * (2 * order - 1) * n_tables;
     const ArcLds at = arc_lds(l, n, order > 0 ? most_arcs : 0);
     if (at.states + (size_t)l.bt * 8 > l.cap || 2 + 2 * most_arcs >= 4096) return 2;
     const size_t room = (l.cap - at.states) / l.elem;

@@ -64,3 +64,11 @@ def test_states_beyond_the_lds(driver):
     whole = driver(BOLD, 4, 4, 0, 4, 100000, 8, 2, 1).split()
     cut = driver(BOLD, 4, 4, 1, 4, int(whole[6]) - 1, 8, 2, 1).split()
     assert whole[0] == cut[0] == "dev" and float(cut[1]) < 1e-9
+
+
+@pytest.mark.parametrize("kind,order", [(BOLD, 0), (BOLD, 1), (BARE, 0), (BARE, 2), (CORR, 0), (SIGMA, 1)])
+def test_model_without_pairs(driver, kind, order):
+    """No interaction pair: the propagator alone at order 0, no diagram above."""
+    n_after = {BARE: 2 * order, SIGMA: 1}.get(kind, order)
+    out = driver(kind, order, n_after, 0, 2, 20000, 8, 0, 1).split()
+    assert out[0] == "dev" and float(out[1]) < 1e-9 and out[3] == out[4]

@@ -88,3 +88,14 @@ def test_scalar_arc_walk(which, order, log2n):
         assert np.abs(p_g - p_c).max() < 1e-10 * np.abs(v_c).max()
         for x, y in zip(g_g, O.correlator_2p(ec, range(0, min(order, 3) + 1), N)):
             assert rel(x, y) < 1e-10
+
+
+@pytest.mark.parametrize("orders", [range(0, 1), range(0, 3)])
+def test_model_without_pairs(orders):
+    """A sector-block model that couples to no bath: the atomic propagator and correlator."""
+    def make():
+        e = fermions(3, particles)
+        return model.Expansion(e.ed, e.grid, [], e.corr_operators)
+    eg, ec = make(), make()
+    assert rel(qiw.inchworm_step(eg, 2, orders, 4)[0], O.inchworm_step(ec, orders, 4, 2)[0]) < 1e-10
+    assert rel(qiw.correlator_2p(eg, eg.grid, orders, 4)[0], O.correlator_2p(ec, orders, 4)[0]) < 1e-10
