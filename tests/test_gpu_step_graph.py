@@ -19,7 +19,7 @@ def test_replay_equals_the_eager_loop(name):
         for what, pairs, N in calls:
             print(f"{name}: {what}, {pairs} pairs, N={N}", flush=True)
             (solve_of if what == "solve" else step_of)(ctx, e := make(pairs), orders, N, prec)
-        assert qiw.stats(ctx).graph_replays > 0
+        assert qiw.stats(ctx)["graph_replays"] > 0
         ctx.check(ctx.lib.qiw_set_graphs(ctx.h, 0))
         solve_of(ctx, f := make(pairs), orders, N, prec)
         assert np.array_equal(e.P, f.P)
