@@ -1342,13 +1342,25 @@ static int ystack_rows(const HostModel &m, int levels) {
 // Samples per task.  The scalar and vector walks map one sample to a lane (64 per task);
 // the block and matrix-core walks evaluate one sample at a time per wavefront, so their
 // tasks are cut smaller until a launch holds at least 4 tasks per SIMD of the device.
-// The arc walk takes a workgroup per sample: its tasks are cut until a launch holds 4096.
-int samples_per_task(const qiw_ctx *c, const HostModel &m, int fmt, int64_t total_samples) {
+// The arc walk takes a workgroup per sample: its tasks are cut until a launch holds 4096, or as
+// many as there may be rows (rows: for its sample blocks; step_rows).
+int samples_per_task(const qiw_ctx *c, const HostModel &m, int fmt, int64_t total_samples, int64_t rows = INT64_MAX) {
     if (fmt == FMT_SCALAR || fmt == FMT_SARC || (fmt == FMT_VEC && m.mmax <= 6)) return QIW_WAVE;
     if (c->tune.samples_per_task > 0) return c->tune.samples_per_task;
     int spt = QIW_WAVE;
-    while (spt > 1 && total_samples / spt < 4096) spt /= 2;
+    while (spt > 1 && total_samples / spt < 4096 && (fmt != FMT_ARC || 2 * total_samples / spt <= rows)) spt /= 2;
     return spt;
+}
+
+// Task rows of a step that fit the scratch array of qiw_inchworm_step_noalloc beside its other
+// per-call buffers (per_call_buffer): n_slots order slots, n_groups groups of n_eval sequences.
+int64_t step_rows(const qiw_ctx *c, const RandPlan &rq, int64_t n_slots, int64_t n_groups) {
+    const HostModel &m = c->m;
+    const bool rqmc = rq.n_seqs > 1;
+    const int64_t row = 8 * (int64_t)m.bt, up = 10 * 256;  // (each buffer starts at 256 bytes)
+    const int64_t others = row * (m.ntau * (1 + n_slots * (rqmc ? 2 : 1)) + n_groups * (rq.n_eval() + (rqmc ? 2 : 0))) +
+                           8 * (int64_t)m.ntau + 4 * (int64_t)m.bt + (rq.scrambled ? 4 * (int64_t)c->sob_m.size() : 0) + up;
+    return std::max<int64_t>(0, (int64_t)kNoAllocScratchBytes - others) / row;
 }
 
 std::vector<int> orders_all(const qiw_run *run) {
@@ -1407,19 +1419,32 @@ void set_format(const HostModel &m, Batch &b, bool arcs) {
 }
 
 // The program parts of a group that get tasks of their own per sample block (QiwTask::chunk
-// and pad_): topology chunks, or for the arc walk all segments (-1), or each segment when
-// the sample blocks alone are fewer than 2048 workgroups.
-std::vector<std::pair<int32_t, int32_t>> task_parts(const Batch &b, const Compiled &cg, bool split_segments) {
+// and pad_): topology chunks, or for the arc walk its segments in up to `most` parts.
+std::vector<std::pair<int32_t, int32_t>> task_parts(const Batch &b, const Compiled &cg, int64_t most) {
     std::vector<std::pair<int32_t, int32_t>> v;
     if (b.fmt != FMT_ARC) {
         for (int32_t ch : cg.chunks) v.push_back({ch, 0});
-    } else if (split_segments && cg.n_segments > 1) {
-        for (int i = 0; i < cg.n_segments; ++i) v.push_back({i, 1});
+    } else if (most > 1 && cg.n_segments > 1) {
+        const int64_t n = std::min<int64_t>(most, cg.n_segments);
+        for (int64_t i = 0; i < n; ++i) {
+            const int32_t first = (int32_t)(i * cg.n_segments / n);
+            v.push_back({first, (int32_t)((i + 1) * cg.n_segments / n) - first});
+        }
     } else {
         v.push_back({-1, 0});
     }
     return v;
 }
+
+// Parts the segments of an arc program may be cut into: as many as there are when the sample
+// blocks alone are fewer than 2048 workgroups, within `rows` task rows for `blocks` blocks.  A
+// program cut by its first pairs has hundreds of segments (three orbitals, order 3, float64: 84),
+// whose rows would take more than the scratch array of a no-alloc step.
+int64_t most_parts(int64_t total_blocks, int64_t blocks, int64_t rows) {
+    return total_blocks < 2048 ? std::max<int64_t>(1, rows / std::max<int64_t>(1, blocks)) : 1;
+}
+// Rows of a call that allocates what it needs: as many as the scratch array would hold.
+int64_t call_rows(const HostModel &m) { return (int64_t)kNoAllocScratchBytes / (8 * (int64_t)m.bt); }
 
 int build_step_batch_as(qiw_ctx *c, const qiw_run *run, bool bare, const std::vector<int> &oall, Batch &b, bool split,
                         bool arcs) {
@@ -1440,7 +1465,9 @@ int build_step_batch_as(qiw_ctx *c, const qiw_run *run, bool bare, const std::ve
     b.precision = run->precision;
     set_format(m, b, arcs);
     const int64_t total = n_groups * b.n_eval * std::max<int64_t>(run->N_samples, 1);
-    b.spt = samples_per_task(c, m, b.fmt, total);
+    const int64_t rows = step_rows(c, rq, (int64_t)oall.size(), n_groups + 1);
+    b.spt = samples_per_task(c, m, b.fmt, total, rows - n_groups * b.n_eval - 1);
+    const int64_t blocks = n_groups * b.n_eval * ((run->N_samples + b.spt - 1) / b.spt) + 1;
     for (int oi = 0; oi < n_o; ++oi) {
         int order = ord[oi];
         if (order > 0 && run->N_samples <= 0) continue;
@@ -1464,7 +1491,7 @@ int build_step_batch_as(qiw_ctx *c, const qiw_run *run, bool bare, const std::ve
             b.lds = std::max(b.lds, lds_slots(cg, m, b.fmt));
             int slot = (int)(std::find(oall.begin(), oall.end(), order) - oall.begin());
             int64_t N = order > 0 ? run->N_samples : 1;
-            const auto parts = task_parts(b, cg, split && total / b.spt < 2048);
+            const auto parts = task_parts(b, cg, split ? most_parts(total / b.spt, blocks, rows) : 1);
             const double flops = (double)N * sample_flops(cg);
             const int64_t leaves = N * cg.leaves_per_sample, evals = N * cg.n_top;
             push_sequences(b, std::move(cg), b.n_eval, [&](int gi) {
@@ -2473,8 +2500,8 @@ int run_inchworm(qiw_ctx *c, const qiw_run *run, bool do_bare, int first_w, int 
     double *ptab = (double *)dev(c, "ptab", (size_t)m.ntau * m.bt * 8, &rc);
     double *porders = (double *)dev(c, "porders", (size_t)n_slots * m.ntau * m.bt * 8, &rc);
     double *lam = (double *)dev(c, "lambda", (size_t)m.ntau * 8, &rc);
-    double *scratch = (double *)dev(c, "fin.scratch",
-                                    std::max(bare_b.r_first.size(), bold_b.r_first.size()) * 2 * m.bt * 8 + 8, &rc);
+    double *scratch = (double *)dev(
+        c, "fin.scratch", (rqmc ? std::max(bare_b.r_first.size(), bold_b.r_first.size()) * 2 * m.bt : 0) * 8 + 8, &rc);
     double *gsum = (double *)dev(c, "fin.gsum",
                                  (size_t)std::max(bare_b.groups.size(), bold_b.groups.size()) * m.bt * 8 + 8, &rc);
     int32_t *diag = (int32_t *)dev(c, "diag", (size_t)m.bt * 4, &rc);
@@ -2839,7 +2866,7 @@ int build_diff_batch_as(qiw_ctx *c, const qiw_run *run, Batch &b, bool arcs) {
         if (cg.g.n_wslots > 255 || m.ns > 255) return fail(c, QIW_E_LIMIT, "too many slots");
         b.lds = std::max(b.lds, lds_slots(cg, m, b.fmt));
         const int64_t N = order == 1 ? 1 : run->N_samples;
-        const auto parts = task_parts(b, cg, total / b.spt < 2048);
+        const auto parts = task_parts(b, cg, most_parts(total / b.spt, total / b.spt + n_groups * b.n_eval, call_rows(m)));
         const double flops = (double)N * sample_flops(cg);
         const int64_t leaves = N * cg.leaves_per_sample, evals = N * cg.n_top;
         push_sequences(b, std::move(cg), b.n_eval, [&](int gi) {
@@ -3290,7 +3317,8 @@ int run_correlator(qiw_ctx *c, const qiw_run *run, double *corr_out, double *cor
                         // tau_A = tau_B: only the leading order-0 group (src/inchworm.jl:1014-1024)
                         if (j == 0 && !(gi == 0 && p.first_is_order0)) continue;
                         int64_t N = b.groups[gi].g.order > 0 ? run->N_samples : 1;
-                        const auto parts = task_parts(b, b.groups[gi], total / b.spt < 2048);
+                        const auto parts = task_parts(
+                            b, b.groups[gi], most_parts(total / b.spt, total / b.spt + (int64_t)m.ntau * ng, call_rows(m)));
                         const int64_t nt64 = (N + b.spt - 1) / b.spt;
                         if (!tasks_fit(b, nt64 * (int64_t)parts.size()))
                             return fail(c, QIW_E_LIMIT, "more than 2^28 workgroups in one launch (lower N_samples)");
