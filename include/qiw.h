@@ -63,8 +63,10 @@ enum {
 /* ---- arithmetic of the chain products ------------------------------------------------ */
 enum {
     QIW_PREC_FP64 = 0,       /* all arithmetic in float64                                */
-    QIW_PREC_FP32 = 1        /* block chain products in float32; Sobol-to-simplex map,
-                                accumulation (compensated) and P bookkeeping in float64  */
+    QIW_PREC_FP32 = 1        /* block chain products in float32 (blocks up to 6, or up to 32
+                                with at most two hybridization functions, orders up to 4;
+                                float64 otherwise); Sobol-to-simplex map, accumulation
+                                (compensated) and P bookkeeping in float64               */
 };
 
 /* One block-sparse operator, the reference's SectorBlockMatrix

@@ -226,6 +226,12 @@ int program_format(const HostModel &m, int max_order, int precision) {
     return FMT_BLOCK;
 }
 
+// Chains are in float32 where a walk of the tries has them so; what runs on the LDS block walk
+// (orders beyond 4, wide blocks of more than two tables) is float64 in the arc walk too.
+int chain_precision(const HostModel &m, int max_order, int precision) {
+    return program_format(m, max_order, precision) == FMT_BLOCK ? QIW_PREC_FP64 : precision;
+}
+
 // Models run the arc walks wherever the states of their groups fit (a CU's LDS; the slots
 // and rows of the scalar walk; compile_group), and the assignment tries otherwise.
 int eval_format(const HostModel &m, int max_order, int precision) {
@@ -1462,7 +1468,7 @@ int build_step_batch_as(qiw_ctx *c, const qiw_run *run, bool bare, const std::ve
     b.scrambled = rq.scrambled;
     b.given = rq.given;
     b.max_order = max_order;
-    b.precision = run->precision;
+    b.precision = chain_precision(m, max_order, run->precision);
     set_format(m, b, arcs);
     const int64_t total = n_groups * b.n_eval * std::max<int64_t>(run->N_samples, 1);
     const int64_t rows = step_rows(c, rq, (int64_t)oall.size(), n_groups + 1);
@@ -2850,7 +2856,7 @@ int build_diff_batch_as(qiw_ctx *c, const qiw_run *run, Batch &b, bool arcs) {
     b.scrambled = rq.scrambled;
     b.given = rq.given;
     b.max_order = max_order;
-    b.precision = run->precision;
+    b.precision = chain_precision(m, max_order, run->precision);
     set_format(m, b, arcs);
     const int64_t total = n_groups * b.n_eval * std::max<int64_t>(run->N_samples, 1);
     b.spt = samples_per_task(c, m, b.fmt, total);
@@ -3166,7 +3172,7 @@ int build_corr_groups_as(qiw_ctx *c, const qiw_run *run, int ci, Batch &b, bool 
     int max_order = 0;
     for (int oi = 0; oi < run->n_orders; ++oi) max_order = std::max(max_order, (int)run->orders[oi]);
     b.max_order = max_order;
-    b.precision = run->precision;
+    b.precision = chain_precision(m, max_order, run->precision);
     set_format(m, b, arcs);
     b.n_eval = rq.n_eval();
     b.scrambled = rq.scrambled;

@@ -99,3 +99,18 @@ def test_model_without_pairs(orders):
     eg, ec = make(), make()
     assert rel(qiw.inchworm_step(eg, 2, orders, 4)[0], O.inchworm_step(ec, orders, 4, 2)[0]) < 1e-10
     assert rel(qiw.correlator_2p(eg, eg.grid, orders, 4)[0], O.correlator_2p(ec, orders, 4)[0]) < 1e-10
+
+
+def test_float32_requests_that_run_in_float64():
+    """Orders beyond 4, and blocks wider than 6 with more than two hybridization functions, have
+    float64 chains whatever is asked for."""
+    def many_tables(e):
+        for i, p in enumerate(e.pairs):
+            p.propagator = p.propagator * (1.0 + 0.1 * i)
+        return e
+    for make, orders, N in ((lambda: fermions(3, particles), range(0, 6), 2),
+                            (lambda: many_tables(fermions(5, particles)), range(0, 3), 4)):
+        v_g, p_g = qiw.inchworm_step(make(), 2, orders, N, precision=abi.QIW_PREC_FP32)
+        v_c, p_c = O.inchworm_step(make(), orders, N, 2)
+        assert rel(v_g, v_c) < 1e-10
+        assert np.abs(p_g - p_c).max() < 1e-10 * np.abs(v_c).max()
