@@ -261,9 +261,11 @@ inline bool arc_graph(const ArcModel &m, int kind, int order, int n_after, int s
 //            the arc values, the propagators and the states, 8.. offsets of the segments
 //   arc      head position | tail position << 8 | table << 16
 //   segment  0 s0 | m0 << 8 | lg << 16, 1 root sector dimension | stride << 8, 2 root operator
-//            block (offset, ARC_NONE: identity), 3 root propagator offset (ARC_NONE: none),
-//            4 root state offset, 5 parts of the closed state, 6 offset of their list,
-//            8.. of each wavefront the offsets of its records and of its joins
+//            block (offset, ARC_NONE: identity), 3 root propagator offset (ARC_NONE: none, the
+//            root is the closed state), 4 root state offset, 5 parts of the closed state, 6 offset
+//            of their list, 7 where the closed state begins: a float64 array, its element
+//            i at offset i of the states (so twice as far behind its beginning in bytes when
+//            the states are float32), 8.. of each wavefront the offsets of its records and of its joins
 // A wavefront reads two streams without a gap, in packets of ArcLayout::slots slots, so that
 // all a packet needs is read while the one before it is at work.  A slot is one or two steps
 // of joins, and what its flags say after them; the slots of a tile follow each other.
@@ -281,7 +283,8 @@ inline bool arc_graph(const ArcModel &m, int kind, int order, int n_after, int s
 constexpr uint32_t ARC_NONE = 0xFFFFFFFFu;
 // Flags of a slot: a barrier before it; the end of the segment; no joins; a second step; the
 // product of the sum of joins with the block; the tile's end: propagator, store.  Without a
-// product the next slot's joins continue the sum.
+// product the next slot's joins continue the sum (float64; a float32 program has a product in
+// every slot).
 enum : uint32_t { ARC_BARRIER = 1, ARC_END = 2, ARC_IDLE = 4, ARC_SECOND = 8, ARC_TIMES = 16, ARC_STORE = 32 };
 // LDS offsets: 16 times, the grid cells of 16 segments (24 bytes each), the arc values.
 constexpr size_t kArcCellsAt = 128, kArcValuesAt = 512;
@@ -292,7 +295,8 @@ constexpr int kArcReadAhead = 6 * 256;   // words a wavefront may read past its 
 // Slots of a packet of the walk whose lanes hold vectors of `rows` values.  The blocks of a packet
 // and of the next one stay in registers: with more slots what spills costs more than the longer
 // read-ahead saves (two-orbital step of orders 0:4, float32: 22.4, 21.1, 21.1 ms with four, three
-// and two slots; three-orbital step of orders 0:3, float32: 31.7 and 31.1 ms with two and one).
+// and two slots; three-orbital step of orders 0:3, float32: 31.7 and 31.1 ms with two and one; both
+// while the sums over diagrams were float32).
 constexpr int arc_slots(int rows) { return rows <= 8 ? 2 : 1; }
 
 struct ArcLayout {
@@ -313,8 +317,8 @@ inline int arc_stride(int m, int mmax) {
 }
 
 // LDS of a group in bytes: the times of the positions and cells of the segments, the arc
-// values, the closed states of all sectors, the propagators of n - 2 segments and one product,
-// then the states (and at the end, in their place, the last propagator).
+// values (float64), the closed states of all sectors, the propagators of n - 2 segments and one
+// product, then the states (and at the end, in their place, the last propagator).
 struct ArcLds {
     size_t fin, arcs, prop, states;
 };
@@ -322,7 +326,7 @@ inline ArcLds arc_lds(const ArcLayout &l, int n, int n_arcs) {
     auto up = [](size_t b) { return (b + 15) & ~(size_t)15; };
     ArcLds r;
     r.arcs = kArcValuesAt;
-    r.fin = r.arcs + up((size_t)(2 + 2 * n_arcs) * l.elem);
+    r.fin = r.arcs + up((size_t)(2 + 2 * n_arcs) * 8);
     r.prop = r.fin + up((size_t)l.bt * 8);
     r.states = r.prop + up((size_t)(n - 1) * l.bt * l.elem);
     return r;
@@ -521,7 +525,7 @@ struct ArcPacker {
 
     struct Plan {
         std::vector<Placed> placed;  // [stage]
-        size_t region = 0;           // elements of the state region, the closed state at its end
+        size_t region = 0;           // elements of the state region, the closed state (float64) at its end
         size_t closed = 0;           // elements of the closed state
         double cost = 0;             // slots on the longest wavefronts, over all column passes
     };
@@ -531,6 +535,7 @@ struct ArcPacker {
     // fit and the steps that they add to the next stage do not cost more.
     bool plan(const ArcGraph &g, int lg, size_t room, Plan &out) const {
         const int cg = 1 << lg, m0 = m.dims[g.s0], per = 64 >> lg;
+        const size_t wide = 8 / l.elem;  // elements a value of the closed state takes
         out = Plan{};
         size_t prev = ((size_t)arc_stride(m.dims[g.levels[0][0].sector], l.mmax) * cg + 3) & ~(size_t)3, reg = prev;
         out.closed = prev;
@@ -563,7 +568,7 @@ struct ArcPacker {
                     else
                         for (size_t i = 0; i < uses.size(); ++i)
                             cost += ((double)p.parts[i].size() - 1.0) * uses[i] / (2.0 * per * l.waves);
-                    const bool fits = last ? reg + p.size <= room : prev + p.size + spare <= room;
+                    const bool fits = last ? reg + wide * p.size <= room : prev + p.size + spare <= room;
                     if (fits && (best_cost < 0 || cost < best_cost)) {
                         best_cost = cost;
                         best = std::move(p);
@@ -582,7 +587,7 @@ struct ArcPacker {
             c += kStageCost + best.deal(l.waves, nullptr);
             out.placed.push_back(std::move(best));
         }
-        out.region = reg + out.closed;
+        out.region = reg + wide * out.closed;
         out.cost = c * ((m0 + cg - 1) / cg);
         return out.region <= room;
     }
@@ -631,7 +636,7 @@ struct ArcPacker {
         b[seg + 3] = n_st == 0 ? ARC_NONE : (uint32_t)(slot_after(1) * l.bt + l.bt_off[s1]);
         std::vector<std::vector<size_t>> src{{0}};
         std::vector<std::vector<Slot>> stream(l.waves);
-        const size_t levels = pn.region - pn.closed;  // elements of the alternating levels
+        const size_t levels = pn.region - 8 / l.elem * pn.closed;  // elements of the alternating levels
         for (size_t s = 0; s < n_st; ++s) {
             const ArcStage &st = g.stages[s];
             const bool last = s + 1 == n_st;
@@ -688,7 +693,7 @@ struct ArcPacker {
                             for (int i = 0; i < per; ++i)
                                 q.second.push_back(i < ns && e + 1 < words[i].size() ? words[i][e + 1] : any);
                         }
-                        if (e + 2 >= most) {
+                        if (e + 2 >= most || l.elem == 4) {
                             q.head[0] |= ARC_TIMES;
                             q.head[2] = blk;
                         }
@@ -745,6 +750,7 @@ struct ArcPacker {
         b[seg + 4] = n_st == 0 ? (uint32_t)levels : 0u;
         b[seg + 5] = (uint32_t)src[0].size();  // the parts of the closed state
         b[seg + 6] = (uint32_t)b.size();
+        b[seg + 7] = (uint32_t)levels;
         for (size_t off : src[0]) b.push_back((uint32_t)off);
         out.n_segments++;
         const double f = graph_flops(g);

@@ -34,9 +34,8 @@ template <typename V>
 __device__ __forceinline__ const V *state_at(const char *lds, uint32_t q, uint32_t coff) {
     return reinterpret_cast<const V *>(lds + ((q & 0xFFFFu) * 4u + coff));
 }
-template <typename V>
-__device__ __forceinline__ V value_at(const char *lds, uint32_t q) {  // bits 16-19 are clear
-    return *reinterpret_cast<const V *>(lds + kArcValuesAt + (q >> (sizeof(V) == 4 ? 18 : 17)));
+__device__ __forceinline__ double value_at(const char *lds, uint32_t q) {  // bits 16-19 are clear
+    return *reinterpret_cast<const double *>(lds + kArcValuesAt + (q >> 17));
 }
 
 // A lane's vector of up to MB values and its products with a block shared by the wavefront.
@@ -49,7 +48,14 @@ __device__ __forceinline__ V value_at(const char *lds, uint32_t q) {  // bits 16
 // rows of every lane, so a lane's vector stays where it is from product to product; the A
 // operand of one (4 rows, column) slice is broadcast to all 16 products from the four lanes
 // that hold it (CBSZ = 4, ABID = the slice).  A register therefore carries 16 slices of a
-// block, read with one 64-lane load.
+// block, read with one 64-lane load.  Only the products are in float32: the sums over joins and
+// over the operators of a tile are in float64 (as the sums over diagrams of the vector and
+// matrix-core walks are) and rounded once, where they enter a product, so a result is no less
+// accurate than the float64 sum of float32 chains.  What they cost against sums in float32: 21.1 ->
+// 23.4 ms in the two-orbital step of orders 0:4 at N = 2^11, 31.1 -> 39.7 in the three-orbital one of
+// orders 0:3 at N = 2^9 (conversions and float64 additions issue at half the rate of float32
+// ones, and the sums take registers).  Every slot ends with its product, so that no sum of
+// joins is kept from slot to slot (27.7 and 42.7 ms with it kept).
 //
 // double: multiply-adds whose block element is broadcast from its lane by the instruction
 // itself (v_fmac_f64 with DPP row_newbcast; every row of 16 lanes holds the same 16
@@ -59,24 +65,25 @@ template <typename V, int MB>
 struct Walk;
 
 // y += w s, s a state of C elements in LDS (a stride of arc_stride: 16-byte aligned from 4
-// floats on, but for 6)
-template <int C>
-__device__ __forceinline__ void join(float *y, float w, const float *s) {
+// floats on, but for 6).  The sums are in float64 for both types of state (FIRST: y = w s).
+template <int C, bool FIRST>
+__device__ __forceinline__ void join(double *y, double w, const float *s) {
+    auto add = [&](int k, float v) { y[k] = FIRST ? w * (double)v : fma(w, (double)v, y[k]); };
     if constexpr (C == 1) {
-        y[0] = fma(w, s[0], y[0]);
+        add(0, s[0]);
     } else if constexpr (C % 4 == 0) {
 #pragma unroll
         for (int k = 0; k < C; k += 4) {
             const f4 v = *(const f4 *)(s + k);
 #pragma unroll
-            for (int q = 0; q < 4; ++q) y[k + q] = fma(w, v[q], y[k + q]);
+            for (int q = 0; q < 4; ++q) add(k + q, v[q]);
         }
     } else {
 #pragma unroll
         for (int k = 0; k < C; k += 2) {
             const f2 v = *(const f2 *)(s + k);
-            y[k] = fma(w, v[0], y[k]);
-            y[k + 1] = fma(w, v[1], y[k + 1]);
+            add(k, v[0]);
+            add(k + 1, v[1]);
         }
     }
 }
@@ -91,6 +98,16 @@ __device__ __forceinline__ void join(double *y, double w, const double *s) {
             y[k] = fma(w, v[0], y[k]);
             y[k + 1] = fma(w, v[1], y[k + 1]);
         }
+    }
+}
+
+template <int C>
+__device__ __forceinline__ void store_sum(double *d, const double *v) {
+    if constexpr (C == 1) {
+        d[0] = v[0];
+    } else {
+#pragma unroll
+        for (int k = 0; k < C; k += 2) *(d2 *)(d + k) = d2{v[k], v[k + 1]};
     }
 }
 
@@ -110,9 +127,9 @@ template <int MB>
 struct Walk<float, MB> {
     static constexpr int NV = (MB / 4 * MB + 15) / 16;  // slice registers of a block
     static constexpr int SL = arc_slots(MB);
-    f4 acc[MB / 4];
-    float y[MB], A[SL][NV], next[SL][NV];  // blocks of the packet and of the next one
-    int rk[NV];                            // row | column << 8 of this lane's element of slice register v
+    double sum[MB];                 // of the products of a tile
+    float A[SL][NV], next[SL][NV];  // blocks of the packet and of the next one
+    int rk[NV];                     // row | column << 8 of this lane's element of slice register v
     int lane;
 
     __device__ __forceinline__ void init(int lane_) {
@@ -124,11 +141,13 @@ struct Walk<float, MB> {
 #pragma unroll
             for (int o = 0; o < SL; ++o) A[o][v] = next[o][v] = 0.f;
         }
-#pragma unroll
-        for (int k = 0; k < MB; ++k) y[k] = 0.f;
         clear();
     }
     __device__ __forceinline__ void clear() {
+#pragma unroll
+        for (int k = 0; k < MB; ++k) sum[k] = 0.0;
+    }
+    static __device__ __forceinline__ void zero(f4 (&acc)[MB / 4]) {
 #pragma unroll
         for (int g = 0; g < MB / 4; ++g) acc[g] = f4{0.f, 0.f, 0.f, 0.f};
     }
@@ -146,26 +165,46 @@ struct Walk<float, MB> {
 #pragma unroll
             for (int v = 0; v < NV; ++v) A[o][v] = next[o][v];
     }
-    // acc += O y, y = 0
+    // sum += O y, the product in float32
     template <int O, int C>
-    __device__ __forceinline__ void product(const float *, uint32_t, int str) {
-        rows<C, 1>(A[O], str);
+    __device__ __forceinline__ void product(const double (&y)[C], int str) {
+        float x[C];
 #pragma unroll
-        for (int k = 0; k < C; ++k) y[k] = 0.f;
+        for (int k = 0; k < C; ++k) x[k] = (float)y[k];
+        rows<C, 1>(A[O], x, str);
     }
     template <int C, int G>
-    __device__ __forceinline__ void rows(const float *a, int str) {
+    __device__ __forceinline__ void rows(const float *a, const float (&x)[C], int str) {
         if constexpr (G < MB / 4) {
             if (str > 4 * G) {
-                rows<C, G + 1>(a, str);
+                rows<C, G + 1>(a, x, str);
                 return;
             }
         }
-        mfma_block<MB, G>(acc, a, y, std::make_integer_sequence<int, C>{});
+        f4 acc[MB / 4];
+        zero(acc);
+        mfma_block<MB, G>(acc, a, x, std::make_integer_sequence<int, C>{});
+        // (downwards, so that the branches of all G end with the same addresses: upwards the
+        // compiler joins their last stores over a pointer, and the array goes to memory)
+#pragma unroll
+        for (int k = 4 * G - 1; k >= 0; --k) sum[k] += (double)acc[k / 4][k % 4];
     }
-    // acc = P acc, P column-major m x m in LDS, C its padded size
+    // d = P sum, P column-major m x m in LDS, C its padded size; sum = 0
     template <int C>
-    __device__ __forceinline__ void propagate(const float *pl, int m) {
+    __device__ __forceinline__ void finish(const float *pl, int m, float *d, bool lanes) {
+        f4 acc[MB / 4];
+        propagate<C>(acc, pl, m);
+        if (lanes) store<C>(acc, d);
+        clear();
+    }
+    // d = sum; sum = 0
+    template <int C>
+    __device__ __forceinline__ void close(double *d, bool lanes) {
+        if (lanes) store_sum<C>(d, sum);
+        clear();
+    }
+    template <int C>
+    __device__ __forceinline__ void propagate(f4 (&acc)[MB / 4], const float *pl, int m) const {
         constexpr int last = ((C + 3) / 4 - 1) * MB + C;
         float P[NV], x[C];
 #pragma unroll
@@ -177,12 +216,12 @@ struct Walk<float, MB> {
                 P[v] = in ? p : 0.f;
             }
 #pragma unroll
-        for (int k = 0; k < C; ++k) x[k] = acc[k / 4][k % 4];
-        clear();
+        for (int k = 0; k < C; ++k) x[k] = (float)sum[k];
+        zero(acc);
         mfma_block<MB, (C + 3) / 4>(acc, P, x, std::make_integer_sequence<int, C>{});
     }
     template <int C>
-    __device__ __forceinline__ void store(float *d) const {
+    static __device__ __forceinline__ void store(const f4 (&acc)[MB / 4], float *d) {
         if constexpr (C == 1) {
             d[0] = acc[0][0];
         } else if constexpr (C % 4 == 0) {
@@ -307,6 +346,16 @@ struct Walk<double, MB> {
         }
     }
     template <int C>
+    __device__ __forceinline__ void finish(const double *pl, int m, double *d, bool lanes) {
+        propagate<C>(pl, m);
+        close<C>(d, lanes);
+    }
+    template <int C>
+    __device__ __forceinline__ void close(double *d, bool lanes) {
+        if (lanes) store_sum<C>(d, acc);
+        clear();
+    }
+    template <int C>
     __device__ __forceinline__ void propagate(const double *pl, int m) {
         double x[C];
 #pragma unroll
@@ -331,15 +380,6 @@ struct Walk<double, MB> {
             else
                 rows<CH, 0>(P, x + K, C);
             prop_chunks<C, K + CH>(pl, x, m);
-        }
-    }
-    template <int C>
-    __device__ __forceinline__ void store(double *d) const {
-        if constexpr (C == 1) {
-            d[0] = acc[0];
-        } else {
-#pragma unroll
-            for (int k = 0; k < C; k += 2) *(d2 *)(d + k) = d2{acc[k], acc[k + 1]};
         }
     }
 };
@@ -376,6 +416,7 @@ template <typename V>
 struct SlotArgs {
     const char *lds;
     V *st;
+    double *closed;  // the closed state by the offsets of the states
     const V *pl, *ops;
     int col, lg;
 };
@@ -384,22 +425,27 @@ struct SlotArgs {
 template <typename V, int MB, int O, int C>
 __device__ __forceinline__ void slot_joins(Walk<V, MB> &w, const Joins<Walk<V, MB>::SL> &jw, const SlotArgs<V> &x,
                                            uint32_t fl, uint32_t blk, int str) {
-    const uint32_t coff = (uint32_t)(x.col * C) * (uint32_t)sizeof(V), q = jw.first[O];
-    join<C>(w.y, value_at<V>(x.lds, q), state_at<V>(x.lds, q, coff));
-    if (fl & ARC_SECOND) {
-        const uint32_t r = jw.second[O];
-        join<C>(w.y, value_at<V>(x.lds, r), state_at<V>(x.lds, r, coff));
+    const uint32_t coff = (uint32_t)(x.col * C) * (uint32_t)sizeof(V), q = jw.first[O], r = jw.second[O];
+    if constexpr (sizeof(V) == 4) {  // every slot ends with its product
+        double y[C];
+        join<C, true>(y, value_at(x.lds, q), state_at<V>(x.lds, q, coff));
+        if (fl & ARC_SECOND) join<C, false>(y, value_at(x.lds, r), state_at<V>(x.lds, r, coff));
+        w.template product<O, C>(y, str);
+    } else {
+        join<C>(w.y, value_at(x.lds, q), state_at<V>(x.lds, q, coff));
+        if (fl & ARC_SECOND) join<C>(w.y, value_at(x.lds, r), state_at<V>(x.lds, r, coff));
+        if (fl & ARC_TIMES) w.template product<O, C>(x.ops, blk, str);
     }
-    if (fl & ARC_TIMES) w.template product<O, C>(x.ops, blk, str);
 }
 // The end of a tile of stride C: propagator and store.
 template <typename V, int MB, int C>
 __device__ __forceinline__ void slot_store(Walk<V, MB> &w, const SlotArgs<V> &x, uint32_t prop, int rows, uint32_t to,
                                            int lanes) {
-    if (prop != kNone) w.template propagate<C>(x.pl + prop, rows);
     const int lane = threadIdx.x & 63;
-    if (lane < lanes) w.template store<C>(x.st + to + lane * C);
-    w.clear();
+    if (prop != kNone)
+        w.template finish<C>(x.pl + prop, rows, x.st + to + lane * C, lane < lanes);
+    else
+        w.template close<C>(x.closed + to + lane * C, lane < lanes);
 }
 
 // Slots O .. of a packet; false after the segment's last one.
@@ -476,9 +522,9 @@ __device__ __forceinline__ double prop_element(const double *ptab, int bt, const
 // blocks 1 4 6 4 1, float32), so a lane cannot own a sample; states of one sector share
 // operator and propagator, so both are wavefront-uniform.  Measured against the walk of the
 // assignment tries (one pass per diagram): two-orbital solve on 50 points, orders 0:2 at
-// N = 2^10, float64 451 -> 15.4 ms; two-orbital step, orders 0:4 at N = 2^11, float32 643 -> 21.2
+// N = 2^10, float64 451 -> 15.4 ms; two-orbital step, orders 0:4 at N = 2^11, float32 643 -> 23.4
 // ms; orders 0:3 at N = 2^12, float64 144 -> 8.8 ms; three-orbital step, orders 0:3 at N =
-// 2^9, float32 399 -> 31.4 ms; orders 0:2 at N = 2^8, float64 63.8 -> 3.2 ms.  Of these the
+// 2^9, float32 399 -> 39.7 ms; orders 0:2 at N = 2^8, float64 63.8 -> 3.2 ms.  Of these the
 // first form of the walk reached 29.9, 43.6, 18.2, 54.8 and 28.8 ms: what it lost were branches
 // on every row and column (one in five instructions), operator blocks and joins read when they
 // were wanted (a load's whole latency each), stages waiting for one wavefront with a tile of
@@ -491,10 +537,10 @@ __device__ __forceinline__ double prop_element(const double *ptab, int bt, const
 // state.  The closed states of all segments are multiplied by the last propagator in float64
 // at the end (segment by segment its gathers and the sums in memory were waited for each time).
 // Wavefronts per SIMD: float64 at MB = 8 takes three (168 registers, what spills is outside the
-// slots; two-orbital step 8.7 ms, 11.0 with two and 11.1 with four), float32 at MB = 20 three
-// (three-orbital step 31.7 ms; 33.7 with two, 39.2 with four).
+// slots; two-orbital step 8.7 ms, 11.0 with two and 11.1 with four), float32 at MB = 20 two
+// (three-orbital step 39.7 ms, 41.7 with three).
 template <typename V, int MB, int NT>
-__global__ __launch_bounds__(NT, (MB == 8 && sizeof(V) == 8) || NT == 768 ? 3 : 2) void k_eval_arcs_t(ArcArgs aa) {
+__global__ __launch_bounds__(NT, MB == 8 && sizeof(V) == 8 ? 3 : 2) void k_eval_arcs_t(ArcArgs aa) {
     extern __shared__ __attribute__((aligned(16))) char lds[];
     const EvalArgs &a = aa.e;
     const int tid = threadIdx.x, nt = blockDim.x;
@@ -507,7 +553,7 @@ __global__ __launch_bounds__(NT, (MB == 8 && sizeof(V) == 8) || NT == 768 ? 3 : 
     const uint32_t *words = reinterpret_cast<const uint32_t *>(a.prog + g.prog_off);
     double *tl = reinterpret_cast<double *>(lds);
     double *fin = reinterpret_cast<double *>(lds + b[4]);
-    V *dv = reinterpret_cast<V *>(lds + kArcValuesAt);
+    double *dv = reinterpret_cast<double *>(lds + kArcValuesAt);
     V *pl = reinterpret_cast<V *>(lds + b[6]);
     V *st = reinterpret_cast<V *>(lds + b[7]);
     const V *ops = reinterpret_cast<const V *>(aa.ops);
@@ -548,13 +594,13 @@ __global__ __launch_bounds__(NT, (MB == 8 && sizeof(V) == 8) || NT == 768 ? 3 : 
         const int na = (int)b[1];
         for (int i = tid; i < na + 1; i += nt) {
             if (i == na) {
-                dv[0] = (V)0;
-                dv[1] = (V)1;
+                dv[0] = 0.0;
+                dv[1] = 1.0;
                 continue;
             }
             const uint32_t arc = words[b[3] + i];
             const ArcPos ap = arc_pos(tl[(arc >> 8) & 255], tl[arc & 255], inv_h, a.n_tau);
-            const V v = (V)delta_value(a.dtab, (int)(arc >> 16), ap);
+            const double v = delta_value(a.dtab, (int)(arc >> 16), ap);
             dv[2 + 2 * i] = v;
             dv[3 + 2 * i] = -v;
         }
@@ -599,6 +645,7 @@ __global__ __launch_bounds__(NT, (MB == 8 && sizeof(V) == 8) || NT == 768 ? 3 : 
             const int m1 = (int)(h[1] & 255), str1 = (int)(h[1] >> 8);
             const uint32_t rblk = h[2], rprop = h[3];
             const int o = aa.bt_off[s0];
+            double *closed = reinterpret_cast<double *>(st + h[7]) - h[7];
             constexpr int SL = Walk<V, MB>::SL;
             const int col = lane & (cg - 1);
             const uint32_t jstep = 4u * (SL * (64u >> lg));  // bytes of a block of joins
@@ -615,7 +662,7 @@ __global__ __launch_bounds__(NT, (MB == 8 && sizeof(V) == 8) || NT == 768 ? 3 : 
                 w.init(lane);
                 fetch_ops<Walk<V, MB>, V, 0>(w, ops, hd);
                 w.rotate();
-                const SlotArgs<V> sa{lds, st, pl, ops, col, lg};
+                const SlotArgs<V> sa{lds, st, closed, pl, ops, col, lg};
                 // position 1: unit columns, or columns of the operator B, times the propagator
                 // that follows
                 for (int i = tid; i < cg * str1; i += nt) {
@@ -629,7 +676,10 @@ __global__ __launch_bounds__(NT, (MB == 8 && sizeof(V) == 8) || NT == 768 ? 3 : 
                         else
                             for (int j = 0; j < m1; ++j) v = fma(pl[rprop + k + j * m1], ops_cm[rblk + c * m1 + j], v);
                     }
-                    st[h[4] + i] = v;
+                    if (rprop == kNone)
+                        closed[h[4] + i] = (double)v;
+                    else
+                        st[h[4] + i] = v;
                 }
                 for (;;) {
                     // the next packet, and the records of the one after it
@@ -651,8 +701,8 @@ __global__ __launch_bounds__(NT, (MB == 8 && sizeof(V) == 8) || NT == 768 ? 3 : 
                 for (int i = wave; i < m0 * cg; i += nw) {
                     const int c = i / m0, r = i - c * m0;
                     if (c0 + c >= m0) break;
-                    double v = lane < np ? (double)st[part + c * stf + r] : 0.0;
-                    for (int p = lane + 64; p < np; p += 64) v += (double)st[words[h[6] + p] + c * stf + r];
+                    double v = lane < np ? closed[part + c * stf + r] : 0.0;
+                    for (int p = lane + 64; p < np; p += 64) v += closed[words[h[6] + p] + c * stf + r];
 #pragma unroll
                     for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d, 64);
                     if (lane == 0) fin[o + (c0 + c) * m0 + r] += v;
@@ -1130,12 +1180,12 @@ void launch_sarcs(hipStream_t st, const EvalArgs &a, int n_tasks, bool bare, siz
 // Vector length of the instantiation for blocks up to mb, and the most wavefronts a
 // workgroup of it can have (its registers).
 int qiw_arc_rows(int mb) { return mb <= 8 ? 8 : mb <= 20 ? 20 : 32; }
-int qiw_arc_waves(int mb, int fp32) { return !fp32 ? 8 : mb <= 8 ? 16 : mb <= 20 ? 12 : 8; }
+int qiw_arc_waves(int mb, int fp32) { return fp32 && mb <= 8 ? 16 : 8; }
 
 hipError_t qiw_launch_eval_arcs(hipStream_t st, const ArcArgs &a, int n_tasks, int mb, int fp32, int waves, size_t lds) {
     if (n_tasks < 1 || mb > 32 || a.e.n_tau < 2) return hipErrorInvalidValue;
     if (mb <= 8) return fp32 ? launch<float, 8, 1024>(st, a, n_tasks, waves, lds) : launch<double, 8, 512>(st, a, n_tasks, waves, lds);
-    if (mb <= 20) return fp32 ? launch<float, 20, 768>(st, a, n_tasks, waves, lds) : launch<double, 20, 512>(st, a, n_tasks, waves, lds);
+    if (mb <= 20) return fp32 ? launch<float, 20, 512>(st, a, n_tasks, waves, lds) : launch<double, 20, 512>(st, a, n_tasks, waves, lds);
     return fp32 ? launch<float, 32, 512>(st, a, n_tasks, waves, lds) : launch<double, 32, 512>(st, a, n_tasks, waves, lds);
 }
 

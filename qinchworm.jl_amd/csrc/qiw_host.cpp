@@ -674,15 +674,14 @@ ArcBlocks arc_blocks(const HostModel &m, int corr, int precision) {
 // 2^12; 11.1 in 40 KB, 11.2 with eight in 80 KB, 13.7 with two).  Wide blocks take all of a
 // CU's LDS: the more columns fit beside each other, the fewer lanes idle in the tiles of one
 // operator (three-orbital step of orders 0:2, N = 2^8, float64: 8.6 ms with two workgroups of
-// 80 KB per CU, which left seven in a hundred lanes at work, 3.1 with one of 160 KB; orders 0:3,
-// N = 2^9, float32: 35.3 and 33.5 ms; 31.2 with twelve wavefronts instead of eight).
+// 80 KB per CU, which left seven in a hundred lanes at work, 3.1 with one of 160 KB).
 struct ArcShape {
     int waves;
     size_t cap;
     int tiles;
 };
 constexpr ArcShape kArcShapes[] = {{2, 40 << 10, 2}, {4, 53 << 10, 12}, {8, 80 << 10, 32}, {16, 160 << 10, 1 << 30}};
-constexpr ArcShape kArcShapesWide[] = {{12, 160 << 10, 1 << 30}};  // mmax > 8; at most qiw_arc_waves
+constexpr ArcShape kArcShapesWide[] = {{8, 160 << 10, 1 << 30}};  // mmax > 8; at most qiw_arc_waves
 
 // Algorithmic real FLOPs of one sample of a compiled group: the scalar walk's multiply per
 // trie edge and leaf, or the block programs' chain products.

@@ -101,6 +101,28 @@ def test_model_without_pairs(orders):
     assert rel(qiw.correlator_2p(eg, eg.grid, orders, 4)[0], O.correlator_2p(ec, orders, 4)[0]) < 1e-10
 
 
+@pytest.mark.parametrize("n_modes", [3, 5])
+def test_float32_sums_keep_small_terms(n_modes):
+    """Float32 chain products, float64 sums (include/qiw.h): three pairs of the same operators whose
+    hybridization functions are the constants 1, 2^-30 and -1 have the same chains, so order 1
+    is 2^-30 times one of them to float32 accuracy.  Summed in float32 nothing of it is left.
+    Blocks up to 3 and up to 10."""
+    out = []
+    for lib in (qiw, O):
+        e = fermions(n_modes, particles)
+        fock = model.FockSpace(list(range(n_modes)))
+        one, small = (model.ScalarGF(np.full(e.grid.n_tau, -1j * v)) for v in (1.0, 2.0 ** -30))
+        pairs = [model.InteractionPair(fock.c_dag(0), fock.c(0), one),
+                 model.InteractionPair(fock.c_dag(0), fock.c(0), small),
+                 model.InteractionPair(-fock.c_dag(0), fock.c(0), one)]
+        e = model.Expansion(e.ed, e.grid, pairs)
+        out.append(qiw.inchworm_step(e, 2, range(0, 2), 8, precision=abi.QIW_PREC_FP32) if lib is qiw
+                   else O.inchworm_step(e, range(0, 2), 8, 2))
+    (v_g, p_g), (v_c, p_c) = out
+    assert rel(v_g, v_c) < 2e-6
+    assert rel(p_g[1], p_c[1]) < 2e-6
+
+
 def test_float32_requests_that_run_in_float64():
     """Orders beyond 4, and blocks wider than 6 with more than two hybridization functions, have
     float64 chains whatever is asked for."""
