@@ -365,14 +365,17 @@ int qiw_get_stats(qiw_ctx *ctx, qiw_stats *out);
 /* ---- work mapping and its tuner ----------------------------------------------------------
  * No counterpart in the reference (its work units are fixed by MPI rank ranges).  How
  * the evaluator's work is cut into workgroups:
- *   chunk_words       flat scalar programs (1x1 sectors): program words per topology chunk;
- *                     each (chunk, 64-sample block) is one workgroup.  0: 896
- *                     (640 for the self-energy batches of qiw_diff_inchworm).
- *   chunk_cost        vector programs (blocks <= 32): program words x replayed columns per
- *                     topology chunk.  0: 2^18.
- *   samples_per_task  walks that evaluate one sample per wavefront at a time (matrix-core
- *                     and LDS block walks): samples per workgroup, a power of 2 <= 64.
- *                     0: the largest that gives >= 4096 workgroups per launch.
+ *   chunk_words       models of 1x1 sectors: the scalar arc walk cuts a program by the pairs of
+ *                     its first two arcs until a segment holds at most this many words (0: as
+ *                     few segments as fit); the flat walk of models whose programs do not fit
+ *                     it has this many words per topology chunk, each (chunk, 64-sample
+ *                     block) one workgroup (0: 896; 640 for the self-energy batches of
+ *                     qiw_diff_inchworm).
+ *   samples_per_task  sector blocks: samples per workgroup of the arc walk and of the
+ *                     matrix-core and LDS block walks of models that do not fit it, a power
+ *                     of 2 <= 64.  0: the largest that gives >= 4096 workgroups per launch.
+ *   chunk_cost        vector and matrix-core walks of models that do not fit the arc walk:
+ *                     program words x replayed columns per topology chunk.  0: 2^18.
  * The settings change only how work is split and summed (results agree to rounding).
  * qiw_set_tuning fixes them; qiw_autotune times candidate settings on one bold step of
  * `run` (tau_w = grid[n_tau/2], the current propagator) and keeps the fastest.  Both last

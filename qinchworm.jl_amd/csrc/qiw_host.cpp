@@ -3707,9 +3707,15 @@ static int qiw_autotune_impl(qiw_ctx *c, const qiw_run *run, qiw_tuning *out) {
     if (run->N_samples <= 0 || run->n_orders == 0) return fail(c, QIW_E_ARG, "autotune needs sampled orders");
     (void)hipSetDevice(c->device);
     const HostModel &m = c->m;
-    int max_order = 0;
-    for (int i = 0; i < run->n_orders; ++i) max_order = std::max(max_order, (int)run->orders[i]);
-    const int fmt = eval_format(m, max_order, run->precision);
+    int fmt;  // of the walk that the step runs on, which need not be the one tried first
+    {
+        qiw_run r = *run;
+        r.n_orders_bare = 0;
+        r.rand_params = nullptr;
+        Batch b;
+        if ((rc = build_step_batch(c, &r, false, std::vector<int>(r.orders, r.orders + r.n_orders), b))) return rc;
+        fmt = b.fmt;
+    }
     std::vector<qiw_tuning> cand;
     if (fmt == FMT_SCALAR || fmt == FMT_SARC) {
         for (int w : {256, 384, 512, 640, 896, 1024, 2048}) cand.push_back(qiw_tuning{w, 0, 0, 0, 0, 0.0});
