@@ -374,6 +374,8 @@ int qiw_get_stats(qiw_ctx *ctx, qiw_stats *out);
  *   samples_per_task  sector blocks: samples per workgroup of the arc walk and of the
  *                     matrix-core and LDS block walks of models that do not fit it, a power
  *                     of 2 <= 64.  0: the largest that gives >= 4096 workgroups per launch.
+ *                     With blocks up to 6 a step takes more where its rows would not fit
+ *                     the array of qiw_inchworm_step_noalloc.
  *   chunk_cost        vector and matrix-core walks of models that do not fit the arc walk:
  *                     program words x replayed columns per topology chunk.  0: 2^18.
  * The settings change only how work is split and summed (results agree to rounding).

@@ -1351,7 +1351,11 @@ static int ystack_rows(const HostModel &m, int levels) {
 // many as there may be rows (rows: for its sample blocks; step_rows).
 int samples_per_task(const qiw_ctx *c, const HostModel &m, int fmt, int64_t total_samples, int64_t rows = INT64_MAX) {
     if (fmt == FMT_SCALAR || fmt == FMT_SARC || (fmt == FMT_VEC && m.mmax <= 6)) return QIW_WAVE;
-    if (c->tune.samples_per_task > 0) return c->tune.samples_per_task;
+    if (c->tune.samples_per_task > 0) {
+        int spt = c->tune.samples_per_task;  // blocks up to 6, whose vector walk takes 64: within the rows
+        while (fmt == FMT_ARC && m.mmax <= 6 && spt < QIW_WAVE && total_samples / spt > rows) spt *= 2;
+        return spt;
+    }
     int spt = QIW_WAVE;
     while (spt > 1 && total_samples / spt < 4096 && (fmt != FMT_ARC || 2 * total_samples / spt <= rows)) spt /= 2;
     return spt;

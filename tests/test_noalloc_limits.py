@@ -79,3 +79,13 @@ def test_rows_of_a_step_fit_the_scratch_array(stub, make, n_tau, order, N, preci
             if parts != [(-1, 0)]:  # (the whole program)
                 assert [p[0] for p in parts] == [0] + [p[0] + p[1] for p in parts[:-1]]
                 assert sum(p[1] for p in parts) == n_segments[g] and min(p[1] for p in parts) > 0
+
+
+def test_tuned_samples_per_workgroup_leave_the_rows_room(stub):  # noqa: F811
+    """A setting that the vector walk did not look at: it must not refuse a step that was taken."""
+    e, orders, N = many_sectors(8), range(0, 2), 2 ** 13
+    qiw.inchworm_step(e, 2, orders, 2, ctx=stub.ctx)
+    stub.ctx.check(stub.lib.qiw_set_tuning(stub.ctx.h, C.byref(abi.qiw_tuning(samples_per_task=1))))
+    qiw.inchworm_step(e, 2, orders, N, ctx=stub.ctx)
+    rc = noalloc(stub, e, orders, N, F64)
+    assert rc == abi.QIW_OK, stub.lib.qiw_last_error(stub.ctx.h).decode()
