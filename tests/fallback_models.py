@@ -6,7 +6,7 @@ from test_gpu_arcs import fermions, parity, particles
 
 
 def many_pairs(n_modes, key, n_pairs=128):
-    e = fermions(n_modes, key)
+    e = fermions(n_modes, key, n_tau=8)
     return model.Expansion(e.ed, e.grid, [e.pairs[i % len(e.pairs)] for i in range(n_pairs)], e.corr_operators)
 
 
