@@ -6,7 +6,7 @@ semi-elliptic baths, D = 2, V = 0.5, 8 pairs; beta = 10, n_tau = 200) solved by 
 at orders 0:4 with N = 2^16 unscrambled Sobol points per (order, n_pts_after) group, the
 chain products in float32 with float64 (compensated) sums and bookkeeping.  One bench step
 is one bold step (all 16 sampled groups and the exact order-0 group in one evaluator
-launch, then the on-device step bookkeeping); K steps are timed at tau_w = grid[100],
+launch per workgroup shape, then the on-device step bookkeeping); K steps are timed at tau_w = grid[100],
 grid[101], ..., and the time to solution of the whole inchworm! is extrapolated as the
 initial step plus 198 bold steps (every bold step does the same work).
 
@@ -45,7 +45,7 @@ def progress(msg):
 
 
 def measured_traffic(path):
-    """HBM bytes per evaluator launch from a committed rocprofv3 FETCH_SIZE/WRITE_SIZE
+    """HBM bytes per evaluator launch (mean of a step's launches) from a committed rocprofv3 FETCH_SIZE/WRITE_SIZE
     summary (copy-calibrated), or None."""
     try:
         for line in open(path):
@@ -571,7 +571,8 @@ def two_orbital_headline(log2n, steps, warmup, sync, with_cpu, cpu_log2n=8, err_
                         "frac": achieved / FP32_PEAK_TFLOPS,
                         "frac_of_unpacked_fp32_valu": achieved / FP32_VALU_UNPACKED_TFLOPS,
                         "traffic": measured_traffic(C2_TRAFFIC_PROFILE), "kernel": "k_eval_arcs_t<float,8,1024>",
-                        "avg_launch_ms": avg_launch_ms, "flops_per_launch": acc["flops"] / max(acc["launches"], 1),
+                        "avg_launch_ms": avg_launch_ms, "launches_per_step": acc["launches"] / steps,
+                        "flops_per_launch": acc["flops"] / max(acc["launches"], 1),
                         "note": "float32 open-arc products on v_mfma_f32_4x4x1 (one lane per column of a state), "
                                 "bound by issue and the stages' barriers; the FLOPs are those of the merged "
                                 "partial diagrams"}}

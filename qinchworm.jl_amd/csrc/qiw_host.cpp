@@ -847,6 +847,9 @@ inline bool tasks_fit(Batch &b, int64_t more) {
     return !b.overflow;
 }
 
+// Evaluator launches of a batch: one per workgroup shape for the arc walks.
+int eval_launches(const Batch &b) { return std::max<int>(1, (int)b.launches.size()); }
+
 // Most task rows of a group (the reduction's block is sized by it).
 int most_rows(const Batch &b) { return b.g_count.empty() ? 0 : *std::max_element(b.g_count.begin(), b.g_count.end()); }
 
@@ -2606,7 +2609,7 @@ int run_inchworm(qiw_ctx *c, const qiw_run *run, bool do_bare, int first_w, int 
         fa.n_known = 0;
         fa.nuse_out = nuse_bare;
         HIPCHK(c, finalize(bare_b, bare_d, -1));
-        ++launches;
+        launches += eval_launches(bare_b);
         if (m.ppgf_kind == QIW_GF_INC_SPLINE) n_known = 2;
         c->stats.flops += bare_b.flops_per_launch;
         c->stats.leaves += bare_b.leaves_per_launch;
@@ -2717,7 +2720,7 @@ int run_inchworm(qiw_ctx *c, const qiw_run *run, bool do_bare, int first_w, int 
             n_known = n_known_start;
             for (int jw = first_w; jw <= last_w; ++jw) {  // host-side state of the loop
                 step_args(jw);
-                ++launches;
+                launches += eval_launches(bold_b);
                 c->stats.flops += bold_b.flops_per_launch;
                 c->stats.leaves += bold_b.leaves_per_launch;
                 c->stats.diagram_evals += bold_b.diagram_evals_per_launch;
@@ -2739,7 +2742,7 @@ int run_inchworm(qiw_ctx *c, const qiw_run *run, bool do_bare, int first_w, int 
             fa.n_known = (m.ppgf_kind == QIW_GF_INC_SPLINE) ? n_known : m.ntau;
             fa.normalize = normalize ? 1 : 0;
             HIPCHK(c, finalize(bold_b, bold_d, next_of(jw)));
-            ++launches;
+            launches += eval_launches(bold_b);
             c->stats.flops += bold_b.flops_per_launch;
             c->stats.leaves += bold_b.leaves_per_launch;
             c->stats.diagram_evals += bold_b.diagram_evals_per_launch;
@@ -3052,7 +3055,7 @@ int run_diff(qiw_ctx *c, const qiw_run *run, double *S_out, double *S_std_out) {
                                              2 * b.max_order));
         if ((rc = launch_eval(c, a, b))) return rc;
         HIPCHK(c, qiw_launch_finalize_diff(c->stream, fa, rqmc ? 1 : 0));
-        ++launches;
+        launches += eval_launches(b);
         c->stats.flops += b.flops_per_launch;
         c->stats.leaves += b.leaves_per_launch;
         c->stats.diagram_evals += b.diagram_evals_per_launch;
@@ -3446,7 +3449,7 @@ int run_correlator(qiw_ctx *c, const qiw_run *run, double *corr_out, double *cor
         HIPCHK(c, hipMemcpyAsync(po.out.data(), dout, po.out.size() * 8, hipMemcpyDeviceToHost, c->stream));
         if (dout_std)
             HIPCHK(c, hipMemcpyAsync(po.out_std.data(), dout_std, m.ntau * 8, hipMemcpyDeviceToHost, c->stream));
-        c->stats.n_kernel_launches += 1;
+        c->stats.n_kernel_launches += eval_launches(b);
         c->stats.flops += b.flops_per_launch;
         c->stats.leaves += b.leaves_per_launch;
         c->stats.diagram_evals += b.diagram_evals_per_launch;
