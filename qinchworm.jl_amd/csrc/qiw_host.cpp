@@ -674,7 +674,10 @@ ArcBlocks arc_blocks(const HostModel &m, int corr, int precision) {
 // 2^12; 11.1 in 40 KB, 11.2 with eight in 80 KB, 13.7 with two).  Wide blocks take all of a
 // CU's LDS: the more columns fit beside each other, the fewer lanes idle in the tiles of one
 // operator (three-orbital step of orders 0:2, N = 2^8, float64: 8.6 ms with two workgroups of
-// 80 KB per CU, which left seven in a hundred lanes at work, 3.1 with one of 160 KB).
+// 80 KB per CU, which left seven in a hundred lanes at work, 3.1 with one of 160 KB).  So do the
+// programs that are cut by their first pairs, whose states did not fit otherwise: two-orbital steps
+// in float64, orders 0:4, 5.1 -> 3.5, 41.8 -> 26.9 and 331 -> 213 ms at N = 2^5, 2^9 and 2^12, orders
+// 0:5 at N = 2^4 118 -> 73 ms, against the first shape that the cut states fit (80 KB).
 struct ArcShape {
     int waves;
     size_t cap;
@@ -741,7 +744,7 @@ int compile_arcs(const HostModel &m, int kind, int order, int n_after, int corr,
     for (int n_fixed = 0; n_fixed <= order && rc == 2; ++n_fixed)
         for (int i = 0; i < n_shapes; ++i) {
             const ArcShape &sh = shapes[i];
-            if (n_fixed == 0 && (widest + 63) / 64 > (size_t)sh.tiles) continue;
+            if (n_fixed == 0 ? (widest + 63) / 64 > (size_t)sh.tiles : i + 1 < n_shapes) continue;
             l.waves = std::min(sh.waves, max_waves);
             l.cap = sh.cap;
             rc = arc_compile(am, l, ob, kind, order, n_after, n_fixed, pg);
