@@ -1451,6 +1451,62 @@ std::vector<std::pair<int32_t, int32_t>> task_parts(const Batch &b, const Compil
     return v;
 }
 
+// Estimated seconds of a batch's evaluator at N samples per sampled group and `rows` tau rows, for
+// the choice between the arc walk and the walks of the assignment tries.  The arc walk takes a
+// workgroup per sample, whose set-up (times, arc values, every sector's propagators) and barriers
+// it pays for however little there is to sum; the vector walk takes a sample per lane and only
+// the blocks of its chains.  So at order 1, and for blocks of two or three at order 2, the vector
+// walk is faster once its launch, as long as one wavefront's walk of the longest program, is
+// full; likewise the LDS block walk for wide blocks in float64.  Measured (arc walk, trie walk; ms):
+//   two orbitals, order 1, N = 2^12 .283 .681, 2^15 1.52 .765, 2^18 11.4 2.68; orders 0:2, N = 2^18
+//   63.8 131 (float32 43.2 47.7); orders 0:3, N = 2^12 8.2 126;
+//   blocks up to 3, order 1, N = 2^18 5.53 .540; orders 0:2, N = 2^12 .582 .896, 2^18 27.7 10.1; orders
+//   0:3, N = 2^12 1.75 9.6;
+//   128 blocks of 4, order 1, N = 2^9 1.58 5.25, 2^12 10.4 5.15, 2^15 76.8 6.34;
+//   blocks up to 10 in float64, order 1, N = 2^15 7.37 2.80; orders 0:2, N = 2^12 6.14 12.4.
+// The rates are fits to these that stay within a factor of two.
+int64_t group_samples(const QiwGroup &g, int64_t N) {
+    return g.order == 0 || (g.kind == QIW_G_SIGMA && g.order == 1) ? 1 : std::max<int64_t>(N, 1);
+}
+double arc_seconds(const HostModel &m, const Batch &b, int64_t N, int64_t rows) {
+    double t = 8e-5;
+    for (const Compiled &cg : b.groups) {
+        // workgroups at a time; a barrier per stage and segment; a lookup per propagator element
+        const double wgs = 256.0 * std::max<size_t>(1, std::min<size_t>(12 / cg.shape, (160 << 10) / std::max<size_t>(cg.lds_bytes, 1)));
+        const double sample = (cg.n_segments * (2.0 * cg.g.order + 1) + 4) * 1.6e-6 / wgs + m.bt * (cg.g.n_nodes - 1.0) * 5e-11;
+        t += (double)rows * group_samples(cg.g, N) * sample * (b.precision == QIW_PREC_FP32 ? 0.7 : 1.0);
+    }
+    return t;
+}
+// least: of an arc batch, what the tries would take at least (4.5 words per diagram, the FLOPs of
+// the merged diagrams).
+double trie_seconds(const HostModel &m, const Batch &b, bool least, int64_t N, int64_t rows) {
+    double longest = 0, t = 0;
+    const bool vec = m.mmax <= 6;
+    for (const Compiled &cg : b.groups) {
+        const double words = least ? 4.5 * cg.leaves_per_sample : (double)cg.prog.size();
+        longest = std::max(longest, words);
+        t += (double)rows * group_samples(cg.g, N) * (vec ? words * m.mmax * 2e-11 : sample_flops(cg) / 1.3e12);
+    }
+    const bool fp32 = b.precision == QIW_PREC_FP32;
+    return vec ? 1e-4 + std::max(longest * m.mmax * (fp32 ? 4.8e-7 : 8e-7), t * (fp32 ? 0.5 : 1.0))
+               : 5e-5 + std::max(longest * m.mmax * 1e-7, t);
+}
+// Whether the batch `arcs` would be faster on the walks of the tries (tries: builds the batch there).
+template <class Build>
+int prefer_tries(const HostModel &m, Batch &arcs, int64_t N, int64_t rows, Build build) {
+    if (arcs.fmt != FMT_ARC || (m.mmax > 6 && arcs.precision == QIW_PREC_FP32)) return 0;
+    if (program_format(m, arcs.max_order, arcs.precision) == FMT_BLOCK && m.mmax <= 6) return 0;
+    const double t = 0.8 * arc_seconds(m, arcs, N, rows);
+    if (trie_seconds(m, arcs, true, N, rows) >= t) return 0;
+    Batch tries;
+    const int rc = build(tries);
+    if (rc) return rc;
+    const bool fits = arcs.groups.empty() || tries.fmt != FMT_BLOCK || (size_t)tries.lds * 8 <= 160 * 1024;
+    if (fits && trie_seconds(m, tries, false, N, rows) < t) arcs = std::move(tries);
+    return 0;
+}
+
 // Parts the segments of an arc program may be cut into: as many as there are when the sample
 // blocks alone are fewer than 2048 workgroups, within `rows` task rows for `blocks` blocks.  A
 // program cut by its first pairs has hundreds of segments (three orbitals, order 3, float64: 84),
@@ -1534,6 +1590,9 @@ int build_step_batch(qiw_ctx *c, const qiw_run *run, bool bare, const std::vecto
                      bool split = true) {
     b = Batch{};
     const int rc = build_step_batch_as(c, run, bare, oall, b, split, true);
+    if (rc == 0)
+        return prefer_tries(c->m, b, run->N_samples, 1,
+                            [&](Batch &t) { return build_step_batch_as(c, run, bare, oall, t, split, false); });
     if (rc != kArcNoFit) return rc;
     b = Batch{};
     return build_step_batch_as(c, run, bare, oall, b, split, false);
@@ -2906,6 +2965,8 @@ int build_diff_batch_as(qiw_ctx *c, const qiw_run *run, Batch &b, bool arcs) {
 int build_diff_batch(qiw_ctx *c, const qiw_run *run, Batch &b) {
     b = Batch{};
     const int rc = build_diff_batch_as(c, run, b, true);
+    if (rc == 0)
+        return prefer_tries(c->m, b, run->N_samples, 1, [&](Batch &t) { return build_diff_batch_as(c, run, t, false); });
     if (rc != kArcNoFit) return rc;
     b = Batch{};
     return build_diff_batch_as(c, run, b, false);
@@ -3210,6 +3271,9 @@ int build_corr_groups_as(qiw_ctx *c, const qiw_run *run, int ci, Batch &b, bool 
 int build_corr_groups(qiw_ctx *c, const qiw_run *run, int ci, Batch &b, bool *first_is_order0) {
     b = Batch{};
     const int rc = build_corr_groups_as(c, run, ci, b, first_is_order0, true);
+    if (rc == 0)
+        return prefer_tries(c->m, b, run->N_samples, c->m.ntau,
+                            [&](Batch &t) { return build_corr_groups_as(c, run, ci, t, first_is_order0, false); });
     if (rc != kArcNoFit) return rc;
     b = Batch{};
     return build_corr_groups_as(c, run, ci, b, first_is_order0, false);
