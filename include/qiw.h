@@ -392,10 +392,11 @@ typedef struct {
 } qiw_tuning;
 int qiw_set_tuning(qiw_ctx *ctx, const qiw_tuning *t);
 /* qiw_set_graphs: no counterpart in the reference.  With on = 1 (the default) the
- * bold-step loop of qiw_inchworm / qiw_inchworm_step on the flat scalar walk (all sectors
- * 1x1, no learned warp) is captured once in a hipGraph and replayed while every launch
- * argument is the same, so a repeated run issues one graph launch instead of two kernel
- * launches per step; results are identical.  on = 0 launches every kernel from the host. */
+ * bold-step loop of qiw_inchworm, of five steps or more and without the learned warp or
+ * caller-drawn sequences, is captured once in a hipGraph and replayed while every launch is the
+ * same, so a repeated run issues one graph launch instead of two or more kernel launches per step;
+ * results are identical.  The LDS block walk stays outside.  on = 0 launches every kernel from
+ * the host. */
 int qiw_set_graphs(qiw_ctx *ctx, int32_t on);
 int qiw_get_tuning(qiw_ctx *ctx, qiw_tuning *out);
 int qiw_autotune(qiw_ctx *ctx, const qiw_run *run, qiw_tuning *out);

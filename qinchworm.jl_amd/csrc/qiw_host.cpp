@@ -1930,12 +1930,11 @@ int stage_arcs(qiw_ctx *c, int precision, ArcArgs *aa) {
     return 0;
 }
 
-// Launches the evaluator matching the model's sector structure.  The vector and matrix-core
-// walks stage their operator tables once per model on their first launch (synchronous
-// copies), so a launch can be captured into a hipGraph only after that
-// (c->vec_staged / c->mfma_staged).  record: append the bytes of every launch (arguments,
-// workgroups, shape, LDS) instead of launching; two calls of one format and precision with the
-// same bytes launch the same.
+// Launches the evaluator matching the model's sector structure.  The arc walk of sector blocks and
+// the vector and matrix-core walks stage their tables on the first call after qiw_set_model
+// (synchronous copies), so a call with `record` comes before a capture.  record: append the bytes of
+// every launch (arguments, workgroups, shape, LDS) instead of launching; two calls of one format
+// and precision with the same bytes launch the same.
 int launch_eval(qiw_ctx *c, const EvalArgs &a, const Batch &batch, std::string *record = nullptr) {
     const HostModel &m = c->m;
     auto put = [&](const auto &args, int count, int shape, size_t lds) {
@@ -2698,14 +2697,12 @@ int run_inchworm(qiw_ctx *c, const qiw_run *run, bool do_bare, int first_w, int 
             fa.n_known = (m.ppgf_kind == QIW_GF_INC_SPLINE) ? n_known : m.ntau;
             fa.normalize = normalize ? 1 : 0;
         };
-        // without the warp the whole loop is one hipGraph, replayed while the launch arguments
-        // are unchanged: the flat scalar walk, the arc walk, and the vector and matrix-core walks once their
-        // tables are staged (from the second call on); the LDS block walk copies host data per
-        // launch and stays eager
-        const bool staged = bold_b.fmt == FMT_SCALAR || bold_b.fmt == FMT_ARC || bold_b.fmt == FMT_SARC ||
-                            (bold_b.fmt == FMT_VEC && (m.mmax > 6 ? c->mfma_staged : c->vec_staged));
+        // without the warp the whole loop is one hipGraph, replayed while its launches are the same;
+        // the walks with tables on the device stage them before the capture (launch_eval, for the
+        // key), but the LDS block walk copies host data per launch and stays eager
         // a few steps launch faster one by one than a graph is replayed, or captured for new times
-        bool graph = c->graphs && staged && !warped && !c->no_alloc && !rq.given && last_w - first_w >= kGraphSteps;
+        bool graph = c->graphs && bold_b.fmt != FMT_BLOCK && !warped && !c->no_alloc && !rq.given &&
+                     last_w - first_w >= kGraphSteps;
         const int n_known_start = n_known;
         if (graph) {
             if (!c->graph) c->graph = new StepGraph;
@@ -2713,7 +2710,7 @@ int run_inchworm(qiw_ctx *c, const qiw_run *run, bool do_bare, int first_w, int 
             const int n_known0 = n_known;
             std::string key;
             auto put = [&](const void *p, size_t n) { key.append((const char *)p, n); };
-            if ((rc = launch_eval(c, a, bold_b, &key))) return rc;  // (stages the arc walk's tables, before a capture)
+            if ((rc = launch_eval(c, a, bold_b, &key))) return rc;
             put(&bold_b.max_order, 4);
             put(&rq.seed, 8);
             const uint32_t *sm = sobm;

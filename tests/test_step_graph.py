@@ -77,3 +77,11 @@ def test_replay_of_an_unchanged_solve(stub):  # noqa: F811
         again, recaptured = solve(stub, make(n), orders, 2 ** 5, prec)
         assert captured == 1 and recaptured == 0
         assert [x[:5] for x in first] == [x[:5] for x in again]
+
+
+def test_first_solve_on_the_vector_walk_is_captured(stub):  # noqa: F811
+    """Its tables are staged before the capture also where the bare step has another walk."""
+    e = two_orbital(8)
+    launched, captured = solve(stub, e, range(0, 2), 2 ** 17, F64)
+    bold = [x for x in launched if "k_eval_vec_t" in x.name]
+    assert captured == 1 and len(bold) >= e.grid.n_tau - 2
