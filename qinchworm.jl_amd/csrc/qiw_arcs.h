@@ -1037,9 +1037,10 @@ struct ScalarPacker {
 
 // Compiles a scalar group.  models: one, whose results are its initial sectors, or several
 // that differ in A and B alone (and their values), with one result each, the sum over the
-// initial sectors (the trace): what they share is computed once.  max_words: cut the graphs by the pairs of their first arcs until
-// a segment holds at most this many words (0: as few segments as fit).  Returns 0, 1 when a diagram ends outside its initial sector, or
-// 2 when the program does not fit the slots, the rows or the tables of the walk.
+// initial sectors (the trace): what they share is computed once.  max_words: cut the graphs by the
+// pairs of their first arcs until a segment holds at most this many words (0: as few segments as
+// fit).  Returns 0, 1 when a diagram ends outside its initial sector, or 2 when the program does
+// not fit the slots, the rows or the tables of the walk.
 inline int arc_compile_scalar(const std::vector<ArcModel> &models, const std::vector<ArcValues> &values, int kind, int order,
                               int n_after, int max_words, ScalarProgram &out) {
     out = ScalarProgram{};

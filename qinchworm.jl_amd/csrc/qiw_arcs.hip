@@ -730,7 +730,6 @@ hipError_t launch(hipStream_t st, const ArcArgs &a, int n_tasks, int waves, size
     return hipGetLastError();
 }
 
-
 // ---------------------------------------------------------------------------------------
 // The scalar arc walk (all sectors 1x1; programs of ScalarPacker, qiw_arcs.h)
 //
@@ -1014,51 +1013,51 @@ __global__ __launch_bounds__(256, SLOTS > kScalarFew ? 3 : DLR ? 4 : 6) void k_e
             tab[i * 64 + lane] = __hiloint2double((int)c[2 * i + 1], (int)c[2 * i]);
     }
     for (int c0 = 0; c0 < na; c0 += 64) {  // records of up to 64 arcs
-    const int nc = min(64, na - c0);
-    if (c0 > 0) arc_records(c0);
-    for (int i0 = wave; i0 < nc; i0 += 4 * UA) {
-        ArcPos ap[UA];
+        const int nc = min(64, na - c0);
+        if (c0 > 0) arc_records(c0);
+        for (int i0 = wave; i0 < nc; i0 += 4 * UA) {
+            ArcPos ap[UA];
 #pragma unroll
-        for (int q = 0; q < UA; ++q) {  // past the last arc: the last one again
-            const uint32_t ends = rlane(rec[0], min(i0 + 4 * q, nc - 1));
-            if constexpr (GRID)
-                ap[q].c = cell((int)(ends >> 8), (int)(ends & 255));
-            else
-                ap[q] = arc_pos(tl[(ends >> 8) * 64 + lane], tl[(ends & 255) * 64 + lane], inv_h, a.n_tau);
-        }
-        for (int tb = 0; tb < a.dtab.n_tables; tb += 2) {
-            double c[UA][2][GRID ? 3 : 4];
-            uint32_t rows[UA];
-#pragma unroll
-            for (int q = 0; q < UA; ++q) {
-                rows[q] = i0 + 4 * q < nc ? rlane(tb ? rec[2] : rec[1], i0 + 4 * q) : 0xFFFFFFFFu;
-#pragma unroll
-                for (int t = 0; t < 2; ++t) {
-                    if (((rows[q] >> (16 * t)) & 0xFFFFu) == 0xFFFFu) continue;
-                    if (DLR && ((a.dtab.dlr_mask >> (tb + t)) & 1)) continue;
-                    const double *co = a.dtab.coef + (int64_t)(tb + t) * (a.n_tau - 1) * 4;
-                    const uint32_t at = 4u * (uint32_t)(GRID || ((a.dtab.grid_mask >> (tb + t)) & 1) ? ap[q].c.d : ap[q].j);
-#pragma unroll
-                    for (int k = 0; k < (GRID ? 3 : 4); ++k) c[q][t][k] = co[at + k];
-                }
+            for (int q = 0; q < UA; ++q) {  // past the last arc: the last one again
+                const uint32_t ends = rlane(rec[0], min(i0 + 4 * q, nc - 1));
+                if constexpr (GRID)
+                    ap[q].c = cell((int)(ends >> 8), (int)(ends & 255));
+                else
+                    ap[q] = arc_pos(tl[(ends >> 8) * 64 + lane], tl[(ends & 255) * 64 + lane], inv_h, a.n_tau);
             }
+            for (int tb = 0; tb < a.dtab.n_tables; tb += 2) {
+                double c[UA][2][GRID ? 3 : 4];
+                uint32_t rows[UA];
 #pragma unroll
-            for (int q = 0; q < UA; ++q)
+                for (int q = 0; q < UA; ++q) {
+                    rows[q] = i0 + 4 * q < nc ? rlane(tb ? rec[2] : rec[1], i0 + 4 * q) : 0xFFFFFFFFu;
 #pragma unroll
-                for (int t = 0; t < 2; ++t) {
-                    const uint32_t r = (rows[q] >> (16 * t)) & 0xFFFFu;
-                    if (r == 0xFFFFu) continue;
-                    double v;
-                    if (DLR && ((a.dtab.dlr_mask >> (tb + t)) & 1))
-                        v = delta_value<DLR>(a.dtab, tb + t, ap[q]);
-                    else if (GRID || ((a.dtab.grid_mask >> (tb + t)) & 1))
-                        v = c[q][t][0] + ap[q].c.wp * c[q][t][1] - ap[q].c.wm * c[q][t][2];
-                    else
-                        v = c[q][t][0] + ap[q].u * (c[q][t][1] + ap[q].u * (c[q][t][2] + ap[q].u * c[q][t][GRID ? 2 : 3]));
-                    tab[r * 64 + lane] = v;
+                    for (int t = 0; t < 2; ++t) {
+                        if (((rows[q] >> (16 * t)) & 0xFFFFu) == 0xFFFFu) continue;
+                        if (DLR && ((a.dtab.dlr_mask >> (tb + t)) & 1)) continue;
+                        const double *co = a.dtab.coef + (int64_t)(tb + t) * (a.n_tau - 1) * 4;
+                        const uint32_t at = 4u * (uint32_t)(GRID || ((a.dtab.grid_mask >> (tb + t)) & 1) ? ap[q].c.d : ap[q].j);
+#pragma unroll
+                        for (int k = 0; k < (GRID ? 3 : 4); ++k) c[q][t][k] = co[at + k];
+                    }
                 }
+#pragma unroll
+                for (int q = 0; q < UA; ++q)
+#pragma unroll
+                    for (int t = 0; t < 2; ++t) {
+                        const uint32_t r = (rows[q] >> (16 * t)) & 0xFFFFu;
+                        if (r == 0xFFFFu) continue;
+                        double v;
+                        if (DLR && ((a.dtab.dlr_mask >> (tb + t)) & 1))
+                            v = delta_value<DLR>(a.dtab, tb + t, ap[q]);
+                        else if (GRID || ((a.dtab.grid_mask >> (tb + t)) & 1))
+                            v = c[q][t][0] + ap[q].c.wp * c[q][t][1] - ap[q].c.wm * c[q][t][2];
+                        else
+                            v = c[q][t][0] + ap[q].u * (c[q][t][1] + ap[q].u * (c[q][t][2] + ap[q].u * c[q][t][GRID ? 2 : 3]));
+                        tab[r * 64 + lane] = v;
+                    }
+            }
         }
-    }
     }
     if (bare) {
         for (int i = wave; i < np; i += 4) {
@@ -1165,7 +1164,8 @@ hipError_t qiw_launch_eval_arcs(hipStream_t st, const ArcArgs &a, int n_tasks, i
     return fp32 ? launch<float, 32, 512>(st, a, n_tasks, waves, lds) : launch<double, 32, 512>(st, a, n_tasks, waves, lds);
 }
 
-// slots: register slots of the programs; bare: its groups are bare ones; lds: scalar_lds_rows of the largest group, 512 bytes each.
+// slots: register slots of the programs; bare: its groups are bare ones; lds: scalar_lds_rows of the
+// largest group, 512 bytes each.
 hipError_t qiw_launch_eval_sarcs(hipStream_t st, const EvalArgs &a, int n_tasks, int slots, bool bare, size_t lds) {
     if (n_tasks < 1 || a.ns > 8 || a.n_out < 1 || a.n_out > 8 || a.dtab.n_tables > 4 || slots > kScalarSlots) return hipErrorInvalidValue;
     if (slots <= kScalarFew)
