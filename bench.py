@@ -606,11 +606,11 @@ def main():
     ap.add_argument("--no-c3", action="store_true", help="skip the three-orbital step line")
     ap.add_argument("--no-rqmc", action="store_true", help="skip the randomized-qMC and differential lines")
     ap.add_argument("--block-models-only", action="store_true",
-                    help="only the two- and three-orbital steps (vector and matrix-core walks), one JSON line")
+                    help="only the two- and three-orbital steps, one JSON line")
     ap.add_argument("--c1-only", action="store_true",
-                    help="only the single-orbital solve (flat scalar walk), no CPU leg (profiling runs)")
+                    help="only the single-orbital solve, no CPU leg (profiling runs)")
     ap.add_argument("--c3-only", type=int, default=0, metavar="LOG2N",
-                    help="only the three-orbital bold step (matrix-core walk) at N=2^LOG2N, no CPU leg "
+                    help="only the three-orbital bold step at N=2^LOG2N, no CPU leg "
                          "(profiling runs)")
     ap.add_argument("--warp-study", action="store_true",
                     help="only run the learned-warp error-versus-samples study and print its JSON line")
