@@ -1484,7 +1484,8 @@ double trie_seconds(const HostModel &m, const Batch &b, bool least, int64_t N, i
     double longest = 0, t = 0;
     const bool vec = m.mmax <= 6;
     for (const Compiled &cg : b.groups) {
-        const double words = least ? 4.5 * cg.leaves_per_sample : (double)cg.prog.size();
+        const Compiled &own = cg.replica_of >= 0 ? b.groups[cg.replica_of] : cg;  // (sequences share a program)
+        const double words = least ? 4.5 * cg.leaves_per_sample : (double)own.prog.size();
         longest = std::max(longest, words);
         t += (double)rows * group_samples(cg.g, N) * (vec ? words * m.mmax * 2e-11 : sample_flops(cg) / 1.3e12);
     }

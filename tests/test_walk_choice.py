@@ -50,3 +50,15 @@ def test_walk_of_the_other_calls(stub, order, log2n, kernel):  # noqa: F811
     stub.clear()
     qiw.diff_inchworm(e, e.grid, orders, 2 ** log2n, ctx=stub.ctx)
     assert all(ARC in x.name for x in stub.launches("k_eval"))  # (order 1 is one sample)
+
+
+@pytest.mark.parametrize("log2n,kernel", [(13, ARC), (18, VEC)])
+def test_walk_of_randomized_steps(stub, log2n, kernel):  # noqa: F811
+    """Every sequence of a group counts: blocks of up to six at order 2 stay on the arc walk, of three
+    do not."""
+    for make, walk in ((two_orbital, ARC), (blocks_of_three, kernel)):
+        stub.clear()
+        qiw.inchworm_step(make(), 3, range(0, 3), 2 ** (log2n - 4), ctx=stub.ctx,
+                          rand_params=qiw.RandomizationParams(5, 16 if make is two_orbital or kernel == VEC else 2, 0.0))
+        names = [x.name for x in stub.launches("k_eval")]
+        assert names and all(walk in n for n in names)
