@@ -65,11 +65,10 @@ enum {
     QIW_PREC_FP64 = 0,       /* all arithmetic in float64                                */
     QIW_PREC_FP32 = 1        /* block chain products in float32 (blocks up to 6, or up to 32
                                 with at most two hybridization functions, orders up to 4;
-                                float64 otherwise); Sobol-to-simplex map, hybridization
-                                functions, sums over diagrams and samples (the latter
-                                compensated) and P bookkeeping in float64.  A sum over
-                                partial diagrams is rounded to float32 only where it enters
-                                a block product.                                         */
+                                float64 otherwise); Sobol-to-simplex map, sums over
+                                diagrams and samples (the latter compensated) and P
+                                bookkeeping in float64.  A sum over partial diagrams is
+                                rounded to float32 only where it enters a block product. */
 };
 
 /* One block-sparse operator, the reference's SectorBlockMatrix
