@@ -1464,7 +1464,8 @@ std::vector<std::pair<int32_t, int32_t>> task_parts(const Batch &b, const Compil
 //   0:3, N = 2^12 1.75 9.6;
 //   128 blocks of 4, order 1, N = 2^9 1.58 5.25, 2^12 10.4 5.15, 2^15 76.8 6.34;
 //   blocks up to 10 in float64, order 1, N = 2^15 7.37 2.80; orders 0:2, N = 2^12 6.14 12.4.
-// The rates are fits to these that stay within a factor of two.
+// The rates are fits to these and to 110 further sizes: the walk chosen is the faster one or within a
+// fifth of it, but for launches below 0.5 ms.
 int64_t group_samples(const QiwGroup &g, int64_t N) {
     return g.order == 0 || (g.kind == QIW_G_SIGMA && g.order == 1) ? 1 : std::max<int64_t>(N, 1);
 }
@@ -1490,7 +1491,7 @@ double trie_seconds(const HostModel &m, const Batch &b, bool least, int64_t N, i
         t += (double)rows * group_samples(cg.g, N) * (vec ? words * m.mmax * 2e-11 : sample_flops(cg) / 1.3e12);
     }
     const bool fp32 = b.precision == QIW_PREC_FP32;
-    return vec ? 1e-4 + std::max(longest * m.mmax * (fp32 ? 4.8e-7 : 8e-7), t * (fp32 ? 0.5 : 1.0))
+    return vec ? 1e-4 + std::max(longest * (m.mmax * 8e-7 + m.bt * 1e-9) * (fp32 ? 0.6 : 1.0), t * (fp32 ? 0.5 : 1.0))
                : 5e-5 + std::max(longest * m.mmax * 1e-7, t);
 }
 // Whether the batch `arcs` would be faster on the walks of the tries (tries: builds the batch there).
@@ -1498,7 +1499,7 @@ template <class Build>
 int prefer_tries(const HostModel &m, Batch &arcs, int64_t N, int64_t rows, Build build) {
     if (arcs.fmt != FMT_ARC || (m.mmax > 6 && arcs.precision == QIW_PREC_FP32)) return 0;
     if (program_format(m, arcs.max_order, arcs.precision) == FMT_BLOCK && m.mmax <= 6) return 0;
-    const double t = 0.8 * arc_seconds(m, arcs, N, rows);
+    const double t = arc_seconds(m, arcs, N, rows);
     if (trie_seconds(m, arcs, true, N, rows) >= t) return 0;
     Batch tries;
     const int rc = build(tries);
